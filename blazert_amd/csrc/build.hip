@@ -770,11 +770,15 @@ __global__ void k_node64(const brt_tree_node *__restrict__ T, uint32_t M, const 
 }
 
 __global__ void k_node4(const brt_tree_node *__restrict__ T, const uint32_t *__restrict__ is_root, uint32_t M,
-                        const uint32_t *__restrict__ k4, Node4 *__restrict__ out) {
+                        const uint32_t *__restrict__ k4, Node4 *__restrict__ out, uint32_t *__restrict__ ord4) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= M || !is_root[i]) return;
-  uint32_t slot[4];
-  const int m = collapse4(T, i, slot);
+  uint32_t slot[4], axis[16] = {};
+  const int m = collapse4(T, i, slot, axis);
+  uint32_t ord[2];
+  visit_order4(axis, m, ord);
+  ord4[2ull * k4[i]] = ord[0];
+  ord4[2ull * k4[i] + 1] = ord[1];
   Node4 nd;
   for (int c = 0; c < 4; c++) {
     for (int k = 0; k < 3; k++) {
@@ -1121,6 +1125,7 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
   const uint32_t n4 = out.root.leaf ? 0u : 1u + last[2] + last[3];
   Node64 *nodes64 = A.get<Node64>(n64);
   Node4 *nodes4 = A.get<Node4>(n4);
+  uint32_t *ord4 = A.get<uint32_t>(2ull * n4);
   size_t rec_size = 0;
   switch (in.type) {
   case TRIANGLES: rec_size = sizeof(TriRec); break;
@@ -1132,7 +1137,7 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
   BRT_CHECK(A.err);
   BRT_LAUNCH(k_assign4<<<blocks_for(M, 256), 256, 0, st>>>(tree, is_root, M, S, k4));
   BRT_LAUNCH(k_node64<<<blocks_for(M, 256), 256, 0, st>>>(tree, M, ni, nodes64));
-  BRT_LAUNCH(k_node4<<<blocks_for(M, 256), 256, 0, st>>>(tree, is_root, M, k4, nodes4));
+  BRT_LAUNCH(k_node4<<<blocks_for(M, 256), 256, 0, st>>>(tree, is_root, M, k4, nodes4, ord4));
   const uint32_t g = blocks_for(n, 256);
   switch (in.type) {
   case TRIANGLES:
@@ -1174,6 +1179,7 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
   out.num_n64 = n64;
   out.n4 = nodes4;
   out.num_n4 = n4;
+  out.ord4 = ord4;
   out.recs = recs;
   out.rec_size = rec_size;
   out.max_depth = std::max(hs.max_depth, ds.max_depth);
@@ -1182,7 +1188,8 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
   out.bad_splits = hs.bad + ds.bad;
   out.max_prims = std::max(hs.max_prims, ds.max_prims);
   out.min_prims = std::min(hs.min_prims, ds.min_prims);
-  for (void *p : {(void *)tree, (void *)idx, (void *)nodes64, (void *)nodes4, (void *)recs}) A.release(p);
+  for (void *p : {(void *)tree, (void *)idx, (void *)nodes64, (void *)nodes4, (void *)ord4, (void *)recs})
+    A.release(p);
   return hipSuccess;
 }
 

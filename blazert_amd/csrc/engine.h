@@ -12,10 +12,13 @@ namespace brt {
 // ones) by its two children in place, so the slots stay in the binary tree's left-to-right order. The internal slots
 // are the roots of further records. Shared by the host flatten and the device build, which give identical records.
 // A record advances a root-to-leaf path by at least one binary level and pushes at most three stack entries.
-__host__ __device__ inline int collapse4(const brt_tree_node *T, uint32_t b, uint32_t slot[4]) {
+// With `axis` the split axis of every slot pair's lowest common ancestor is reported too: axis[4 * i + j], i < j.
+__host__ __device__ inline int collapse4(const brt_tree_node *T, uint32_t b, uint32_t slot[4],
+                                         uint32_t *axis = nullptr) {
 #pragma clang fp contract(off)
   slot[0] = T[b].children[0];
   slot[1] = T[b].children[1];
+  if (axis) axis[1] = T[b].axis;
   int m = 2;
   while (m < 4) {
     int best = -1;
@@ -35,9 +38,32 @@ __host__ __device__ inline int collapse4(const brt_tree_node *T, uint32_t b, uin
     for (int c = m; c > best + 1; c--) slot[c] = slot[c - 1];
     slot[best] = T[e].children[0];
     slot[best + 1] = T[e].children[1];
+    if (axis) {
+      uint32_t old[16];
+      for (int i = 0; i < 16; i++) old[i] = axis[i];
+      const auto from = [&](int c) { return c > best ? c - 1 : c; };  // slot c's place before the split
+      for (int i = 0; i <= m; i++)
+        for (int j = i + 1; j <= m; j++)
+          axis[4 * i + j] = (i == best && j == best + 1) ? T[e].axis : old[4 * from(i) + from(j)];
+    }
     m++;
   }
   return m;
+}
+
+// The visiting order of a record's m slots (NodeQ::ord) from the split axes collapse4 reports: of two slots the left
+// one comes first when the direction is not negative along the axis that parts them (blazert/bvh/accel.h:95-104).
+__host__ __device__ inline void visit_order4(const uint32_t axis[16], int m, uint32_t ord[2]) {
+  ord[0] = ord[1] = 0;
+  for (uint32_t oct = 0; oct < 4; oct++) {
+    uint32_t later = 0;
+    for (int i = 0; i < m; i++)
+      for (int j = i + 1; j < m; j++) {
+        const bool right_first = (oct >> axis[4 * i + j]) & 1u;
+        later |= right_first ? 1u << (4 * j + i) : 1u << (4 * i + j);
+      }
+    ord[oct >> 1] |= later << (16 * (oct & 1u));
+  }
 }
 
 // Device counters of one traversal launch, in a group cleared by the launch itself: the persistent schedule's ray
@@ -50,7 +76,13 @@ constexpr int COUNTER_DEFERRED = 1;
 constexpr int COUNTER_DEFERRED_POOL = 2;
 constexpr int CLAIM_COUNTERS = 8;
 constexpr int COUNTER_STRIDE = 16;
-constexpr int COUNTER_GROUP = CLAIM_COUNTERS * COUNTER_STRIDE;  // slots per group (1 KiB)
+constexpr int COUNTER_CLEARED = CLAIM_COUNTERS * COUNTER_STRIDE;  // slots a launch clears (1 KiB)
+// Rays whose fast triangle traversal could not be certified (k_trace_tri) are listed behind the counters, for the
+// exact launch that follows: COUNTER_LISTED counts them, and when there are more than LIST_CAPACITY that launch traces
+// every ray.
+constexpr int COUNTER_LISTED = 3;
+constexpr int LIST_CAPACITY = 3968;
+constexpr int COUNTER_GROUP = COUNTER_CLEARED + LIST_CAPACITY;  // slots per group (32 KiB)
 
 constexpr uint32_t SCHEDULE_PERSISTENT = 0;  // persistent waves with per-lane ray refill (default)
 constexpr uint32_t SCHEDULE_PER_THREAD = 1;  // one ray per thread, grid-stride
@@ -66,6 +98,7 @@ struct TraceLaunch {
   const uint32_t *order;        // optional ray permutation (sorted launches); kernels trace rays[order[k]]
   uint32_t ring = 0;            // LDS stack slots per lane: 4, 8 or 16 (0 = default of the precision)
   uint32_t pool = 0;            // persistent: ray indices per claim, 32, 64 or 128 (0 = 64)
+  bool fast = false;            // batches: every job's triangle tree has reference-order nodes (BvhView::nodesq)
   bool overwrite = false;       // every hit replaces the record (traverse semantics), not only closer ones
 };
 
@@ -102,10 +135,10 @@ hipError_t sort_workspace_reserve(SortWorkspace &ws, uint64_t n);
 hipError_t sort_workspace_in(SortWorkspace &ws, void *base, size_t bytes, uint64_t n);
 
 // Device scratch of the allocation-free intersect (brt_intersect_noalloc): a file-scope __device__ array, one copy
-// per GPU, holding a launch counter group in its first 256 bytes and then the workspace of a ray sort of up to
+// per GPU, holding a launch counter group at its start and then the workspace of a ray sort of up to
 // NOALLOC_MAX_SORTED_RAYS rays.
 constexpr uint64_t NOALLOC_MAX_SORTED_RAYS = 1ull << 20;
-constexpr size_t NOALLOC_SCRATCH_BYTES = 24ull << 20;
+constexpr size_t NOALLOC_SCRATCH_BYTES = (24ull << 20) + COUNTER_GROUP * 8;
 // This device's address of the scratch array (looked up once per device with hipGetSymbolAddress).
 hipError_t noalloc_scratch(unsigned char **ptr);
 // Computes the sort keys (mode 1: direction octant + origin Morton code, mode 2: Morton only) and radix-sorts the
@@ -124,6 +157,10 @@ hipError_t launch_tri_filter_records(const void *recs, uint32_t n, void *out, hi
 hipError_t launch_sph_filter_records(const void *recs, uint32_t n, void *out, hipStream_t stream);
 // Split precision: writes the bounding-sphere pre-test records (SphFilt, n + SPH_FILTER_PAD) of n leaf-order CylRecs.
 hipError_t launch_cyl_filter_records(const void *recs, uint32_t n, void *out, hipStream_t stream);
+
+// Triangles: assembles the reference-order nodes (NodeQ) from n Node4 records and their visiting orders (two words per
+// record, visit_order4).
+hipError_t launch_nodeq_records(const Node4 *nodes4, const uint32_t *ord, uint32_t n, NodeQ *out, hipStream_t stream);
 
 // Enqueues the traversal of one geometry type over n rays on `stream` (asynchronous).
 hipError_t launch_trace(GeomType type, const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint64_t n,
@@ -198,6 +235,7 @@ struct DeviceBuildOut {
   uint32_t num_n64;
   Node4 *n4;
   uint32_t num_n4;
+  uint32_t *ord4;       // visiting order of every Node4's slots, two words each (visit_order4)
   void *recs;           // primitive records in leaf order
   size_t rec_size;
   brt_tree_node root;   // host copy of node 0

@@ -165,23 +165,21 @@ __device__ __forceinline__ bool slab32(const float *b, const Ray32 &q, float &ke
 //   det:    5.1 u sa sb                      (n rounded once from the FP64 test's own n)
 //   t:      6.1 u sa sb Pm
 //   w = |det| - u - v: the sum of those plus 2 u (|det| + |u| + |v|) <= 0.2 Ed + 0.18 (Eu + Ev)
-// The bounds used (Eu = kub Pm, Ev = kua Pm, Ed = ed, Et = 1.2 ed Pm, Ew = 1.3 ed + 1.2 (kua + kub) Pm) keep a
-// margin for the rounding of the bounds themselves; ed and Et hold an absolute 1e-29, Eu, Ev and Ew the reference's
-// tolerance, for results in the FP32 denormal range. The reference accepts u, v, w >= -4 DBL_EPSILON (tol), t >= |det| tmin and |det| h > t with the signs
+// The bounds used (Ed = ed, Et = 1.2 ed Pm, and for u, v and w alike E = kw Pm + cw, with kw = 1.2 * 16 u (sa + sb) and
+// cw = 1.3 ed + tol) keep a margin for the rounding of the bounds themselves; ed and Et hold an absolute 1e-29, E the
+// reference's tolerance, for results in the FP32 denormal range. The reference accepts u, v, w >= -4 DBL_EPSILON (tol), t >= |det| tmin and |det| h > t with the signs
 // taken from det; where the sign of det is not certain (|det| <= Ed) the triangle passes. Scenes and ray origins
 // above FILTER_MAX_EXTENT are not pre-tested, so no value here overflows; every rejection is a comparison that is
 // false for NaN operands.
 __device__ __forceinline__ bool tri_filter(const TriFilt &T, const float D[3], const float O[3], float om,
                                            float tmin32, float h32) {
   const float u = 5.9604644775390625e-08f;
-  const float tol = 9e-16f;  // 4 DBL_EPSILON rounded up
   // fused multiply-adds round once where a product and a sum round twice, so the bounds below hold for them too
   auto dot3 = [](float a0, float a1, float a2, float b0, float b1, float b2) {
     return __builtin_fmaf(a0, b0, __builtin_fmaf(a1, b1, a2 * b2));
   };
   const float det = dot3(T.n[0], T.n[1], T.n[2], D[0], D[1], D[2]);
   const float ad = fabsf(det);
-  if (!(ad > T.ed)) return true;  // the sign of det is not certain
   const float c0 = T.v0[0] - O[0], c1 = T.v0[1] - O[1], c2 = T.v0[2] - O[2];
   const float rx = __builtin_fmaf(D[1], c2, -(D[2] * c1));
   const float ry = __builtin_fmaf(D[2], c0, -(D[0] * c2));
@@ -190,19 +188,16 @@ __device__ __forceinline__ bool tri_filter(const TriFilt &T, const float D[3], c
   const float *a = T.e1, *b = T.e2;
   const float us = product_sign(dot3(rx, ry, rz, b[0], b[1], b[2]), det);
   const float vs = product_sign(dot3(rx, ry, rz, a[0], a[1], a[2]), det);
-  if (us < -__builtin_fmaf(T.kub, Pm, tol) || vs < -__builtin_fmaf(T.kua, Pm, tol)) return false;
-  const float Ew = __builtin_fmaf(1.2f * (T.kua + T.kub), Pm, __builtin_fmaf(1.3f, T.ed, tol));
-  if ((ad - us) - vs < -Ew) return false;
+  const float E = __builtin_fmaf(T.kw, Pm, T.cw);
   const float ts = product_sign(dot3(T.n[0], T.n[1], T.n[2], c0, c1, c2), det);
   const float Et = __builtin_fmaf(1.2f * T.ed, Pm, 1e-29f);
-  // t >= |det| tmin: a lower bound of the right side (tmin32 <= tmin; no bound for negative tmin)
-  if (tmin32 >= 0.0f) {
-    const float L = tmin32 > 0.0f ? ((ad - T.ed) * tmin32) * (1.0f - 4.0f * u) : 0.0f;
-    if (ts + Et < L) return false;
-  }
+  // t >= |det| tmin: a lower bound of the right side (tmin32 <= tmin; none for negative tmin)
+  const float L = (ad - T.ed) * (tmin32 >= 0.0f ? tmin32 * (1.0f - 4.0f * u) : -__builtin_inff());
   // |det| h > t: an upper bound of the left side (h32 >= h)
-  if (ts - Et >= ((ad + T.ed) * h32) * (1.0f + 4.0f * u)) return false;
-  return true;
+  const float H = (ad + T.ed) * (h32 * (1.0f + 4.0f * u));
+  // without branches: lanes of a wave rarely agree on one, and the tests of a group overlap
+  const bool out = (fminf(fminf(us, vs), (ad - us) - vs) < -E) | (ts + Et < L) | (ts - Et >= H);
+  return !(ad > T.ed) | !out;  // where the sign of det is not certain the triangle passes
 }
 
 // Conservative FP32 pre-test of one sphere for the split path: returns false only when the FP64 test isect_sph
@@ -262,10 +257,10 @@ using Hit = HitT<double>;
 // Every intersector runs in the scene type of its record (Rec::real): the same operation sequence for double and
 // float, with the reference's constants of that type.
 
-// blazert/primitives/trimesh.h:153-181
-template <class Rec>
+// blazert/primitives/trimesh.h:153-181. accepted(u, v, w, t, |det|, |det| h) is called on a hit, before s is updated.
+template <class Rec, class F>
 __device__ __forceinline__ bool isect_tri(const Rec &T, const RayT<typename Rec::real> &r,
-                                          HitT<typename Rec::real> &s, uint32_t idx) {
+                                          HitT<typename Rec::real> &s, uint32_t idx, F accepted) {
   using R = typename Rec::real;
   const R tol = R(4) * Real<R>::eps;
   const R c0 = T.v0[0] - r.o[0], c1 = T.v0[1] - r.o[1], c2 = T.v0[2] - r.o[2];
@@ -293,6 +288,7 @@ __device__ __forceinline__ bool isect_tri(const Rec &T, const RayT<typename Rec:
   if (u >= -tol && v >= -tol && w >= -tol) {
     const R t = product_sign(nx * c0 + ny * c1 + nz * c2, det);
     if (t >= abs_det * r.tmin && abs_det * s.h > t) {
+      accepted(u, v, w, t, abs_det, abs_det * s.h);
       const R inv_det = R(1) / abs_det;
       s.h = t * inv_det;
       s.u = u * inv_det;
@@ -303,6 +299,13 @@ __device__ __forceinline__ bool isect_tri(const Rec &T, const RayT<typename Rec:
     }
   }
   return false;
+}
+
+template <class Rec>
+__device__ __forceinline__ bool isect_tri(const Rec &T, const RayT<typename Rec::real> &r,
+                                          HitT<typename Rec::real> &s, uint32_t idx) {
+  using R = typename Rec::real;
+  return isect_tri(T, r, s, idx, [](R, R, R, R, R, R) {});
 }
 
 template <class R>
@@ -1058,6 +1061,40 @@ __device__ __forceinline__ void start_ray(const BvhView &bvh, const RaysViewT<R>
   s.leaf_idx = INVALID_ID;
 }
 
+// Rays whose reference traversal the FP32 bounds enclose: no slab term can be NaN or leave the FP32 range, tmin >= 0
+// and a direction of unit length (its slab distances are then the hit distances; a longer one only makes the reference
+// skip less, except through tmin).
+__device__ __forceinline__ bool fast_ray(const Ray &r, double len2, double S) {
+  bool ok = (r.sign & RAY_NAN_FREE) && r.tmin >= 0.0 && len2 >= 1.0 - 0x1p-20 && len2 <= 1e20 &&
+            (len2 <= 1.0 + 0x1p-20 || r.tmin == 0.0);
+#pragma unroll
+  for (int k = 0; k < 3; k++) ok = ok && fabs(r.inv[k]) * (S + fabs(r.o[k])) <= 1e36 && fabs(r.inv[k]) <= 1e30;
+  return ok && fabs(r.o[0]) <= FILTER_MAX_EXTENT && fabs(r.o[1]) <= FILTER_MAX_EXTENT &&
+         fabs(r.o[2]) <= FILTER_MAX_EXTENT;
+}
+
+// A ray's columns as they stand in memory.
+struct RawRay {
+  double org[3], dir[3], tmin, tmax;
+};
+__device__ __forceinline__ RawRay load_ray(const RaysView &V, uint64_t i) {
+  return RawRay{{ld_stream(V.ox, i), ld_stream(V.oy, i), ld_stream(V.oz, i)},
+                {ld_stream(V.dx, i), ld_stream(V.dy, i), ld_stream(V.dz, i)},
+                V.tmin ? ld_stream(V.tmin, i) : V.tmin0,
+                V.tmax ? ld_stream(V.tmax, i) : V.tmax0};
+}
+__device__ __forceinline__ double squared_length(const RawRay &w) {
+  return w.dir[0] * w.dir[0] + w.dir[1] * w.dir[1] + w.dir[2] * w.dir[2];
+}
+
+// The same predicate from the ray's columns.
+__device__ __forceinline__ bool fast_ray(const RaysView &V, uint64_t i, double S) {
+  const RawRay w = load_ray(V, i);
+  Ray r;
+  setup_ray(w.org, w.dir, w.tmin, w.tmax, r);
+  return fast_ray(r, squared_length(w), S);
+}
+
 // One ray per thread (grid-stride).
 template <class Rec, bool SPLIT>
 __global__ void __launch_bounds__(256) k_trace(BvhView bvh, RaysViewT<typename Rec::real> rays,
@@ -1185,7 +1222,21 @@ __device__ __forceinline__ T lds_fresh(const uint64_t *src) {
   return out;
 }
 
-template <class Rec, bool SPLIT>
+// What the exact launch behind k_trace_tri has to trace: positions [0, scan) (of the rays k_trace_tri passed over, or
+// of all rays when more were listed than the list holds) and then `listed` entries of the list.
+struct Leftover {
+  uint64_t scan, listed;
+  bool all;
+};
+__device__ __forceinline__ Leftover leftover(const unsigned long long *group, uint64_t n) {
+  const uint64_t listed = __atomic_load_n(group + COUNTER_LISTED, __ATOMIC_RELAXED);
+  const bool all = listed > (uint64_t)LIST_CAPACITY;
+  const bool passed = __atomic_load_n(group + COUNTER_DEFERRED, __ATOMIC_RELAXED) != 0ull;
+  return Leftover{all || passed ? n : 0ull, all ? 0ull : listed, all};
+}
+
+// AFTER_FAST: the launch behind k_trace_tri (see leftover).
+template <class Rec, bool SPLIT, bool AFTER_FAST = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BRT_WAVES_PER_EU)))
 k_trace_persistent(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<typename Rec::real> hits, uint64_t n,
                    uint32_t flags, uint32_t first, uint32_t is_tri, double S, unsigned long long *counter,
@@ -1194,8 +1245,14 @@ k_trace_persistent(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<ty
   using R = typename Rec::real;
   extern __shared__ unsigned char smem[];
   const bool any_hit = (flags & FLAG_ANY_HIT) != 0;
-  const bool deferred_only = !SPLIT && (flags & FLAG_DEFERRED_ONLY);
+  const bool deferred_only = !SPLIT && !AFTER_FAST && (flags & FLAG_DEFERRED_ONLY);
   if (deferred_only && __atomic_load_n(deferred, __ATOMIC_RELAXED) == 0ull) return;
+  Leftover left{};
+  if constexpr (AFTER_FAST) {
+    left = leftover(deferred - COUNTER_DEFERRED, n);
+    n = left.scan + left.listed;
+    if (n == 0) return;
+  }
   constexpr bool LDS_VIEWS = Rec::kind == TRIANGLES;
   constexpr int RW = (int)(sizeof(RaysViewT<R>) / 8), HW = (int)(sizeof(HitsViewT<R>) / 8);
   __shared__ uint64_t views[RW + HW];
@@ -1236,11 +1293,18 @@ k_trace_persistent(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<ty
         uint64_t cand = 0;
         pool_refill(pool, counter, n, chunk, idle, nidle, lane, got, cand, exhausted);
         if (got) {
-          idx = order ? (uint64_t)order[cand] : cand;
-          start_ray<SPLIT>(bvh, rays_view(), idx, S, r, q, s);
+          bool trace = true;
+          if (AFTER_FAST && cand >= left.scan) {
+            idx = deferred[COUNTER_CLEARED - COUNTER_DEFERRED + (cand - left.scan)];
+            start_ray<SPLIT>(bvh, rays_view(), idx, S, r, q, s);
+          } else {
+            idx = order ? (uint64_t)order[cand] : cand;
+            start_ray<SPLIT>(bvh, rays_view(), idx, S, r, q, s);
+            if constexpr (AFTER_FAST) trace = left.all || !fast_ray(rays_view(), idx, S);
+          }
           if (SPLIT && deferred_to_exact(r)) {
             __atomic_store_n(deferred, 1ull, __ATOMIC_RELAXED);
-          } else if (!deferred_only || deferred_to_exact(r)) {
+          } else if (trace && (!deferred_only || deferred_to_exact(r))) {
             has_ray = true;
             trav_begin<SPLIT>(bvh, r, q, s, t);
             st.reset();
@@ -1277,15 +1341,21 @@ __device__ __forceinline__ uint32_t find_job(const BatchJob *jobs, uint32_t njob
   return lo;
 }
 
-template <class Rec, bool SPLIT>
+template <class Rec, bool SPLIT, bool AFTER_FAST = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BRT_WAVES_PER_EU)))
 k_trace_batch(const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t total, uint32_t flags,
               unsigned long long *counter, uint32_t refill, uint32_t ring, unsigned long long *deferred,
               uint32_t chunk) {
   extern __shared__ unsigned char smem[];
   const bool any_hit = (flags & FLAG_ANY_HIT) != 0;
-  const bool deferred_only = !SPLIT && (flags & FLAG_DEFERRED_ONLY);
+  const bool deferred_only = !SPLIT && !AFTER_FAST && (flags & FLAG_DEFERRED_ONLY);
   if (deferred_only && __atomic_load_n(deferred, __ATOMIC_RELAXED) == 0ull) return;
+  Leftover left{};
+  if constexpr (AFTER_FAST) {
+    left = leftover(deferred - COUNTER_DEFERRED, total);
+    total = left.scan + left.listed;
+    if (total == 0) return;
+  }
   // Finishing a ray needs its job's hit columns and flags: for batches of up to BATCH_LDS_JOBS jobs every block
   // keeps them in LDS, so that a finish does not wait on a load from the job table.
   constexpr int JW = (int)(sizeof(HitsView) / 8) + 1;  // hit column pointers, then first | is_tri << 32
@@ -1323,6 +1393,11 @@ k_trace_batch(const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t total,
         pool_refill(pool, counter, total, chunk, idle, nidle, lane, got, g, exhausted);
         // A claim is a run of consecutive indices and usually lies in one job: find the jobs of its first and last
         // index once per wave (wave-uniform, so scalar loads), and search per lane only when they differ.
+        bool from_list = false;
+        if constexpr (AFTER_FAST) {
+          from_list = got && g >= left.scan;
+          if (from_list) g = deferred[COUNTER_CLEARED - COUNTER_DEFERRED + (g - left.scan)];
+        }
         const unsigned long long gm = __ballot(got);
         if (gm) {
           const int lo = __ffsll((long long)gm) - 1, hi = 63 - __clzll((long long)gm);
@@ -1331,7 +1406,8 @@ k_trace_batch(const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t total,
           const uint64_t g_hi = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(g >> 32), hi) << 32) |
                                 (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)g, hi);
           const uint32_t j_lo = find_job(jobs, njobs, g_lo);
-          const bool one_job = j_lo + 1u >= njobs || jobs[j_lo + 1u].offset > g_hi;
+          // (indices from the list are in no order)
+          const bool one_job = !AFTER_FAST && (j_lo + 1u >= njobs || jobs[j_lo + 1u].offset > g_hi);
           if (got) {
             j = one_job ? j_lo : find_job(jobs, njobs, g);
             const BatchJob &J = jobs[j];
@@ -1339,9 +1415,11 @@ k_trace_batch(const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t total,
             idx = J.order ? (uint64_t)J.order[local] : local;
             bv = J.bvh;
             start_ray<SPLIT>(bv, J.rays, idx, J.extent, r, q, s);
+            bool trace = true;
+            if constexpr (AFTER_FAST) trace = from_list || left.all || !fast_ray(J.rays, idx, J.extent);
             if (SPLIT && deferred_to_exact(r)) {
               __atomic_store_n(deferred, 1ull, __ATOMIC_RELAXED);
-            } else if (!deferred_only || deferred_to_exact(r)) {
+            } else if (trace && (!deferred_only || deferred_to_exact(r))) {
               has_ray = true;
               trav_begin<SPLIT>(bv, r, q, s, t);
               st.reset();
@@ -1374,6 +1452,653 @@ k_trace_batch(const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t total,
   }
 }
 
+// ------------------------------------------------------------------------------------------------ triangles, fast
+// Closest hits of a triangle tree, bit-identical to the exact FP64 kernels (k_trace_persistent<TriRec, false>), at
+// the cost of FP32 boxes and pre-tests.
+//
+// The reference's depth-first order is kept (NodeQ::ord), with the reference's own hit distance at every point of it.
+// A box is skipped only when the FP32 bounds prove that the reference's slab test or its pop test skips it (Ray32
+// below), a triangle only when tri_filter proves that the FP64 test rejects it, and every other triangle gets the FP64
+// test itself, in leaf order. So the primitives tested are the reference's, in its order, plus some of boxes that its
+// FP64 slab test rejects by a rounding. Those change nothing unless one is accepted. Every accepted hit is therefore
+// checked (certified): one that lies inside its triangle by more than the rounding of the test, and clear of the earlier
+// hit distance and of tmin by more than the error of its own distance, lies inside every box above it by more than the
+// rounding of the slab test (whose far planes are widened by 4 eps), so the reference tests it too, with the same hit
+// distance, and accepts it. A ray with a hit that fails the check writes nothing and is listed for the exact kernel that
+// follows on the stream. Rays outside the assumptions of the argument (fast_ray) go there as well.
+//
+// What bounds it (4,194,304 incoherent rays, 1.31M triangles): the data path of the vector L1 (87% busy: every step reads a
+// 128-byte record per lane in eight loads) and the vector ALU (73%, a quarter of the lanes active), with 5.7 TB/s of
+// lines beyond L2. Near and far rows are therefore chosen by address instead of by selects, references carry no second
+// word, the pre-test has no branches and finished rays are written together.
+//
+// Once a wave's pool is exhausted, its idle lanes take over stack entries of the busy ones: always the bottom entry,
+// the last subtree in the lane's part of the order, with the lane's hit distance as it stands. That distance is at
+// least the one the reference would have there, so the helper tests a superset of the reference's primitives; an
+// accepted hit is certified as before, and one nearer than the hit of the parts before it would have been accepted in
+// the reference's order too. A part also skips what lies behind a hit of a part before it (never of one after it). The
+// parts' hits are merged by distance when the last of them ends, and a ray whose parts have two hits within their error
+// bounds of each other is listed. Sharing takes the incoherent set from 3.57 to 3.16 ms and 50,000 rays on 328k triangles
+// from 450 to 268 us; the camera set, whose rays mostly end at their first hit, loses 4%.
+struct RayQ {
+  float inv[3];
+  float offn[3], offf[3];  // entry / exit plane offsets, rounded apart (make_ray32)
+  float D[3], O[3];        // unit direction and origin, for the pre-test
+  float om, tmin;
+  float slack;             // >= 1 - |raw direction|
+  // bits 0-4: shift of the octant's order mask, bit 5: its word, bits 6-8: direction signs, bit 9: mask complemented
+  uint32_t code;
+};
+
+__device__ __forceinline__ void make_rayq(const Ray &r, double len2, double S, RayQ &q) {
+  Ray32 a;
+  make_ray32(r, S, a);
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    q.inv[k] = a.inv[k];
+    q.offn[k] = a.offn[k];
+    q.offf[k] = a.offf[k];
+    q.D[k] = (float)r.d[k];
+    q.O[k] = (float)r.o[k];
+  }
+  q.om = a.om;
+  q.tmin = fmaxf(a.tmin, 0.0f);
+  q.slack = len2 < 1.0 ? f32_up(1.0 - len2) : 0.0f;
+  const uint32_t s = r.sign & 7u, c = (s & 4u) ? (~s & 3u) : s;
+  q.code = ((c & 1u) << 4) | ((c >> 1) << 5) | (s << 6) | ((s >> 2) << 9);
+}
+
+// Whether an accepted hit is one that the reference's traversal must reach as well (see above). `thr` is |det| times
+// the hit distance before it, `slack` what the ray's direction falls short of unit length. The FP64 test's errors are
+// those of tri_filter's table with u = 2^-53; 32 u covers them and the rounding of the record's edges and of the
+// normalised direction. The distance h = t / |det| is then known to err / |det|, err = 4 (Et + Ed h), twice over; `rel` is
+// that relative to h.
+struct Certificate {
+  bool sure;
+  float rel;
+};
+__device__ __forceinline__ Certificate certified(const TriRec &T, const double o[3], double tmin, double slack, double u,
+                                                 double v, double w, double t, double ad, double thr) {
+  const double sa = fabs(T.e1[0]) + fabs(T.e1[1]) + fabs(T.e1[2]);
+  const double sb = fabs(T.e2[0]) + fabs(T.e2[1]) + fabs(T.e2[2]);
+  const double Pm = fmax(fabs(T.v0[0]), fmax(fabs(T.v0[1]), fabs(T.v0[2]))) +
+                    fmax(fabs(o[0]), fmax(fabs(o[1]), fabs(o[2])));
+  const double k = 32.0 * 0x1p-53;
+  const double Ed = k * sa * sb + 1e-290, Eu = k * Pm * sb + 1e-290, Ev = k * Pm * sa + 1e-290, Et = Ed * Pm + 1e-290;
+  const double err = 4.0 * (Et + Ed * (t * (1.0 / ad)));
+  Certificate c;
+  c.sure = u > Eu && v > Ev && w > Eu + Ev + Ed && ad >= 0x1p12 * Ed && t >= 0x1p12 * Et &&
+           t - err >= ad * tmin * (1.0 + 0x1p-46) && t + err < thr * (1.0 - (0x1p-46 + slack));
+  c.rel = (float)(err * (1.0 / t)) * (1.0f + 0x1p-20f);
+  return c;
+}
+
+__device__ __forceinline__ float max3_nn(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+__device__ __forceinline__ float min3_nn(float a, float b, float c) {
+  float r;
+  asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+// One entry: a node or leaf reference, and its entry distance with the low 8 bits (rounded towards 0; keys are not
+// negative) replaced by the leaf's primitive count.
+struct TriEntry {
+  uint32_t ref, key;
+};
+constexpr uint32_t TRI_SPILL = 192;  // three entries per level, at most 63 levels (stack_cap)
+
+// The lane's stack: entries [bot, sp), of which [lo, sp) lie in the LDS ring and the older ones in private memory.
+// Entries below bot have been given away.
+struct TriStack {
+  BRT_LDS uint32_t *ring;  // the lane's slot 0; slot i: reference at [128 i], key at [128 i + 64]
+  uint64_t *spill;
+  int sp, lo, bot;
+  int mask;  // ring slots - 1
+
+  __device__ __forceinline__ void reset() { sp = lo = bot = 0; }
+  __device__ __forceinline__ void room(int n) {  // n more entries fit the ring
+    while (sp + n - lo > mask + 1) {
+      spill[lo] = slot(lo);
+      lo++;
+    }
+  }
+  __device__ __forceinline__ void put(int i, uint32_t ref, uint32_t key) {
+    BRT_LDS uint32_t *e = ring + (i & mask) * 128;
+    e[0] = ref;
+    e[64] = key;
+  }
+  __device__ __forceinline__ uint64_t slot(int i) const {
+    BRT_LDS uint32_t *e = ring + (i & mask) * 128;
+    return ((uint64_t)e[64] << 32) | e[0];
+  }
+  __device__ __forceinline__ TriEntry pop() {  // requires sp > bot
+    sp--;
+    uint64_t e;
+    if (sp < lo) {
+      lo = sp;
+      e = spill[sp];
+    } else {
+      e = slot(sp);
+    }
+    return TriEntry{(uint32_t)e, (uint32_t)(e >> 32)};
+  }
+  __device__ __forceinline__ uint64_t take_bottom() {  // requires sp > bot
+    uint64_t e;
+    if (bot < lo) e = spill[bot];
+    else e = slot(bot);
+    bot++;
+    lo = lo < bot ? bot : lo;
+    return e;
+  }
+};
+
+struct TriTrees {
+  const NodeQ *nodes;
+  const TriFilt *filt;
+  const TriRec *recs;
+};
+
+// A lane's traversal: cur is a node, or LEAF_BIT | the next primitive of a leaf with `cnt` of them left; cand marks
+// the members of the current pre-test group that still need the FP64 test.
+struct TriTrav {
+  uint32_t cur, cnt, cand;
+  float h32;
+  float rel;  // largest relative error bound of the accepted hits
+  bool active, listed;
+};
+
+// One unit of the traversal: an internal node, the pre-test of a leaf's next FILTER_GROUP triangles, or the FP64 test of
+// one that passed. As in trav_step, every lane fetches its record by the same instructions and waits once.
+__device__ __forceinline__ void tri_step(const TriTrees &T, const Ray &r, const RayQ &q, Hit &s, TriTrav &t,
+                                         TriStack &st) {
+  using u32x4 = unsigned int __attribute__((ext_vector_type(4)));
+  using Bytes = const __attribute__((address_space(1))) unsigned char;
+  using GlobalChunk = const __attribute__((address_space(1))) u32x4;
+  const bool at_leaf = (t.cur & LEAF_BIT) != 0;
+  const bool test = t.cand != 0u;
+  const uint32_t first = t.cur & ~LEAF_BIT;
+  const uint32_t p = first + (uint32_t)__builtin_ctz(t.cand | 0x80000000u);
+  // without pre-test records every triangle of the leaf gets the FP64 test (the fetch then reads node 0)
+  Bytes *base = !at_leaf          ? (Bytes *)(T.nodes + t.cur)
+                : test            ? (Bytes *)(T.recs + p)
+                : T.filt != nullptr ? (Bytes *)(T.filt + first)
+                                  : (Bytes *)T.nodes;
+  // node lanes read the near row of each axis into chunk a and the far row into chunk 4 + a; the others read 16-byte
+  // chunks in order
+  const uint32_t code = at_leaf ? 0u : q.code;
+  const uint32_t near0 = code & 64u, near1 = (code >> 1) & 64u, near2 = (code >> 2) & 64u;
+  u32x4 c0, c1, c2, c3, c4, c5, c6, c7;
+  c0 = *(GlobalChunk *)(base + near0);
+  c1 = *(GlobalChunk *)(base + near1 + 16);
+  c2 = *(GlobalChunk *)(base + near2 + 32);
+  c3 = *(GlobalChunk *)(base + 48);
+  c4 = *(GlobalChunk *)(base + (64u - near0));
+  if (!test) {  // a triangle record ends with chunk 4
+    c5 = *(GlobalChunk *)(base + (64u - near1) + 16);
+    c6 = *(GlobalChunk *)(base + (64u - near2) + 32);
+    c7 = *(GlobalChunk *)(base + 112);
+  }
+  asm volatile("" : "+v"(c0), "+v"(c1), "+v"(c2), "+v"(c3), "+v"(c4), "+v"(c5), "+v"(c6), "+v"(c7));
+  if (!at_leaf) {
+    uint32_t m = 0;
+    uint32_t key[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const float n0 = __builtin_fmaf(__uint_as_float(c0[c]), q.inv[0], q.offn[0]);
+      const float n1 = __builtin_fmaf(__uint_as_float(c1[c]), q.inv[1], q.offn[1]);
+      const float n2 = __builtin_fmaf(__uint_as_float(c2[c]), q.inv[2], q.offn[2]);
+      const float f0 = __builtin_fmaf(__uint_as_float(c4[c]), q.inv[0], q.offf[0]);
+      const float f1 = __builtin_fmaf(__uint_as_float(c5[c]), q.inv[1], q.offf[1]);
+      const float f2 = __builtin_fmaf(__uint_as_float(c6[c]), q.inv[2], q.offf[2]);
+      const float A = max_nn(max3_nn(n0, n1, n2), q.tmin);
+      const float M = min_nn(min3_nn(f0, f1, f2), t.h32);
+      key[c] = __float_as_uint(A);
+      m |= A <= M ? 1u << c : 0u;
+    }
+    if (m) {
+      // the visiting order: slot c goes below the entries of the slots before it, i.e. at sp + the number of entered
+      // slots after it; the first one is visited next
+      const uint32_t word = (code & 32u) ? c7[1] : c7[0];
+      const uint32_t later = (word >> (code & 31u)) ^ (uint32_t)(((int)(code << 22)) >> 31);
+      const int n = __popc(m);
+      st.room(n - 1);
+      uint32_t ncur = 0, ncnt = 0;
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        if ((m >> c) & 1u) {
+          const int rank = __popc(m & (later >> (4 * c)) & (15u & ~(1u << c)));
+          const uint32_t k = __builtin_amdgcn_perm(key[c], c7[2], 0x07060500u | (uint32_t)c);
+          if (rank == n - 1) {
+            ncur = c3[c];
+            ncnt = k & 255u;
+          } else {
+            st.put(st.sp + rank, c3[c], k);
+          }
+        }
+      }
+      st.sp += n - 1;
+      t.cur = ncur;
+      t.cnt = ncnt;
+      return;
+    }
+  } else if (!test) {
+    TriFilt g[2];
+    u32x4 raw[8] = {c0, c1, c2, c3, c4, c5, c6, c7};
+    __builtin_memcpy(g, raw, sizeof g);
+    bool p0 = true, p1 = true;
+    if (T.filt != nullptr) {
+      p0 = tri_filter(g[0], q.D, q.O, q.om, q.tmin, t.h32);
+      p1 = tri_filter(g[1], q.D, q.O, q.om, q.tmin, t.h32);
+    }
+    t.cand = (p0 ? 1u : 0u) | (p1 && t.cnt > 1u ? 2u : 0u);
+    if (t.cand) return;
+    if (t.cnt > 2u) {
+      t.cnt -= 2u;
+      t.cur += 2u;
+      return;
+    }
+  } else {
+    TriRec rec;
+    u32x4 raw[5] = {c0, c1, c2, c3, c4};
+    __builtin_memcpy(&rec, raw, sizeof rec);
+    Certificate c{true, 0.0f};
+    if (isect_tri(rec, r, s, p, [&](double u, double v, double w, double tt, double ad, double thr) {
+          c = certified(rec, r.o, r.tmin, (double)q.slack, u, v, w, tt, ad, thr);
+        })) {
+      t.h32 = f32_up(s.h);
+      t.listed = t.listed || !c.sure;
+      t.rel = fmaxf(t.rel, c.rel);
+    }
+    t.cand &= t.cand - 1u;
+    if (t.cand) return;
+    if (t.cnt > 2u) {
+      t.cnt -= 2u;
+      t.cur += 2u;
+      return;
+    }
+  }
+  while (st.sp > st.bot) {
+    const TriEntry e = st.pop();
+    if (!(t.h32 < __uint_as_float(e.key & ~255u))) {
+      t.cur = e.ref;
+      t.cnt = e.key & 255u;
+      return;
+    }
+  }
+  t.active = false;
+}
+
+// Starts a ray: its root test, with the FP32 bounds.
+struct TriRoot {
+  float lo[3], hi[3];
+  uint32_t ref, cnt;
+};
+__device__ __forceinline__ TriRoot tri_root(const BvhView &bvh) {
+  return TriRoot{{bvh.root_min32[0], bvh.root_min32[1], bvh.root_min32[2]},
+                 {bvh.root_max32[0], bvh.root_max32[1], bvh.root_max32[2]}, bvh.root_ref4, bvh.root_cnt};
+}
+__device__ __forceinline__ void tri_begin(const TriRoot &root, const Ray &r, const RayQ &q, const Hit &s, TriTrav &t) {
+  t.cur = root.ref;
+  t.cnt = root.cnt;
+  t.cand = 0;
+  t.listed = false;
+  t.rel = 0.0f;
+  t.h32 = f32_up(s.h);
+  float A = q.tmin, M = t.h32;
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const bool sg = (r.sign >> a) & 1u;
+    const float lo = root.lo[a], hi = root.hi[a];
+    A = fmaxf(A, __builtin_fmaf(sg ? hi : lo, q.inv[a], q.offn[a]));
+    M = fminf(M, __builtin_fmaf(sg ? lo : hi, q.inv[a], q.offf[a]));
+  }
+  t.active = A <= M;
+}
+
+// A value of another lane, for the lanes that take over its work.
+__device__ __forceinline__ uint32_t lane_get(uint32_t x, int src) {
+  return (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)x);
+}
+template <class V>
+__device__ __forceinline__ void lane_take(V &x, int src, bool take) {
+  static_assert(sizeof(V) % 4 == 0, "words");
+  uint32_t w[sizeof(V) / 4];
+  __builtin_memcpy(w, &x, sizeof(V));
+#pragma unroll
+  for (size_t k = 0; k < sizeof(V) / 4; k++) {
+    const uint32_t y = lane_get(w[k], src);
+    w[k] = take ? y : w[k];
+  }
+  __builtin_memcpy(&x, w, sizeof(V));
+}
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Rays whose parts several lanes trace. Sharing starts with at least SHARE_MIN_IDLE idle lanes and no rays left to
+// start, so at most SHARE_SLOTS rays of a wave are ever shared.
+constexpr uint32_t SHARE_MIN_IDLE = 32;
+constexpr uint32_t SHARE_SLOTS = 32;
+static_assert(64u - SHARE_MIN_IDLE <= SHARE_SLOTS, "a slot for every ray left");
+struct TriShare {
+  double h[SHARE_SLOTS], u[SHARE_SLOTS], v[SHARE_SLOTS];
+  uint32_t prim[SHARE_SLOTS];
+  uint32_t parts[SHARE_SLOTS];  // parts still running; bit 31: the ray is to be listed
+  float rel[SHARE_SLOTS];
+  // smallest accepted hit distance so far, as the bits of its FP32 upper bound above the position of the part that
+  // accepted it in the traversal order: the parts after that one skip what lies behind it
+  unsigned long long bound[SHARE_SLOTS];
+};
+
+__device__ __forceinline__ unsigned long long bound_of(float h32, uint32_t pos) {
+  return ((unsigned long long)__float_as_uint(h32) << 32) | pos;  // h32 >= 0: its bits order as it does
+}
+
+// Persistent waves as in k_trace_persistent. BATCH: the rays of many jobs, as in k_trace_batch.
+template <bool BATCH>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BRT_WAVES_PER_EU)))
+k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t n,
+            uint32_t flags, uint32_t first, double S, unsigned long long *group, uint32_t refill,
+            const uint32_t *order, uint32_t ring, uint32_t chunk, uint32_t fixed) {
+  extern __shared__ unsigned char smem[];
+  __shared__ TriShare shares[4];
+  constexpr int RW = (int)(sizeof(RaysView) / 8), HW = (int)(sizeof(HitsView) / 8);
+  __shared__ uint64_t views[RW + HW];  // ray and hit columns, read back where they are used (see k_trace_persistent)
+  if constexpr (!BATCH) {
+    if (threadIdx.x == 0) {
+      lds_store(views, rays);
+      lds_store(views + RW, hits);
+    }
+    __syncthreads();
+  }
+  // as in k_trace_batch, with the geometry id in place of is_tri
+  constexpr int JW = HW + 1;
+  __shared__ uint64_t job_fin[BATCH ? BATCH_LDS_JOBS * JW : 1];
+  const bool fin_lds = njobs <= BATCH_LDS_JOBS;
+  if constexpr (BATCH) {
+    if (fin_lds) {
+      for (uint32_t k = threadIdx.x; k < njobs; k += blockDim.x) {
+        lds_store(job_fin + k * JW, jobs[k].hits);
+        job_fin[k * JW + JW - 1] = (uint64_t)jobs[k].first | ((uint64_t)jobs[k].bvh.geom_id << 32);
+      }
+      __syncthreads();
+    }
+  }
+  const uint32_t lane = __lane_id(), wave = threadIdx.x / 64;
+  BRT_LDS volatile TriShare *sh = (BRT_LDS volatile TriShare *)&shares[wave];
+  uint64_t spill[TRI_SPILL];
+  TriStack st;
+  st.ring = (BRT_LDS uint32_t *)smem + (size_t)wave * ring * 128 + lane;
+  st.spill = spill;
+  st.mask = (int)ring - 1;
+  st.reset();
+  TriTrees T{bvh.nodesq, bvh.tri_filter, reinterpret_cast<const TriRec *>(bvh.prims)};
+  Ray r;
+  RayQ q;
+  Hit s;
+  TriTrav t;
+  t.active = false;
+  t.cand = 0;
+  bool has_ray = false, shared = false;
+  bool done = false;       // a traced ray, still to be written
+  bool exhausted = false;  // wave-uniform
+  uint32_t pos = 0, pos_end = 0;  // shared rays: this part's positions in the traversal order
+  uint32_t slot = 0, slots = 0;  // the share slot of this lane's ray; slots given out (wave-uniform)
+  uint64_t idx = 0;        // ray index, within its job
+  uint32_t j = 0;
+  // Finished rays are written together, when the wave refills: a ray ends in almost every iteration, and writing it
+  // there would run this code for a lane or two each time.
+  auto write_rays = [&]() {
+    if (done) {
+      done = false;
+      if (t.listed) {
+        const unsigned long long k = atomicAdd(group + COUNTER_LISTED, 1ull);
+        if (k < (unsigned long long)LIST_CAPACITY) {
+          group[COUNTER_CLEARED + k] = BATCH ? jobs[j].offset + idx : idx;
+        }
+      } else {
+        r.tmax = s.leaf_idx == INVALID_ID ? -__builtin_inf() : __builtin_inf();  // hit or not, for finish_ray
+        if constexpr (BATCH) {
+          HitsView hv;
+          BvhView fb{};
+          uint32_t jfirst;
+          if (fin_lds) {
+            __builtin_memcpy(&hv, job_fin + j * JW, sizeof(HitsView));
+            const uint64_t w = job_fin[j * JW + JW - 1];
+            jfirst = (uint32_t)w;
+            fb.geom_id = (uint32_t)(w >> 32);
+          } else {
+            hv = jobs[j].hits;
+            jfirst = jobs[j].first;
+            fb.geom_id = jobs[j].bvh.geom_id;
+          }
+          if (hv.nx) {
+            fb.faces = jobs[j].bvh.faces;
+            fb.vnormals = jobs[j].bvh.vnormals;
+          }
+          finish_ray<TriRec>(fb, hv, idx, r, s, flags, jfirst, 1u);
+        } else {
+          finish_ray<TriRec>(bvh, lds_fresh<HitsView>(views + RW), idx, r, s, flags, first, 1u);
+        }
+      }
+    }
+  };
+  WavePool pool;
+  if (fixed) {  // a small launch: `fixed` rays per wave, no claims, and the other lanes help from the start
+    const uint64_t w = (uint64_t)blockIdx.x * (blockDim.x / 64) + wave;
+    pool.next = w * fixed < n ? w * fixed : n;
+    pool.end = pool.next + fixed < n ? pool.next + fixed : n;
+    pool.last = true;
+  }
+  uint32_t turn = 0;
+  for (;;) {
+    if (!exhausted) {
+      const unsigned long long idle = __ballot(!has_ray);
+      const uint32_t nidle = (uint32_t)__popcll(idle);
+      if (nidle >= refill || nidle == 64u) {
+        write_rays();
+        bool got;
+        uint64_t cand = 0;
+        pool_refill(pool, group + COUNTER_POOL, n, chunk, idle, nidle, lane, got, cand, exhausted);
+        double ext = S;
+        TriRoot root{};
+        RawRay raw{};
+        if constexpr (BATCH) {
+          const unsigned long long gm = __ballot(got);
+          if (gm) {
+            // The jobs of the claim's first and last index, once per wave. Nearly always they are one job, whose record
+            // is then read by scalar loads; otherwise every lane searches for its own.
+            const int lo = __ffsll((long long)gm) - 1, hi = 63 - __clzll((long long)gm);
+            const uint64_t g_lo = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(cand >> 32), lo) << 32) |
+                                  (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cand, lo);
+            const uint64_t g_hi = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(cand >> 32), hi) << 32) |
+                                  (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cand, hi);
+            const uint32_t j_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)find_job(jobs, njobs, g_lo));
+            const bool one_job = j_lo + 1u >= njobs || jobs[j_lo + 1u].offset > g_hi;
+            const auto take = [&](const BatchJob &J) {
+              idx = cand - J.offset;  // batches trace in input order
+              ext = J.extent;
+              T = TriTrees{J.bvh.nodesq, J.bvh.tri_filter, reinterpret_cast<const TriRec *>(J.bvh.prims)};
+              root = tri_root(J.bvh);
+              raw = load_ray(J.rays, idx);
+            };
+            if (one_job) {
+              const BatchJob &J = jobs[j_lo];
+              if (got) {
+                j = j_lo;
+                take(J);
+              }
+            } else if (got) {
+              j = find_job(jobs, njobs, cand);
+              take(jobs[j]);
+            }
+          }
+        } else if (got) {
+          idx = order ? (uint64_t)order[cand] : cand;
+          root = tri_root(bvh);
+          raw = load_ray(lds_fresh<RaysView>(views), idx);
+        }
+        if (got) {
+          setup_ray(raw.org, raw.dir, raw.tmin, raw.tmax, r);
+          const double len2 = squared_length(raw);
+          if (fast_ray(r, len2, ext)) {
+            has_ray = true;
+            make_rayq(r, len2, ext, q);
+            s.h = r.tmax;
+            s.u = s.v = 0.0;
+            s.leaf_idx = INVALID_ID;
+            tri_begin(root, r, q, s, t);
+            st.reset();
+          } else if (r.o[2] != r.o[2] || r.inv[2] != r.inv[2]) {
+            // NaN far-plane terms on the last axis: the reference rejects every box, the root first (a mirror ray
+            // that has left the scene)
+            has_ray = true;
+            s.leaf_idx = INVALID_ID;
+            t.active = t.listed = false;
+          } else {
+            __atomic_store_n(group + COUNTER_DEFERRED, 1ull, __ATOMIC_RELAXED);
+          }
+        }
+      }
+    }
+    const unsigned long long busy = __ballot(has_ray);
+    if (exhausted) {
+      if (!busy) {
+        write_rays();
+        break;
+      }
+      const unsigned long long can = __ballot(has_ray && st.sp > st.bot);
+      const uint32_t nidle = 64u - (uint32_t)__popcll(busy);
+      // in every other iteration: sharing costs about as many instructions as a traversal step (every one: 3-5% slower)
+      if (nidle >= SHARE_MIN_IDLE && can && (++turn & 1u) == 0u) {
+        write_rays();  // the helpers' state is overwritten
+        const unsigned long long below = (1ull << lane) - 1ull;
+        const uint32_t ncan = (uint32_t)__popcll(can), k = nidle < ncan ? nidle : ncan;
+        const uint32_t rank = (uint32_t)__popcll((has_ray ? can : ~busy) & below);
+        const bool donor = ((can >> lane) & 1ull) && rank < k, helper = !has_ray && rank < k;
+        const uint32_t pos_end0 = shared ? pos_end : 0xffffffffu;
+        // the r-th helper takes from the r-th donor, whose lane number lane r receives
+        const unsigned long long fresh = __ballot(donor && !shared);
+        uint64_t e = 0;
+        if (donor) {
+          e = st.take_bottom();
+          if (!shared) {
+            shared = true;
+            slot = slots + (uint32_t)__popcll(fresh & below);
+            sh->parts[slot] = 1u;
+            sh->prim[slot] = INVALID_ID;
+            sh->h[slot] = __builtin_inf();
+            sh->rel[slot] = 0.0f;
+            sh->bound[slot] = bound_of(t.h32, 0u);
+            pos = 0u;
+            pos_end = 0xffffffffu;
+          }
+          pos_end -= (pos_end - pos) >> 3;  // the helper's part is the last eighth of the positions
+        }
+        slots += (uint32_t)__popcll(fresh);
+        wave_fence();
+        if (donor) atomicAdd(&shares[wave].parts[slot], 1u);
+        // (at most 32 donors: lane 63 takes what the others push)
+        const uint32_t by_rank = (uint32_t)__builtin_amdgcn_ds_permute((donor ? (int)rank : 63) << 2, (int)lane);
+        const uint32_t from = lane_get(by_rank, (int)rank);  // with all lanes: a permute reads active lanes only
+        const int src = helper ? (int)from : (int)lane;
+        lane_take(e, src, helper);
+        lane_take(r.o, src, helper);
+        lane_take(r.d, src, helper);
+        lane_take(r.tmin, src, helper);
+        lane_take(q, src, helper);
+        lane_take(s.h, src, helper);
+        lane_take(t.h32, src, helper);
+        lane_take(idx, src, helper);
+        lane_take(slot, src, helper);
+        {
+          const uint32_t from_end = lane_get(pos_end, src), old_end = lane_get(pos_end0, src);
+          pos = helper ? from_end : pos;
+          pos_end = helper ? old_end : pos_end;
+        }
+        if constexpr (BATCH) {
+          lane_take(T, src, helper);
+          lane_take(j, src, helper);
+        }
+        if (helper) {
+          has_ray = true;
+          shared = true;
+          s.leaf_idx = INVALID_ID;
+          t.cur = (uint32_t)e;
+          t.cnt = (uint32_t)(e >> 32) & 255u;
+          t.cand = 0;
+          t.listed = false;
+          t.rel = 0.0f;
+          t.active = !(t.h32 < __uint_as_float((uint32_t)(e >> 32) & ~255u));
+          st.reset();
+        }
+        wave_fence();
+      }
+    }
+    if (has_ray && t.active) {
+      if (shared) {
+        const unsigned long long b = sh->bound[slot];
+        const float h32 = __uint_as_float((uint32_t)(b >> 32));
+        if ((uint32_t)b < pos && h32 < t.h32) {  // an earlier part's hit: this part's own, if it lies behind, is void
+          t.h32 = h32;
+          s.h = (double)h32;
+          s.leaf_idx = INVALID_ID;
+        }
+      }
+      const uint32_t before = s.leaf_idx;
+      tri_step(T, r, q, s, t, st);
+      if (shared && s.leaf_idx != before && s.h >= 0.0) atomicMin(&shares[wave].bound[slot], bound_of(t.h32, pos));
+    }
+    bool fin = has_ray && !t.active;
+    if (exhausted) {
+      // the parts of a shared ray are merged one lane at a time; the last one writes the ray
+      unsigned long long m = __ballot(fin && shared);
+      while (m) {
+        const uint32_t l = (uint32_t)__ffsll((long long)m) - 1u;
+        m &= m - 1ull;
+        if (lane == l) {
+          uint32_t parts = sh->parts[slot];
+          if (t.listed) parts |= 0x80000000u;
+          if (s.leaf_idx != INVALID_ID) {
+            const double h = sh->h[slot];
+            const float rel = fmaxf(t.rel, sh->rel[slot]);
+            sh->rel[slot] = rel;
+            if (fabs(s.h - h) <= (2.0 * (double)rel + 0x1p-46) * s.h) parts |= 0x80000000u;
+            if (s.h < h) {
+              sh->h[slot] = s.h;
+              sh->u[slot] = s.u;
+              sh->v[slot] = s.v;
+              sh->prim[slot] = s.leaf_idx;
+            }
+          }
+          parts--;
+          sh->parts[slot] = parts;
+          has_ray = false;
+          shared = false;
+          if ((parts & 0x7fffffffu) == 0u) {
+            s.h = sh->h[slot];
+            s.u = sh->u[slot];
+            s.v = sh->v[slot];
+            s.leaf_idx = sh->prim[slot];
+            t.listed = (parts >> 31) != 0u;
+          } else {
+            fin = false;
+          }
+        }
+        wave_fence();
+      }
+    }
+    done = done || fin;
+    if (fin) has_ray = false;
+  }
+}
+
 // Split-precision pre-test records of the triangles in leaf order (TriFilt), from their FP64 records; the FILTER_PAD
 // records after the last one are zero.
 __global__ void k_tri_filter_records(const TriRec *__restrict__ recs, uint32_t n, TriFilt *out, uint32_t total) {
@@ -1397,9 +2122,9 @@ __global__ void k_tri_filter_records(const TriRec *__restrict__ recs, uint32_t n
       // upper bounds (the FP64 sums and products of non-negative terms are within a few ulps of exact)
       const double up = 1.0 + 0x1p-48, u = 0x1p-24;
       f.vmax = f32_up(vm * up);
-      f.kua = f32_up(16.0 * u * sa * up);
-      f.kub = f32_up(16.0 * u * sb * up);
       f.ed = f32_up((10.0 * u * sa * sb + 1e-29) * up);
+      f.kw = f32_up(1.2 * 16.0 * u * (sa + sb) * up);
+      f.cw = f32_up((1.3 * (double)f.ed + 9e-16) * up);  // 9e-16: 4 DBL_EPSILON rounded up
     }
     out[i] = f;
   }
@@ -1451,9 +2176,29 @@ __global__ void k_cyl_filter_records(const CylRec *__restrict__ recs, uint32_t n
   }
 }
 
+__global__ void k_nodeq_records(const Node4 *__restrict__ in, const uint32_t *__restrict__ ord, uint32_t n,
+                                NodeQ *__restrict__ out) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const Node4 a = in[i];
+  NodeQ b;
+  for (int c = 0; c < 4; c++) {
+    for (int k = 0; k < 3; k++) {
+      b.lo[k][c] = a.lo[k][c];
+      b.hi[k][c] = a.hi[k][c];
+    }
+    b.ref[c] = a.ref[c];
+    b.cnt[c] = a.cnt[c] == EMPTY_SLOT ? 0 : (uint8_t)a.cnt[c];
+  }
+  b.ord[0] = ord[2ull * i];
+  b.ord[1] = ord[2ull * i + 1];
+  b.pad = 0;
+  out[i] = b;
+}
+
 // Clears a launch's counter group (a fill kernel, not hipMemsetAsync, so that graph captures replay correctly).
 __global__ void k_zero_counters(unsigned long long *c) {
-  for (uint32_t k = threadIdx.x; k < (uint32_t)COUNTER_GROUP; k += blockDim.x) c[k] = 0ull;
+  for (uint32_t k = threadIdx.x; k < (uint32_t)COUNTER_CLEARED; k += blockDim.x) c[k] = 0ull;
 }
 
 // 3 x 9-bit Morton interleave
@@ -1562,6 +2307,88 @@ hipError_t launch_kernel(const BvhView &bvh, const RaysViewT<typename Rec::real>
   return hipGetLastError();
 }
 
+// Rays per wave of a launch that the device's `waves` resident waves take in one go (up to a full wave each; 262,144 on
+// 256 CUs): the waves then have idle lanes from the start, which share their rays' work, and none waits for a claim.
+// 0 for larger launches, whose waves claim. Incoherent rays, 82k-triangle mesh: 2,000 rays 123 -> 74 us against claims
+// of 64; 328k-triangle mesh: 50,000 rays 265 -> 202 us, 200,000 rays 375 -> 324 us; a 200x150 camera 394 -> 250 us.
+constexpr uint64_t FIXED_RAYS = 64;
+uint32_t fixed_rays(uint64_t n, uint64_t waves) {
+  const uint64_t per = (n + waves - 1) / waves;
+  return per <= FIXED_RAYS ? (uint32_t)per : 0u;
+}
+
+// The fast triangle traversal (k_trace_tri) takes closest-hit launches on the persistent schedule, in either precision:
+// 1.31M-triangle mesh, 4,194,304 incoherent rays 3.03 ms, against 5.6-5.8 ms for the exact FP64 kernel and 3.8 ms for
+// nearest-first split precision; a 1920x1080 camera with normals 2.24 against 3.57 ms. Any-hit launches return the first
+// hit of their own visiting order and keep the kernels that define it; the one-ray-per-thread schedule keeps its kernel.
+bool fast_triangles(const TraceLaunch &cfg) {
+  return cfg.schedule == SCHEDULE_PERSISTENT && !(cfg.flags & FLAG_ANY_HIT);
+}
+constexpr uint32_t TRI_RING = 16, TRI_REFILL = 16;
+constexpr size_t tri_lds_bytes(uint32_t block, uint32_t ring) { return (size_t)block * ring * sizeof(uint64_t); }
+
+hipError_t launch_tri(const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint64_t n,
+                      const TraceLaunch &cfg, const SplitParams &sp, hipStream_t stream) {
+  const uint32_t block = cfg.block ? cfg.block : 256;
+  const uint32_t ring = cfg.ring ? cfg.ring : TRI_RING;
+  const uint32_t first = cfg.first ? 1u : 0u;
+  const size_t lds = tri_lds_bytes(block, ring);
+  unsigned long long *grp = cfg.counter;
+  if (!grp) return hipErrorInvalidValue;
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
+  uint64_t blocks = 0;
+  hipError_t e = persistent_blocks(k_trace_tri<false>, block, lds, n * 64, blocks);
+  if (e != hipSuccess) return e;
+  const uint32_t wpb = block / 64, fixed = fixed_rays(n, blocks * wpb);
+  const uint64_t need = fixed ? (n + fixed * wpb - 1) / (fixed * wpb) : (n + block - 1) / block;
+  if (blocks > need) blocks = need;
+  hipLaunchKernelGGL(k_trace_tri<false>, dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits,
+                     (const BatchJob *)nullptr, 0u, n, cfg.flags, first, sp.scene_extent, grp,
+                     cfg.refill ? cfg.refill : TRI_REFILL, cfg.order, ring, cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  // the rays it left to the exact kernel (default launch shape of the exact path)
+  const uint32_t ring64 = ring_default<TriRec, false>();
+  const size_t lds64 = ring_lds_bytes<false, double>(256, ring64);
+  e = persistent_blocks(k_trace_persistent<TriRec, false, true>, 256, lds64, n, blocks);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_trace_persistent<TriRec, false, true>), dim3((uint32_t)blocks), dim3(256), lds64, stream, bvh,
+                     rays, hits, n, cfg.flags, first, 1u, sp.scene_extent, grp + COUNTER_DEFERRED_POOL,
+                     refill_default<TriRec, false>(), cfg.order, ring64, grp + COUNTER_DEFERRED, POOL_CHUNK);
+  return hipGetLastError();
+}
+
+hipError_t launch_tri_batch(const BatchJob *jobs, uint32_t njobs, uint64_t total, const TraceLaunch &cfg,
+                            hipStream_t stream) {
+  const uint32_t block = cfg.block ? cfg.block : 256;
+  const uint32_t ring = cfg.ring ? cfg.ring : TRI_RING;
+  const size_t lds = tri_lds_bytes(block, ring);
+  unsigned long long *grp = cfg.counter;
+  if (!grp || njobs == 0) return hipErrorInvalidValue;
+  if (total == 0) return hipSuccess;
+  uint64_t blocks = 0;
+  hipError_t e = persistent_blocks(k_trace_tri<true>, block, lds, total * 64, blocks);
+  if (e != hipSuccess) return e;
+  const uint32_t wpb = block / 64, fixed = fixed_rays(total, blocks * wpb);
+  const uint64_t need = fixed ? (total + fixed * wpb - 1) / (fixed * wpb) : (total + block - 1) / block;
+  if (blocks > need) blocks = need;
+  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
+  hipLaunchKernelGGL(k_trace_tri<true>, dim3((uint32_t)blocks), dim3(block), lds, stream, BvhView{}, RaysView{},
+                     HitsView{}, jobs, njobs, total, cfg.flags, 0u, 0.0, grp, cfg.refill ? cfg.refill : TRI_REFILL,
+                     (const uint32_t *)nullptr, ring, cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const uint32_t ring64 = ring_default<TriRec, false>();
+  const size_t lds64 = ring_lds_bytes<false>(256, ring64);
+  e = persistent_blocks(k_trace_batch<TriRec, false, true>, 256, lds64, total, blocks);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_trace_batch<TriRec, false, true>), dim3((uint32_t)blocks), dim3(256), lds64, stream, jobs,
+                     njobs, total, cfg.flags, grp + COUNTER_DEFERRED_POOL, refill_default<TriRec, false>(), ring64,
+                     grp + COUNTER_DEFERRED, POOL_CHUNK);
+  return hipGetLastError();
+}
+
 template <class Rec, bool SPLIT>
 hipError_t launch_batch_kernel(const BatchJob *jobs, uint32_t njobs, uint64_t total, const TraceLaunch &cfg,
                                hipStream_t stream) {
@@ -1602,7 +2429,9 @@ hipError_t launch_typed(const BvhView &bvh, const RaysView &rays, const HitsView
 hipError_t launch_trace(GeomType type, const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint64_t n,
                         const TraceLaunch &cfg, const SplitParams &split, hipStream_t stream) {
   switch (type) {
-  case TRIANGLES: return launch_typed<TriRec>(bvh, rays, hits, n, cfg, split, 1u, stream);
+  case TRIANGLES:
+    if (bvh.nodesq && fast_triangles(cfg)) return launch_tri(bvh, rays, hits, n, cfg, split, stream);
+    return launch_typed<TriRec>(bvh, rays, hits, n, cfg, split, 1u, stream);
   case SPHERES: return launch_typed<SphRec>(bvh, rays, hits, n, cfg, split, cfg.overwrite ? 1u : 0u, stream);
   case PLANES: return launch_typed<PlaRec>(bvh, rays, hits, n, cfg, split, cfg.overwrite ? 1u : 0u, stream);
   default: return launch_typed<CylRec>(bvh, rays, hits, n, cfg, split, cfg.overwrite ? 1u : 0u, stream);
@@ -1624,6 +2453,12 @@ hipError_t launch_cyl_filter_records(const void *recs, uint32_t n, void *out, hi
   if (blocks > 65536) blocks = 65536;
   hipLaunchKernelGGL(k_cyl_filter_records, dim3(blocks), dim3(256), 0, stream, static_cast<const CylRec *>(recs), n,
                      static_cast<SphFilt *>(out), total);
+  return hipGetLastError();
+}
+
+hipError_t launch_nodeq_records(const Node4 *nodes4, const uint32_t *ord, uint32_t n, NodeQ *out, hipStream_t stream) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_nodeq_records, dim3((n + 255) / 256), dim3(256), 0, stream, nodes4, ord, n, out);
   return hipGetLastError();
 }
 
@@ -1714,6 +2549,7 @@ hipError_t launch_trace_batch(GeomType type, const BatchJob *jobs, uint32_t njob
   const bool split = cfg.precision != PREC_FP64;
   switch (type) {
   case TRIANGLES:
+    if (cfg.fast && fast_triangles(cfg)) return launch_tri_batch(jobs, njobs, total, cfg, stream);
     return split ? launch_batch_kernel<TriRec, true>(jobs, njobs, total, cfg, stream)
                  : launch_batch_kernel<TriRec, false>(jobs, njobs, total, cfg, stream);
   case SPHERES:

@@ -38,6 +38,23 @@ struct alignas(128) Node4 {
 };
 static_assert(sizeof(Node4) == 128, "Node4 must be one 128-byte line");
 
+// Reference-order FP32 4-wide node of a triangle tree, 128 B: a Node4's child boxes and references, and the order in
+// which the reference's depth-first traversal visits its slots. Planes are child-minor rows; the lo and hi rows of an
+// axis lie 64 bytes apart, so a lane loads the near and the far row of an axis by address. ord: for the octants 0..3 of
+// the direction signs (x, y; z positive), 16 bits each: bits 4c..4c+3 are the slots visited after slot c; the masks of
+// the other octants are the complements of those of the opposite octant. cnt: leaf counts (a tree with a leaf of more
+// than NODEQ_MAX_LEAF primitives has no such nodes). Unused slots have an inverted infinite box, which no ray enters.
+constexpr uint32_t NODEQ_MAX_LEAF = 255;
+struct alignas(128) NodeQ {
+  float lo[3][4];
+  uint32_t ref[4];
+  float hi[3][4];
+  uint32_t ord[2];
+  uint8_t cnt[4];
+  uint32_t pad;
+};
+static_assert(sizeof(NodeQ) == 128, "NodeQ must be one 128-byte line");
+
 // Triangle record in leaf order: v0, e1 = v0 - v1, e2 = v2 - v0 (blazert/primitives/trimesh.h:26-27) and the user
 // primitive id (prim_ids at this leaf position), which a hit takes from the record it has just read instead of a
 // dependent lookup when the ray finishes. The FP64 record does not carry n = cross(e1, e2): the 16 more bytes per
@@ -55,15 +72,15 @@ static_assert(sizeof(TriRec) == 80, "TriRec size");
 
 // Split precision: FP32 pre-test record of a triangle, in leaf order beside the TriRec array: v0, e1, e2 and the
 // FP64 test's n = cross(e1, e2), each rounded to nearest, and the constants of the pre-test's error bound, rounded
-// up from FP64: vmax >= max |v0_i|, kua = 16 u sum |e1_i|, kub = 16 u sum |e2_i|, ed = 10 u sum |e1_i| sum |e2_i|
-// + 1e-29 (u = 2^-24). Built on the device from the TriRec array; FILTER_PAD records of padding follow the last one,
+// up from FP64: vmax >= max |v0_i|, ed = 10 u sum |e1_i| sum |e2_i| + 1e-29, kw = 19.2 u (sum |e1_i| + sum |e2_i|),
+// cw = 1.3 ed + 4 DBL_EPSILON (u = 2^-24). Built on the device from the TriRec array; FILTER_PAD records of padding follow the last one,
 // so a group of FILTER_GROUP records read from any leaf start stays in bounds.
 struct alignas(16) TriFilt {
   float v0[3];
   float e1[3];
   float e2[3];
   float n[3];
-  float vmax, kua, kub, ed;
+  float vmax, kw, cw, ed;
 };
 static_assert(sizeof(TriFilt) == 64, "TriFilt size");
 #ifndef BRT_FILTER_GROUP
@@ -174,6 +191,7 @@ struct BvhView {
   const double *vertices;     // triangles only: user vertices (3 per vertex), for mirror tracing and its adjoint
   const Node32 *nodes32;      // Scene<float>: FP32 nodes (nodes64 / nodes4 unused)
   const TriFilt *tri_filter;  // split precision, triangles: FP32 pre-test records (NULL: every test in FP64)
+  const NodeQ *nodesq;        // triangles: reference-order FP32 nodes (NULL: the exact kernels trace the type)
   const SphFilt *sph_filter;  // split precision, spheres and cylinders: FP32 (bounding) spheres (NULL: all in FP64)
   const float *vnormals32;    // Scene<float> triangles: vertex normals
   double root_min[3], root_max[3];

@@ -156,6 +156,7 @@ struct GeometryT {
   // flattened
   std::vector<Node64> n64;  // double scenes
   std::vector<Node4> n4;
+  std::vector<uint32_t> ord4;  // visiting order of every n4 record's slots, two words each
   std::vector<Node32> n32;  // Scene<float>
   RecordBytes recs;
   size_t rec_size = 0;
@@ -530,6 +531,7 @@ void flatten(Geometry &g, GeomType type) {
   // 4-wide FP32 records: every Node4 stands for one binary internal node, with up to four slots taken from its
   // subtree by collapse4 (largest internal slot opened first). Depth-first allocation keeps subtrees together.
   g.n4.clear();
+  g.ord4.clear();
   uint32_t root4 = INVALID_ID;
   if (!T.empty() && !T[0].leaf) {
     std::vector<std::pair<uint32_t, uint32_t>> work;  // (binary internal node, its Node4 index)
@@ -539,8 +541,10 @@ void flatten(Geometry &g, GeomType type) {
     while (!work.empty()) {
       const auto [bi, k4] = work.back();
       work.pop_back();
-      uint32_t slot[4];
-      const int m = collapse4(T.data(), bi, slot);
+      uint32_t slot[4], axis[16] = {};
+      const int m = collapse4(T.data(), bi, slot, axis);
+      g.ord4.resize(2 * g.n4.size());
+      visit_order4(axis, m, &g.ord4[2ull * k4]);
       Node4 nd{};
       for (int c = 0; c < 4; c++) {
         for (int k = 0; k < 3; k++) {
@@ -975,6 +979,25 @@ hipError_t make_prim_filter(DeviceScene &d, BvhView &v, uint32_t type, double ex
   return e;
 }
 
+// Triangles: the reference-order FP32 nodes of the fast closest-hit traversal, made on the device from its Node4
+// records and waited for. None (every trace then takes the exact kernels) for a tree that split precision does not take,
+// one with an inverted or NaN box, or one with a leaf of more than NODEQ_MAX_LEAF primitives.
+hipError_t make_nodesq(DeviceScene &d, BvhView &v, const Geometry &g, uint32_t num_n4, const uint32_t *ord4,
+                       uint32_t max_leaf, hipStream_t st, uint64_t *device_bytes) {
+  v.nodesq = nullptr;
+  if (!g.extent_ok || v.irregular_boxes || max_leaf > NODEQ_MAX_LEAF) return hipSuccess;
+  const size_t bytes = std::max<size_t>(num_n4, 1) * sizeof(NodeQ);  // a root leaf has no records
+  void *p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e != hipSuccess) return e;
+  d.allocs.push_back(p);
+  if (num_n4) e = launch_nodeq_records(v.nodes4, ord4, num_n4, static_cast<NodeQ *>(p), st);
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  v.nodesq = static_cast<const NodeQ *>(p);
+  *device_bytes += bytes;
+  return e;
+}
+
 // Copies one host-built geometry to the device.
 int put_geometry(DeviceScene &d, Geometry &g, uint32_t t) {
   if (g.stats.max_tree_depth >= 64) return fail(BRT_ERR_UNSUPPORTED, "tree deeper than the 64-entry device stack");
@@ -991,6 +1014,12 @@ int put_geometry(DeviceScene &d, Geometry &g, uint32_t t) {
     if (e == hipSuccess) e = d.put(g.vertices, &v.vertices);
   }
   if (e == hipSuccess) e = make_prim_filter(d, v, t, g.extent, nullptr, &g.stats.device_bytes);
+  if (e == hipSuccess && t == TRIANGLES) {
+    const uint32_t *ord4 = nullptr;
+    e = d.put(g.ord4, &ord4);
+    if (e == hipSuccess)
+      e = make_nodesq(d, v, g, g.num_n4, ord4, g.stats.max_num_prims_per_leaf, nullptr, &g.stats.device_bytes);
+  }
   if (e != hipSuccess) return device_error(e, "upload failed");
   d.views[t] = v;
   return BRT_OK;
@@ -1095,11 +1124,13 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
     hipError_t e = device_build(in, r, st);
     if (e != hipSuccess)
       return device_error(e, ("device build failed (build.hip:" + std::to_string(r.failed_line) + ")").c_str());
-    for (void *p : {(void *)r.tree, (void *)r.order, (void *)r.n64, (void *)r.n4, r.recs}) d->allocs.push_back(p);
+    for (void *p : {(void *)r.tree, (void *)r.order, (void *)r.n64, (void *)r.n4, (void *)r.ord4, r.recs})
+      d->allocs.push_back(p);
     g.tree.clear();
     g.order.clear();
     g.n64.clear();
     g.n4.clear();
+    g.ord4.clear();
     g.recs.clear();
     g.rec_size = r.rec_size;
     g.num_n4 = r.num_n4;
@@ -1148,6 +1179,9 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
                       g.vertices.size() * 8;
     if (hipError_t fe = make_prim_filter(*d, v, t, g.extent, st, &bs.device_bytes))
       return device_error(fe, "pre-test records");
+    if (t == TRIANGLES)
+      if (hipError_t fe = make_nodesq(*d, v, g, r.num_n4, r.ord4, r.max_prims, st, &bs.device_bytes))
+        return device_error(fe, "fast traversal nodes");
     d->views[t] = v;
     bs.build_time_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   }
@@ -1906,6 +1940,7 @@ struct brt_batch {
   void *d_jobs[NUM_TYPES] = {nullptr, nullptr, nullptr, nullptr};
   uint32_t njobs[NUM_TYPES] = {0, 0, 0, 0};
   uint64_t total[NUM_TYPES] = {0, 0, 0, 0};
+  bool fast = true;  // every triangle job's tree has the fast traversal's nodes
   unsigned long long *counters = nullptr;
   std::vector<size_t> empty_items;  // items whose scene holds no primitive: their hits are initialised
   hipGraph_t graph = nullptr;
@@ -1928,6 +1963,7 @@ int batch_enqueue(brt_batch *b, hipStream_t st) {
                     b->counters + (size_t)t * COUNTER_GROUP, nullptr};
     cfg.ring = b->L.stack_ring;
     cfg.pool = b->L.pool_size;
+    cfg.fast = b->fast;
     hipError_t e = launch_trace_batch((GeomType)t, static_cast<const BatchJob *>(b->d_jobs[t]), b->njobs[t],
                                       b->total[t], cfg, st);
     if (e != hipSuccess) return fail(BRT_ERR_DEVICE, std::string("batch launch failed: ") + hipGetErrorString(e));
@@ -1983,6 +2019,7 @@ int brt_batch_create(const brt_batch_item *items, uint32_t count, const brt_laun
       }
       BatchJob j{};
       j.bvh = s->dev->views[t];
+      if (t == TRIANGLES && !j.bvh.nodesq) b->fast = false;
       j.rays = RaysView{it.rays.ox, it.rays.oy, it.rays.oz, it.rays.dx, it.rays.dy, it.rays.dz, it.rays.tmin,
                         it.rays.tmax};
       j.hits = HitsView{it.hits.t,  it.hits.u,  it.hits.v,  it.hits.prim_id, it.hits.geom_id,

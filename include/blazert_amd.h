@@ -40,7 +40,7 @@ extern "C" {
 #define BRT_GEOM_CYLINDERS 3u
 
 /* traversal precision (launch option) */
-#define BRT_PRECISION_FP64 0u              /* drop-in: FP64 everywhere, bit-identical to the reference */
+#define BRT_PRECISION_FP64 0u              /* drop-in: FP64 hits, bit-identical to the reference */
 #define BRT_PRECISION_FP32_TRAV_FP64_HIT 1u /* FP32 conservative slab tests, FP64 primitive tests */
 
 /* launch flags */
@@ -114,10 +114,10 @@ typedef struct brt_launch {
   uint32_t block_size; /* threads per block: 64, 128, 192 or 256; 0 = library default (256; 128 for FP64 spheres) */
   uint32_t schedule;   /* BRT_SCHEDULE_* */
   uint32_t refill;     /* persistent: refill a wave once this many of its 64 lanes are idle; 0 = default (32 for
-                          triangles on the exact paths, 16 otherwise) */
+                          any-hit FP64 triangles and FP32 triangles, 16 otherwise) */
   uint32_t sort;       /* BRT_SORT_*: trace rays in a sorted order (results are written in input order) */
-  uint32_t stack_ring; /* traversal-stack entries per lane kept in LDS: 4, 8 or 16; 0 = 16 for split-precision
-                          triangles, 8 otherwise.
+  uint32_t stack_ring; /* traversal-stack entries per lane kept in LDS: 4, 8 or 16; 0 = 16 for FP64 and
+                          split-precision triangles (8 for any-hit FP64), 8 otherwise.
                           Deeper entries spill to private memory; a deeper ring spills less but takes more LDS */
   uint32_t pool_size;  /* persistent: ray indices a wave claims at once: 32, 64 or 128; 0 = 64. Smaller claims
                           balance image-order (coherent) rays better, larger ones cost fewer atomics on the launch's
