@@ -23,6 +23,8 @@
 
 #include "../../include/blazert_amd/user_geometry.h"  // RingStack: LDS stack ring with a private spill area
 #include "engine.h"
+#include "f32_round.h"
+#include "wave.h"
 
 namespace brt {
 
@@ -328,9 +330,9 @@ constexpr uint32_t CLOSEST_BLOCK = 128;
 using ClosestStack = blazert_amd::RingStack<double, CLOSEST_RING>;
 
 // Depth-first search of one BVH, nearer child first. `bound` is the best distance of earlier geometry types.
-template <int TYPE>
+template <int TYPE, class Stack>
 __device__ void closest_in_bvh(const BvhView &bvh, const double *leaf_vertices, const double *p, double margin,
-                               double bound, Best &best, ClosestStack &st) {
+                               double bound, Best &best, Stack &st) {
   st.sp = st.lo = 0;
   auto limit = [&]() { return best.d < bound ? best.d : bound; };
   if (box_gap(bvh.root_min, bvh.root_max, p) - margin > limit()) return;
@@ -396,7 +398,320 @@ __device__ void closest_scan(const BvhView &bvh, const double *p, Best &best) {
   for (uint32_t k = 0; k < bvh.n_prims; k++) consider(best, rec_distance(recs[k], p), bvh.prim_ids[k]);
 }
 
-__global__ void k_closest_surface(ClosestViews V, const double *__restrict__ px, const double *__restrict__ py,
+// ------------------------------------------------------------------------------------------------ closest, triangles
+// The triangles of a scene with 4-wide FP32 nodes (NodeQ), one point per lane, nearest child first. A box or a triangle is
+// skipped only when an FP32 lower bound of its distance, less the error of that bound, exceeds the best distance; every
+// other triangle gets the FP64 distance, and the smallest (distance, id) does not depend on the visiting order.
+//
+// With u = 2^-24, Sm = max |p_i| + the largest |coordinate| of the boxes, and FP32 boxes rounded outward, the box gap
+// computed here exceeds the exact one by at most 9 u Sm (three differences of inputs rounded once, and their norm). For a
+// triangle and any vector w, |p - q| >= min_i (p - v_i).w / |w| over its vertices; w is taken from the centroid to p, which is
+// nearly exact for a triangle that is small against its distance, and as the plane's normal. Those dot products are within
+// 26 u Sm |w| of exact (each p - v_i within 4 u Sm per component, each dot within 3 u of its factors' norms).
+// slack = 32 u Sm covers both, and the FP64 distance's own 1e-10 Sm.
+constexpr uint32_t WIDE_RING = 16;
+constexpr uint32_t WIDE_BLOCK = 256;
+
+// The FP64 search with its stack in private memory.
+__device__ __attribute__((noinline)) void closest_exact(const BvhView &bvh, const double *leaf_vertices, const double *p,
+                                                        double margin, Best &best) {
+  struct Stack {
+    double key[64];
+    uint32_t ref[64], cnt[64];
+    int sp = 0, lo = 0;
+    __device__ bool empty() const { return sp == 0; }
+    __device__ void push(uint32_t r, uint32_t c, double k) {
+      key[sp] = k;
+      ref[sp] = r;
+      cnt[sp++] = c;
+    }
+    __device__ void pop(uint32_t &r, uint32_t &c, double &k) {
+      k = key[--sp];
+      r = ref[sp];
+      c = cnt[sp];
+    }
+  } st;
+  closest_in_bvh<TRIANGLES>(bvh, leaf_vertices, p, margin, __builtin_inf(), best, st);
+}
+
+// Whether the triangle may hold a point nearer than lim (the best distance plus slack, rounded up).
+__device__ __forceinline__ bool tri_in_reach(const TriFilt &T, const float P[3], float lim) {
+  const float u = 5.9604644775390625e-08f;
+  auto dot = [](float a0, float a1, float a2, float b0, float b1, float b2) {
+    return __builtin_fmaf(a0, b0, __builtin_fmaf(a1, b1, a2 * b2));
+  };
+  const float c0 = P[0] - T.v0[0], c1 = P[1] - T.v0[1], c2 = P[2] - T.v0[2];  // p - v0; v1 = v0 - e1, v2 = v0 + e2
+  const float k = 1.0f / 3.0f;
+  const float w0 = __builtin_fmaf(k, T.e1[0] - T.e2[0], c0), w1 = __builtin_fmaf(k, T.e1[1] - T.e2[1], c1),
+              w2 = __builtin_fmaf(k, T.e1[2] - T.e2[2], c2);
+  const float cw = dot(c0, c1, c2, w0, w1, w2);
+  const float m = fminf(cw, fminf(cw + dot(T.e1[0], T.e1[1], T.e1[2], w0, w1, w2),
+                                  cw - dot(T.e2[0], T.e2[1], T.e2[2], w0, w1, w2)));
+  const float ww = dot(w0, w1, w2, w0, w1, w2);
+  const float cn = dot(c0, c1, c2, T.n[0], T.n[1], T.n[2]);
+  const float nn = dot(T.n[0], T.n[1], T.n[2], T.n[0], T.n[1], T.n[2]);
+  const float l2 = (lim * lim) * (1.0f + 16.0f * u);
+  // products below 1e-30 may have lost digits to the denormal range: no rejection (nor on infinities and NaN)
+  return !((m > 0.0f) & (m * m > l2 * ww) & (l2 * ww > 1e-30f)) & !((cn * cn > l2 * nn) & (l2 * nn > 1e-30f));
+}
+
+__device__ __forceinline__ void order_pair(uint32_t &ka, uint32_t &ra, uint32_t &kb, uint32_t &rb) {
+  const bool sw = kb < ka;
+  const uint32_t k = ka, r = ra;
+  ka = sw ? kb : ka;
+  ra = sw ? rb : ra;
+  kb = sw ? k : kb;
+  rb = sw ? r : rb;
+}
+
+// Points whose parts several lanes search.
+struct ClosestShare {
+  double d[SHARE_SLOTS];
+  unsigned long long bound[SHARE_SLOTS];  // bits of the smallest distance any part has found (distances are >= 0)
+  uint32_t id[SHARE_SLOTS];
+  uint32_t parts[SHARE_SLOTS];  // parts still running
+};
+
+// What bounds it: 1,048,576 points in [-2,2]^3 around 1.31M triangles take 3.65 ms (6.5 with binary FP64 nodes and FP64
+// distances only, one point per thread), about 90 steps a point with a far from even spread; lines beyond L2 at 3.7 TB/s.
+// 1,000 points on 82k triangles 351 -> 130 us, 50,000 on 328k 735 -> 463 us.
+//
+// Persistent waves as in the ray traversal (or `fixed` points per wave): lanes whose point is done start the wave's next
+// ones, and once there are none, idle lanes take over stack entries of the busy ones, whose best distances they share.
+__global__ void __launch_bounds__(WIDE_BLOCK)
+k_closest_triangles(ClosestViews V, const double *__restrict__ px, const double *__restrict__ py,
+                    const double *__restrict__ pz, uint64_t n, unsigned long long *group, uint32_t fixed,
+                    double *__restrict__ dist, uint32_t *__restrict__ prim, uint32_t *__restrict__ geom) {
+  using u32x4 = unsigned int __attribute__((ext_vector_type(4)));
+  using Bytes = const __attribute__((address_space(1))) unsigned char;
+  typedef u32x4 __attribute__((aligned(8))) Chunk;  // the vertices are 72-byte records
+  using GlobalChunk = const __attribute__((address_space(1))) Chunk;
+  __shared__ uint64_t ring[WIDE_RING * WIDE_BLOCK];
+  __shared__ ClosestShare shares[WIDE_BLOCK / 64];
+  const BvhView &bvh = V.view[TRIANGLES];
+  const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  BRT_LDS volatile ClosestShare *sh = (BRT_LDS volatile ClosestShare *)&shares[wave];
+  uint64_t spill[WIDE_SPILL];
+  WideStack st;
+  st.ring = (BRT_LDS uint32_t *)ring + (size_t)wave * WIDE_RING * 128 + lane;
+  st.spill = spill;
+  st.mask = (int)WIDE_RING - 1;
+  st.reset();
+  WavePool pool;
+  if (fixed) pool.take_fixed(((uint64_t)blockIdx.x * (WIDE_BLOCK / 64) + wave) * fixed, fixed, n);
+  bool exhausted = false;  // wave-uniform
+  uint64_t i = 0;
+  double p[3] = {0.0, 0.0, 0.0};
+  float P[3] = {0.0f, 0.0f, 0.0f}, slack = 0.0f;
+  float lim = 0.0f;  // best distance + slack, rounded up
+  Best best{__builtin_inf(), INVALID_ID};
+  uint32_t cur = 0, cnt = 0, cand = 0;
+  bool busy = false, shared = false;
+  uint32_t slot = 0, slots = 0, turn = 0;
+  for (;;) {
+    const unsigned long long working = __ballot(busy);
+    const uint32_t nidle = 64u - (uint32_t)__popcll(working);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    if (!exhausted) {
+      if (nidle >= 16u) {
+        bool got;
+        pool_refill(pool, group + COUNTER_POOL, n, POOL_CHUNK, ~working, nidle, lane, got, i, exhausted);
+        if (got) {
+          p[0] = px[i];
+          p[1] = py[i];
+          p[2] = pz[i];
+          const double pm = fmax(fabs(p[0]), fmax(fabs(p[1]), fabs(p[2])));
+          best = Best{__builtin_inf(), INVALID_ID};
+          if (pm <= FILTER_MAX_EXTENT && p[0] == p[0] && p[1] == p[1] && p[2] == p[2]) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) P[k] = (float)p[k];
+            slack = f32_up(32.0 * 0x1p-24 * (pm + V.extent[TRIANGLES]));
+            lim = __builtin_inff();
+            cur = bvh.root_ref4;
+            cnt = bvh.root_cnt;
+            cand = 0;
+            busy = true;
+            st.reset();
+          } else {
+            // a point outside the FP32 bounds' range, or not a number: the FP64 search
+            closest_exact(bvh, V.leaf_vertices, p, 1e-10 * (pm + V.extent[TRIANGLES]), best);
+            const bool found = best.d < __builtin_inf();
+            dist[i] = found ? best.d : __builtin_inf();
+            prim[i] = found ? best.id : INVALID_ID;
+            geom[i] = found ? bvh.geom_id : INVALID_ID;
+          }
+        }
+      }
+    } else {
+      if (!working) break;
+      const unsigned long long can = __ballot(busy && st.sp > st.bot);
+            if (nidle >= SHARE_MIN_IDLE && can && (++turn & 1u) == 0u) {
+        const uint32_t ncan = (uint32_t)__popcll(can), k = nidle < ncan ? nidle : ncan;
+        const uint32_t rank = (uint32_t)__popcll((busy ? can : ~working) & below);
+        const bool donor = ((can >> lane) & 1ull) && rank < k, helper = !busy && rank < k;
+        const unsigned long long fresh = __ballot(donor && !shared);
+        uint64_t e = 0;
+        if (donor) {
+          const WideEntry t = st.pop();  // the nearest entry: the bottom one would mostly be out of reach in the end
+          e = ((uint64_t)t.key << 32) | t.ref;
+          if (!shared) {
+            shared = true;
+            slot = slots + (uint32_t)__popcll(fresh & below);
+            sh->d[slot] = __builtin_inf();
+            sh->bound[slot] = (unsigned long long)__double_as_longlong(best.d);
+            sh->id[slot] = INVALID_ID;
+            sh->parts[slot] = 1u;
+          }
+        }
+        slots += (uint32_t)__popcll(fresh);
+        wave_fence();
+        if (donor) atomicAdd(&shares[wave].parts[slot], 1u);
+        // the r-th helper takes from the r-th donor, whose lane number lane r receives (at most 32 donors: lane 63 takes
+        // what the others push); both permutes with all lanes, since they serve active lanes only
+        const uint32_t by_rank = (uint32_t)__builtin_amdgcn_ds_permute((donor ? (int)rank : 63) << 2, (int)lane);
+        const uint32_t from = lane_get(by_rank, (int)rank);
+        const int src = helper ? (int)from : (int)lane;
+        lane_take(e, src, helper);
+        lane_take(p, src, helper);
+        lane_take(P, src, helper);
+        lane_take(slack, src, helper);
+        lane_take(lim, src, helper);
+        lane_take(slot, src, helper);
+        lane_take(i, src, helper);
+        if (helper) {
+          busy = shared = true;
+          best = Best{__builtin_inf(), INVALID_ID};
+          cur = (uint32_t)e;
+          cnt = (uint32_t)(e >> 32) & 255u;
+          cand = 0;
+          st.reset();
+        }
+        wave_fence();
+      }
+    }
+    bool fin = false;
+    if (busy) {
+      if (shared) {
+        const double d = __longlong_as_double((long long)sh->bound[slot]);
+        lim = fminf(lim, f32_up((double)f32_up(d) + (double)slack));
+      }
+      // one unit per iteration, as in the ray traversal: a node, a pre-test of two triangles or an FP64 distance
+      const bool at_leaf = (cur & LEAF_BIT) != 0, test = cand != 0u;
+      const uint32_t first = cur & ~LEAF_BIT;
+      const uint32_t q = first + (uint32_t)__builtin_ctz(cand | 0x80000000u);
+      Bytes *base = !at_leaf ? (Bytes *)(bvh.nodesq + cur)
+                    : test   ? (Bytes *)(V.leaf_vertices + 9ull * q)
+                             : (Bytes *)(bvh.tri_filter + first);
+      u32x4 c[8];
+#pragma unroll
+      for (int k = 0; k < 4; k++) c[k] = *(GlobalChunk *)(base + 16 * k);
+      if (!test) {
+#pragma unroll
+        for (int k = 4; k < 8; k++) c[k] = *(GlobalChunk *)(base + 16 * k);
+      } else {
+        const __attribute__((address_space(1))) uint32_t *w = (const __attribute__((address_space(1))) uint32_t *)(base + 64);
+        c[4][0] = w[0];
+        c[4][1] = w[1];
+      }
+#pragma unroll
+      for (int k = 0; k < 8; k++) asm volatile("" : "+v"(c[k]));
+      bool pop = true;
+      if (!at_leaf) {
+        const float l2 = (lim * lim) * (1.0f + 0x1p-20f);
+        uint32_t key[4], ref[4];
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+          float g2 = 0.0f;
+#pragma unroll
+          for (int a = 0; a < 3; a++) {
+            const float g = fmaxf(fmaxf(__uint_as_float(c[a][s]) - P[a], P[a] - __uint_as_float(c[4 + a][s])), 0.0f);
+            g2 = __builtin_fmaf(g, g, g2);
+          }
+          // (an unused slot's inverted box is infinitely far)
+          const bool in = g2 <= l2 && g2 < __builtin_inff();
+          key[s] = in ? __builtin_amdgcn_perm(__float_as_uint(g2), c[7][2], 0x07060500u | (uint32_t)s) : 0xFFFFFFFFu;
+          ref[s] = c[3][s];
+        }
+        order_pair(key[0], ref[0], key[1], ref[1]);
+        order_pair(key[2], ref[2], key[3], ref[3]);
+        order_pair(key[0], ref[0], key[2], ref[2]);
+        order_pair(key[1], ref[1], key[3], ref[3]);
+        order_pair(key[1], ref[1], key[2], ref[2]);
+        if (key[0] != 0xFFFFFFFFu) {
+          st.room(3);
+#pragma unroll
+          for (int s = 3; s > 0; s--)
+            if (key[s] != 0xFFFFFFFFu) st.put(st.sp++, ref[s], key[s]);
+          cur = ref[0];
+          cnt = key[0] & 255u;
+          pop = false;
+        }
+      } else if (!test) {
+        TriFilt g[2];
+        __builtin_memcpy(g, c, sizeof g);
+        cand = (tri_in_reach(g[0], P, lim) ? 1u : 0u) | (tri_in_reach(g[1], P, lim) && cnt > 1u ? 2u : 0u);
+        pop = cand == 0u;
+      } else {
+        double v[9];
+        __builtin_memcpy(v, c, sizeof v);
+        const double d = triangle_distance(v, v + 3, v + 6, p);
+        if (d <= best.d) {
+          consider(best, d, bvh.prim_ids[q]);
+          lim = fminf(lim, f32_up((double)f32_up(best.d) + (double)slack));
+          if (shared) atomicMin(&shares[wave].bound[slot], (unsigned long long)__double_as_longlong(best.d));
+        }
+        cand &= cand - 1u;
+        pop = cand == 0u;
+      }
+      if (pop) {
+        if (at_leaf && cnt > 2u) {
+          cnt -= 2u;
+          cur += 2u;
+        } else {
+          const float l2 = (lim * lim) * (1.0f + 0x1p-20f);
+          fin = true;
+          while (st.sp > st.bot) {
+            const WideEntry e = st.pop();
+            if (!(__uint_as_float(e.key & ~255u) > l2)) {
+              cur = e.ref;
+              cnt = e.key & 255u;
+              fin = false;
+              break;
+            }
+          }
+        }
+      }
+    }
+    if (exhausted) {
+      // the parts of a shared point are merged one lane at a time; the last one writes it
+      unsigned long long m = __ballot(fin && shared);
+      while (m) {
+        const uint32_t l = (uint32_t)__ffsll((long long)m) - 1u;
+        m &= m - 1ull;
+        if (lane == l) {
+          consider(best, sh->d[slot], sh->id[slot]);
+          sh->d[slot] = best.d;
+          sh->id[slot] = best.id;
+          const uint32_t parts = sh->parts[slot] - 1u;
+          sh->parts[slot] = parts;
+          busy = shared = false;
+          fin = parts == 0u;
+        }
+        wave_fence();
+      }
+    }
+    if (fin) {
+      busy = false;
+      const bool found = best.d < __builtin_inf();
+      dist[i] = found ? best.d : __builtin_inf();
+      prim[i] = found ? best.id : INVALID_ID;
+      geom[i] = found ? bvh.geom_id : INVALID_ID;
+    }
+  }
+}
+
+// `from`: the geometry types before it are done, their result is in the output arrays.
+__global__ void k_closest_surface(ClosestViews V, int from, const double *__restrict__ px, const double *__restrict__ py,
                                   const double *__restrict__ pz, uint64_t n, double *__restrict__ dist,
                                   uint32_t *__restrict__ prim, uint32_t *__restrict__ geom) {
   __shared__ double lkey[CLOSEST_RING * CLOSEST_BLOCK];
@@ -410,7 +725,12 @@ __global__ void k_closest_surface(ClosestViews V, const double *__restrict__ px,
   const double pm = fmax(fabs(p[0]), fmax(fabs(p[1]), fabs(p[2])));
   double gd = __builtin_inf();
   uint32_t gp = INVALID_ID, gg = INVALID_ID;
-  for (int t = 0; t < NUM_TYPES; t++) {
+  if (from) {
+    gd = dist[i];
+    gp = prim[i];
+    gg = geom[i];
+  }
+  for (int t = from; t < NUM_TYPES; t++) {
     const BvhView &bvh = V.view[t];
     if (!V.present[t] || bvh.n_prims == 0) continue;
     Best b{__builtin_inf(), INVALID_ID};
@@ -464,10 +784,35 @@ hipError_t launch_distance_pairs(GeomType type, const BvhView &bvh, const uint32
 }
 
 hipError_t launch_closest_surface(const ClosestViews &views, const double *px, const double *py, const double *pz,
-                                  uint64_t n, double *dist, uint32_t *prim, uint32_t *geom, hipStream_t stream) {
+                                  uint64_t n, double *dist, uint32_t *prim, uint32_t *geom, unsigned long long *group,
+                                  hipStream_t stream) {
   if (n == 0) return hipSuccess;
+  int from = 0;
+  const BvhView &tri = views.view[TRIANGLES];
+  if (views.present[TRIANGLES] && tri.nodesq && tri.tri_filter) {
+    if (!group) return hipErrorInvalidValue;
+    int dev = 0, cus = 0, per_cu = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e == hipSuccess)
+      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_closest_triangles, WIDE_BLOCK, 0);
+    if (e == hipSuccess) e = launch_zero_counters(group, stream);
+    if (e != hipSuccess) return e;
+    constexpr uint32_t waves = WIDE_BLOCK / 64;
+    uint64_t blocks = (uint64_t)(cus > 0 ? cus : 1) * (uint64_t)(per_cu > 0 ? per_cu : 1);
+    const uint32_t fixed = fixed_per_wave(n, blocks * waves);
+    const uint64_t need = fixed ? (n + fixed * waves - 1) / (fixed * waves) : (n + WIDE_BLOCK - 1) / WIDE_BLOCK;
+    if (blocks > need) blocks = need;
+    k_closest_triangles<<<(uint32_t)blocks, WIDE_BLOCK, 0, stream>>>(views, px, py, pz, n, group, fixed, dist, prim, geom);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    from = TRIANGLES + 1;
+    bool more = false;
+    for (int t = from; t < NUM_TYPES; t++) more = more || views.present[t];
+    if (!more) return hipSuccess;
+  }
   k_closest_surface<<<(uint32_t)((n + CLOSEST_BLOCK - 1) / CLOSEST_BLOCK), CLOSEST_BLOCK, 0, stream>>>(
-      views, px, py, pz, n, dist, prim, geom);
+      views, from, px, py, pz, n, dist, prim, geom);
   return hipGetLastError();
 }
 

@@ -162,6 +162,9 @@ hipError_t launch_cyl_filter_records(const void *recs, uint32_t n, void *out, hi
 // record, visit_order4).
 hipError_t launch_nodeq_records(const Node4 *nodes4, const uint32_t *ord, uint32_t n, NodeQ *out, hipStream_t stream);
 
+// Clears the counters of a group on the stream.
+hipError_t launch_zero_counters(unsigned long long *group, hipStream_t stream);
+
 // Enqueues the traversal of one geometry type over n rays on `stream` (asynchronous).
 hipError_t launch_trace(GeomType type, const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint64_t n,
                         const TraceLaunch &cfg, const SplitParams &split, hipStream_t stream);
@@ -211,8 +214,10 @@ struct ClosestViews {
 // Gathers the triangles' vertices in leaf order (9 doubles per triangle) for the closest-surface query.
 hipError_t launch_leaf_vertices(const uint32_t *order, const uint32_t *faces, const double *vertices, uint32_t n,
                                 double *out, hipStream_t stream);
+// group: the stream's launch counters (used for triangles).
 hipError_t launch_closest_surface(const ClosestViews &views, const double *px, const double *py, const double *pz,
-                                  uint64_t n, double *dist, uint32_t *prim, uint32_t *geom, hipStream_t stream);
+                                  uint64_t n, double *dist, uint32_t *prim, uint32_t *geom, unsigned long long *group,
+                                  hipStream_t stream);
 
 // Device build of one geometry type's BVH (build.hip): the host builder's tree, primitive order and flattened
 // records, bit for bit, provided no primitive box coordinate is NaN or -0.0 (the caller checks) and

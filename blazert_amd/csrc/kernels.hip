@@ -23,6 +23,7 @@
 #include "../../include/blazert_amd/device/exact.h"
 #include "engine.h"
 #include "f32_round.h"
+#include "wave.h"
 
 namespace brt {
 
@@ -664,10 +665,6 @@ constexpr uint32_t block_default() { return (!SPLIT && std::is_same<Rec, SphRec>
 template <bool SPLIT, class R>
 using StackKey = typename std::conditional<SPLIT, float, R>::type;
 
-// LDS pointers of the ring stack carry the LDS address space explicitly: as generic pointers the compiler had to
-// resolve their address space at run time in places (flat accesses), which costs time on the coherent sets.
-#define BRT_LDS __attribute__((address_space(3)))
-
 template <bool SPLIT, class R = double>
 struct SpillArea {  // private (scratch) memory for entries pushed deeper than the ring
   using Key = StackKey<SPLIT, R>;
@@ -1129,67 +1126,6 @@ __global__ void __launch_bounds__(256) k_trace(BvhView bvh, RaysViewT<typename R
   }
 }
 
-// Persistent waves: every lane owns one ray at a time; when at least `refill` lanes of a wave are idle, they start
-// the next indices of the wave's pool. Skewed per-ray work (many rays miss the root box, a few visit hundreds of
-// nodes) then no longer idles the wave until its slowest ray ends. The pool is a chunk of `chunk` consecutive indices
-// (POOL_CHUNK unless the launch asks for 32 or 128) claimed with one atomic add. Claims on one address serialise
-// across the GPU (about 14 ns each), which bounded short launches and image-order rays, so they are spread over
-// CLAIM_COUNTERS counters on separate 128-byte lines: counter k hands out chunks k, k + CLAIM_COUNTERS,
-// k + 2 CLAIM_COUNTERS, ... A wave starts at the counter of its block (block index mod CLAIM_COUNTERS: blocks are
-// dealt to the eight XCDs in turn, so each XCD's waves start at a counter of their own) and moves on to the next
-// counter once one has passed n. When all have, the pool is exhausted; every lane leaves the loop once its pool is
-// exhausted and its own ray is done, so the grid always drains.
-constexpr uint32_t POOL_CHUNK = 64;
-
-// Wave-uniform pool of claimed, not yet started ray indices [next, end).
-struct WavePool {
-  uint64_t next = 0, end = 0;
-  bool last = false;  // every counter has passed n
-};
-
-// Called by every lane of a wave with the same pool state when the wave refills. An idle lane handed an index gets
-// it in `idx` and `got`; `exhausted` is set once nothing is left to hand out. `counter` is the first of the
-// launch's CLAIM_COUNTERS counters (COUNTER_STRIDE slots apart).
-__device__ __forceinline__ void pool_refill(WavePool &P, unsigned long long *counter, uint64_t n, uint32_t chunk,
-                                            unsigned long long idle, uint32_t nidle, uint32_t lane, bool &got,
-                                            uint64_t &idx, bool &exhausted) {
-  got = false;
-  if (P.next == P.end && !P.last) {
-    unsigned long long base = n;
-    const uint32_t leader = (uint32_t)__ffsll((long long)idle) - 1u;
-    if (lane == leader) {
-      const uint32_t home = blockIdx.x % (uint32_t)CLAIM_COUNTERS;
-      for (uint32_t a = 0; a < (uint32_t)CLAIM_COUNTERS; a++) {
-        const uint32_t k = (home + a) % (uint32_t)CLAIM_COUNTERS;
-        const unsigned long long c = atomicAdd(counter + k * COUNTER_STRIDE, 1ull);
-        const unsigned long long start = (c * CLAIM_COUNTERS + k) * chunk;
-        if (start < n) {
-          base = start;
-          break;
-        }
-      }
-    }
-    const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)base, (int)leader);
-    const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(base >> 32), (int)leader);
-    base = ((unsigned long long)hi << 32) | lo;
-    if (base >= n) {
-      P.last = true;
-      P.next = P.end = n;
-    } else {
-      P.next = base;
-      P.end = base + chunk < n ? base + chunk : n;
-    }
-  }
-  const uint64_t avail = P.end - P.next;
-  const uint32_t take = avail < nidle ? (uint32_t)avail : nidle;
-  const uint32_t rank = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-  if (((idle >> lane) & 1ull) && rank < take) {
-    idx = P.next + rank;
-    got = true;
-  }
-  P.next += take;
-  if (P.last && P.next == P.end) exhausted = true;
-}
 // Occupancy target of the persistent kernels (waves per SIMD the register allocation must allow).
 #ifndef BRT_WAVES_PER_EU
 #define BRT_WAVES_PER_EU 4
@@ -1544,58 +1480,6 @@ __device__ __forceinline__ float min3_nn(float a, float b, float c) {
   return r;
 }
 
-// One entry: a node or leaf reference, and its entry distance with the low 8 bits (rounded towards 0; keys are not
-// negative) replaced by the leaf's primitive count.
-struct TriEntry {
-  uint32_t ref, key;
-};
-constexpr uint32_t TRI_SPILL = 192;  // three entries per level, at most 63 levels (stack_cap)
-
-// The lane's stack: entries [bot, sp), of which [lo, sp) lie in the LDS ring and the older ones in private memory.
-// Entries below bot have been given away.
-struct TriStack {
-  BRT_LDS uint32_t *ring;  // the lane's slot 0; slot i: reference at [128 i], key at [128 i + 64]
-  uint64_t *spill;
-  int sp, lo, bot;
-  int mask;  // ring slots - 1
-
-  __device__ __forceinline__ void reset() { sp = lo = bot = 0; }
-  __device__ __forceinline__ void room(int n) {  // n more entries fit the ring
-    while (sp + n - lo > mask + 1) {
-      spill[lo] = slot(lo);
-      lo++;
-    }
-  }
-  __device__ __forceinline__ void put(int i, uint32_t ref, uint32_t key) {
-    BRT_LDS uint32_t *e = ring + (i & mask) * 128;
-    e[0] = ref;
-    e[64] = key;
-  }
-  __device__ __forceinline__ uint64_t slot(int i) const {
-    BRT_LDS uint32_t *e = ring + (i & mask) * 128;
-    return ((uint64_t)e[64] << 32) | e[0];
-  }
-  __device__ __forceinline__ TriEntry pop() {  // requires sp > bot
-    sp--;
-    uint64_t e;
-    if (sp < lo) {
-      lo = sp;
-      e = spill[sp];
-    } else {
-      e = slot(sp);
-    }
-    return TriEntry{(uint32_t)e, (uint32_t)(e >> 32)};
-  }
-  __device__ __forceinline__ uint64_t take_bottom() {  // requires sp > bot
-    uint64_t e;
-    if (bot < lo) e = spill[bot];
-    else e = slot(bot);
-    bot++;
-    lo = lo < bot ? bot : lo;
-    return e;
-  }
-};
-
 struct TriTrees {
   const NodeQ *nodes;
   const TriFilt *filt;
@@ -1614,7 +1498,7 @@ struct TriTrav {
 // One unit of the traversal: an internal node, the pre-test of a leaf's next FILTER_GROUP triangles, or the FP64 test of
 // one that passed. As in trav_step, every lane fetches its record by the same instructions and waits once.
 __device__ __forceinline__ void tri_step(const TriTrees &T, const Ray &r, const RayQ &q, Hit &s, TriTrav &t,
-                                         TriStack &st) {
+                                         WideStack &st) {
   using u32x4 = unsigned int __attribute__((ext_vector_type(4)));
   using Bytes = const __attribute__((address_space(1))) unsigned char;
   using GlobalChunk = const __attribute__((address_space(1))) u32x4;
@@ -1722,7 +1606,7 @@ __device__ __forceinline__ void tri_step(const TriTrees &T, const Ray &r, const 
     }
   }
   while (st.sp > st.bot) {
-    const TriEntry e = st.pop();
+    const WideEntry e = st.pop();
     if (!(t.h32 < __uint_as_float(e.key & ~255u))) {
       t.cur = e.ref;
       t.cnt = e.key & 255u;
@@ -1759,33 +1643,7 @@ __device__ __forceinline__ void tri_begin(const TriRoot &root, const Ray &r, con
   t.active = A <= M;
 }
 
-// A value of another lane, for the lanes that take over its work.
-__device__ __forceinline__ uint32_t lane_get(uint32_t x, int src) {
-  return (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)x);
-}
-template <class V>
-__device__ __forceinline__ void lane_take(V &x, int src, bool take) {
-  static_assert(sizeof(V) % 4 == 0, "words");
-  uint32_t w[sizeof(V) / 4];
-  __builtin_memcpy(w, &x, sizeof(V));
-#pragma unroll
-  for (size_t k = 0; k < sizeof(V) / 4; k++) {
-    const uint32_t y = lane_get(w[k], src);
-    w[k] = take ? y : w[k];
-  }
-  __builtin_memcpy(&x, w, sizeof(V));
-}
-__device__ __forceinline__ void wave_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Rays whose parts several lanes trace. Sharing starts with at least SHARE_MIN_IDLE idle lanes and no rays left to
-// start, so at most SHARE_SLOTS rays of a wave are ever shared.
-constexpr uint32_t SHARE_MIN_IDLE = 32;
-constexpr uint32_t SHARE_SLOTS = 32;
-static_assert(64u - SHARE_MIN_IDLE <= SHARE_SLOTS, "a slot for every ray left");
+// Rays whose parts several lanes trace.
 struct TriShare {
   double h[SHARE_SLOTS], u[SHARE_SLOTS], v[SHARE_SLOTS];
   uint32_t prim[SHARE_SLOTS];
@@ -1832,8 +1690,8 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
   }
   const uint32_t lane = __lane_id(), wave = threadIdx.x / 64;
   BRT_LDS volatile TriShare *sh = (BRT_LDS volatile TriShare *)&shares[wave];
-  uint64_t spill[TRI_SPILL];
-  TriStack st;
+  uint64_t spill[WIDE_SPILL];
+  WideStack st;
   st.ring = (BRT_LDS uint32_t *)smem + (size_t)wave * ring * 128 + lane;
   st.spill = spill;
   st.mask = (int)ring - 1;
@@ -1890,12 +1748,8 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
     }
   };
   WavePool pool;
-  if (fixed) {  // a small launch: `fixed` rays per wave, no claims, and the other lanes help from the start
-    const uint64_t w = (uint64_t)blockIdx.x * (blockDim.x / 64) + wave;
-    pool.next = w * fixed < n ? w * fixed : n;
-    pool.end = pool.next + fixed < n ? pool.next + fixed : n;
-    pool.last = true;
-  }
+  if (fixed)  // a small launch: no claims, and the other lanes help from the start
+    pool.take_fixed(((uint64_t)blockIdx.x * (blockDim.x / 64) + wave) * fixed, fixed, n);
   uint32_t turn = 0;
   for (;;) {
     if (!exhausted) {
@@ -2307,16 +2161,6 @@ hipError_t launch_kernel(const BvhView &bvh, const RaysViewT<typename Rec::real>
   return hipGetLastError();
 }
 
-// Rays per wave of a launch that the device's `waves` resident waves take in one go (up to a full wave each; 262,144 on
-// 256 CUs): the waves then have idle lanes from the start, which share their rays' work, and none waits for a claim.
-// 0 for larger launches, whose waves claim. Incoherent rays, 82k-triangle mesh: 2,000 rays 123 -> 74 us against claims
-// of 64; 328k-triangle mesh: 50,000 rays 265 -> 202 us, 200,000 rays 375 -> 324 us; a 200x150 camera 394 -> 250 us.
-constexpr uint64_t FIXED_RAYS = 64;
-uint32_t fixed_rays(uint64_t n, uint64_t waves) {
-  const uint64_t per = (n + waves - 1) / waves;
-  return per <= FIXED_RAYS ? (uint32_t)per : 0u;
-}
-
 // The fast triangle traversal (k_trace_tri) takes closest-hit launches on the persistent schedule, in either precision:
 // 1.31M-triangle mesh, 4,194,304 incoherent rays 3.03 ms, against 5.6-5.8 ms for the exact FP64 kernel and 3.8 ms for
 // nearest-first split precision; a 1920x1080 camera with normals 2.24 against 3.57 ms. Any-hit launches return the first
@@ -2340,7 +2184,7 @@ hipError_t launch_tri(const BvhView &bvh, const RaysView &rays, const HitsView &
   uint64_t blocks = 0;
   hipError_t e = persistent_blocks(k_trace_tri<false>, block, lds, n * 64, blocks);
   if (e != hipSuccess) return e;
-  const uint32_t wpb = block / 64, fixed = fixed_rays(n, blocks * wpb);
+  const uint32_t wpb = block / 64, fixed = fixed_per_wave(n, blocks * wpb);
   const uint64_t need = fixed ? (n + fixed * wpb - 1) / (fixed * wpb) : (n + block - 1) / block;
   if (blocks > need) blocks = need;
   hipLaunchKernelGGL(k_trace_tri<false>, dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits,
@@ -2370,7 +2214,7 @@ hipError_t launch_tri_batch(const BatchJob *jobs, uint32_t njobs, uint64_t total
   uint64_t blocks = 0;
   hipError_t e = persistent_blocks(k_trace_tri<true>, block, lds, total * 64, blocks);
   if (e != hipSuccess) return e;
-  const uint32_t wpb = block / 64, fixed = fixed_rays(total, blocks * wpb);
+  const uint32_t wpb = block / 64, fixed = fixed_per_wave(total, blocks * wpb);
   const uint64_t need = fixed ? (total + fixed * wpb - 1) / (fixed * wpb) : (total + block - 1) / block;
   if (blocks > need) blocks = need;
   hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
@@ -2453,6 +2297,11 @@ hipError_t launch_cyl_filter_records(const void *recs, uint32_t n, void *out, hi
   if (blocks > 65536) blocks = 65536;
   hipLaunchKernelGGL(k_cyl_filter_records, dim3(blocks), dim3(256), 0, stream, static_cast<const CylRec *>(recs), n,
                      static_cast<SphFilt *>(out), total);
+  return hipGetLastError();
+}
+
+hipError_t launch_zero_counters(unsigned long long *group, hipStream_t stream) {
+  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, group);
   return hipGetLastError();
 }
 

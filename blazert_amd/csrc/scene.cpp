@@ -1539,7 +1539,9 @@ int brt_closest_surface(const brt_scene *cs, const brt_points *points, uint64_t 
     }
     cv.leaf_vertices = s->dev->leaf_vertices;
   }
-  hipError_t e = launch_closest_surface(cv, points->x, points->y, points->z, n, distance, prim_id, geom_id,
+  unsigned long long *group = s->dev->counter_group(static_cast<hipStream_t>(stream));
+  if (!group) return fail(BRT_ERR_OUT_OF_MEMORY, "launch counters");
+  hipError_t e = launch_closest_surface(cv, points->x, points->y, points->z, n, distance, prim_id, geom_id, group,
                                         static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return device_error(e, "launch failed");
   return BRT_OK;
