@@ -160,13 +160,27 @@ __device__ __forceinline__ uint32_t block_rank(bool flag, uint32_t *wave_tot, ui
 }
 
 // ------------------------------------------------------------------------------------------------ inputs
-// Triangle boxes and centers exactly as the host collection precompute (blazert/primitives/trimesh.h:78-130).
+// What the triangles' inputs mean for the device build.
+struct MeshFlags {
+  uint32_t refused;   // some box coordinate is not finite or is -0.0: the order-free reductions would not be exact
+  uint32_t max_fan;   // most corners at one vertex of a long fan; 2^32 - 1 when some face normal is NaN
+  uint32_t num_long;  // vertices of more than FAN_SHORT corners
+};
+constexpr uint32_t FAN_SHORT = 64;    // corners one thread sums
+constexpr uint32_t FAN_LONG = 4096;   // corners one block sums; beyond, the host computes the normals
+
+// Triangle boxes and centers exactly as the host collection precompute (blazert/primitives/trimesh.h:78-130), each face's
+// share of its vertices' normals, normalize(cross(v1 - v0, v2 - v0)) / 3, and the number of corners at every vertex.
 __global__ void k_tri_boxes(const double *__restrict__ V, const uint32_t *__restrict__ F, uint32_t n,
-                            double *__restrict__ lo, double *__restrict__ hi, double *__restrict__ ctr) {
+                            double *__restrict__ lo, double *__restrict__ hi, double *__restrict__ ctr,
+                            double *__restrict__ fn3, uint32_t *__restrict__ fan, MeshFlags *__restrict__ flags) {
   const uint32_t f = blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= n) return;
-  const double *v0 = V + 3ull * F[3ull * f], *v1 = V + 3ull * F[3ull * f + 1], *v2 = V + 3ull * F[3ull * f + 2];
+  const uint32_t i0 = F[3ull * f], i1 = F[3ull * f + 1], i2 = F[3ull * f + 2];
+  const double *v0 = V + 3ull * i0, *v1 = V + 3ull * i1, *v2 = V + 3ull * i2;
   const double third = 1.0 / 3.0;
+  bool odd = false;
+  double a[3], b[3];
   for (int k = 0; k < 3; k++) {
     double l = v0[k], h = v0[k];
     l = (l < v1[k]) ? l : v1[k];
@@ -176,6 +190,93 @@ __global__ void k_tri_boxes(const double *__restrict__ V, const uint32_t *__rest
     lo[3ull * f + k] = l;
     hi[3ull * f + k] = h;
     ctr[3ull * f + k] = ((v0[k] + v1[k]) + v2[k]) * third;
+    const u64 neg0 = 0x8000000000000000ull;
+    odd = odd || !(fabs(l) <= DBL_MAX) || !(fabs(h) <= DBL_MAX) || (u64)__double_as_longlong(l) == neg0 ||
+          (u64)__double_as_longlong(h) == neg0;
+    a[k] = v1[k] - v0[k];
+    b[k] = v2[k] - v0[k];
+  }
+  if (odd) flags->refused = 1u;
+  const double c[3] = {a[1] * b[2] - a[2] * b[1], a[2] * b[0] - a[0] * b[2], a[0] * b[1] - a[1] * b[0]};
+  const double len = __builtin_sqrt(c[0] * c[0] + c[1] * c[1] + c[2] * c[2]);
+  const double il = (len != 0.0) ? 1.0 / len : 0.0;
+  bool nan = false;
+  for (int k = 0; k < 3; k++) {
+    const double x = (c[k] * il) * third;
+    fn3[3ull * f + k] = x;
+    nan = nan || x != x;
+  }
+  if (nan) flags->max_fan = 0xFFFFFFFFu;  // a NaN's sign and payload are the host's to choose
+  atomicAdd(&fan[i0], 1u);
+  atomicAdd(&fan[i1], 1u);
+  atomicAdd(&fan[i2], 1u);
+}
+
+__global__ void k_zero_words(uint32_t *p, uint64_t n) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0u;
+}
+
+// Corner c = 3 face + k goes to one of its vertex's places [start[v], start[v] + fan[v]), in no particular order;
+// `left` starts as the fans and counts down.
+__global__ void k_corners(const uint32_t *__restrict__ F, uint32_t corners, const uint32_t *__restrict__ start,
+                          uint32_t *__restrict__ left, uint32_t *__restrict__ at) {
+  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= corners) return;
+  const uint32_t v = F[c];
+  at[start[v] + atomicSub(&left[v], 1u) - 1u] = c;
+}
+
+// Vertex normals as the host sums them (trimesh.h:91-93): every corner's share in ascending corner order. A short fan is
+// summed by one thread, which looks for the next larger corner each time (six of them as a rule); long ones are listed.
+__global__ void k_vertex_normals(const uint32_t *__restrict__ start, const uint32_t *__restrict__ ends, uint32_t nv,
+                                 const uint32_t *__restrict__ at, const double *__restrict__ fn3,
+                                 double *__restrict__ out, uint32_t *__restrict__ longs, MeshFlags *__restrict__ flags) {
+  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= nv) return;
+  const uint32_t b = start[v], m = ends[v] - b;
+  if (m > FAN_SHORT) {
+    longs[atomicAdd(&flags->num_long, 1u)] = v;
+    atomicMax(&flags->max_fan, m);  // (after k_tri_boxes: a NaN's mark stays)
+    return;
+  }
+  double s[3] = {0.0, 0.0, 0.0};
+  uint32_t from = 0;
+  for (uint32_t k = 0; k < m; k++) {
+    uint32_t c = 0xFFFFFFFFu;
+    for (uint32_t j = 0; j < m; j++) {
+      const uint32_t x = at[b + j];
+      c = (x >= from && x < c) ? x : c;
+    }
+    const double *f = fn3 + 3ull * (c / 3u);
+    for (int a = 0; a < 3; a++) s[a] = s[a] + f[a];
+    from = c + 1u;
+  }
+  for (int a = 0; a < 3; a++) out[3ull * v + a] = s[a];
+}
+
+// Long fans, one block each: every corner's rank by counting, then the sum in order.
+__global__ void k_vertex_normals_long(const uint32_t *__restrict__ start, const uint32_t *__restrict__ ends,
+                                      const uint32_t *__restrict__ at, const double *__restrict__ fn3,
+                                      const uint32_t *__restrict__ longs, const MeshFlags *__restrict__ flags,
+                                      double *__restrict__ out) {
+  __shared__ uint32_t sorted[FAN_LONG];
+  for (uint32_t l = blockIdx.x; l < flags->num_long; l += gridDim.x) {
+    const uint32_t v = longs[l], b = start[v], m = ends[v] - b;
+    if (m > FAN_LONG) continue;
+    for (uint32_t i = threadIdx.x; i < m; i += blockDim.x) {
+      const uint32_t x = at[b + i];
+      uint32_t rank = 0;
+      for (uint32_t j = 0; j < m; j++) rank += at[b + j] < x ? 1u : 0u;
+      sorted[rank] = x;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+      double s = 0.0;
+      for (uint32_t i = 0; i < m; i++) s = s + fn3[3ull * (sorted[i] / 3u) + threadIdx.x];
+      out[3ull * v + threadIdx.x] = s;
+    }
+    __syncthreads();
   }
 }
 
@@ -934,8 +1035,31 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
   double *lo = A.get<double>(3ull * n), *hi = A.get<double>(3ull * n), *ctr = A.get<double>(3ull * n);
   uint32_t *idx = A.get<uint32_t>(n), *pos_r = A.get<uint32_t>(n);
   BRT_CHECK(A.err);
+  MeshFlags *d_flags = nullptr, hflags{};
+  double *vnormals = nullptr;
   if (in.type == TRIANGLES) {
-    BRT_LAUNCH(k_tri_boxes<<<blocks_for(n, 256), 256, 0, st>>>(in.vertices, in.faces, n, lo, hi, ctr));
+    const uint32_t nv = in.num_vertices, corners = 3u * n;
+    double *fn3 = A.get<double>(3ull * n);
+    // fans and their running ends (the scan's extra element), corner places, the list of long fans
+    uint32_t *fan = A.get<uint32_t>(nv + 1ull), *start = A.get<uint32_t>(nv + 1ull), *at = A.get<uint32_t>(corners);
+    uint32_t *longs = A.get<uint32_t>(corners / FAN_SHORT + 1);
+    d_flags = A.get<MeshFlags>(1);
+    vnormals = A.get<double>(3ull * nv);
+    size_t tb = 0;
+    BRT_CHECK(A.err);
+    BRT_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, fan, start, (int)(nv + 1), st));
+    unsigned char *tmp_scan = A.get<unsigned char>(tb);
+    BRT_CHECK(A.err);
+    BRT_LAUNCH(k_zero_words<<<blocks_for(nv + 1ull, 256), 256, 0, st>>>(fan, nv + 1ull));
+    BRT_LAUNCH(k_zero_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t *>(d_flags), sizeof(MeshFlags) / 4));
+    BRT_LAUNCH(k_tri_boxes<<<blocks_for(n, 256), 256, 0, st>>>(in.vertices, in.faces, n, lo, hi, ctr, fn3, fan, d_flags));
+    BRT_CHECK(hipcub::DeviceScan::ExclusiveSum(tmp_scan, tb, fan, start, (int)(nv + 1), st));
+    BRT_LAUNCH(k_corners<<<blocks_for(corners, 256), 256, 0, st>>>(in.faces, corners, start, fan, at));
+    if (nv)
+      BRT_LAUNCH(k_vertex_normals<<<blocks_for(nv, 256), 256, 0, st>>>(start, start + 1, nv, at, fn3, vnormals, longs,
+                                                                      d_flags));
+    BRT_LAUNCH(k_vertex_normals_long<<<256, 256, 0, st>>>(start, start + 1, at, fn3, longs, d_flags, vnormals));
+    BRT_CHECK(hipMemcpyAsync(&hflags, d_flags, sizeof hflags, hipMemcpyDeviceToHost, st));
   } else {
     BRT_CHECK(hipMemcpyAsync(lo, in.box_lo, 3ull * n * 8, hipMemcpyHostToDevice, st));
     BRT_CHECK(hipMemcpyAsync(hi, in.box_hi, 3ull * n * 8, hipMemcpyHostToDevice, st));
@@ -1007,6 +1131,10 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
     BRT_LAUNCH(k_lv_swap<<<nblocks, BLOCK, 0, st>>>(L, idx, ctr, pos_r));
     BRT_CHECK(hipMemcpyAsync(hn.data(), d_nodes, m * sizeof(LNode), hipMemcpyDeviceToHost, st));
     BRT_CHECK(hipStreamSynchronize(st));
+    if (hflags.refused) {
+      out.refused = true;
+      return hipSuccess;
+    }
     std::vector<uint32_t> next;
     for (uint32_t i = 0; i < m; i++) {
       const LNode &x = hn[i];
@@ -1052,6 +1180,11 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
   BRT_CHECK(hipMemcpyAsync(hsizes.data(), sizes, ns * 4, hipMemcpyDeviceToHost, st));
   BRT_CHECK(hipMemcpyAsync(&ds, d_stats, sizeof ds, hipMemcpyDeviceToHost, st));
   BRT_CHECK(hipStreamSynchronize(st));
+  if (hflags.refused) {
+    out.refused = true;
+    return hipSuccess;
+  }
+  out.host_normals = hflags.max_fan > FAN_LONG;
 
   // ---- pre-order numbering of the large nodes and placement of the small subtrees
   std::vector<uint32_t> pre_top(top.size(), INVALID_ID);
@@ -1180,6 +1313,7 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
   out.n4 = nodes4;
   out.num_n4 = n4;
   out.ord4 = ord4;
+  out.vnormals = vnormals;
   out.recs = recs;
   out.rec_size = rec_size;
   out.max_depth = std::max(hs.max_depth, ds.max_depth);
@@ -1188,7 +1322,7 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
   out.bad_splits = hs.bad + ds.bad;
   out.max_prims = std::max(hs.max_prims, ds.max_prims);
   out.min_prims = std::min(hs.min_prims, ds.min_prims);
-  for (void *p : {(void *)tree, (void *)idx, (void *)nodes64, (void *)nodes4, (void *)ord4, (void *)recs})
+  for (void *p : {(void *)tree, (void *)idx, (void *)nodes64, (void *)nodes4, (void *)ord4, (void *)recs, (void *)vnormals})
     A.release(p);
   return hipSuccess;
 }

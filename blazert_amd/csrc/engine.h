@@ -226,8 +226,9 @@ struct DeviceBuildIn {
   GeomType type;
   uint32_t n;  // primitives (> 0)
   uint32_t min_leaf, max_depth, nbins;
-  const double *vertices;  // triangles: device vertices and faces (the boxes are computed on the device)
+  const double *vertices;  // triangles: device vertices and faces (boxes and normals are computed on the device)
   const uint32_t *faces;
+  uint32_t num_vertices;
   const double *box_lo, *box_hi, *box_ctr;  // other types: host boxes and centers, 3 per primitive
   const double *centers, *radii, *dxs, *dys, *rot, *sa, *sb, *heights;  // other types: host record inputs
 };
@@ -242,6 +243,9 @@ struct DeviceBuildOut {
   uint32_t num_n4;
   uint32_t *ord4;       // visiting order of every Node4's slots, two words each (visit_order4)
   void *recs;           // primitive records in leaf order
+  double *vnormals;     // triangles: vertex normals
+  bool host_normals;    // triangles: some vertex has too many corners, vnormals are left to the host
+  bool refused;         // triangles: some box coordinate is not finite or is -0.0; nothing else is set
   size_t rec_size;
   brt_tree_node root;   // host copy of node 0
   uint32_t max_depth, leaves, branches, bad_splits, max_prims, min_prims;

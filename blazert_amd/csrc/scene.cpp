@@ -149,6 +149,9 @@ struct GeometryT {
   std::vector<uint32_t> faces;
   std::vector<R> vnormals;
   std::vector<R> centers, radii, dxs, dys, rot, sa, sb, heights;
+  // triangles: the boxes and vertex normals are made when a host build needs them (host_precompute); the device build makes
+  // its own
+  bool precomputed = false;
   // build output
   std::vector<brt_tree_node> tree;  // reference form, pre-order
   std::vector<uint32_t> order;      // primitive ids in leaf order
@@ -201,6 +204,14 @@ void mesh_precompute(GeometryT<R> &g, uint32_t nv) {
     for (uint32_t vi : {i0, i1, i2})
       for (int k = 0; k < 3; k++) g.vnormals[3ull * vi + k] = g.vnormals[3ull * vi + k] + fn3[k];
   }
+}
+
+template <class R>
+void host_precompute(GeometryT<R> &g) {
+  if (g.faces.empty() || g.precomputed) return;
+  mesh_precompute(g, (uint32_t)(g.vertices.size() / 3));
+  g.boxes.classify();
+  g.precomputed = true;
 }
 
 template <class R>
@@ -772,6 +783,7 @@ void flatten_f32(GeometryF &g, GeomType type) {
 
 template <class R>
 void build_geometry(GeometryT<R> &g, GeomType type, const brt_build_options &o) {
+  if (type == TRIANGLES) host_precompute(g);
   const auto t0 = std::chrono::steady_clock::now();
   g.built_on_device = false;
   g.dtree = nullptr;
@@ -1087,9 +1099,13 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
       build_geometry(g, (GeomType)t, o);
       continue;
     }
-    if (!g.boxes.device_buildable || !device_build_supported(o.bin_size, o.max_tree_depth)) {
+    const auto on_host = [&]() -> int {
       build_geometry(g, (GeomType)t, o);
-      if (int rc = put_geometry(*d, g, t)) return rc;
+      return put_geometry(*d, g, t);
+    };
+    if ((t != TRIANGLES && !g.boxes.device_buildable) || g.vertices.size() / 3 >= 0x7fffffffu ||
+        !device_build_supported(o.bin_size, o.max_tree_depth)) {
+      if (int rc = on_host()) return rc;
       continue;
     }
     const auto t0 = std::chrono::steady_clock::now();
@@ -1102,11 +1118,11 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
     in.nbins = o.bin_size;
     if (t == TRIANGLES) {
       hipError_t e = d->put(g.faces, &v.faces);
-      if (e == hipSuccess) e = d->put(g.vnormals, &v.vnormals);
       if (e == hipSuccess) e = d->put(g.vertices, &v.vertices);
       if (e != hipSuccess) return device_error(e, "upload failed");
       in.vertices = v.vertices;
       in.faces = v.faces;
+      in.num_vertices = (uint32_t)(g.vertices.size() / 3);
     } else {
       in.box_lo = g.boxes.lo.data();
       in.box_hi = g.boxes.hi.data();
@@ -1124,8 +1140,22 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
     hipError_t e = device_build(in, r, st);
     if (e != hipSuccess)
       return device_error(e, ("device build failed (build.hip:" + std::to_string(r.failed_line) + ")").c_str());
-    for (void *p : {(void *)r.tree, (void *)r.order, (void *)r.n64, (void *)r.n4, (void *)r.ord4, r.recs})
-      d->allocs.push_back(p);
+    if (r.refused) {
+      for (const void *p : {(const void *)v.faces, (const void *)v.vertices}) {
+        d->allocs.erase(std::remove(d->allocs.begin(), d->allocs.end(), p), d->allocs.end());
+        (void)hipFree(const_cast<void *>(p));
+      }
+      if (int rc = on_host()) return rc;
+      continue;
+    }
+    for (void *p : {(void *)r.tree, (void *)r.order, (void *)r.n64, (void *)r.n4, (void *)r.ord4, r.recs,
+                    (void *)r.vnormals})
+      if (p) d->allocs.push_back(p);
+    v.vnormals = r.vnormals;
+    if (r.host_normals) {
+      host_precompute(g);
+      if (hipError_t pe = d->put(g.vnormals, &v.vnormals)) return device_error(pe, "upload failed");
+    }
     g.tree.clear();
     g.order.clear();
     g.n64.clear();
@@ -1165,7 +1195,8 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
     v.n_prims = g.boxes.n;
     v.n_nodes = r.num_n64;
     v.depth = r.max_depth;
-    v.irregular_boxes = g.boxes.ordered ? 0u : 1u;  // finite boxes (device_buildable): only the order can fail
+    // finite boxes: only the order can fail, and a triangle's box is ordered
+    v.irregular_boxes = (t == TRIANGLES || g.boxes.ordered) ? 0u : 1u;
     g.view = v;
     g.extent = extent;
     g.extent_ok = extent < 1e30;
@@ -1175,8 +1206,7 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
     v.prims = r.recs;
     v.prim_ids = r.order;
     bs.device_bytes = (uint64_t)r.num_n64 * sizeof(Node64) + (uint64_t)r.num_n4 * sizeof(Node4) +
-                      (uint64_t)g.boxes.n * (r.rec_size + 4) + g.faces.size() * 4 + g.vnormals.size() * 8 +
-                      g.vertices.size() * 8;
+                      (uint64_t)g.boxes.n * (r.rec_size + 4) + g.faces.size() * 4 + 2 * g.vertices.size() * 8;
     if (hipError_t fe = make_prim_filter(*d, v, t, g.extent, st, &bs.device_bytes))
       return device_error(fe, "pre-test records");
     if (t == TRIANGLES)
@@ -1224,14 +1254,14 @@ int add_mesh_t(brt_scene *s, const R *vertices, uint32_t nv, const uint32_t *fac
   int rc = add_common<R>(s, TRIANGLES, geom_id);
   if (rc) return rc;
   if ((nv && !vertices) || (nf && !faces)) return fail(BRT_ERR_INVALID_ARGUMENT, "NULL vertex or face array");
-  for (uint64_t i = 0; i < 3ull * nf; i++)
-    if (faces[i] >= nv) return fail(BRT_ERR_INVALID_ARGUMENT, "face index out of range");
+  uint32_t top = 0;
+  for (uint64_t i = 0; i < 3ull * nf; i++) top = std::max(top, faces[i]);
+  if (nf && top >= nv) return fail(BRT_ERR_INVALID_ARGUMENT, "face index out of range");
   if (nf >= (1u << 30)) return fail(BRT_ERR_UNSUPPORTED, "too many triangles");
   GeometryT<R> &g = geo_of<R>(s)[TRIANGLES];
   g.vertices.assign(vertices, vertices + 3ull * nv);
   g.faces.assign(faces, faces + 3ull * nf);
-  mesh_precompute(g, nv);
-  g.boxes.classify();
+  g.boxes.n = nf;
   finish_add<R>(s, TRIANGLES, geom_id);
   return BRT_OK;
 }
