@@ -11,9 +11,12 @@
 //     the i-th element of the left part [begin, begin + T) that fails the predicate with the i-th element of the
 //     right part that passes it, counted from the right end, and leaves every other element in place (T = number
 //     of passing elements). Ranks from prefix counts therefore give its exact result.
-// Nodes with more than SMALL primitives are processed level by level, several blocks per node; each subtree of at
-// most SMALL primitives is then built depth first by one wave out of LDS. The host numbers the nodes in pre-order
-// (subtree sizes are known by then), and prefix scans flatten the tree into the traversal records.
+// Nodes with more than SMALL primitives are processed level by level, several blocks per node; the nodes of more than TINY
+// primitives in a subtree of at most SMALL are then split by one wave out of LDS, and each subtree of at most TINY by 16
+// lanes, one primitive per lane, all its nodes of a level at once. Nodes are numbered in pre-order in closed form: a node
+// whose primitives begin at b and whose path from the root has l left turns is number 2 L(b) + l, L(b) being the number of
+// leaves that begin before b (the left subtrees hanging off its path hold 2 L(b) nodes less one for every right turn, and
+// its ancestors are as many as the turns). Its number among the internal nodes is L(b) + l.
 #include <hip/hip_runtime.h>
 
 #include <float.h>
@@ -24,6 +27,7 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include "../../include/blazert_amd/device/exact.h"
 #include "engine.h"
 #include "f32_round.h"
 
@@ -33,11 +37,11 @@ namespace {
 
 typedef unsigned long long u64;
 
-constexpr uint32_t SMALL = 256;          // subtrees of at most this many primitives are built by one wave
+constexpr uint32_t SMALL = 256;          // subtrees of at most this many primitives are split by one wave
+constexpr uint32_t TINY = 16;            // subtrees of at most this many primitives are built by 16 lanes
 constexpr uint32_t CHUNK = 2048;         // primitives per block in the level passes
 constexpr uint32_t BLOCK = 256;          // threads per block in the level passes
 constexpr uint32_t STACK = 64;           // depth-first stack of the subtree waves (max_depth <= 62)
-constexpr uint32_t SMALL_REF = 0x80000000u;  // host-side child tag: a small subtree (else a large node)
 
 // Order-preserving unsigned key of a double (NaN excluded): min / max of keys = min / max of values.
 __device__ __forceinline__ u64 okey(double x) {
@@ -564,23 +568,42 @@ __global__ void k_lv_swap(Level L, uint32_t *__restrict__ idx, const double *__r
 
 // ------------------------------------------------------------------------------------------------ small subtrees
 struct SmallRoot {
-  uint32_t begin, n, depth, pad;
+  uint32_t begin, n, depth, left;  // left: left turns on the path from the tree's root
 };
 
 struct BuildStatsDev {
-  uint32_t max_depth, leaves, branches, bad, max_prims, min_prims;
+  uint32_t max_depth, bad, max_prims, min_prims;
+};
+__device__ __forceinline__ void add_stats(BuildStatsDev &a, const BuildStatsDev &b) {
+  a.max_depth = a.max_depth > b.max_depth ? a.max_depth : b.max_depth;
+  a.bad += b.bad;
+  a.max_prims = a.max_prims > b.max_prims ? a.max_prims : b.max_prims;
+  a.min_prims = a.min_prims < b.min_prims ? a.min_prims : b.min_prims;
+}
+
+// A node before it has its number: internal nodes are kept at the position that parts their children, which no two share,
+// leaves at their first position.
+struct RawNode {
+  double lo[3], hi[3];
+  uint32_t begin;
+  uint32_t info;  // internal: split axis; leaf: primitives
+  uint32_t left;  // left turns on the path from the root
+  uint32_t pad;
+};
+static_assert(sizeof(RawNode) == 64, "RawNode size");
+struct RawTree {
+  RawNode *inner, *leaf;
+  uint32_t *is_inner, *is_leaf;  // 0 / 1 per position
 };
 
-// One wave builds the whole subtree of a small root depth first (build_recursive, blazert/bvh/builder.h:85-115), its
-// primitives' boxes and centers staged in LDS and permuted through an LDS index array. Nodes are written in the
-// subtree's own pre-order to tmp[2 * begin ...] (a subtree of n primitives has at most 2n - 1 nodes) with
-// subtree-local child indices; sizes[s] receives the node count.
+// One wave splits the nodes of more than TINY primitives of a small subtree depth first (build_recursive,
+// blazert/bvh/builder.h:85-115), its primitives' boxes and centers staged in LDS and permuted through an LDS index array.
+// The subtrees of at most TINY primitives that remain are listed at tiny[R.begin ...], their number in num_tiny.
 __global__ void __launch_bounds__(64) k_small(const SmallRoot *__restrict__ roots, uint32_t *__restrict__ idx,
                                               const double *__restrict__ lo, const double *__restrict__ hi,
                                               const double *__restrict__ ctr, uint32_t nb, uint32_t min_leaf,
-                                              uint32_t max_depth, brt_tree_node *__restrict__ tmp,
-                                              uint32_t *__restrict__ sizes,
-                                              BuildStatsDev *__restrict__ stats) {
+                                              uint32_t max_depth, RawTree raw, SmallRoot *__restrict__ tiny,
+                                              uint32_t *__restrict__ num_tiny, BuildStatsDev *__restrict__ stats) {
   __shared__ uint32_t e_idx[SMALL];
   __shared__ double e_lo[3][SMALL], e_hi[3][SMALL], e_ctr[3][SMALL];
   __shared__ uint16_t perm[SMALL];
@@ -591,6 +614,15 @@ __global__ void __launch_bounds__(64) k_small(const SmallRoot *__restrict__ root
 
   const SmallRoot R = roots[blockIdx.x];
   const uint32_t lane = threadIdx.x;
+  BuildStatsDev st{0, 0, 0, 0xFFFFFFFFu};
+  if (R.n <= TINY) {
+    if (lane == 0) {
+      tiny[R.begin] = R;
+      num_tiny[blockIdx.x] = 1;
+      stats[blockIdx.x] = st;
+    }
+    return;
+  }
   for (uint32_t k = lane; k < R.n; k += 64) {
     const uint32_t p = idx[R.begin + k];
     e_idx[k] = p;
@@ -601,21 +633,18 @@ __global__ void __launch_bounds__(64) k_small(const SmallRoot *__restrict__ root
     }
     perm[k] = (uint16_t)k;
   }
-  brt_tree_node *out = tmp + 2ull * R.begin;
-  BuildStatsDev st{0, 0, 0, 0, 0, 0xFFFFFFFFu};
   if (lane == 0) {
     stk[0][0] = 0;
     stk[0][1] = R.n;
     stk[0][2] = R.depth;
-    stk[0][3] = INVALID_ID;
+    stk[0][3] = R.left;
   }
   __syncthreads();
-  uint32_t sp = 1, count = 0;
+  uint32_t sp = 1, tinies = 0;
   while (sp > 0) {
     sp--;
-    const uint32_t b = stk[sp][0], e = stk[sp][1], d = stk[sp][2], parent = stk[sp][3];
+    const uint32_t b = stk[sp][0], e = stk[sp][1], d = stk[sp][2], left = stk[sp][3];
     __syncthreads();
-    const uint32_t self = count++;
     const uint32_t n = e - b;
     // bounds
     double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
@@ -632,24 +661,13 @@ __global__ void __launch_bounds__(64) k_small(const SmallRoot *__restrict__ root
         mx[c] = dmax(mx[c], __shfl_xor(mx[c], off));
       }
     st.max_depth = d > st.max_depth ? d : st.max_depth;
-    brt_tree_node node;
-    for (int c = 0; c < 3; c++) {
-      node.min[c] = mn[c];
-      node.max[c] = mx[c];
-    }
-    node.children[0] = node.children[1] = INVALID_ID;
-    node.prim_begin = node.prim_count = 0;
+    RawNode node{{mn[0], mn[1], mn[2]}, {mx[0], mx[1], mx[2]}, R.begin + b, n, left, 0};
     if (n <= min_leaf || d >= max_depth) {
-      node.leaf = 1;
-      node.axis = INVALID_ID;
-      node.prim_begin = R.begin + b;
-      node.prim_count = n;
-      st.leaves++;
       st.max_prims = n > st.max_prims ? n : st.max_prims;
       st.min_prims = n < st.min_prims ? n : st.min_prims;
       if (lane == 0) {
-        out[self] = node;
-        if (parent != INVALID_ID) out[parent].children[1] = self;
+        raw.leaf[R.begin + b] = node;
+        raw.is_leaf[R.begin + b] = 1u;
       }
       continue;
     }
@@ -729,62 +747,334 @@ __global__ void __launch_bounds__(64) k_small(const SmallRoot *__restrict__ root
       }
       __syncthreads();
     }
-    node.leaf = 0;
-    node.axis = axis;
-    node.children[0] = self + 1;
-    st.branches++;
+    node.info = axis;
     if (lane == 0) {
-      out[self] = node;
-      if (parent != INVALID_ID) out[parent].children[1] = self;
-      stk[sp][0] = mid;
-      stk[sp][1] = e;
-      stk[sp][2] = d + 1;
-      stk[sp][3] = self;
-      stk[sp + 1][0] = b;
-      stk[sp + 1][1] = mid;
-      stk[sp + 1][2] = d + 1;
-      stk[sp + 1][3] = INVALID_ID;
+      raw.inner[R.begin + mid] = node;
+      raw.is_inner[R.begin + mid] = 1u;
     }
-    sp += 2;
+    for (int c = 1; c >= 0; c--) {
+      const uint32_t cb = c ? mid : b, ce = c ? e : mid, cl = c ? left : left + 1u;
+      if (ce - cb <= TINY) {
+        if (lane == 0) tiny[R.begin + tinies] = SmallRoot{R.begin + cb, ce - cb, d + 1, cl};
+        tinies++;
+      } else {
+        if (lane == 0) {
+          stk[sp][0] = cb;
+          stk[sp][1] = ce;
+          stk[sp][2] = d + 1;
+          stk[sp][3] = cl;
+        }
+        sp++;
+      }
+    }
     __syncthreads();
   }
   for (uint32_t k = lane; k < R.n; k += 64) idx[R.begin + k] = e_idx[perm[k]];
   if (lane == 0) {
-    sizes[blockIdx.x] = count;
-    atomicMax(&stats->max_depth, st.max_depth);
-    atomicAdd(&stats->leaves, st.leaves);
-    atomicAdd(&stats->branches, st.branches);
-    atomicAdd(&stats->bad, st.bad);
-    atomicMax(&stats->max_prims, st.max_prims);
-    atomicMin(&stats->min_prims, st.min_prims);
+    num_tiny[blockIdx.x] = tinies;
+    stats[blockIdx.x] = st;
+  }
+}
+
+// The lists of the small subtrees' waves, one after the other.
+__global__ void k_tiny_list(const SmallRoot *__restrict__ roots, const uint32_t *__restrict__ num_tiny,
+                            const uint32_t *__restrict__ at, const SmallRoot *__restrict__ tiny,
+                            SmallRoot *__restrict__ list) {
+  const uint32_t r = blockIdx.x;
+  for (uint32_t k = threadIdx.x; k < num_tiny[r]; k += blockDim.x) list[at[r] + k] = tiny[roots[r].begin + k];
+}
+
+// Rotates a value by one lane within the row of 16.
+__device__ __forceinline__ uint32_t row_next(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x121, 0xf, 0xf, false);
+}
+__device__ __forceinline__ double row_next(double x) {
+  const u64 b = (u64)__double_as_longlong(x);
+  return __longlong_as_double((long long)(((u64)row_next((uint32_t)(b >> 32)) << 32) | row_next((uint32_t)b)));
+}
+
+// Subtrees of at most TINY primitives, four per wave: a row of 16 lanes holds one primitive per lane and splits all nodes of
+// a level at once, each lane seeing the others of its node as their values rotate through the row. A bin boundary that
+// can be chosen is one after an occupied bin (the boundaries behind empty bins cost the same and come later), so every lane
+// evaluates the one after its own bin, on each axis. The primitives stay in their lanes; `pos` is the order.
+__global__ void __launch_bounds__(256) k_tiny(const SmallRoot *__restrict__ list, const uint32_t *__restrict__ total,
+                                              uint32_t *__restrict__ idx, const double *__restrict__ lo,
+                                              const double *__restrict__ hi, const double *__restrict__ ctr, uint32_t nb,
+                                              uint32_t min_leaf, uint32_t max_depth, RawTree raw,
+                                              BuildStatsDev *__restrict__ stats) {
+  using exact::max_nn;
+  using exact::min_nn;
+  const uint32_t lane = threadIdx.x & 63u, in_row = lane & 15u;
+  const uint32_t waves = gridDim.x * (blockDim.x >> 6), wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const uint32_t count = *total;
+  const double scale = (double)(nb - 1);
+  constexpr uint32_t GONE = 0xFFu;
+  BuildStatsDev st{0, 0, 0, 0xFFFFFFFFu};
+  for (uint32_t first = 4u * wave; first < count; first += 4u * waves) {  // wave-uniform
+    const uint32_t g = first + (lane >> 4);
+    const SmallRoot R = g < count ? list[g] : SmallRoot{0, 0, 0, 0};
+    const bool mine = in_row < R.n;
+    const uint32_t prim = mine ? idx[R.begin + in_row] : 0u;
+    double l[3], h[3], c[3];
+    for (int k = 0; k < 3; k++) {
+      l[k] = mine ? lo[3ull * prim + k] : 0.0;
+      h[k] = mine ? hi[3ull * prim + k] : 0.0;
+      c[k] = mine ? ctr[3ull * prim + k] : 0.0;
+    }
+    uint32_t node = mine ? 0u : GONE;  // first position of this lane's node in the subtree
+    uint32_t size = R.n, depth = R.depth, left = R.left, pos = in_row;
+    while (__ballot(node != GONE)) {
+      // bounds of the node
+      double mn[3], mx[3];
+      {
+        double ol[3], oh[3];
+        uint32_t on = node;
+        for (int k = 0; k < 3; k++) {
+          ol[k] = mn[k] = l[k];
+          oh[k] = mx[k] = h[k];
+        }
+#pragma unroll 1
+        for (int r = 1; r < 16; r++) {
+          on = row_next(on);
+          const bool same = on == node;
+#pragma unroll
+          for (int k = 0; k < 3; k++) {
+            ol[k] = row_next(ol[k]);
+            oh[k] = row_next(oh[k]);
+            mn[k] = min_nn(mn[k], same ? ol[k] : mn[k]);
+            mx[k] = max_nn(mx[k], same ? oh[k] : mx[k]);
+          }
+        }
+      }
+      if (node != GONE) st.max_depth = depth > st.max_depth ? depth : st.max_depth;
+      if (node != GONE && (size <= min_leaf || depth >= max_depth)) {
+        if (pos == node) {
+          const uint32_t at = R.begin + node;
+          raw.leaf[at] = RawNode{{mn[0], mn[1], mn[2]}, {mx[0], mx[1], mx[2]}, at, size, left, 0};
+          raw.is_leaf[at] = 1u;
+          st.max_prims = size > st.max_prims ? size : st.max_prims;
+          st.min_prims = size < st.min_prims ? size : st.min_prims;
+        }
+        node = GONE;
+      }
+      if (!__ballot(node != GONE)) break;
+      // bins of the three axes, packed
+      uint32_t bins = 0;
+      double step[3];
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const double len = mx[k] - mn[k];
+        const double inv = (len > 0.0) ? 1.0 / len : 0.0;
+        bins |= bin_of(((c[k] - mn[k]) * inv) * scale, nb - 1) << (8 * k);
+        step[k] = len / (double)nb;
+      }
+      // the cost of the boundary after this lane's bin, and the node's least one with its first bin
+      double cost[3];
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        double ll[3], lh[3], rl[3], rh[3];
+        uint32_t nl = 1, nr = 0;
+        double ol[3], oh[3];
+        uint32_t on = node, ob = (bins >> (8 * j)) & 255u;
+        const uint32_t mine_b = ob;
+        for (int k = 0; k < 3; k++) {
+          ll[k] = ol[k] = l[k];
+          lh[k] = oh[k] = h[k];
+          rl[k] = DBL_MAX;
+          rh[k] = -DBL_MAX;
+        }
+#pragma unroll 1
+        for (int r = 1; r < 16; r++) {
+          on = row_next(on);
+          ob = row_next(ob);
+          const bool same = on == node, is_l = same && ob <= mine_b, is_r = same && ob > mine_b;
+          nl += is_l ? 1u : 0u;
+          nr += is_r ? 1u : 0u;
+#pragma unroll
+          for (int k = 0; k < 3; k++) {
+            ol[k] = row_next(ol[k]);
+            oh[k] = row_next(oh[k]);
+            ll[k] = min_nn(ll[k], is_l ? ol[k] : DBL_MAX);
+            lh[k] = max_nn(lh[k], is_l ? oh[k] : -DBL_MAX);
+            rl[k] = min_nn(rl[k], is_r ? ol[k] : DBL_MAX);
+            rh[k] = max_nn(rh[k], is_r ? oh[k] : -DBL_MAX);
+          }
+        }
+        const double x = (double)nl * surface(ll, lh) + (double)nr * surface(rl, rh);
+        cost[j] = (nr > 0u && x < DBL_MAX) ? x : __builtin_inf();  // an empty right side costs NaN in the sweep
+      }
+      double cut[3], least[3];
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        double m = cost[j], oc = cost[j];
+        uint32_t mb = (bins >> (8 * j)) & 255u, ob = mb, on = node;
+#pragma unroll 1
+        for (int r = 1; r < 16; r++) {
+          on = row_next(on);
+          ob = row_next(ob);
+          oc = row_next(oc);
+          const bool take = on == node && (oc < m || (oc == m && ob < mb));
+          m = take ? oc : m;
+          mb = take ? ob : mb;
+        }
+        const bool any = m < DBL_MAX;
+        least[j] = any ? m : DBL_MAX;
+        cut[j] = (double)(any ? mb + 1u : 1u) * step[j] + mn[j];
+      }
+      uint32_t axis = 0;
+      if (least[0] > least[1]) axis = 1;
+      if ((axis ? least[1] : least[0]) > least[2]) axis = 2;
+      // elements left of each axis's cut, counted over the node (packed), and the partition attempts
+      const uint32_t pass3 = (c[0] < cut[0] ? 1u : 0u) | (c[1] < cut[1] ? 0x100u : 0u) | (c[2] < cut[2] ? 0x10000u : 0u);
+      uint32_t T3 = pass3;
+      {
+        uint32_t on = node, op = pass3;
+#pragma unroll 1
+        for (int r = 1; r < 16; r++) {
+          on = row_next(on);
+          op = row_next(op);
+          T3 += on == node ? op : 0u;
+        }
+      }
+      uint32_t mid = 0, bad = 0;  // mid: within the node
+      bool split = false;
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        if (!split) {
+          const uint32_t T = (T3 >> (8 * axis)) & 255u;
+          if (T == 0 || T == size) {
+            bad++;
+            mid = size >> 1;
+            axis = axis == 2 ? 0u : axis + 1u;
+          } else {
+            mid = T;
+            split = true;
+          }
+        }
+      }
+      // the r-th failing element of the left part trades places with the r-th passing one of the right part from the end
+      const bool pass = ((pass3 >> (8 * axis)) & 1u) != 0u;
+      const uint32_t at = pos - node;
+      const bool out_l = split && at < mid && !pass, out_r = split && at >= mid && pass;
+      // tag: 0 in place, else side (1 left, 2 right); rank among the misplaced of the side
+      const uint32_t side = node == GONE ? 0u : out_l ? 1u : out_r ? 2u : 0u;
+      uint32_t rank = 0;
+      {
+        uint32_t o = (node << 16) | (side << 8) | pos;
+        const uint32_t self = o;
+#pragma unroll 1
+        for (int r = 1; r < 16; r++) {
+          o = row_next(o);
+          const bool same = (o & 0xFFFFFF00u) == (self & 0xFFFFFF00u);
+          const uint32_t op = o & 255u;
+          rank += same && (side == 1u ? op < pos : op > pos) ? 1u : 0u;
+        }
+      }
+      uint32_t to = pos;
+      {
+        uint32_t o = (node << 24) | (side << 16) | (rank << 8) | pos;
+        const uint32_t want = (node << 24) | ((3u - side) << 16) | (rank << 8);
+#pragma unroll 1
+        for (int r = 1; r < 16; r++) {
+          o = row_next(o);
+          if (side && (o & 0xFFFFFF00u) == want) to = o & 255u;
+        }
+      }
+      if (node != GONE) {
+        if (pos == node) {
+          raw.inner[R.begin + node + mid] =
+              RawNode{{mn[0], mn[1], mn[2]}, {mx[0], mx[1], mx[2]}, R.begin + node, axis, left, 0};
+          raw.is_inner[R.begin + node + mid] = 1u;
+          st.bad += bad;
+        }
+        pos = to;
+        const bool right = pos - node >= mid;
+        node = right ? node + mid : node;
+        size = right ? size - mid : mid;
+        left += right ? 0u : 1u;
+        depth++;
+      }
+    }
+    if (mine) idx[R.begin + pos] = prim;
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    BuildStatsDev o;
+    o.max_depth = __shfl_xor(st.max_depth, off);
+    o.bad = __shfl_xor(st.bad, off);
+    o.max_prims = __shfl_xor(st.max_prims, off);
+    o.min_prims = __shfl_xor(st.min_prims, off);
+    add_stats(st, o);
+  }
+  if (lane == 0) stats[wave] = st;
+}
+
+// One block: the waves' statistics added up into stats[0].
+__global__ void k_sum_stats(BuildStatsDev *stats, uint32_t n) {
+  __shared__ BuildStatsDev part[256];
+  BuildStatsDev st{0, 0, 0, 0xFFFFFFFFu};
+  for (uint32_t i = threadIdx.x; i < n; i += 256) add_stats(st, stats[i]);
+  part[threadIdx.x] = st;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < 256; i++) add_stats(st, part[i]);
+    stats[0] = st;
   }
 }
 
 // ------------------------------------------------------------------------------------------------ assembly
-struct TopPut {
-  brt_tree_node node;
-  uint32_t pre, pad;
+struct RawPut {
+  RawNode node;
+  uint32_t at, leaf;
 };
 
-__global__ void k_put_top(const TopPut *__restrict__ tops, uint32_t m, brt_tree_node *__restrict__ tree) {
+__global__ void k_put_raw(const RawPut *__restrict__ puts, uint32_t m, RawTree raw) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= m) return;
-  tree[tops[i].pre] = tops[i].node;
+  const RawPut p = puts[i];
+  if (p.leaf) {
+    raw.leaf[p.at] = p.node;
+    raw.is_leaf[p.at] = 1u;
+  } else {
+    raw.inner[p.at] = p.node;
+    raw.is_inner[p.at] = 1u;
+  }
 }
 
-// Moves each small subtree from its scratch slot to its pre-order position (base[s]), making child indices global.
-__global__ void k_reloc(const SmallRoot *__restrict__ roots, const uint32_t *__restrict__ sizes,
-                        const uint32_t *__restrict__ bases, const brt_tree_node *__restrict__ tmp,
-                        brt_tree_node *__restrict__ tree) {
-  const uint32_t s = blockIdx.x, base = bases[s];
-  const size_t from = 2ull * roots[s].begin;
-  for (uint32_t j = threadIdx.x; j < sizes[s]; j += blockDim.x) {
-    brt_tree_node nd = tmp[from + j];
-    if (!nd.leaf) {
-      nd.children[0] += base;
-      nd.children[1] += base;
+// Writes every node at its number. before[p]: leaves that begin before position p; ni: number among the internal nodes.
+__global__ void k_emit(RawTree raw, uint32_t n, const uint32_t *__restrict__ before, brt_tree_node *__restrict__ tree,
+                       uint32_t *__restrict__ ni) {
+  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  if (raw.is_leaf[p]) {
+    const RawNode r = raw.leaf[p];
+    brt_tree_node t;
+    for (int k = 0; k < 3; k++) {
+      t.min[k] = r.lo[k];
+      t.max[k] = r.hi[k];
     }
-    tree[base + j] = nd;
+    t.leaf = 1;
+    t.axis = t.children[0] = t.children[1] = INVALID_ID;
+    t.prim_begin = p;
+    t.prim_count = r.info;
+    const uint32_t i = 2u * before[p] + r.left;
+    tree[i] = t;
+    ni[i] = 0;
+  }
+  if (raw.is_inner[p]) {
+    const RawNode r = raw.inner[p];
+    brt_tree_node t;
+    for (int k = 0; k < 3; k++) {
+      t.min[k] = r.lo[k];
+      t.max[k] = r.hi[k];
+    }
+    const uint32_t b = before[r.begin], i = 2u * b + r.left;
+    t.leaf = 0;
+    t.axis = r.info;
+    t.children[0] = i + 1u;
+    t.children[1] = 2u * before[p] + r.left;
+    t.prim_begin = t.prim_count = 0;
+    tree[i] = t;
+    ni[i] = b + r.left;
   }
 }
 
@@ -825,10 +1115,9 @@ __global__ void k_roots4(const brt_tree_node *__restrict__ T, uint32_t M, uint32
 }
 
 __global__ void k_flags(const brt_tree_node *__restrict__ T, const uint32_t *__restrict__ is_root, uint32_t M,
-                        uint32_t *__restrict__ internal, uint32_t *__restrict__ islots) {
+                        uint32_t *__restrict__ islots) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= M) return;
-  internal[i] = T[i].leaf ? 0u : 1u;
   uint32_t s = 0;
   if (is_root[i]) {
     uint32_t slot[4];
@@ -1001,9 +1290,7 @@ hipError_t to_device(Arena &A, const T *host, size_t count, const T **dst, hipSt
 }
 
 struct HostTop {
-  uint32_t begin, n, depth, leaf, axis;
-  uint32_t child[2];
-  double lo[3], hi[3];
+  uint32_t begin, n, depth, left;
 };
 
 }  // namespace
@@ -1079,20 +1366,15 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
   Level L{d_nodes, d_map, d_map + cap_blocks, d_cnt4, d_cnt4 + cap_blocks, d_cnt4 + 2 * cap_blocks,
           d_cnt4 + 3 * cap_blocks, Bins{bcnt, bklo, bkhi}};
 
-  BuildStatsDev hs{0, 0, 0, 0, 0, 0xFFFFFFFFu};
-  std::vector<HostTop> top;
+  BuildStatsDev hs{0, 0, 0, 0xFFFFFFFFu};
   std::vector<SmallRoot> small;
-  auto add_child = [&](uint32_t begin, uint32_t cnt, uint32_t depth, std::vector<uint32_t> &next) -> uint32_t {
-    if (cnt > SMALL) {
-      top.push_back(HostTop{begin, cnt, depth, 0, INVALID_ID, {INVALID_ID, INVALID_ID}, {0, 0, 0}, {0, 0, 0}});
-      next.push_back((uint32_t)top.size() - 1);
-      return (uint32_t)top.size() - 1;
-    }
-    small.push_back(SmallRoot{begin, cnt, depth, 0});
-    return SMALL_REF | ((uint32_t)small.size() - 1);
+  std::vector<RawPut> puts;  // the large nodes
+  auto add_child = [&](uint32_t begin, uint32_t cnt, uint32_t depth, uint32_t left, std::vector<HostTop> &next) {
+    if (cnt > SMALL) next.push_back(HostTop{begin, cnt, depth, left});
+    else small.push_back(SmallRoot{begin, cnt, depth, left});
   };
-  std::vector<uint32_t> level;
-  const uint32_t root_ref = add_child(0, n, 0, level);
+  std::vector<HostTop> level;
+  add_child(0, n, 0, 0, level);
   std::vector<LNode> hn;
   std::vector<uint32_t> hmap;
   while (!level.empty()) {
@@ -1101,7 +1383,7 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
     hmap.clear();
     uint32_t nblocks = 0;
     for (uint32_t i = 0; i < m; i++) {
-      const HostTop &t = top[level[i]];
+      const HostTop &t = level[i];
       LNode &x = hn[i];
       x.begin = t.begin;
       x.n = t.n;
@@ -1135,49 +1417,62 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
       out.refused = true;
       return hipSuccess;
     }
-    std::vector<uint32_t> next;
+    std::vector<HostTop> next;
     for (uint32_t i = 0; i < m; i++) {
       const LNode &x = hn[i];
-      const uint32_t ti = level[i];
-      for (int k = 0; k < 3; k++) {
-        top[ti].lo[k] = x.lo[k];
-        top[ti].hi[k] = x.hi[k];
-      }
+      const uint32_t left = level[i].left;
       hs.max_depth = std::max(hs.max_depth, x.depth);
+      RawPut put{{{x.lo[0], x.lo[1], x.lo[2]}, {x.hi[0], x.hi[1], x.hi[2]}, x.begin, x.leaf ? x.n : x.axis, left, 0},
+                 x.leaf ? x.begin : x.mid, x.leaf};
+      puts.push_back(put);
       if (x.leaf) {
-        top[ti].leaf = 1;
-        hs.leaves++;
         hs.max_prims = std::max(hs.max_prims, x.n);
         hs.min_prims = std::min(hs.min_prims, x.n);
         continue;
       }
-      hs.branches++;
       hs.bad += x.bad;
-      top[ti].axis = x.axis;
-      const uint32_t c0 = add_child(x.begin, x.mid - x.begin, x.depth + 1, next);
-      const uint32_t c1 = add_child(x.mid, x.begin + x.n - x.mid, x.depth + 1, next);
-      top[ti].child[0] = c0;
-      top[ti].child[1] = c1;
+      add_child(x.begin, x.mid - x.begin, x.depth + 1, left + 1, next);
+      add_child(x.mid, x.begin + x.n - x.mid, x.depth + 1, left, next);
     }
     level.swap(next);
   }
 
-  // ---- small subtrees
+  // ---- small and tiny subtrees
   const uint32_t ns = (uint32_t)small.size();
-  brt_tree_node *tmp = A.get<brt_tree_node>(2ull * n);
-  uint32_t *sizes = A.get<uint32_t>(ns), *bases = A.get<uint32_t>(ns);
-  SmallRoot *d_small = A.get<SmallRoot>(ns);
-  BuildStatsDev *d_stats = A.get<BuildStatsDev>(1);
+  const uint32_t tiny_blocks = std::min(blocks_for(n, 64), 4096u), tiny_waves = tiny_blocks * 4u;
+  RawTree raw{A.get<RawNode>(n), A.get<RawNode>(n), A.get<uint32_t>(n), A.get<uint32_t>(n + 1ull)};
+  uint32_t *before = A.get<uint32_t>(n + 1ull);
+  SmallRoot *tiny = A.get<SmallRoot>(n), *list = A.get<SmallRoot>(n), *d_small = A.get<SmallRoot>(ns);
+  uint32_t *num_tiny = A.get<uint32_t>(ns + 1ull), *tiny_at = A.get<uint32_t>(ns + 1ull);
+  BuildStatsDev *d_stats = A.get<BuildStatsDev>((size_t)ns + tiny_waves);
+  RawPut *d_puts = A.get<RawPut>(puts.size());
+  size_t tb_tiny = 0, tb_before = 0;
   BRT_CHECK(A.err);
-  BuildStatsDev init{0, 0, 0, 0, 0, 0xFFFFFFFFu};
-  BRT_CHECK(hipMemcpyAsync(d_stats, &init, sizeof init, hipMemcpyHostToDevice, st));
-  BRT_CHECK(hipMemcpyAsync(d_small, small.data(), ns * sizeof(SmallRoot), hipMemcpyHostToDevice, st));
-  if (ns)
-    BRT_LAUNCH(k_small<<<ns, 64, 0, st>>>(d_small, idx, lo, hi, ctr, nb, in.min_leaf, in.max_depth, tmp, sizes,
+  BRT_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb_tiny, num_tiny, tiny_at, (int)(ns + 1), st));
+  BRT_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb_before, raw.is_leaf, before, (int)(n + 1), st));
+  unsigned char *scan_tmp = A.get<unsigned char>(std::max(tb_tiny, tb_before));
+  BRT_CHECK(A.err);
+  BRT_LAUNCH(k_zero_words<<<blocks_for(n, 256), 256, 0, st>>>(raw.is_inner, n));
+  BRT_LAUNCH(k_zero_words<<<blocks_for(n + 1ull, 256), 256, 0, st>>>(raw.is_leaf, n + 1ull));
+  BRT_LAUNCH(k_zero_words<<<1, 64, 0, st>>>(num_tiny + ns, 1));
+  if (!puts.empty()) {
+    BRT_CHECK(hipMemcpyAsync(d_puts, puts.data(), puts.size() * sizeof(RawPut), hipMemcpyHostToDevice, st));
+    BRT_LAUNCH(k_put_raw<<<blocks_for(puts.size(), 64), 64, 0, st>>>(d_puts, (uint32_t)puts.size(), raw));
+  }
+  if (ns) {
+    BRT_CHECK(hipMemcpyAsync(d_small, small.data(), ns * sizeof(SmallRoot), hipMemcpyHostToDevice, st));
+    BRT_LAUNCH(k_small<<<ns, 64, 0, st>>>(d_small, idx, lo, hi, ctr, nb, in.min_leaf, in.max_depth, raw, tiny, num_tiny,
                                           d_stats));
-  std::vector<uint32_t> hsizes(ns), hbases(ns);
+  }
+  BRT_CHECK(hipcub::DeviceScan::ExclusiveSum(scan_tmp, tb_tiny, num_tiny, tiny_at, (int)(ns + 1), st));
+  if (ns) BRT_LAUNCH(k_tiny_list<<<ns, 64, 0, st>>>(d_small, num_tiny, tiny_at, tiny, list));
+  BRT_LAUNCH(k_tiny<<<tiny_blocks, 256, 0, st>>>(list, tiny_at + ns, idx, lo, hi, ctr, nb, in.min_leaf, in.max_depth, raw,
+                                                 d_stats + ns));
+  BRT_LAUNCH(k_sum_stats<<<1, 256, 0, st>>>(d_stats, ns + tiny_waves));
+  BRT_CHECK(hipcub::DeviceScan::ExclusiveSum(scan_tmp, tb_before, raw.is_leaf, before, (int)(n + 1), st));
   BuildStatsDev ds{};
-  BRT_CHECK(hipMemcpyAsync(hsizes.data(), sizes, ns * 4, hipMemcpyDeviceToHost, st));
+  uint32_t leaves = 0;
+  BRT_CHECK(hipMemcpyAsync(&leaves, before + n, 4, hipMemcpyDeviceToHost, st));
   BRT_CHECK(hipMemcpyAsync(&ds, d_stats, sizeof ds, hipMemcpyDeviceToHost, st));
   BRT_CHECK(hipStreamSynchronize(st));
   if (hflags.refused) {
@@ -1186,76 +1481,31 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
   }
   out.host_normals = hflags.max_fan > FAN_LONG;
 
-  // ---- pre-order numbering of the large nodes and placement of the small subtrees
-  std::vector<uint32_t> pre_top(top.size(), INVALID_ID);
-  uint32_t M = 0;
-  {
-    std::vector<uint32_t> stack{root_ref};
-    while (!stack.empty()) {
-      const uint32_t r = stack.back();
-      stack.pop_back();
-      if (r & SMALL_REF) {
-        const uint32_t s = r & ~SMALL_REF;
-        hbases[s] = M;
-        M += hsizes[s];
-      } else {
-        pre_top[r] = M++;
-        if (!top[r].leaf) {
-          stack.push_back(top[r].child[1]);
-          stack.push_back(top[r].child[0]);
-        }
-      }
-    }
-  }
-  auto final_index = [&](uint32_t r) { return (r & SMALL_REF) ? hbases[r & ~SMALL_REF] : pre_top[r]; };
-  std::vector<TopPut> puts(top.size());
-  for (size_t t = 0; t < top.size(); t++) {
-    TopPut &p = puts[t];
-    const HostTop &h = top[t];
-    for (int k = 0; k < 3; k++) {
-      p.node.min[k] = h.lo[k];
-      p.node.max[k] = h.hi[k];
-    }
-    p.node.leaf = h.leaf;
-    p.node.axis = h.leaf ? INVALID_ID : h.axis;
-    p.node.children[0] = h.leaf ? INVALID_ID : final_index(h.child[0]);
-    p.node.children[1] = h.leaf ? INVALID_ID : final_index(h.child[1]);
-    p.node.prim_begin = h.leaf ? h.begin : 0u;
-    p.node.prim_count = h.leaf ? h.n : 0u;
-    p.pre = pre_top[t];
-    p.pad = 0;
-  }
+  // ---- numbering
+  const uint32_t M = 2u * leaves - 1u;
   brt_tree_node *tree = A.get<brt_tree_node>(M);
-  const TopPut *d_puts = nullptr;
+  uint32_t *ni = A.get<uint32_t>(M);
   BRT_CHECK(A.err);
-  BRT_CHECK(to_device(A, puts.data(), puts.size(), &d_puts, st));
-  BRT_CHECK(hipMemcpyAsync(bases, hbases.data(), ns * 4, hipMemcpyHostToDevice, st));
-  if (!puts.empty())
-    BRT_LAUNCH(k_put_top<<<blocks_for(puts.size(), 64), 64, 0, st>>>(d_puts, (uint32_t)puts.size(), tree));
-  if (ns) BRT_LAUNCH(k_reloc<<<ns, 256, 0, st>>>(d_small, sizes, bases, tmp, tree));
+  BRT_LAUNCH(k_emit<<<blocks_for(n, 256), 256, 0, st>>>(raw, n, before, tree, ni));
 
   // ---- flatten
-  uint32_t *internal = A.get<uint32_t>(M), *islots = A.get<uint32_t>(M), *ni = A.get<uint32_t>(M),
-           *S = A.get<uint32_t>(M), *k4 = A.get<uint32_t>(M), *is_root = A.get<uint32_t>(M);
+  uint32_t *islots = A.get<uint32_t>(M), *S = A.get<uint32_t>(M), *k4 = A.get<uint32_t>(M),
+           *is_root = A.get<uint32_t>(M);
   BRT_CHECK(A.err);
   BRT_LAUNCH(k_roots4<<<blocks_for(M, 256), 256, 0, st>>>(tree, M, is_root));
-  BRT_LAUNCH(k_flags<<<blocks_for(M, 256), 256, 0, st>>>(tree, is_root, M, internal, islots));
-  size_t tb1 = 0, tb2 = 0;
-  BRT_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb1, internal, ni, (int)M, st));
+  BRT_LAUNCH(k_flags<<<blocks_for(M, 256), 256, 0, st>>>(tree, is_root, M, islots));
+  size_t tb2 = 0;
   BRT_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb2, islots, S, (int)M, st));
-  unsigned char *tstore = A.get<unsigned char>(std::max(tb1, tb2));
+  unsigned char *tstore = A.get<unsigned char>(tb2);
   BRT_CHECK(A.err);
-  BRT_CHECK(hipcub::DeviceScan::ExclusiveSum(tstore, tb1, internal, ni, (int)M, st));
   BRT_CHECK(hipcub::DeviceScan::ExclusiveSum(tstore, tb2, islots, S, (int)M, st));
-  uint32_t last[4] = {0, 0, 0, 0};
-  BRT_CHECK(hipMemcpyAsync(&last[0], ni + M - 1, 4, hipMemcpyDeviceToHost, st));
-  BRT_CHECK(hipMemcpyAsync(&last[1], internal + M - 1, 4, hipMemcpyDeviceToHost, st));
-  BRT_CHECK(hipMemcpyAsync(&last[2], S + M - 1, 4, hipMemcpyDeviceToHost, st));
-  BRT_CHECK(hipMemcpyAsync(&last[3], islots + M - 1, 4, hipMemcpyDeviceToHost, st));
+  uint32_t last[2] = {0, 0};
+  BRT_CHECK(hipMemcpyAsync(&last[0], S + M - 1, 4, hipMemcpyDeviceToHost, st));
+  BRT_CHECK(hipMemcpyAsync(&last[1], islots + M - 1, 4, hipMemcpyDeviceToHost, st));
   BRT_CHECK(hipMemcpyAsync(&out.root, tree, sizeof(brt_tree_node), hipMemcpyDeviceToHost, st));
   BRT_CHECK(hipStreamSynchronize(st));
-  const uint32_t n64 = last[0] + last[1];
-  const uint32_t n4 = out.root.leaf ? 0u : 1u + last[2] + last[3];
+  const uint32_t n64 = leaves - 1u;
+  const uint32_t n4 = out.root.leaf ? 0u : 1u + last[0] + last[1];
   Node64 *nodes64 = A.get<Node64>(n64);
   Node4 *nodes4 = A.get<Node4>(n4);
   uint32_t *ord4 = A.get<uint32_t>(2ull * n4);
@@ -1317,8 +1567,8 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
   out.recs = recs;
   out.rec_size = rec_size;
   out.max_depth = std::max(hs.max_depth, ds.max_depth);
-  out.leaves = hs.leaves + ds.leaves;
-  out.branches = hs.branches + ds.branches;
+  out.leaves = leaves;
+  out.branches = leaves - 1u;
   out.bad_splits = hs.bad + ds.bad;
   out.max_prims = std::max(hs.max_prims, ds.max_prims);
   out.min_prims = std::min(hs.min_prims, ds.min_prims);
