@@ -1252,18 +1252,19 @@ __global__ void k_cyl_recs(const uint32_t *__restrict__ order, const double *__r
 // ------------------------------------------------------------------------------------------------ host driver
 inline uint32_t blocks_for(uint64_t n, uint32_t t) { return (uint32_t)((n + t - 1) / t); }
 
-// Device allocations of one build; temporaries are released by the destructor (after the build's stream has
+// Device allocations of one build; temporaries go back to the pool in the destructor (after the build's stream has
 // drained, also on an error path), results are handed over.
 struct Arena {
   hipStream_t stream;
+  int device = -1;
   std::vector<void *> ptrs;
   hipError_t err = hipSuccess;
-  explicit Arena(hipStream_t s) : stream(s) {}
+  explicit Arena(hipStream_t s) : stream(s) { err = hipGetDevice(&device); }
   template <class T>
   T *get(size_t count) {
     if (err != hipSuccess) return nullptr;
     void *p = nullptr;
-    err = hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T));
+    err = pool_get(device, std::max<size_t>(count, 1) * sizeof(T), &p);
     if (err != hipSuccess) return nullptr;
     ptrs.push_back(p);
     return static_cast<T *>(p);
@@ -1273,9 +1274,9 @@ struct Arena {
       if (q == p) q = nullptr;
   }
   ~Arena() {
-    (void)hipStreamSynchronize(stream);
+    const bool idle = hipStreamSynchronize(stream) == hipSuccess;
     for (void *p : ptrs)
-      if (p) (void)hipFree(p);
+      if (p) pool_put(device, p, idle);
   }
 };
 

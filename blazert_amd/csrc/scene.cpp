@@ -23,6 +23,7 @@
 #include <string>
 #include <thread>
 #include <type_traits>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/blazert_amd.h"
@@ -816,6 +817,36 @@ void build_geometry(GeometryT<R> &g, GeomType type, const brt_build_options &o) 
 }
 
 // ------------------------------------------------------------------------------------------------ device
+struct DevicePool {
+  struct Block {
+    void *p;
+    size_t bytes;
+    bool idle;
+  };
+  std::mutex mu;
+  std::vector<Block> free_blocks;
+  std::unordered_map<void *, size_t> sizes;  // every block handed out
+  size_t held = 0;                           // bytes in free_blocks
+  int users = 0;                             // scenes on the device
+};
+
+// One pool per device; never destroyed, since the HIP runtime may end before static objects do.
+DevicePool &pool_of(int device) {
+  static std::mutex mu;
+  static auto *pools = new std::unordered_map<int, std::unique_ptr<DevicePool>>();
+  std::lock_guard<std::mutex> lk(mu);
+  auto &p = (*pools)[device];
+  if (!p) p = std::make_unique<DevicePool>();
+  return *p;
+}
+
+// Frees every kept block; the caller holds the pool's mutex.
+void pool_trim(DevicePool &P) {
+  for (auto &b : P.free_blocks) (void)hipFree(b.p);
+  P.free_blocks.clear();
+  P.held = 0;
+}
+
 struct DeviceScene {
   int device = -1;
   std::vector<void *> allocs;
@@ -829,11 +860,19 @@ struct DeviceScene {
   double *leaf_vertices = nullptr;    // triangles' vertices in leaf order, made on the first closest-surface query
   std::mutex sort_mu;
   std::vector<std::pair<hipStream_t, std::unique_ptr<SortWorkspace>>> sorts;  // one ray-sort workspace per stream
+  explicit DeviceScene(int dev) : device(dev) { pool_retain(device); }
   ~DeviceScene() {
     for (auto &w : sorts)
       if (w.second->base) (void)hipFree(w.second->base);
-    for (auto &c : stream_counters) (void)hipFree(c.second);
-    for (void *p : allocs) (void)hipFree(p);
+    for (auto &c : stream_counters) pool_put(device, c.second, false);
+    for (void *p : allocs) pool_put(device, p, false);
+    pool_release(device);
+  }
+  // Device memory that lives as long as the scene.
+  hipError_t alloc(size_t bytes, void **p) {
+    const hipError_t e = pool_get(device, bytes, p);
+    if (e == hipSuccess) allocs.push_back(*p);
+    return e;
   }
   // The counter group of `st`, allocated on the stream's first launch (NULL if that allocation fails).
   unsigned long long *counter_group(hipStream_t st) {
@@ -841,7 +880,7 @@ struct DeviceScene {
     for (auto &c : stream_counters)
       if (c.first == st) return c.second;
     void *p = nullptr;
-    if (hipMalloc(&p, COUNTER_GROUP * sizeof(unsigned long long)) != hipSuccess) return nullptr;
+    if (pool_get(device, COUNTER_GROUP * sizeof(unsigned long long), &p) != hipSuccess) return nullptr;
     stream_counters.emplace_back(st, static_cast<unsigned long long *>(p));
     return stream_counters.back().second;
   }
@@ -857,9 +896,8 @@ struct DeviceScene {
     *dst = nullptr;
     if (v.empty()) return hipSuccess;
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, v.size() * sizeof(T));
+    hipError_t e = alloc(v.size() * sizeof(T), &p);
     if (e != hipSuccess) return e;
-    allocs.push_back(p);
     e = hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice);
     *dst = static_cast<const T *>(p);
     return e;
@@ -870,6 +908,66 @@ struct DeviceScene {
 }  // namespace brt
 
 namespace brt {
+
+hipError_t pool_get(int device, size_t bytes, void **p) {
+  // sizes in steps of a sixteenth, so that a scene rebuilt with a few nodes more finds the blocks of the last one
+  size_t step = 4096;
+  while (step * 32 <= bytes) step *= 2;
+  const size_t want = (bytes + step - 1) / step * step;
+  DevicePool &P = pool_of(device);
+  std::lock_guard<std::mutex> lk(P.mu);
+  auto best = P.free_blocks.end();
+  for (auto it = P.free_blocks.begin(); it != P.free_blocks.end(); ++it)
+    if (it->bytes >= want && it->bytes <= want + want / 4 && (best == P.free_blocks.end() || it->bytes < best->bytes))
+      best = it;
+  if (best != P.free_blocks.end()) {
+    if (!best->idle) {
+      const hipError_t e = hipDeviceSynchronize();
+      if (e != hipSuccess) return e;
+      for (auto &b : P.free_blocks) b.idle = true;
+    }
+    *p = best->p;
+    P.held -= best->bytes;
+    P.sizes[best->p] = best->bytes;
+    P.free_blocks.erase(best);
+    return hipSuccess;
+  }
+  hipError_t e = hipMalloc(p, want);
+  if (e == hipErrorOutOfMemory && !P.free_blocks.empty()) {
+    (void)hipGetLastError();
+    pool_trim(P);
+    e = hipMalloc(p, want);
+  }
+  if (e == hipSuccess) P.sizes[*p] = want;
+  return e;
+}
+
+void pool_put(int device, void *p, bool idle) {
+  if (!p) return;
+  DevicePool &P = pool_of(device);
+  std::lock_guard<std::mutex> lk(P.mu);
+  const auto it = P.sizes.find(p);
+  const size_t bytes = it == P.sizes.end() ? 0 : it->second;
+  if (it != P.sizes.end()) P.sizes.erase(it);
+  if (!bytes || P.users == 0 || P.held + bytes > POOL_BYTES) {
+    (void)hipFree(p);
+    return;
+  }
+  P.free_blocks.push_back({p, bytes, idle});
+  P.held += bytes;
+}
+
+void pool_retain(int device) {
+  DevicePool &P = pool_of(device);
+  std::lock_guard<std::mutex> lk(P.mu);
+  P.users++;
+}
+
+void pool_release(int device) {
+  DevicePool &P = pool_of(device);
+  std::lock_guard<std::mutex> lk(P.mu);
+  if (--P.users == 0) pool_trim(P);
+}
 
 int check_launch(const brt_launch &L) {
   if (L.precision > BRT_PRECISION_FP32_TRAV_FP64_HIT) return fail(BRT_ERR_INVALID_ARGUMENT, "unknown precision");
@@ -938,9 +1036,7 @@ int double_only(const brt_scene *s, const char *what) {
 }
 
 hipError_t new_device_scene(int dev, std::unique_ptr<DeviceScene> &out) {
-  auto d = std::make_unique<DeviceScene>();
-  d->device = dev;
-  out = std::move(d);
+  out = std::make_unique<DeviceScene>(dev);
   return hipSuccess;
 }
 
@@ -978,9 +1074,8 @@ hipError_t make_prim_filter(DeviceScene &d, BvhView &v, uint32_t type, double ex
   const size_t bytes = type == TRIANGLES ? (size_t)(v.n_prims + FILTER_PAD) * sizeof(TriFilt)
                                          : (size_t)(v.n_prims + SPH_FILTER_PAD) * sizeof(SphFilt);
   void *p = nullptr;
-  hipError_t e = hipMalloc(&p, bytes);
+  hipError_t e = d.alloc(bytes, &p);
   if (e != hipSuccess) return e;
-  d.allocs.push_back(p);
   e = type == TRIANGLES ? launch_tri_filter_records(v.prims, v.n_prims, p, st)
       : type == SPHERES  ? launch_sph_filter_records(v.prims, v.n_prims, p, st)
                          : launch_cyl_filter_records(v.prims, v.n_prims, p, st);
@@ -1000,9 +1095,8 @@ hipError_t make_nodesq(DeviceScene &d, BvhView &v, const Geometry &g, uint32_t n
   if (!g.extent_ok || v.irregular_boxes || max_leaf > NODEQ_MAX_LEAF) return hipSuccess;
   const size_t bytes = std::max<size_t>(num_n4, 1) * sizeof(NodeQ);  // a root leaf has no records
   void *p = nullptr;
-  hipError_t e = hipMalloc(&p, bytes);
+  hipError_t e = d.alloc(bytes, &p);
   if (e != hipSuccess) return e;
-  d.allocs.push_back(p);
   if (num_n4) e = launch_nodeq_records(v.nodes4, ord4, num_n4, static_cast<NodeQ *>(p), st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   v.nodesq = static_cast<const NodeQ *>(p);
@@ -1143,7 +1237,7 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
     if (r.refused) {
       for (const void *p : {(const void *)v.faces, (const void *)v.vertices}) {
         d->allocs.erase(std::remove(d->allocs.begin(), d->allocs.end(), p), d->allocs.end());
-        (void)hipFree(const_cast<void *>(p));
+        pool_put(dev, const_cast<void *>(p), true);
       }
       if (int rc = on_host()) return rc;
       continue;
@@ -1519,9 +1613,8 @@ int brt_distance_to_surface(const brt_scene *cs, uint32_t type, const brt_points
     uint32_t *&slot = s->dev->inv_order[type];
     if (!slot) {
       void *p = nullptr;
-      hipError_t e = hipMalloc(&p, (size_t)g.boxes.n * 4);
+      hipError_t e = s->dev->alloc((size_t)g.boxes.n * 4, &p);
       if (e != hipSuccess) return device_error(e, "inverse order allocation");
-      s->dev->allocs.push_back(p);
       e = launch_inverse_order(v.prim_ids, g.boxes.n, static_cast<uint32_t *>(p), st);
       if (e == hipSuccess) e = hipStreamSynchronize(st);  // complete before a query on another stream reads it
       if (e != hipSuccess) return device_error(e, "launch failed");
@@ -1558,9 +1651,8 @@ int brt_closest_surface(const brt_scene *cs, const brt_points *points, uint64_t 
       const Geometry &g = s->geo[TRIANGLES];
       const BvhView &v = s->dev->views[TRIANGLES];
       void *p = nullptr;
-      hipError_t e = hipMalloc(&p, (size_t)g.boxes.n * 9 * sizeof(double));
+      hipError_t e = s->dev->alloc((size_t)g.boxes.n * 9 * sizeof(double), &p);
       if (e != hipSuccess) return device_error(e, "leaf-order vertex allocation");
-      s->dev->allocs.push_back(p);
       const hipStream_t st = static_cast<hipStream_t>(stream);
       e = launch_leaf_vertices(v.prim_ids, v.faces, v.vertices, g.boxes.n, static_cast<double *>(p), st);
       if (e == hipSuccess) e = hipStreamSynchronize(st);  // complete before a query on another stream reads it
