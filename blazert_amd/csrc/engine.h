@@ -168,6 +168,10 @@ hipError_t launch_zero_counters(unsigned long long *group, hipStream_t stream);
 // Enqueues the traversal of one geometry type over n rays on `stream` (asynchronous).
 hipError_t launch_trace(GeomType type, const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint64_t n,
                         const TraceLaunch &cfg, const SplitParams &split, hipStream_t stream);
+// The closest hit of one ray (index 0) among the triangles of an FP64 scene whose view has nodesq. hits.merged is required
+// and set to RAY_LEFT where the ray needs launch_trace, and nothing else is then written.
+hipError_t launch_tri_lone(const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint32_t flags,
+                           const SplitParams &split, hipStream_t stream);
 
 // Mirror tracing: the next bounce's rays from this bounce's hits (positions o + t normalize(d), mirror directions;
 // NaN for misses). pos / dir are x, y, z arrays of n doubles.
@@ -226,6 +230,11 @@ hipError_t launch_closest_surface(const ClosestViews &views, const double *px, c
 constexpr size_t POOL_BYTES = 2ull << 30;
 hipError_t pool_get(int device, size_t bytes, void **p);
 void pool_put(int device, void *p, bool idle);
+// Host memory that kernels read and write in place, LONE_SLOT_BYTES of it: kept and given back like the device memory, up
+// to LONE_SLOTS of them. The caller has waited for the kernels that use it (`idle`), or it isn't kept.
+constexpr size_t LONE_SLOT_BYTES = 256, LONE_SLOTS = 64;
+hipError_t pool_get_slot(int device, void **p);
+void pool_put_slot(int device, void *p, bool idle);
 void pool_retain(int device);
 void pool_release(int device);
 

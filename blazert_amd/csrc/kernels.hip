@@ -1658,8 +1658,9 @@ __device__ __forceinline__ unsigned long long bound_of(float h32, uint32_t pos) 
   return ((unsigned long long)__float_as_uint(h32) << 32) | pos;  // h32 >= 0: its bits order as it does
 }
 
-// Persistent waves as in k_trace_persistent. BATCH: the rays of many jobs, as in k_trace_batch.
-template <bool BATCH>
+// Persistent waves as in k_trace_persistent. BATCH: the rays of many jobs, as in k_trace_batch. LONE: one ray by one wave,
+// without counters; where it would be listed or deferred, `merged` says so (RAY_LEFT) and nothing else is written.
+template <bool BATCH, bool LONE = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BRT_WAVES_PER_EU)))
 k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t n,
             uint32_t flags, uint32_t first, double S, unsigned long long *group, uint32_t refill,
@@ -1716,9 +1717,13 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
     if (done) {
       done = false;
       if (t.listed) {
-        const unsigned long long k = atomicAdd(group + COUNTER_LISTED, 1ull);
-        if (k < (unsigned long long)LIST_CAPACITY) {
-          group[COUNTER_CLEARED + k] = BATCH ? jobs[j].offset + idx : idx;
+        if constexpr (LONE) {
+          st_stream(lds_fresh<HitsView>(views + RW).merged, idx, RAY_LEFT);
+        } else {
+          const unsigned long long k = atomicAdd(group + COUNTER_LISTED, 1ull);
+          if (k < (unsigned long long)LIST_CAPACITY) {
+            group[COUNTER_CLEARED + k] = BATCH ? jobs[j].offset + idx : idx;
+          }
         }
       } else {
         r.tmax = s.leaf_idx == INVALID_ID ? -__builtin_inf() : __builtin_inf();  // hit or not, for finish_ray
@@ -1815,6 +1820,8 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
             has_ray = true;
             s.leaf_idx = INVALID_ID;
             t.active = t.listed = false;
+          } else if constexpr (LONE) {
+            st_stream(lds_fresh<HitsView>(views + RW).merged, idx, RAY_LEFT);
           } else {
             __atomic_store_n(group + COUNTER_DEFERRED, 1ull, __ATOMIC_RELAXED);
           }
@@ -2280,6 +2287,16 @@ hipError_t launch_trace(GeomType type, const BvhView &bvh, const RaysView &rays,
   case PLANES: return launch_typed<PlaRec>(bvh, rays, hits, n, cfg, split, cfg.overwrite ? 1u : 0u, stream);
   default: return launch_typed<CylRec>(bvh, rays, hits, n, cfg, split, cfg.overwrite ? 1u : 0u, stream);
   }
+}
+
+// The closest hit of one ray among the triangles, by a wave whose lanes share the ray's tree: the chain of dependent
+// reads bounds it, which one lane alone follows through every node. `hits.merged` is required.
+hipError_t launch_tri_lone(const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint32_t flags,
+                           const SplitParams &sp, hipStream_t stream) {
+  hipLaunchKernelGGL((k_trace_tri<false, true>), dim3(1), dim3(64), tri_lds_bytes(64, TRI_RING), stream, bvh, rays, hits,
+                     (const BatchJob *)nullptr, 0u, (uint64_t)1, flags, 0u, sp.scene_extent,
+                     (unsigned long long *)nullptr, TRI_REFILL, (const uint32_t *)nullptr, TRI_RING, POOL_CHUNK, 1u);
+  return hipGetLastError();
 }
 
 hipError_t launch_sph_filter_records(const void *recs, uint32_t n, void *out, hipStream_t stream) {

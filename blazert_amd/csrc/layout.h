@@ -213,12 +213,14 @@ struct RaysViewT {
   R tmin0 = R(0);
   R tmax0 = std::numeric_limits<R>::max();
 };
+constexpr uint32_t RAY_LEFT = 2u;  // in HitsViewT::merged: a kernel left the ray to another one
+
 template <class R>
 struct HitsViewT {
   R *t, *u, *v;
   uint32_t *prim_id, *geom_id;
   R *nx, *ny, *nz;
-  uint32_t *merged;  // optional: set to 1 where a geometry type's hit was merged (intersect1's return value)
+  uint32_t *merged;  // optional: set to 1 where a geometry type's hit was merged (intersect1's return value), or RAY_LEFT
 };
 using RaysView = RaysViewT<double>;
 using HitsView = HitsViewT<double>;

@@ -827,6 +827,7 @@ struct DevicePool {
   std::vector<Block> free_blocks;
   std::unordered_map<void *, size_t> sizes;  // every block handed out
   size_t held = 0;                           // bytes in free_blocks
+  std::vector<void *> slots;                 // kept host memory (pool_get_slot)
   int users = 0;                             // scenes on the device
 };
 
@@ -845,6 +846,8 @@ void pool_trim(DevicePool &P) {
   for (auto &b : P.free_blocks) (void)hipFree(b.p);
   P.free_blocks.clear();
   P.held = 0;
+  for (void *p : P.slots) (void)hipHostFree(p);
+  P.slots.clear();
 }
 
 struct DeviceScene {
@@ -955,6 +958,31 @@ void pool_put(int device, void *p, bool idle) {
   }
   P.free_blocks.push_back({p, bytes, idle});
   P.held += bytes;
+}
+
+hipError_t pool_get_slot(int device, void **p) {
+  DevicePool &P = pool_of(device);
+  {
+    std::lock_guard<std::mutex> lk(P.mu);
+    if (!P.slots.empty()) {
+      *p = P.slots.back();
+      P.slots.pop_back();
+      return hipSuccess;
+    }
+  }
+  return hipHostMalloc(p, LONE_SLOT_BYTES, hipHostMallocMapped | hipHostMallocPortable);
+}
+
+void pool_put_slot(int device, void *p, bool idle) {
+  DevicePool &P = pool_of(device);
+  if (idle) {
+    std::lock_guard<std::mutex> lk(P.mu);
+    if (P.users && P.slots.size() < LONE_SLOTS) {
+      P.slots.push_back(p);
+      return;
+    }
+  }
+  (void)hipHostFree(p);
 }
 
 void pool_retain(int device) {
@@ -1418,56 +1446,64 @@ template <class R, class H>
 int intersect1_t(const brt_scene *s, const R org[3], const R dir[3], R tmin, R tmax, uint32_t flags, H *hit,
                  int *hit_out) {
   if (!s || !org || !dir || !hit) return fail(BRT_ERR_INVALID_ARGUMENT, "NULL argument");
-  // one ray through the batched kernels, keeping RayHit's in/out semantics: 8 ray values, 6 hit values,
-  // then prim id, geom id and the merged flag
-  R host[14] = {org[0], org[1], org[2], dir[0], dir[1], dir[2], tmin, tmax,
-                     hit->t, hit->u, hit->v, hit->normal[0], hit->normal[1], hit->normal[2]};
-  uint32_t ids[3] = {hit->prim_id, hit->geom_id, 0u};
-  char *d = nullptr;
-  hipError_t e = hipMalloc(reinterpret_cast<void **>(&d), sizeof host + sizeof ids);
-  if (e != hipSuccess) return fail(BRT_ERR_DEVICE, std::string("hipMalloc: ") + hipGetErrorString(e));
-  R *dd = reinterpret_cast<R *>(d);
-  uint32_t *di = reinterpret_cast<uint32_t *>(d + sizeof host);
-  e = hipMemcpy(d, host, sizeof host, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(di, ids, sizeof ids, hipMemcpyHostToDevice);
-  int rc = BRT_OK;
   brt_scene *ms = const_cast<brt_scene *>(s);
-  if (e == hipSuccess && !ms->committed) rc = fail(BRT_ERR_STATE, "scene not committed");
-  if (e == hipSuccess && rc == BRT_OK) rc = upload(ms);
-  if (e == hipSuccess && rc == BRT_OK) {
-    RaysViewT<R> rv{dd, dd + 1, dd + 2, dd + 3, dd + 4, dd + 5, dd + 6, dd + 7};
-    HitsViewT<R> hv{dd + 8, dd + 9, dd + 10, di, di + 1, dd + 11, dd + 12, dd + 13, di + 2};
-    for (uint32_t t = 0; t < NUM_TYPES && e == hipSuccess; t++) {
-      const GeometryT<R> &g = geo_of<R>(ms)[t];
-      if (!g.present || g.boxes.n == 0) continue;
-      TraceLaunch cfg{BRT_PRECISION_FP64, flags | BRT_FLAG_HITS_INOUT, 64, false, SCHEDULE_PER_THREAD, 0,
-                      ms->dev->counter_group(nullptr), nullptr};
-      if (!cfg.counter) {
-        e = hipErrorOutOfMemory;
-        break;
+  if (!ms->committed) return fail(BRT_ERR_STATE, "scene not committed");
+  if (int rc = upload(ms)) return rc;
+  // One ray through the batched kernels, keeping RayHit's in/out semantics. The ray and its hit stand in host memory that
+  // the kernels read and write in place: a few words across the link cost about 2 us, against four copies and a device
+  // allocation around the launch (one ray, 5,120 triangles: 106 us a call with those).
+  struct Slot {
+    R ray[8], hit[6];  // origin, direction, tmin, tmax; t, u, v, normal
+    uint32_t prim_id, geom_id, merged;
+  };
+  static_assert(sizeof(Slot) <= LONE_SLOT_BYTES, "one ray and its hit");
+  const int dev = ms->dev->device;
+  void *mem = nullptr;
+  hipError_t e = pool_get_slot(dev, &mem);
+  if (e != hipSuccess) return fail(BRT_ERR_DEVICE, std::string("hipHostMalloc: ") + hipGetErrorString(e));
+  Slot *q = new (mem) Slot{{org[0], org[1], org[2], dir[0], dir[1], dir[2], tmin, tmax},
+                           {hit->t, hit->u, hit->v, hit->normal[0], hit->normal[1], hit->normal[2]},
+                           hit->prim_id, hit->geom_id, 0u};
+  const RaysViewT<R> rv{&q->ray[0], &q->ray[1], &q->ray[2], &q->ray[3], &q->ray[4], &q->ray[5], &q->ray[6], &q->ray[7]};
+  const HitsViewT<R> hv{&q->hit[0], &q->hit[1], &q->hit[2], &q->prim_id, &q->geom_id,
+                        &q->hit[3], &q->hit[4], &q->hit[5], &q->merged};
+  bool pending = false;
+  for (uint32_t t = 0; t < NUM_TYPES && e == hipSuccess; t++) {
+    const GeometryT<R> &g = geo_of<R>(ms)[t];
+    if (!g.present || g.boxes.n == 0) continue;
+    if constexpr (std::is_same<R, double>::value) {
+      if (t == TRIANGLES && ms->dev->views[t].nodesq && !(flags & BRT_FLAG_ANY_HIT)) {
+        e = launch_tri_lone(ms->dev->views[t], rv, hv, flags | BRT_FLAG_HITS_INOUT, SplitParams{g.extent}, nullptr);
+        if (e == hipSuccess) e = hipDeviceSynchronize();
+        if (e != hipSuccess || q->merged != RAY_LEFT) continue;
+        q->merged = 0u;
       }
-      if constexpr (std::is_same<R, float>::value)
-        e = launch_trace_f32((GeomType)t, ms->dev->views[t], rv, hv, 1, cfg, nullptr);
-      else
-        e = launch_trace((GeomType)t, ms->dev->views[t], rv, hv, 1, cfg, SplitParams{g.extent}, nullptr);
     }
-    if (e == hipSuccess) e = hipDeviceSynchronize();
-    if (e == hipSuccess) e = hipMemcpy(host, d, sizeof host, hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(ids, di, sizeof ids, hipMemcpyDeviceToHost);
-    if (e == hipSuccess) {
-      hit->t = host[8];
-      hit->u = host[9];
-      hit->v = host[10];
-      hit->normal[0] = host[11];
-      hit->normal[1] = host[12];
-      hit->normal[2] = host[13];
-      hit->prim_id = ids[0];
-      hit->geom_id = ids[1];
-      if (hit_out) *hit_out = ids[2] ? 1 : 0;
+    TraceLaunch cfg{BRT_PRECISION_FP64, flags | BRT_FLAG_HITS_INOUT, 64, false, SCHEDULE_PER_THREAD, 0,
+                    ms->dev->counter_group(nullptr), nullptr};
+    if (!cfg.counter) {
+      e = hipErrorOutOfMemory;
+      break;
     }
+    if constexpr (std::is_same<R, float>::value)
+      e = launch_trace_f32((GeomType)t, ms->dev->views[t], rv, hv, 1, cfg, nullptr);
+    else
+      e = launch_trace((GeomType)t, ms->dev->views[t], rv, hv, 1, cfg, SplitParams{g.extent}, nullptr);
+    if (e == hipSuccess) pending = true;
   }
-  (void)hipFree(d);
-  if (rc != BRT_OK) return rc;
+  if (e == hipSuccess && pending) e = hipDeviceSynchronize();
+  if (e == hipSuccess) {
+    hit->t = q->hit[0];
+    hit->u = q->hit[1];
+    hit->v = q->hit[2];
+    hit->normal[0] = q->hit[3];
+    hit->normal[1] = q->hit[4];
+    hit->normal[2] = q->hit[5];
+    hit->prim_id = q->prim_id;
+    hit->geom_id = q->geom_id;
+    if (hit_out) *hit_out = q->merged ? 1 : 0;
+  }
+  pool_put_slot(dev, mem, e == hipSuccess);
   if (e != hipSuccess) return fail(BRT_ERR_DEVICE, std::string("intersect1: ") + hipGetErrorString(e));
   return BRT_OK;
 }
