@@ -1798,16 +1798,16 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
               take(jobs[j]);
             }
           }
-        } else if (got) {
+        } else if (LONE || got) {
           idx = order ? (uint64_t)order[cand] : cand;
           root = tri_root(bvh);
           raw = load_ray(lds_fresh<RaysView>(views), idx);
         }
-        if (got) {
+        if (LONE || got) {
           setup_ray(raw.org, raw.dir, raw.tmin, raw.tmax, r);
           const double len2 = squared_length(raw);
           if (fast_ray(r, len2, ext)) {
-            has_ray = true;
+            has_ray = got;
             make_rayq(r, len2, ext, q);
             s.h = r.tmax;
             s.u = s.v = 0.0;
@@ -1817,7 +1817,7 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
           } else if (r.o[2] != r.o[2] || r.inv[2] != r.inv[2]) {
             // NaN far-plane terms on the last axis: the reference rejects every box, the root first (a mirror ray
             // that has left the scene)
-            has_ray = true;
+            has_ray = got;
             s.leaf_idx = INVALID_ID;
             t.active = t.listed = false;
           } else if constexpr (LONE) {
@@ -1836,8 +1836,9 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
       }
       const unsigned long long can = __ballot(has_ray && st.sp > st.bot);
       const uint32_t nidle = 64u - (uint32_t)__popcll(busy);
-      // in every other iteration: sharing costs about as many instructions as a traversal step (every one: 3-5% slower)
-      if (nidle >= SHARE_MIN_IDLE && can && (++turn & 1u) == 0u) {
+      // in every other iteration: sharing costs about as many instructions as a traversal step (every one: 3-5% slower);
+      // a lone ray has the instruction slots to itself and shares in every one (41.4 -> 38.4 us a call; not at all: 46.0 us)
+      if (nidle >= SHARE_MIN_IDLE && can && (LONE || (++turn & 1u) == 0u)) {
         write_rays();  // the helpers' state is overwritten
         const unsigned long long below = (1ull << lane) - 1ull;
         const uint32_t ncan = (uint32_t)__popcll(can), k = nidle < ncan ? nidle : ncan;
@@ -1870,14 +1871,16 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
         const uint32_t from = lane_get(by_rank, (int)rank);  // with all lanes: a permute reads active lanes only
         const int src = helper ? (int)from : (int)lane;
         lane_take(e, src, helper);
-        lane_take(r.o, src, helper);
-        lane_take(r.d, src, helper);
-        lane_take(r.tmin, src, helper);
-        lane_take(q, src, helper);
+        if constexpr (!LONE) {  // all lanes hold a lone ray, in slot 0
+          lane_take(r.o, src, helper);
+          lane_take(r.d, src, helper);
+          lane_take(r.tmin, src, helper);
+          lane_take(q, src, helper);
+          lane_take(idx, src, helper);
+          lane_take(slot, src, helper);
+        }
         lane_take(s.h, src, helper);
         lane_take(t.h32, src, helper);
-        lane_take(idx, src, helper);
-        lane_take(slot, src, helper);
         {
           const uint32_t from_end = lane_get(pos_end, src), old_end = lane_get(pos_end0, src);
           pos = helper ? from_end : pos;
