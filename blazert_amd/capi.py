@@ -135,6 +135,7 @@ SIGNATURES = {
     "brt_scene_upload": (C.c_int, [_P]),
     "brt_scene_commit_device": (C.c_int, [_P, _P]),
     "brt_distance_to_surface": (C.c_int, [_P, C.c_uint32, C.POINTER(Points), _P, C.c_uint64, _P, _P]),
+    "brt_rows_to_columns": (C.c_int, [_P, C.c_uint32, C.c_uint64, _P, _P]),
     "brt_closest_surface": (C.c_int, [_P, C.POINTER(Points), C.c_uint64, _P, _P, _P, _P]),
     "brt_scene_read_device_array": (C.c_int, [_P, C.c_uint32, C.c_uint32, C.c_void_p, C.c_uint64,
                                               C.POINTER(C.c_uint64)]),

@@ -168,6 +168,8 @@ hipError_t launch_zero_counters(unsigned long long *group, hipStream_t stream);
 // Enqueues the traversal of one geometry type over n rays on `stream` (asynchronous).
 hipError_t launch_trace(GeomType type, const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint64_t n,
                         const TraceLaunch &cfg, const SplitParams &split, hipStream_t stream);
+// n rows of three elements (4 or 8 bytes each) to three columns of n, one after another.
+hipError_t launch_rows_to_columns(const void *rows, uint32_t elem_bytes, uint64_t n, void *columns, hipStream_t stream);
 // The closest hit of one ray (index 0) among the triangles of an FP64 scene whose view has nodesq. hits.merged is required
 // and set to RAY_LEFT where the ray needs launch_trace, and nothing else is then written.
 hipError_t launch_tri_lone(const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint32_t flags,

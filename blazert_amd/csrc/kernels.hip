@@ -2112,6 +2112,31 @@ __global__ void k_init_hits(HitsViewT<R> hits, uint64_t n) {
 }
 
 // Blocks of a persistent launch: as many as fit on the device at once, but no more than the rays need.
+// (n, 3) rows to three columns of n. Memory bound: the rows are read once (the second and third loads of a wave hit the
+// lines of the first) and each column written in whole lines.
+constexpr uint32_t ROWS_PER_THREAD = 4;
+template <class T>
+__global__ void __launch_bounds__(256) k_rows_to_columns(const T *__restrict__ rows, uint64_t n, T *__restrict__ x,
+                                                         T *__restrict__ y, T *__restrict__ z) {
+  const uint64_t i0 = (uint64_t)blockIdx.x * (256u * ROWS_PER_THREAD) + threadIdx.x;
+  T r[ROWS_PER_THREAD][3];
+#pragma unroll
+  for (uint32_t k = 0; k < ROWS_PER_THREAD; k++) {
+    const uint64_t i = i0 + k * 256u;
+    if (i < n)
+      for (int a = 0; a < 3; a++) r[k][a] = rows[3 * i + a];
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < ROWS_PER_THREAD; k++) {
+    const uint64_t i = i0 + k * 256u;
+    if (i < n) {
+      x[i] = r[k][0];
+      y[i] = r[k][1];
+      z[i] = r[k][2];
+    }
+  }
+}
+
 template <class K>
 hipError_t persistent_blocks(K kernel, uint32_t block, size_t lds, uint64_t n, uint64_t &blocks) {
   int dev = 0, cus = 0, per_cu = 0;
@@ -2299,6 +2324,21 @@ hipError_t launch_tri_lone(const BvhView &bvh, const RaysView &rays, const HitsV
   hipLaunchKernelGGL((k_trace_tri<false, true>), dim3(1), dim3(64), tri_lds_bytes(64, TRI_RING), stream, bvh, rays, hits,
                      (const BatchJob *)nullptr, 0u, (uint64_t)1, flags, 0u, sp.scene_extent,
                      (unsigned long long *)nullptr, TRI_REFILL, (const uint32_t *)nullptr, TRI_RING, POOL_CHUNK, 1u);
+  return hipGetLastError();
+}
+
+hipError_t launch_rows_to_columns(const void *rows, uint32_t elem_bytes, uint64_t n, void *columns, hipStream_t stream) {
+  if (n == 0) return hipSuccess;
+  const uint64_t blocks = (n + 256u * ROWS_PER_THREAD - 1) / (256u * ROWS_PER_THREAD);
+  if (blocks > 0x7fffffffu) return hipErrorInvalidValue;
+  const auto run = [&](auto zero) {
+    using T = decltype(zero);
+    T *c = static_cast<T *>(columns);
+    hipLaunchKernelGGL(k_rows_to_columns<T>, dim3((uint32_t)blocks), dim3(256), 0, stream, static_cast<const T *>(rows), n,
+                       c, c + n, c + 2 * n);
+  };
+  if (elem_bytes == 8) run(uint64_t{});
+  else run(uint32_t{});
   return hipGetLastError();
 }
 

@@ -1705,6 +1705,16 @@ int brt_closest_surface(const brt_scene *cs, const brt_points *points, uint64_t 
   return BRT_OK;
 }
 
+int brt_rows_to_columns(const void *rows, uint32_t elem_bytes, uint64_t n, void *columns, void *stream) {
+  if (elem_bytes != 4 && elem_bytes != 8) return fail(BRT_ERR_INVALID_ARGUMENT, "elements must have 4 or 8 bytes");
+  if (n == 0) return BRT_OK;
+  if (!rows || !columns) return fail(BRT_ERR_INVALID_ARGUMENT, "NULL argument");
+  if (((uintptr_t)rows | (uintptr_t)columns) % elem_bytes) return fail(BRT_ERR_INVALID_ARGUMENT, "misaligned array");
+  const hipError_t e = launch_rows_to_columns(rows, elem_bytes, n, columns, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return device_error(e, "launch failed");
+  return BRT_OK;
+}
+
 int brt_scene_upload(brt_scene *s) {
   if (!s) return fail(BRT_ERR_INVALID_ARGUMENT, "scene is NULL");
   if (!s->committed) return fail(BRT_ERR_STATE, "scene not committed");

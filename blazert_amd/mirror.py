@@ -13,7 +13,7 @@ import ctypes as C
 
 from . import capi
 from .capi import check, lib
-from .scene import Scene, _columns, _OnStream, _scalar_col
+from .scene import Scene, _columns, _OnStream, _packed_rows, _rows_to_columns, _scalar_col
 
 DEFAULT_BOUNCE_TMIN = 1e-9
 
@@ -94,7 +94,14 @@ def mirror_adjoint(scene: Scene, org, dirs, prim_id, grad_t=None, grad_position=
     if grad_position is not None and tuple(grad_position.shape) != (3, B, n):
         raise ValueError("grad_position must have shape (3, bounces, n)")
     gt = None if grad_t is None else grad_t.to(torch.float64).contiguous()
-    gp = None if grad_position is None else grad_position.to(torch.float64).contiguous()
+    gp = None
+    if grad_position is not None:
+        rows = grad_position.permute(1, 2, 0)
+        rows = rows.reshape(-1, 3) if rows.is_contiguous() else None
+        if rows is not None and _packed_rows(rows, torch.float64):
+            gp = _rows_to_columns(rows).view(3, B, n)
+        else:
+            gp = grad_position.to(torch.float64).contiguous()
     if grad_vertices is None:
         grad_vertices = torch.zeros((scene.num_vertices, 3), dtype=torch.float64, device=dev)
     elif (tuple(grad_vertices.shape) != (scene.num_vertices, 3) or grad_vertices.dtype != torch.float64

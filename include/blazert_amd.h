@@ -212,6 +212,10 @@ int brt_distance_to_surface(const brt_scene *scene, uint32_t geom_type, const br
 int brt_closest_surface(const brt_scene *scene, const brt_points *points, uint64_t n, double *distance,
                         uint32_t *prim_id, uint32_t *geom_id, void *stream);
 
+/* n packed rows of three elements (elem_bytes 4 or 8) to three columns of n, one after another in `columns`, which does not
+ * overlap the rows: device arrays aligned to elem_bytes. Asynchronous on `stream`; allocates nothing. */
+int brt_rows_to_columns(const void *rows, uint32_t elem_bytes, uint64_t n, void *columns, void *stream);
+
 /* Batched intersect1 (blazert/scene.h:161-211) for n rays resident on the device, enqueued on `stream`
  * (a hipStream_t, NULL = default stream). launch may be NULL (FP64, no flags, persistent). Asynchronous.
  * The launches keep a few device counters per scene and stream, allocated on the first launch on that stream
