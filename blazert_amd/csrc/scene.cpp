@@ -882,6 +882,9 @@ struct DeviceScene {
     std::lock_guard<std::mutex> lk(counter_mu);
     for (auto &c : stream_counters)
       if (c.first == st) return c.second;
+    // a first launch under capture is refused, as the allocation it needs would be; kept memory must not change that
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return nullptr;
     void *p = nullptr;
     if (pool_get(device, COUNTER_GROUP * sizeof(unsigned long long), &p) != hipSuccess) return nullptr;
     stream_counters.emplace_back(st, static_cast<unsigned long long *>(p));
