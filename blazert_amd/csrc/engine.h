@@ -160,6 +160,7 @@ hipError_t launch_cyl_filter_records(const void *recs, uint32_t n, void *out, hi
 
 // Triangles: assembles the reference-order nodes (NodeQ) from n Node4 records and their visiting orders (two words per
 // record, visit_order4).
+hipError_t launch_leaf_boxes(const BvhView &bvh, uint32_t num_nodes, double *out, hipStream_t stream);
 hipError_t launch_nodeq_records(const Node4 *nodes4, const uint32_t *ord, uint32_t n, NodeQ *out, hipStream_t stream);
 
 // Clears the counters of a group on the stream.

@@ -239,6 +239,30 @@ __device__ __forceinline__ bool sph_filter(const SphFilt &S, const float D[3], c
   return true;
 }
 
+// Conservative FP32 pre-test of one cylinder: returns false only when the FP64 test cyl_eval
+// (blazert/primitives/cylinder.h:181-495) reports no hit, whatever the hit distance (its last hit counts, at any t >= 0).
+//
+// A hit's point lies in the bounding sphere (sph_filter with the window [0, inf)), and the ray's line, projected along the
+// axis, reaches the ellipse of semi-axes a, b: in the local frame (org, dir) = R^T (o - c, d) the shell's quadratic needs
+// T^2 <= a^2 k^2 + b^2 j^2 for T = j y0 - k x0, a cap's point is on or in the ellipse and so is an origin inside, up to
+// roundings of 2e-15 (P^2 + max(a,b)^2) in T^2. T = (o - c) . (d x axis) for the record's axis, and the right side is at most
+// max(a,b)^2 (|d x axis|^2 + 1e-5) for a rotation within 1e-6 of orthonormal (others have infinite radii and pass). In FP32 T
+// is within 27 u P, u = 2^-24; the test rejects when it is outside by 32 u P, whose square covers the FP64 roundings too.
+__device__ __forceinline__ bool cyl_filter(const CylFilt &C, const float D[3], const float O[3], float om) {
+  const float u = 5.9604644775390625e-08f;
+  const SphFilt sphere{{C.c[0], C.c[1], C.c[2]}, C.r};
+  const float cm = fmaxf(fabsf(C.c[0]), fmaxf(fabsf(C.c[1]), fabsf(C.c[2])));
+  const float P = (cm + om) * (1.0f + 4.0f * u);
+  const float v0 = O[0] - C.c[0], v1 = O[1] - C.c[1], v2 = O[2] - C.c[2];
+  const float nx = __builtin_fmaf(D[1], C.axis[2], -(D[2] * C.axis[1]));
+  const float ny = __builtin_fmaf(D[2], C.axis[0], -(D[0] * C.axis[2]));
+  const float nz = __builtin_fmaf(D[0], C.axis[1], -(D[1] * C.axis[0]));
+  const float n2 = __builtin_fmaf(nx, nx, __builtin_fmaf(ny, ny, nz * nz));
+  const float T = fabsf(__builtin_fmaf(v0, nx, __builtin_fmaf(v1, ny, v2 * nz))) - 32.0f * u * P;
+  if (T > 0.0f && T * T > (C.shell * C.shell) * (n2 * (1.0f + 16.0f * u) + 2e-5f)) return false;
+  return sph_filter(sphere, D, O, om, 0.0f, __builtin_inff());
+}
+
 // ------------------------------------------------------------------------------------------------ intersectors
 // Closest-hit state of one traversal (prepare_traversal: hit = tmax, uv = 0, prim invalid).
 template <class R>
@@ -807,7 +831,8 @@ __device__ __forceinline__ void trav_step(const BvhView &bvh, const RayT<typenam
   // without waiting in between.
   // split precision, triangles, spheres and cylinders: FP32 pre-test records, FG of them per step
   constexpr bool FILTER = SPLIT && (Rec::kind == TRIANGLES || Rec::kind == SPHERES || Rec::kind == CYLINDERS);
-  using Filt = typename std::conditional<Rec::kind == TRIANGLES, TriFilt, SphFilt>::type;
+  using Filt = typename std::conditional<Rec::kind == TRIANGLES, TriFilt,
+                                         typename std::conditional<Rec::kind == CYLINDERS, CylFilt, SphFilt>::type>::type;
   constexpr uint32_t FG = Rec::kind == TRIANGLES ? FILTER_GROUP : SPH_FILTER_GROUP;
   constexpr int NODE_Q = SPLIT ? 8 : (sizeof(R) == 8 ? 7 : 4);  // 16-byte chunks of the record used (Node64: 112 B)
   constexpr int REC_Q = (int)(sizeof(Rec) / 16);
@@ -821,6 +846,7 @@ __device__ __forceinline__ void trav_step(const BvhView &bvh, const RayT<typenam
   const Filt *frecs = nullptr;
   if constexpr (FILTER) {
     if constexpr (Rec::kind == TRIANGLES) frecs = bvh.tri_filter;
+    else if constexpr (Rec::kind == CYLINDERS) frecs = bvh.cyl_filter;
     else frecs = bvh.sph_filter;
   }
   const bool filt = FILTER && frecs != nullptr;  // the same for every lane of a launch
@@ -944,7 +970,7 @@ __device__ __forceinline__ void trav_step(const BvhView &bvh, const RayT<typenam
         bool pass;
         if constexpr (Rec::kind == TRIANGLES) pass = tri_filter(g[j], D, O, q.om, q.tmin, t.h32);
         else if constexpr (Rec::kind == SPHERES) pass = sph_filter(g[j], D, O, q.om, q.tmin, t.h32);
-        else pass = sph_filter(g[j], D, O, q.om, 0.0f, __builtin_inff());  // cylinders: any hit at t >= 0 counts
+        else pass = cyl_filter(g[j], D, O, q.om);
         if (j < left && pass) mask |= 1u << j;
       }
       t.cand = mask;
@@ -1070,6 +1096,15 @@ __device__ __forceinline__ bool fast_ray(const Ray &r, double len2, double S) {
          fabs(r.o[2]) <= FILTER_MAX_EXTENT;
 }
 
+// Rays of k_trace_wide (spheres, cylinders): the FP32 bounds enclose the reference's traversal, whatever the length of the direction.
+__device__ __forceinline__ bool wide_ray(const Ray &r, double S) {
+  bool ok = (r.sign & RAY_NAN_FREE) && r.tmin >= 0.0;
+#pragma unroll
+  for (int k = 0; k < 3; k++)
+    ok = ok && fabs(r.inv[k]) * (S + fabs(r.o[k])) <= 1e36 && fabs(r.inv[k]) <= 1e30 && fabs(r.o[k]) <= FILTER_MAX_EXTENT;
+  return ok;
+}
+
 // A ray's columns as they stand in memory.
 struct RawRay {
   double org[3], dir[3], tmin, tmax;
@@ -1084,12 +1119,13 @@ __device__ __forceinline__ double squared_length(const RawRay &w) {
   return w.dir[0] * w.dir[0] + w.dir[1] * w.dir[1] + w.dir[2] * w.dir[2];
 }
 
-// The same predicate from the ray's columns.
+// The type's predicate from the ray's columns.
+template <class Rec>
 __device__ __forceinline__ bool fast_ray(const RaysView &V, uint64_t i, double S) {
   const RawRay w = load_ray(V, i);
   Ray r;
   setup_ray(w.org, w.dir, w.tmin, w.tmax, r);
-  return fast_ray(r, squared_length(w), S);
+  return Rec::kind == TRIANGLES ? fast_ray(r, squared_length(w), S) : wide_ray(r, S);
 }
 
 // One ray per thread (grid-stride).
@@ -1236,7 +1272,7 @@ k_trace_persistent(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<ty
           } else {
             idx = order ? (uint64_t)order[cand] : cand;
             start_ray<SPLIT>(bvh, rays_view(), idx, S, r, q, s);
-            if constexpr (AFTER_FAST) trace = left.all || !fast_ray(rays_view(), idx, S);
+            if constexpr (AFTER_FAST) trace = left.all || !fast_ray<Rec>(rays_view(), idx, S);
           }
           if (SPLIT && deferred_to_exact(r)) {
             __atomic_store_n(deferred, 1ull, __ATOMIC_RELAXED);
@@ -1352,7 +1388,7 @@ k_trace_batch(const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t total,
             bv = J.bvh;
             start_ray<SPLIT>(bv, J.rays, idx, J.extent, r, q, s);
             bool trace = true;
-            if constexpr (AFTER_FAST) trace = from_list || left.all || !fast_ray(J.rays, idx, J.extent);
+            if constexpr (AFTER_FAST) trace = from_list || left.all || !fast_ray<Rec>(J.rays, idx, J.extent);
             if (SPLIT && deferred_to_exact(r)) {
               __atomic_store_n(deferred, 1ull, __ATOMIC_RELAXED);
             } else if (trace && (!deferred_only || deferred_to_exact(r))) {
@@ -1963,6 +1999,281 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
   }
 }
 
+// ------------------------------------------------------------------------------------------------ spheres and cylinders, fast
+// Closest hits of spheres and cylinders, bit-identical to the exact FP64 kernel (k_trace_persistent<Rec, false>), with the
+// FP32 boxes and the visiting order of k_trace_tri. No certificate is needed: when a primitive reports a hit and its leaf has
+// not been checked yet, the reference's own FP64 slab and pop tests of the leaf's box, at the hit distance as it stands,
+// decide whether the reference tests the leaf at all. That leaf's test decides for the boxes above it too. They hold its box
+// and every operation of the slab test is monotone, so they pass the slab test with it, with an entry distance no larger. As
+// to their pop tests: of the boxes above it, those popped before the last accepted hit are boxes above that hit's leaf as
+// well (a depth-first stack holds only siblings of the path), which was checked; those popped since saw the hit distance
+// that the leaf's test sees. An FP32 pop test (at most the reference's entry distance against at least its hit distance)
+// skips only what the reference skips. So does a box left out of the stack, since hit distances only shrink: a ray on which
+// a sphere's grows by a rounding is listed for the exact kernel; a cylinder's last hit counts, so its distance may grow, and
+// only the slab test leaves its boxes out.
+//
+// What bounds it (8,388,608 incoherent rays): the vector ALU, 74% busy with a quarter of the lanes active, since a wave runs
+// the node, pre-test and FP64 branches in almost every iteration for a few lanes each. Lanes with an FP64 test, or with a
+// pre-test, therefore wait until WIDE_MIN_LANES of the wave have one (or no other lane has anything else to do): 50,000
+// spheres 4.19 -> 3.24 ms (8 lanes: 3.36, 24: 3.62), against 4.44 ms for the exact kernel; 10,000 cylinders 3.65 -> 3.46 ms,
+// against 5.45 ms. (k_trace_tri, bound by the data path of the L1, gains nothing from it.) A wave with no rays left to take
+// doesn't wait: there the longest ray counts.
+constexpr int WIDE_MIN_LANES = 16;
+
+struct WideTrav {
+  uint32_t cur, cnt, cand;
+  uint32_t leaf;  // first primitive of the leaf
+  float h32;
+  bool active, listed, seen;  // seen: the reference tests this leaf
+};
+
+// One unit of the traversal: an internal node, the pre-test of a leaf's next SPH_FILTER_GROUP primitives, or the FP64 test
+// of one.
+template <class Rec, class Inv>
+__device__ __forceinline__ void wide_step(const BvhView &bvh, const Ray &r, const RayQ &q, Hit &s, WideTrav &t,
+                                          WideStack &st, Inv &&load_inv, bool wait) {
+  using u32x4 = unsigned int __attribute__((ext_vector_type(4)));
+  using Bytes = const __attribute__((address_space(1))) unsigned char;
+  using GlobalChunk = const __attribute__((address_space(1))) u32x4;
+  constexpr bool GROWS = Rec::kind == CYLINDERS;
+  constexpr uint32_t FG = SPH_FILTER_GROUP;
+  using Filt = typename std::conditional<GROWS, CylFilt, SphFilt>::type;
+  constexpr int REC_Q = (int)(sizeof(Rec) / 16), FILT_Q = (int)(FG * sizeof(Filt) / 16);
+  const Filt *filt;
+  if constexpr (GROWS) filt = bvh.cyl_filter;
+  else filt = bvh.sph_filter;
+  const bool at_leaf = (t.cur & LEAF_BIT) != 0;
+  const bool test = t.cand != 0u;
+  if (wait) {
+    const bool group = at_leaf && !test;
+    const int tests = __popcll(__ballot(test)), groups = __popcll(__ballot(group));
+    const int nodes = __popcll(__ballot(true)) - tests - groups;
+    if (test && tests < WIDE_MIN_LANES && nodes + groups != 0) return;
+    if (group && groups < WIDE_MIN_LANES && nodes != 0) return;
+  }
+  const uint32_t first = t.cur & ~LEAF_BIT;
+  const uint32_t p = first + (uint32_t)__builtin_ctz(t.cand | 0x80000000u);
+  // without pre-test records every primitive gets the FP64 test (the fetch then reads node 0)
+  Bytes *base = !at_leaf          ? (Bytes *)(bvh.nodesq + t.cur)
+                : test            ? (Bytes *)(reinterpret_cast<const Rec *>(bvh.prims) + p)
+                : filt != nullptr ? (Bytes *)(filt + first)
+                                  : (Bytes *)bvh.nodesq;
+  const uint32_t code = at_leaf ? 0u : q.code;
+  const uint32_t near0 = code & 64u, near1 = (code >> 1) & 64u, near2 = (code >> 2) & 64u;
+  u32x4 c0, c1, c2, c3, c4, c5, c6, c7;
+  c0 = *(GlobalChunk *)(base + near0);
+  c1 = *(GlobalChunk *)(base + near1 + 16);
+  if (REC_Q > 2 || !test) {
+    c2 = *(GlobalChunk *)(base + near2 + 32);
+    c3 = *(GlobalChunk *)(base + 48);
+  }
+  if (!at_leaf || (test ? REC_Q > 4 : FILT_Q > 4)) {
+    c4 = *(GlobalChunk *)(base + (64u - near0));
+    c5 = *(GlobalChunk *)(base + (64u - near1) + 16);
+    c6 = *(GlobalChunk *)(base + (64u - near2) + 32);
+    c7 = *(GlobalChunk *)(base + 112);
+  }
+  asm volatile("" : "+v"(c0), "+v"(c1), "+v"(c2), "+v"(c3), "+v"(c4), "+v"(c5), "+v"(c6), "+v"(c7));
+  if (!at_leaf) {
+    uint32_t m = 0;
+    uint32_t key[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const float n0 = __builtin_fmaf(__uint_as_float(c0[c]), q.inv[0], q.offn[0]);
+      const float n1 = __builtin_fmaf(__uint_as_float(c1[c]), q.inv[1], q.offn[1]);
+      const float n2 = __builtin_fmaf(__uint_as_float(c2[c]), q.inv[2], q.offn[2]);
+      const float f0 = __builtin_fmaf(__uint_as_float(c4[c]), q.inv[0], q.offf[0]);
+      const float f1 = __builtin_fmaf(__uint_as_float(c5[c]), q.inv[1], q.offf[1]);
+      const float f2 = __builtin_fmaf(__uint_as_float(c6[c]), q.inv[2], q.offf[2]);
+      const float A = max_nn(max3_nn(n0, n1, n2), q.tmin);
+      float M = min3_nn(f0, f1, f2);
+      if constexpr (!GROWS) M = min_nn(M, t.h32);  // a cylinder's hit distance may have grown when the entry is popped
+      key[c] = __float_as_uint(A);
+      m |= A <= M ? 1u << c : 0u;
+    }
+    if (m) {
+      const uint32_t word = (code & 32u) ? c7[1] : c7[0];
+      const uint32_t later = (word >> (code & 31u)) ^ (uint32_t)(((int)(code << 22)) >> 31);
+      const int n = __popc(m);
+      st.room(n - 1);
+      uint32_t ncur = 0, ncnt = 0;
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        if ((m >> c) & 1u) {
+          const int rank = __popc(m & (later >> (4 * c)) & (15u & ~(1u << c)));
+          const uint32_t k = __builtin_amdgcn_perm(key[c], c7[2], 0x07060500u | (uint32_t)c);
+          if (rank == n - 1) {
+            ncur = c3[c];
+            ncnt = k;
+          } else {
+            st.put(st.sp + rank, c3[c], k);
+          }
+        }
+      }
+      st.sp += n - 1;
+      if (!GROWS || !(t.h32 < __uint_as_float(ncnt & ~255u))) {
+        t.cur = ncur;
+        t.cnt = ncnt & 255u;
+        t.leaf = ncur & ~LEAF_BIT;
+        t.seen = false;
+        return;
+      }
+    }
+  } else if (!test) {
+    Filt g[FG];
+    u32x4 raw[8] = {c0, c1, c2, c3, c4, c5, c6, c7};
+    __builtin_memcpy(g, raw, sizeof g);
+    uint32_t mask = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < FG; j++) {
+      bool pass = true;
+      if (filt != nullptr) {
+        if constexpr (GROWS) pass = cyl_filter(g[j], q.D, q.O, q.om);
+        else pass = sph_filter(g[j], q.D, q.O, q.om, q.tmin, t.h32);
+      }
+      if (j < t.cnt && pass) mask |= 1u << j;
+    }
+    t.cand = mask;
+    if (mask) return;
+    if (t.cnt > FG) {
+      t.cnt -= FG;
+      t.cur += FG;
+      return;
+    }
+  } else {
+    Rec rec;
+    u32x4 raw[8] = {c0, c1, c2, c3, c4, c5, c6, c7};
+    __builtin_memcpy(&rec, raw, sizeof rec);
+    const Hit old = s;
+    if (isect(rec, r, s, p)) {
+      if (!t.seen) {
+        Ray x = r;
+        load_inv(x);
+        const double *b = bvh.leaf_boxes + 6ull * t.leaf;
+        const double box[6] = {gmem(b)[0], gmem(b)[1], gmem(b)[2], gmem(b)[3], gmem(b)[4], gmem(b)[5]};
+        double key;
+        t.seen = slab_exact(box, x, key) && !(old.h < key);
+      }
+      if (t.seen) {
+        t.h32 = f32_up(s.h);
+        if constexpr (!GROWS) t.listed = t.listed || !(s.h <= old.h);
+      } else {  // not a leaf of the reference's: none of its primitives counts
+        s = old;
+        t.cnt = 0;
+        t.cand = 0;
+      }
+    }
+    t.cand &= t.cand - 1u;
+    if (t.cand) return;
+    if (t.cnt > FG) {
+      t.cnt -= FG;
+      t.cur += FG;
+      return;
+    }
+  }
+  while (st.sp > 0) {
+    const WideEntry e = st.pop();
+    if (!(t.h32 < __uint_as_float(e.key & ~255u))) {
+      t.cur = e.ref;
+      t.cnt = e.key & 255u;
+      t.leaf = e.ref & ~LEAF_BIT;
+      t.seen = false;
+      return;
+    }
+  }
+  t.active = false;
+}
+
+template <class Rec>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BRT_WAVES_PER_EU)))
+k_trace_wide(BvhView bvh, RaysView rays, HitsView hits, uint64_t n, uint32_t flags, uint32_t first, uint32_t is_tri,
+             double S, unsigned long long *group, uint32_t refill, const uint32_t *order, uint32_t ring, uint32_t chunk,
+             uint32_t fixed) {
+  extern __shared__ unsigned char smem[];
+  constexpr int RW = (int)(sizeof(RaysView) / 8), HW = (int)(sizeof(HitsView) / 8);
+  __shared__ uint64_t views[RW + HW];  // ray and hit columns, read back where they are used (see k_trace_persistent)
+  if (threadIdx.x == 0) {
+    lds_store(views, rays);
+    lds_store(views + RW, hits);
+  }
+  __syncthreads();
+  const uint32_t lane = __lane_id(), wave = threadIdx.x / 64;
+  uint64_t spill[WIDE_SPILL];
+  WideStack st;
+  st.ring = (BRT_LDS uint32_t *)smem + (size_t)wave * ring * 128 + lane;
+  st.spill = spill;
+  st.mask = (int)ring - 1;
+  st.reset();
+  Ray r;
+  RayQ q;
+  Hit s;
+  WideTrav t;
+  t.active = false;
+  t.cand = 0;
+  bool has_ray = false, done = false, exhausted = false;
+  uint64_t idx = 0;
+  const auto write_rays = [&]() {  // finished rays are written together (see k_trace_tri)
+    if (done) {
+      done = false;
+      if (t.listed) {
+        const unsigned long long k = atomicAdd(group + COUNTER_LISTED, 1ull);
+        if (k < (unsigned long long)LIST_CAPACITY) group[COUNTER_CLEARED + k] = idx;
+      } else {
+        finish_ray<Rec>(bvh, lds_fresh<HitsView>(views + RW), idx, r, s, flags, first, is_tri);
+      }
+    }
+  };
+  const auto load_inv = [&](Ray &x) {
+    const RaysView V = lds_fresh<RaysView>(views);
+    x.inv[0] = 1.0 / V.dx[idx];
+    x.inv[1] = 1.0 / V.dy[idx];
+    x.inv[2] = 1.0 / V.dz[idx];
+  };
+  WavePool pool;
+  if (fixed) pool.take_fixed(((uint64_t)blockIdx.x * (blockDim.x / 64) + wave) * fixed, fixed, n);
+  for (;;) {
+    if (!exhausted) {
+      const unsigned long long idle = __ballot(!has_ray);
+      const uint32_t nidle = (uint32_t)__popcll(idle);
+      if (nidle >= refill || nidle == 64u) {
+        write_rays();
+        bool got;
+        uint64_t cand = 0;
+        pool_refill(pool, group + COUNTER_POOL, n, chunk, idle, nidle, lane, got, cand, exhausted);
+        if (got) {
+          idx = order ? (uint64_t)order[cand] : cand;
+          const RawRay raw = load_ray(lds_fresh<RaysView>(views), idx);
+          setup_ray(raw.org, raw.dir, raw.tmin, raw.tmax, r);
+          if (wide_ray(r, S)) {
+            has_ray = true;
+            make_rayq(r, 1.0, S, q);
+            s.h = r.tmax;
+            s.u = s.v = 0.0;
+            s.leaf_idx = INVALID_ID;
+            TriTrav b;
+            tri_begin(tri_root(bvh), r, q, s, b);
+            t = WideTrav{b.cur, b.cnt, 0u, b.cur & ~LEAF_BIT, b.h32, b.active, false, false};
+            st.reset();
+          } else {
+            __atomic_store_n(group + COUNTER_DEFERRED, 1ull, __ATOMIC_RELAXED);
+          }
+        }
+      }
+    }
+    if (exhausted && !__ballot(has_ray)) {
+      write_rays();
+      break;
+    }
+    if (has_ray) {
+      if (t.active) wide_step<Rec>(bvh, r, q, s, t, st, load_inv, !exhausted);
+      if (!t.active) {
+        done = true;
+        has_ray = false;
+      }
+    }
+  }
+}
+
 // Split-precision pre-test records of the triangles in leaf order (TriFilt), from their FP64 records; the FILTER_PAD
 // records after the last one are zero.
 __global__ void k_tri_filter_records(const TriRec *__restrict__ recs, uint32_t n, TriFilt *out, uint32_t total) {
@@ -2009,17 +2320,16 @@ __global__ void k_sph_filter_records(const SphRec *__restrict__ recs, uint32_t n
   }
 }
 
-// Split-precision pre-test records of the cylinders: each one's bounding sphere, for sph_filter with the window
-// [0, inf). The cylinder test (cylinder.h:181-495) accepts any hit at t >= 0, with no distance check, at a point of
-// the local frame org + t dir = R^T (o + t d - c) with |z| <= h/2 and, up to the rounding of the test, on or inside
-// the elliptic shell of semi-axes a, b; for an orthonormal R that point lies within sqrt(max(a,b)^2 + (h/2)^2) of c.
-// The radius is enlarged by 2^-10 of itself and 2^-20 of the coordinate magnitude, far above any rounding of the
-// FP64 test, and is infinite (never rejects) when R R^T differs from the identity by more than 1e-6 or an input is
-// not finite.
-__global__ void k_cyl_filter_records(const CylRec *__restrict__ recs, uint32_t n, SphFilt *out, uint32_t total) {
+// Pre-test records of the cylinders (cyl_filter). The cylinder test (cylinder.h:181-495) accepts any hit at t >= 0, with no
+// distance check, at a point of the local frame org + t dir = R^T (o + t d - c) with |z| <= h/2 and, up to the rounding of
+// the test, on or inside the elliptic shell of semi-axes a, b; for an orthonormal R that point lies within
+// sqrt(max(a,b)^2 + (h/2)^2) of c. Both radii are enlarged by 2^-10 of themselves, the sphere's also by 2^-20 of the
+// coordinate magnitude, far above any rounding of the FP64 test, and are infinite (never reject) when R R^T differs from
+// the identity by more than 1e-6 or an input is not finite.
+__global__ void k_cyl_filter_records(const CylRec *__restrict__ recs, uint32_t n, CylFilt *out, uint32_t total) {
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-    SphFilt f{};
+    CylFilt f{};
     if (i < n) {
       const CylRec &C = recs[i];
       double dev = 0.0;
@@ -2032,9 +2342,15 @@ __global__ void k_cyl_filter_records(const CylRec *__restrict__ recs, uint32_t n
       const double rb = sqrt(ab * ab + hh * hh);
       const double cm = fmax(fabs(C.c[0]), fmax(fabs(C.c[1]), fabs(C.c[2])));
       double rad = rb * (1.0 + 0x1p-10) + 0x1p-20 * (cm + rb);
-      if (!(dev <= 1e-6) || !(rad < 1e300)) rad = __builtin_inf();
+      double shell = ab * (1.0 + 0x1p-10);
+      if (!(dev <= 1e-6) || !(rad < 1e300)) rad = shell = __builtin_inf();
+      for (int k = 0; k < 3; k++) {  // first column of R x second
+        const int x = (k + 1) % 3, y = (k + 2) % 3;
+        f.axis[k] = (float)(C.R[3 * x] * C.R[3 * y + 1] - C.R[3 * y] * C.R[3 * x + 1]);
+      }
       for (int k = 0; k < 3; k++) f.c[k] = (float)C.c[k];
       f.r = f32_up(rad);
+      f.shell = f32_up(shell);
     }
     out[i] = f;
   }
@@ -2058,6 +2374,20 @@ __global__ void k_nodeq_records(const Node4 *__restrict__ in, const uint32_t *__
   b.ord[1] = ord[2ull * i + 1];
   b.pad = 0;
   out[i] = b;
+}
+
+// The FP64 boxes of the leaves, each at its first primitive's place (six doubles). A root leaf's box is the tree's.
+__global__ void k_leaf_boxes(const Node64 *__restrict__ nodes, uint32_t n, BvhView bvh, double *__restrict__ out) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0 && n == 0)
+    for (int k = 0; k < 3; k++) {
+      out[k] = bvh.root_min[k];
+      out[3 + k] = bvh.root_max[k];
+    }
+  if (i >= n) return;
+  for (int c = 0; c < 2; c++)
+    if (nodes[i].ref[c] & LEAF_BIT)
+      for (int k = 0; k < 6; k++) out[6ull * (nodes[i].ref[c] & ~LEAF_BIT) + k] = nodes[i].b[6 * c + k];
 }
 
 // Clears a launch's counter group (a fill kernel, not hipMemsetAsync, so that graph captures replay correctly).
@@ -2203,6 +2533,12 @@ hipError_t launch_kernel(const BvhView &bvh, const RaysViewT<typename Rec::real>
 bool fast_triangles(const TraceLaunch &cfg) {
   return cfg.schedule == SCHEDULE_PERSISTENT && !(cfg.flags & FLAG_ANY_HIT);
 }
+// Spheres' and cylinders' (k_trace_wide), in FP64 (split precision has a visiting order of its own): 8,388,608 incoherent
+// rays, 50,000 spheres 3.24 against 4.44 ms, 10,000 cylinders 3.48 against 5.45 ms; a 512x512 camera over 1,024 spheres 0.094
+// against 0.137 ms a call. 100 planes 1.75 against 1.61 ms: they keep the exact kernel.
+bool fast_wide(const BvhView &bvh, const TraceLaunch &cfg) {
+  return bvh.nodesq && bvh.leaf_boxes && cfg.precision == PREC_FP64 && fast_triangles(cfg);
+}
 constexpr uint32_t TRI_RING = 16, TRI_REFILL = 16;
 constexpr size_t tri_lds_bytes(uint32_t block, uint32_t ring) { return (size_t)block * ring * sizeof(uint64_t); }
 
@@ -2235,6 +2571,38 @@ hipError_t launch_tri(const BvhView &bvh, const RaysView &rays, const HitsView &
   hipLaunchKernelGGL((k_trace_persistent<TriRec, false, true>), dim3((uint32_t)blocks), dim3(256), lds64, stream, bvh,
                      rays, hits, n, cfg.flags, first, 1u, sp.scene_extent, grp + COUNTER_DEFERRED_POOL,
                      refill_default<TriRec, false>(), cfg.order, ring64, grp + COUNTER_DEFERRED, POOL_CHUNK);
+  return hipGetLastError();
+}
+
+template <class Rec>
+hipError_t launch_wide(const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint64_t n, const TraceLaunch &cfg,
+                       const SplitParams &sp, uint32_t is_tri, hipStream_t stream) {
+  const uint32_t block = cfg.block ? cfg.block : 256;
+  const uint32_t ring = cfg.ring ? cfg.ring : TRI_RING;
+  const uint32_t first = cfg.first ? 1u : 0u;
+  const size_t lds = tri_lds_bytes(block, ring);
+  unsigned long long *grp = cfg.counter;
+  if (!grp) return hipErrorInvalidValue;
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
+  uint64_t blocks = 0;
+  hipError_t e = persistent_blocks(k_trace_wide<Rec>, block, lds, n * 64, blocks);
+  if (e != hipSuccess) return e;
+  const uint32_t wpb = block / 64, fixed = fixed_per_wave(n, blocks * wpb);
+  const uint64_t need = fixed ? (n + fixed * wpb - 1) / (fixed * wpb) : (n + block - 1) / block;
+  if (blocks > need) blocks = need;
+  hipLaunchKernelGGL(k_trace_wide<Rec>, dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits, n, cfg.flags,
+                     first, is_tri, sp.scene_extent, grp, cfg.refill ? cfg.refill : TRI_REFILL, cfg.order, ring,
+                     cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const uint32_t ring64 = ring_default<Rec, false>();
+  const size_t lds64 = ring_lds_bytes<false, double>(256, ring64);
+  e = persistent_blocks(k_trace_persistent<Rec, false, true>, 256, lds64, n, blocks);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_trace_persistent<Rec, false, true>), dim3((uint32_t)blocks), dim3(256), lds64, stream, bvh, rays,
+                     hits, n, cfg.flags, first, is_tri, sp.scene_extent, grp + COUNTER_DEFERRED_POOL,
+                     refill_default<Rec, false>(), cfg.order, ring64, grp + COUNTER_DEFERRED, POOL_CHUNK);
   return hipGetLastError();
 }
 
@@ -2303,6 +2671,14 @@ hipError_t launch_typed(const BvhView &bvh, const RaysView &rays, const HitsView
   return launch_kernel<Rec, true>(bvh, rays, hits, n, cfg, sp, is_tri, stream);
 }
 
+template <class Rec>
+hipError_t launch_other(const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint64_t n, const TraceLaunch &cfg,
+                        const SplitParams &sp, hipStream_t stream) {
+  const uint32_t ow = cfg.overwrite ? 1u : 0u;
+  if (fast_wide(bvh, cfg)) return launch_wide<Rec>(bvh, rays, hits, n, cfg, sp, ow, stream);
+  return launch_typed<Rec>(bvh, rays, hits, n, cfg, sp, ow, stream);
+}
+
 }  // namespace
 
 hipError_t launch_trace(GeomType type, const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint64_t n,
@@ -2311,9 +2687,9 @@ hipError_t launch_trace(GeomType type, const BvhView &bvh, const RaysView &rays,
   case TRIANGLES:
     if (bvh.nodesq && fast_triangles(cfg)) return launch_tri(bvh, rays, hits, n, cfg, split, stream);
     return launch_typed<TriRec>(bvh, rays, hits, n, cfg, split, 1u, stream);
-  case SPHERES: return launch_typed<SphRec>(bvh, rays, hits, n, cfg, split, cfg.overwrite ? 1u : 0u, stream);
+  case SPHERES: return launch_other<SphRec>(bvh, rays, hits, n, cfg, split, stream);
   case PLANES: return launch_typed<PlaRec>(bvh, rays, hits, n, cfg, split, cfg.overwrite ? 1u : 0u, stream);
-  default: return launch_typed<CylRec>(bvh, rays, hits, n, cfg, split, cfg.overwrite ? 1u : 0u, stream);
+  default: return launch_other<CylRec>(bvh, rays, hits, n, cfg, split, stream);
   }
 }
 
@@ -2356,12 +2732,17 @@ hipError_t launch_cyl_filter_records(const void *recs, uint32_t n, void *out, hi
   uint32_t blocks = (total + 255) / 256;
   if (blocks > 65536) blocks = 65536;
   hipLaunchKernelGGL(k_cyl_filter_records, dim3(blocks), dim3(256), 0, stream, static_cast<const CylRec *>(recs), n,
-                     static_cast<SphFilt *>(out), total);
+                     static_cast<CylFilt *>(out), total);
   return hipGetLastError();
 }
 
 hipError_t launch_zero_counters(unsigned long long *group, hipStream_t stream) {
   hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, group);
+  return hipGetLastError();
+}
+
+hipError_t launch_leaf_boxes(const BvhView &bvh, uint32_t num_nodes, double *out, hipStream_t stream) {
+  hipLaunchKernelGGL(k_leaf_boxes, dim3(num_nodes / 256 + 1), dim3(256), 0, stream, bvh.nodes64, num_nodes, bvh, out);
   return hipGetLastError();
 }
 

@@ -38,7 +38,7 @@ struct alignas(128) Node4 {
 };
 static_assert(sizeof(Node4) == 128, "Node4 must be one 128-byte line");
 
-// Reference-order FP32 4-wide node of a triangle tree, 128 B: a Node4's child boxes and references, and the order in
+// Reference-order FP32 4-wide node, 128 B: a Node4's child boxes and references, and the order in
 // which the reference's depth-first traversal visits its slots. Planes are child-minor rows; the lo and hi rows of an
 // axis lie 64 bytes apart, so a lane loads the near and the far row of an axis by address. ord: for the octants 0..3 of
 // the direction signs (x, y; z positive), 16 bits each: bits 4c..4c+3 are the slots visited after slot c; the masks of
@@ -90,8 +90,7 @@ constexpr uint32_t FILTER_GROUP = BRT_FILTER_GROUP;  // triangles pre-tested per
 constexpr uint32_t FILTER_PAD = FILTER_GROUP - 1;
 
 // Split precision: FP32 pre-test record of a sphere, in leaf order beside the SphRec array: the center rounded to
-// nearest and |r| rounded up; for a cylinder, its bounding sphere, enlarged (k_cyl_filter_records). Built on the
-// device from the SphRec / CylRec array; SPH_FILTER_PAD zero records follow the last one, so a group of
+// nearest and |r| rounded up. Built on the device from the SphRec array; SPH_FILTER_PAD zero records follow the last one, so a group of
 // SPH_FILTER_GROUP records read from any leaf start stays in bounds.
 struct alignas(16) SphFilt {
   float c[3];
@@ -101,8 +100,18 @@ static_assert(sizeof(SphFilt) == 16, "SphFilt size");
 #ifndef BRT_SPH_FILTER_GROUP
 #define BRT_SPH_FILTER_GROUP 4
 #endif
-constexpr uint32_t SPH_FILTER_GROUP = BRT_SPH_FILTER_GROUP;  // spheres pre-tested per traversal step
+constexpr uint32_t SPH_FILTER_GROUP = BRT_SPH_FILTER_GROUP;  // spheres or cylinders pre-tested per traversal step
 constexpr uint32_t SPH_FILTER_PAD = SPH_FILTER_GROUP - 1;
+// Pre-test record of a cylinder beside the CylRec array: the center and the radius of its bounding sphere, the axis
+// (cross product of the rotation's first two columns) and the larger semi-axis, the radii enlarged (k_cyl_filter_records);
+// padded as the spheres' records.
+struct alignas(16) CylFilt {
+  float c[3];
+  float r;
+  float axis[3];
+  float shell;
+};
+static_assert(sizeof(CylFilt) == 32, "CylFilt size");
 // Largest scene extent (and ray origin magnitude) for which the FP32 pre-test is used: below it no product of the
 // pre-test or of its error bound can overflow FP32.
 constexpr double FILTER_MAX_EXTENT = 1e12;
@@ -191,8 +200,10 @@ struct BvhView {
   const double *vertices;     // triangles only: user vertices (3 per vertex), for mirror tracing and its adjoint
   const Node32 *nodes32;      // Scene<float>: FP32 nodes (nodes64 / nodes4 unused)
   const TriFilt *tri_filter;  // split precision, triangles: FP32 pre-test records (NULL: every test in FP64)
-  const NodeQ *nodesq;        // triangles: reference-order FP32 nodes (NULL: the exact kernels trace the type)
-  const SphFilt *sph_filter;  // split precision, spheres and cylinders: FP32 (bounding) spheres (NULL: all in FP64)
+  const NodeQ *nodesq;        // reference-order FP32 nodes (NULL: the exact kernels trace the type)
+  const double *leaf_boxes;   // spheres, cylinders: the FP64 box of each leaf at its first primitive (6 values)
+  const SphFilt *sph_filter;  // spheres: FP32 pre-test records (NULL: every test in FP64)
+  const CylFilt *cyl_filter;  // cylinders: the same
   const float *vnormals32;    // Scene<float> triangles: vertex normals
   double root_min[3], root_max[3];
   float root_min32[3], root_max32[3];

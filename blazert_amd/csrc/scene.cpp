@@ -1090,20 +1090,22 @@ int device_error(hipError_t e, const char *what) {
               std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// Split precision: the FP32 pre-test records of a triangle (TriFilt) or sphere (SphFilt) geometry, made on the
+// The FP32 pre-test records of a triangle (TriFilt), sphere (SphFilt) or cylinder (CylFilt) geometry, made on the
 // device from its uploaded FP64 records and waited for; none for other types, or when the scene's extent is above
 // FILTER_MAX_EXTENT. BLAZERT_AMD_SPLIT_PRETEST=0 in the environment at upload time leaves them out (every
-// split-precision primitive test then runs in FP64; the hits are the same, which the tests check).
+// primitive test then runs in FP64; the hits are the same, which the tests check).
 hipError_t make_prim_filter(DeviceScene &d, BvhView &v, uint32_t type, double extent, hipStream_t st,
                             uint64_t *device_bytes) {
   v.tri_filter = nullptr;
   v.sph_filter = nullptr;
+  v.cyl_filter = nullptr;
   if (type != TRIANGLES && type != SPHERES && type != CYLINDERS) return hipSuccess;
   if (!(extent <= FILTER_MAX_EXTENT) || v.n_prims == 0 || !v.prims) return hipSuccess;
   const char *env = std::getenv("BLAZERT_AMD_SPLIT_PRETEST");
   if (env && env[0] == '0') return hipSuccess;
   const size_t bytes = type == TRIANGLES ? (size_t)(v.n_prims + FILTER_PAD) * sizeof(TriFilt)
-                                         : (size_t)(v.n_prims + SPH_FILTER_PAD) * sizeof(SphFilt);
+                       : type == SPHERES ? (size_t)(v.n_prims + SPH_FILTER_PAD) * sizeof(SphFilt)
+                                         : (size_t)(v.n_prims + SPH_FILTER_PAD) * sizeof(CylFilt);
   void *p = nullptr;
   hipError_t e = d.alloc(bytes, &p);
   if (e != hipSuccess) return e;
@@ -1112,23 +1114,35 @@ hipError_t make_prim_filter(DeviceScene &d, BvhView &v, uint32_t type, double ex
                          : launch_cyl_filter_records(v.prims, v.n_prims, p, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (type == TRIANGLES) v.tri_filter = static_cast<const TriFilt *>(p);
-  else v.sph_filter = static_cast<const SphFilt *>(p);
+  else if (type == SPHERES) v.sph_filter = static_cast<const SphFilt *>(p);
+  else v.cyl_filter = static_cast<const CylFilt *>(p);
   *device_bytes += bytes;
   return e;
 }
 
-// Triangles: the reference-order FP32 nodes of the fast closest-hit traversal, made on the device from its Node4
-// records and waited for. None (every trace then takes the exact kernels) for a tree that split precision does not take,
-// one with an inverted or NaN box, or one with a leaf of more than NODEQ_MAX_LEAF primitives.
-hipError_t make_nodesq(DeviceScene &d, BvhView &v, const Geometry &g, uint32_t num_n4, const uint32_t *ord4,
-                       uint32_t max_leaf, hipStream_t st, uint64_t *device_bytes) {
+// The reference-order FP32 nodes of the fast closest-hit traversals, made on the device from the type's Node4 records and
+// waited for, and for spheres and cylinders the leaves' FP64 boxes. None (every trace then takes the exact kernels) for
+// planes, for a tree that split precision does not take, one with an inverted or NaN box, or one with a leaf of more than
+// NODEQ_MAX_LEAF primitives.
+hipError_t make_nodesq(DeviceScene &d, BvhView &v, uint32_t type, const Geometry &g, uint32_t num_n4,
+                       const uint32_t *ord4, uint32_t max_leaf, hipStream_t st, uint64_t *device_bytes) {
   v.nodesq = nullptr;
-  if (!g.extent_ok || v.irregular_boxes || max_leaf > NODEQ_MAX_LEAF) return hipSuccess;
+  v.leaf_boxes = nullptr;
+  if (type == PLANES || !g.extent_ok || v.irregular_boxes || max_leaf > NODEQ_MAX_LEAF) return hipSuccess;
   const size_t bytes = std::max<size_t>(num_n4, 1) * sizeof(NodeQ);  // a root leaf has no records
   void *p = nullptr;
   hipError_t e = d.alloc(bytes, &p);
   if (e != hipSuccess) return e;
   if (num_n4) e = launch_nodeq_records(v.nodes4, ord4, num_n4, static_cast<NodeQ *>(p), st);
+  if (type != TRIANGLES && e == hipSuccess) {
+    const size_t box_bytes = (size_t)v.n_prims * 6 * sizeof(double);
+    void *b = nullptr;
+    e = d.alloc(box_bytes, &b);
+    if (e != hipSuccess) return e;
+    e = launch_leaf_boxes(v, v.n_nodes, static_cast<double *>(b), st);
+    v.leaf_boxes = static_cast<const double *>(b);
+    *device_bytes += box_bytes;
+  }
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   v.nodesq = static_cast<const NodeQ *>(p);
   *device_bytes += bytes;
@@ -1151,11 +1165,11 @@ int put_geometry(DeviceScene &d, Geometry &g, uint32_t t) {
     if (e == hipSuccess) e = d.put(g.vertices, &v.vertices);
   }
   if (e == hipSuccess) e = make_prim_filter(d, v, t, g.extent, nullptr, &g.stats.device_bytes);
-  if (e == hipSuccess && t == TRIANGLES) {
+  if (e == hipSuccess) {
     const uint32_t *ord4 = nullptr;
     e = d.put(g.ord4, &ord4);
     if (e == hipSuccess)
-      e = make_nodesq(d, v, g, g.num_n4, ord4, g.stats.max_num_prims_per_leaf, nullptr, &g.stats.device_bytes);
+      e = make_nodesq(d, v, t, g, g.num_n4, ord4, g.stats.max_num_prims_per_leaf, nullptr, &g.stats.device_bytes);
   }
   if (e != hipSuccess) return device_error(e, "upload failed");
   d.views[t] = v;
@@ -1334,9 +1348,8 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
                       (uint64_t)g.boxes.n * (r.rec_size + 4) + g.faces.size() * 4 + 2 * g.vertices.size() * 8;
     if (hipError_t fe = make_prim_filter(*d, v, t, g.extent, st, &bs.device_bytes))
       return device_error(fe, "pre-test records");
-    if (t == TRIANGLES)
-      if (hipError_t fe = make_nodesq(*d, v, g, r.num_n4, r.ord4, r.max_prims, st, &bs.device_bytes))
-        return device_error(fe, "fast traversal nodes");
+    if (hipError_t fe = make_nodesq(*d, v, t, g, r.num_n4, r.ord4, r.max_prims, st, &bs.device_bytes))
+      return device_error(fe, "fast traversal nodes");
     d->views[t] = v;
     bs.build_time_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   }
