@@ -160,7 +160,7 @@ hipError_t launch_cyl_filter_records(const void *recs, uint32_t n, void *out, hi
 
 // Triangles: assembles the reference-order nodes (NodeQ) from n Node4 records and their visiting orders (two words per
 // record, visit_order4).
-hipError_t launch_leaf_boxes(const BvhView &bvh, uint32_t num_nodes, double *out, hipStream_t stream);
+hipError_t launch_leaf_boxes(const BvhView &bvh, bool f32, void *out, hipStream_t stream);
 hipError_t launch_nodeq_records(const Node4 *nodes4, const uint32_t *ord, uint32_t n, NodeQ *out, hipStream_t stream);
 
 // Clears the counters of a group on the stream.
@@ -202,7 +202,7 @@ hipError_t launch_init_hits(const HitsView &hits, uint64_t n, hipStream_t stream
 
 // Scene<float>: traversal of one geometry type in FP32 (bvh.nodes32 and FP32 records), and the FP32 default RayHit.
 hipError_t launch_trace_f32(GeomType type, const BvhView &bvh, const RaysViewF &rays, const HitsViewF &hits,
-                            uint64_t n, const TraceLaunch &cfg, hipStream_t stream);
+                            uint64_t n, const TraceLaunch &cfg, double extent, hipStream_t stream);
 hipError_t launch_init_hits_f32(const HitsViewF &hits, uint64_t n, hipStream_t stream);
 
 // Distance queries (distance.hip). inv maps primitive ids to leaf positions (spheres, planes, cylinders; built by

@@ -198,10 +198,10 @@ struct BvhView {
   const uint32_t *faces;      // triangles only: user faces (3 per primitive id)
   const double *vnormals;     // triangles only: vertex normals (3 per vertex)
   const double *vertices;     // triangles only: user vertices (3 per vertex), for mirror tracing and its adjoint
-  const Node32 *nodes32;      // Scene<float>: FP32 nodes (nodes64 / nodes4 unused)
+  const Node32 *nodes32;      // Scene<float>: FP32 nodes (nodes64 unused, nodes4 dropped once nodesq is made)
   const TriFilt *tri_filter;  // split precision, triangles: FP32 pre-test records (NULL: every test in FP64)
   const NodeQ *nodesq;        // reference-order FP32 nodes (NULL: the exact kernels trace the type)
-  const double *leaf_boxes;   // spheres, cylinders: the FP64 box of each leaf at its first primitive (6 values)
+  const void *leaf_boxes;     // k_trace_wide's types: the box of each leaf at its first primitive (6 values of the scene type)
   const SphFilt *sph_filter;  // spheres: FP32 pre-test records (NULL: every test in FP64)
   const CylFilt *cyl_filter;  // cylinders: the same
   const float *vnormals32;    // Scene<float> triangles: vertex normals

@@ -500,6 +500,58 @@ float f32_up(double x) {
   return f;
 }
 
+// 4-wide FP32 records: every Node4 stands for one binary internal node, with up to four slots taken from its subtree by
+// collapse4 (largest internal slot opened first). Depth-first allocation keeps subtrees together. Returns the root's record,
+// or INVALID_ID for a root leaf.
+uint32_t make_nodes4(const std::vector<brt_tree_node> &T, std::vector<Node4> &n4, std::vector<uint32_t> &ord4) {
+  n4.clear();
+  ord4.clear();
+  uint32_t root4 = INVALID_ID;
+  if (!T.empty() && !T[0].leaf) {
+    std::vector<std::pair<uint32_t, uint32_t>> work;  // (binary internal node, its Node4 index)
+    n4.push_back(Node4{});
+    root4 = 0;
+    work.emplace_back(0u, 0u);
+    while (!work.empty()) {
+      const auto [bi, k4] = work.back();
+      work.pop_back();
+      uint32_t slot[4], axis[16] = {};
+      const int m = collapse4(T.data(), bi, slot, axis);
+      ord4.resize(2 * n4.size());
+      visit_order4(axis, m, &ord4[2ull * k4]);
+      Node4 nd{};
+      for (int c = 0; c < 4; c++) {
+        for (int k = 0; k < 3; k++) {
+          nd.lo[k][c] = __builtin_inff();
+          nd.hi[k][c] = -__builtin_inff();
+        }
+        nd.ref[c] = 0;
+        nd.cnt[c] = EMPTY_SLOT;
+      }
+      std::vector<std::pair<uint32_t, uint32_t>> children;
+      for (int c = 0; c < m; c++) {
+        const brt_tree_node &sn = T[slot[c]];
+        for (int k = 0; k < 3; k++) {
+          nd.lo[k][c] = f32_down(sn.min[k]);
+          nd.hi[k][c] = f32_up(sn.max[k]);
+        }
+        if (sn.leaf) {
+          nd.ref[c] = LEAF_BIT | sn.prim_begin;
+          nd.cnt[c] = sn.prim_count;
+        } else {
+          nd.ref[c] = (uint32_t)n4.size();
+          nd.cnt[c] = 0;
+          n4.push_back(Node4{});
+          children.emplace_back(slot[c], nd.ref[c]);
+        }
+      }
+      n4[k4] = nd;
+      for (auto it = children.rbegin(); it != children.rend(); ++it) work.push_back(*it);
+    }
+  }
+  return root4;
+}
+
 // Flattens the reference-form tree into children-in-parent records and leaf-order primitive records.
 void flatten(Geometry &g, GeomType type) {
   const auto &T = g.tree;
@@ -540,53 +592,7 @@ void flatten(Geometry &g, GeomType type) {
     }
     a.cnt[1] |= T[i].axis << AXIS_SHIFT;
   }
-  // 4-wide FP32 records: every Node4 stands for one binary internal node, with up to four slots taken from its
-  // subtree by collapse4 (largest internal slot opened first). Depth-first allocation keeps subtrees together.
-  g.n4.clear();
-  g.ord4.clear();
-  uint32_t root4 = INVALID_ID;
-  if (!T.empty() && !T[0].leaf) {
-    std::vector<std::pair<uint32_t, uint32_t>> work;  // (binary internal node, its Node4 index)
-    g.n4.push_back(Node4{});
-    root4 = 0;
-    work.emplace_back(0u, 0u);
-    while (!work.empty()) {
-      const auto [bi, k4] = work.back();
-      work.pop_back();
-      uint32_t slot[4], axis[16] = {};
-      const int m = collapse4(T.data(), bi, slot, axis);
-      g.ord4.resize(2 * g.n4.size());
-      visit_order4(axis, m, &g.ord4[2ull * k4]);
-      Node4 nd{};
-      for (int c = 0; c < 4; c++) {
-        for (int k = 0; k < 3; k++) {
-          nd.lo[k][c] = __builtin_inff();
-          nd.hi[k][c] = -__builtin_inff();
-        }
-        nd.ref[c] = 0;
-        nd.cnt[c] = EMPTY_SLOT;
-      }
-      std::vector<std::pair<uint32_t, uint32_t>> children;
-      for (int c = 0; c < m; c++) {
-        const brt_tree_node &sn = T[slot[c]];
-        for (int k = 0; k < 3; k++) {
-          nd.lo[k][c] = f32_down(sn.min[k]);
-          nd.hi[k][c] = f32_up(sn.max[k]);
-        }
-        if (sn.leaf) {
-          nd.ref[c] = LEAF_BIT | sn.prim_begin;
-          nd.cnt[c] = sn.prim_count;
-        } else {
-          nd.ref[c] = (uint32_t)g.n4.size();
-          nd.cnt[c] = 0;
-          g.n4.push_back(Node4{});
-          children.emplace_back(slot[c], nd.ref[c]);
-        }
-      }
-      g.n4[k4] = nd;
-      for (auto it = children.rbegin(); it != children.rend(); ++it) work.push_back(*it);
-    }
-  }
+  const uint32_t root4 = make_nodes4(T, g.n4, g.ord4);
   g.num_n4 = (uint32_t)g.n4.size();
   BvhView &v = g.view;
   v = BvhView{};
@@ -720,6 +726,18 @@ void flatten_f32(GeometryF &g, GeomType type) {
   }
   child_ref(0, v.root_ref, v.root_cnt);
   v.root_ref4 = v.root_ref;
+  // for the fast traversal; the records' FP32 boxes are the tree's
+  g.extent = 0.0;
+  g.num_n4 = 0;
+  if (type != USER_COLLECTION && type != PLANES && !irregular) {
+    if (make_nodes4(T, g.n4, g.ord4) != INVALID_ID) v.root_ref4 = 0;
+    g.num_n4 = (uint32_t)g.n4.size();
+  }
+  for (int k = 0; k < 3; k++) {
+    v.root_min32[k] = f32_down(T[0].min[k]);
+    v.root_max32[k] = f32_up(T[0].max[k]);
+    g.extent = std::max(g.extent, std::max(std::fabs(T[0].min[k]), std::fabs(T[0].max[k])));
+  }
   v.geom_id = g.geom_id;
   v.n_prims = g.boxes.n;
   v.n_nodes = ni;
@@ -876,6 +894,13 @@ struct DeviceScene {
     const hipError_t e = pool_get(device, bytes, p);
     if (e == hipSuccess) allocs.push_back(*p);
     return e;
+  }
+  // Gives memory from alloc() back early.
+  void release(const void *p) {
+    const auto it = std::find(allocs.begin(), allocs.end(), p);
+    if (!p || it == allocs.end()) return;
+    allocs.erase(it);
+    pool_put(device, const_cast<void *>(p), false);
   }
   // The counter group of `st`, allocated on the stream's first launch (NULL if that allocation fails).
   unsigned long long *counter_group(hipStream_t st) {
@@ -1121,26 +1146,26 @@ hipError_t make_prim_filter(DeviceScene &d, BvhView &v, uint32_t type, double ex
 }
 
 // The reference-order FP32 nodes of the fast closest-hit traversals, made on the device from the type's Node4 records and
-// waited for, and for spheres and cylinders the leaves' FP64 boxes. None (every trace then takes the exact kernels) for
+// waited for, and the leaves' boxes (not for an FP64 scene's triangles). None (every trace then takes the exact kernels) for
 // planes, for a tree that split precision does not take, one with an inverted or NaN box, or one with a leaf of more than
 // NODEQ_MAX_LEAF primitives.
-hipError_t make_nodesq(DeviceScene &d, BvhView &v, uint32_t type, const Geometry &g, uint32_t num_n4,
+hipError_t make_nodesq(DeviceScene &d, BvhView &v, uint32_t type, bool f32, double extent, uint32_t num_n4,
                        const uint32_t *ord4, uint32_t max_leaf, hipStream_t st, uint64_t *device_bytes) {
   v.nodesq = nullptr;
   v.leaf_boxes = nullptr;
-  if (type == PLANES || !g.extent_ok || v.irregular_boxes || max_leaf > NODEQ_MAX_LEAF) return hipSuccess;
+  if (type == PLANES || !(extent < 1e30) || v.irregular_boxes || max_leaf > NODEQ_MAX_LEAF) return hipSuccess;
   const size_t bytes = std::max<size_t>(num_n4, 1) * sizeof(NodeQ);  // a root leaf has no records
   void *p = nullptr;
   hipError_t e = d.alloc(bytes, &p);
   if (e != hipSuccess) return e;
   if (num_n4) e = launch_nodeq_records(v.nodes4, ord4, num_n4, static_cast<NodeQ *>(p), st);
-  if (type != TRIANGLES && e == hipSuccess) {
-    const size_t box_bytes = (size_t)v.n_prims * 6 * sizeof(double);
+  if ((type != TRIANGLES || f32) && e == hipSuccess) {
+    const size_t box_bytes = (size_t)v.n_prims * 6 * (f32 ? sizeof(float) : sizeof(double));
     void *b = nullptr;
     e = d.alloc(box_bytes, &b);
     if (e != hipSuccess) return e;
-    e = launch_leaf_boxes(v, v.n_nodes, static_cast<double *>(b), st);
-    v.leaf_boxes = static_cast<const double *>(b);
+    e = launch_leaf_boxes(v, f32, b, st);
+    v.leaf_boxes = b;
     *device_bytes += box_bytes;
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -1169,7 +1194,8 @@ int put_geometry(DeviceScene &d, Geometry &g, uint32_t t) {
     const uint32_t *ord4 = nullptr;
     e = d.put(g.ord4, &ord4);
     if (e == hipSuccess)
-      e = make_nodesq(d, v, t, g, g.num_n4, ord4, g.stats.max_num_prims_per_leaf, nullptr, &g.stats.device_bytes);
+      e = make_nodesq(d, v, t, false, g.extent_ok ? g.extent : INFINITY, g.num_n4, ord4,
+                      g.stats.max_num_prims_per_leaf, nullptr, &g.stats.device_bytes);
   }
   if (e != hipSuccess) return device_error(e, "upload failed");
   d.views[t] = v;
@@ -1188,6 +1214,17 @@ int put_geometry_f32(DeviceScene &d, GeometryF &g, uint32_t t) {
   if (t == TRIANGLES) {
     if (e == hipSuccess) e = d.put(g.faces, &v.faces);
     if (e == hipSuccess) e = d.put(g.vnormals, &v.vnormals32);
+  }
+  if (e == hipSuccess && (g.num_n4 || (v.root_ref & LEAF_BIT))) {
+    const uint32_t *ord4 = nullptr;
+    e = d.put(g.n4, &v.nodes4);
+    if (e == hipSuccess) e = d.put(g.ord4, &ord4);
+    if (e == hipSuccess)
+      e = make_nodesq(d, v, t, true, g.extent, g.num_n4, ord4, g.stats.max_num_prims_per_leaf, nullptr,
+                      &g.stats.device_bytes);
+    d.release(v.nodes4);  // only the nodes made from them are used
+    d.release(ord4);
+    v.nodes4 = nullptr;
   }
   if (e != hipSuccess) return device_error(e, "upload failed");
   d.views[t] = v;
@@ -1348,7 +1385,8 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
                       (uint64_t)g.boxes.n * (r.rec_size + 4) + g.faces.size() * 4 + 2 * g.vertices.size() * 8;
     if (hipError_t fe = make_prim_filter(*d, v, t, g.extent, st, &bs.device_bytes))
       return device_error(fe, "pre-test records");
-    if (hipError_t fe = make_nodesq(*d, v, t, g, r.num_n4, r.ord4, r.max_prims, st, &bs.device_bytes))
+    if (hipError_t fe = make_nodesq(*d, v, t, false, g.extent_ok ? g.extent : INFINITY, r.num_n4, r.ord4, r.max_prims, st,
+                                    &bs.device_bytes))
       return device_error(fe, "fast traversal nodes");
     d->views[t] = v;
     bs.build_time_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
@@ -1502,7 +1540,7 @@ int intersect1_t(const brt_scene *s, const R org[3], const R dir[3], R tmin, R t
       break;
     }
     if constexpr (std::is_same<R, float>::value)
-      e = launch_trace_f32((GeomType)t, ms->dev->views[t], rv, hv, 1, cfg, nullptr);
+      e = launch_trace_f32((GeomType)t, ms->dev->views[t], rv, hv, 1, cfg, g.extent, nullptr);
     else
       e = launch_trace((GeomType)t, ms->dev->views[t], rv, hv, 1, cfg, SplitParams{g.extent}, nullptr);
     if (e == hipSuccess) pending = true;
@@ -1962,7 +2000,7 @@ int brt_intersect_f32(const brt_scene *cs, const brt_rays_f32 *rays, const brt_h
     cfg.pool = L.pool_size;
     cfg.counter = s->dev->counter_group(st);
     if (!cfg.counter) return fail(BRT_ERR_OUT_OF_MEMORY, "launch counters");
-    hipError_t e = launch_trace_f32((GeomType)t, s->dev->views[t], rv, hv, n, cfg, st);
+    hipError_t e = launch_trace_f32((GeomType)t, s->dev->views[t], rv, hv, n, cfg, s->geoF[t].extent, st);
     if (e != hipSuccess) return fail(BRT_ERR_DEVICE, std::string("launch failed: ") + hipGetErrorString(e));
     first = false;
   }
