@@ -16,11 +16,14 @@
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
+#include <future>
 #include <memory>
 #include <mutex>
 #include <new>
 #include <numeric>
+#include <optional>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <type_traits>
 #include <unordered_map>
@@ -506,6 +509,8 @@ float f32_up(double x) {
 uint32_t make_nodes4(const std::vector<brt_tree_node> &T, std::vector<Node4> &n4, std::vector<uint32_t> &ord4) {
   n4.clear();
   ord4.clear();
+  n4.reserve(T.size() / 4 + 1);
+  ord4.reserve(T.size() / 2 + 2);
   uint32_t root4 = INVALID_ID;
   if (!T.empty() && !T[0].leaf) {
     std::vector<std::pair<uint32_t, uint32_t>> work;  // (binary internal node, its Node4 index)
@@ -517,7 +522,7 @@ uint32_t make_nodes4(const std::vector<brt_tree_node> &T, std::vector<Node4> &n4
       work.pop_back();
       uint32_t slot[4], axis[16] = {};
       const int m = collapse4(T.data(), bi, slot, axis);
-      ord4.resize(2 * n4.size());
+      ord4.resize(std::max(ord4.size(), 2 * n4.size()));
       visit_order4(axis, m, &ord4[2ull * k4]);
       Node4 nd{};
       for (int c = 0; c < 4; c++) {
@@ -528,7 +533,8 @@ uint32_t make_nodes4(const std::vector<brt_tree_node> &T, std::vector<Node4> &n4
         nd.ref[c] = 0;
         nd.cnt[c] = EMPTY_SLOT;
       }
-      std::vector<std::pair<uint32_t, uint32_t>> children;
+      std::pair<uint32_t, uint32_t> children[4];
+      int nc = 0;
       for (int c = 0; c < m; c++) {
         const brt_tree_node &sn = T[slot[c]];
         for (int k = 0; k < 3; k++) {
@@ -542,19 +548,42 @@ uint32_t make_nodes4(const std::vector<brt_tree_node> &T, std::vector<Node4> &n4
           nd.ref[c] = (uint32_t)n4.size();
           nd.cnt[c] = 0;
           n4.push_back(Node4{});
-          children.emplace_back(slot[c], nd.ref[c]);
+          children[nc++] = {slot[c], nd.ref[c]};
         }
       }
       n4[k4] = nd;
-      for (auto it = children.rbegin(); it != children.rend(); ++it) work.push_back(*it);
+      while (nc) work.push_back(children[--nc]);
     }
   }
   return root4;
 }
 
+// make_nodes4 beside the caller's own work on a larger tree (327,680 triangles: 15 of 135 ms of a Scene<float> commit).
+class Nodes4Job {
+public:
+  template <class R>
+  explicit Nodes4Job(GeometryT<R> &g) {
+    const auto run = [&g] { return make_nodes4(g.tree, g.n4, g.ord4); };
+    if (g.tree.size() >= 4096) {
+      try {
+        later = std::async(std::launch::async, run);
+        return;
+      } catch (const std::system_error &) {  // no thread to be had
+      }
+    }
+    root = run();
+  }
+  uint32_t get() { return later.valid() ? root = later.get() : root; }
+
+private:
+  std::future<uint32_t> later;
+  uint32_t root = INVALID_ID;
+};
+
 // Flattens the reference-form tree into children-in-parent records and leaf-order primitive records.
 void flatten(Geometry &g, GeomType type) {
   const auto &T = g.tree;
+  Nodes4Job nodes4(g);
   std::vector<uint32_t> internal(T.size(), INVALID_ID);
   uint32_t ni = 0;
   for (size_t i = 0; i < T.size(); i++)
@@ -592,8 +621,6 @@ void flatten(Geometry &g, GeomType type) {
     }
     a.cnt[1] |= T[i].axis << AXIS_SHIFT;
   }
-  const uint32_t root4 = make_nodes4(T, g.n4, g.ord4);
-  g.num_n4 = (uint32_t)g.n4.size();
   BvhView &v = g.view;
   v = BvhView{};
   for (int k = 0; k < 3; k++) {
@@ -606,7 +633,6 @@ void flatten(Geometry &g, GeomType type) {
     if (T[0].min[k] > T[0].max[k]) irregular = true;  // a root leaf's box is not among the children checked above
   }
   child_ref(0, v.root_ref, v.root_cnt);
-  v.root_ref4 = (root4 == INVALID_ID) ? v.root_ref : root4;
   v.geom_id = g.geom_id;
   v.n_prims = g.boxes.n;
   v.n_nodes = ni;
@@ -678,6 +704,9 @@ void flatten(Geometry &g, GeomType type) {
     break;
   }
   }
+  const uint32_t root4 = nodes4.get();
+  g.num_n4 = (uint32_t)g.n4.size();
+  v.root_ref4 = (root4 == INVALID_ID) ? v.root_ref : root4;
 }
 
 unsigned hw_threads() {
@@ -688,6 +717,8 @@ unsigned hw_threads() {
 // Scene<float>: the same children-in-parent layout with FP32 boxes, and FP32 records in leaf order.
 void flatten_f32(GeometryF &g, GeomType type) {
   const auto &T = g.tree;
+  std::optional<Nodes4Job> nodes4;  // for the fast traversal; the records' FP32 boxes are the tree's
+  if (type != USER_COLLECTION && type != PLANES) nodes4.emplace(g);
   std::vector<uint32_t> internal(T.size(), INVALID_ID);
   uint32_t ni = 0;
   for (size_t i = 0; i < T.size(); i++)
@@ -726,13 +757,7 @@ void flatten_f32(GeometryF &g, GeomType type) {
   }
   child_ref(0, v.root_ref, v.root_cnt);
   v.root_ref4 = v.root_ref;
-  // for the fast traversal; the records' FP32 boxes are the tree's
   g.extent = 0.0;
-  g.num_n4 = 0;
-  if (type != USER_COLLECTION && type != PLANES && !irregular) {
-    if (make_nodes4(T, g.n4, g.ord4) != INVALID_ID) v.root_ref4 = 0;
-    g.num_n4 = (uint32_t)g.n4.size();
-  }
   for (int k = 0; k < 3; k++) {
     v.root_min32[k] = f32_down(T[0].min[k]);
     v.root_max32[k] = f32_up(T[0].max[k]);
@@ -798,6 +823,8 @@ void flatten_f32(GeometryF &g, GeomType type) {
     });
     break;
   }
+  if (nodes4 && nodes4->get() != INVALID_ID) v.root_ref4 = 0;
+  g.num_n4 = (uint32_t)g.n4.size();
 }
 
 template <class R>
