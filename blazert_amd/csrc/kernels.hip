@@ -1099,14 +1099,16 @@ __device__ __forceinline__ bool fast_ray(const Ray &r, double len2, double S) {
          fabs(r.o[2]) <= FILTER_MAX_EXTENT;
 }
 
-// Rays of k_trace_wide: the FP32 bounds enclose the reference's traversal, whatever the length of the direction.
+// Rays of k_trace_wide: the FP32 bounds enclose the reference's traversal, whatever the length of the direction, within
+// limits that keep 1/d a normal FP32 number: as 0 it would make the infinite planes of a node's unused slots NaN, and the
+// slots passable.
 template <class R>
 __device__ __forceinline__ bool wide_ray(const RayT<R> &r, double S) {
   bool ok = (r.sign & RAY_NAN_FREE) && r.tmin >= R(0);
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     const double inv = fabs((double)r.inv[k]), o = fabs((double)r.o[k]);
-    ok = ok && inv * (S + o) <= 1e36 && inv <= 1e30 && o <= FILTER_MAX_EXTENT;
+    ok = ok && inv * (S + o) <= 1e36 && inv <= 1e30 && inv >= 1e-30 && o <= FILTER_MAX_EXTENT;
   }
   return ok;
 }
