@@ -2327,6 +2327,319 @@ k_trace_wide(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<typename
   }
 }
 
+// ------------------------------------------------------------------------------------------------ any hit, fast
+// Any hit of triangles in split precision: the first hit in the visiting order of trav_step<TriRec, true> (nearest box first,
+// ties as its sorting network leaves them), bit for bit. The hit distance never shrinks before the ray ends, so an entry
+// that was pushed is always visited: the stack needs no keys, and the parts of a ray are independent. A wave with nothing
+// left to start therefore shares its rays' bottom stack entries (the last parts of the order, as k_trace_tri does), and the
+// hit of the first part in the order that has one is the ray's; parts behind a hit are dropped.
+//
+// What bounds it (500,009 shadow rays, 100k triangles): the longest rays; k_trace_persistent<TriRec, true> kept the CUs busy
+// for 59% of the launch. Shared work, stack entries of two words and planes chosen by address take 20,000 rays from 136 to
+// 88 us a call, 500,009 from 318 to 302, 2,000,000 on 400k triangles from 1.10 to 0.98 ms; of that, waves that refill at 32 idle
+// lanes instead of 16 give 3%.
+struct AnyShare {
+  double h[SHARE_SLOTS], u[SHARE_SLOTS], v[SHARE_SLOTS];
+  uint32_t prim[SHARE_SLOTS];
+  uint32_t parts[SHARE_SLOTS];  // parts still running
+  uint32_t first[SHARE_SLOTS];  // position of the first part with a hit
+};
+
+struct AnyRay {
+  Ray32 b;
+  float D[3], O[3];
+};
+
+struct AnyTrav {
+  uint32_t cur, cnt, cand;
+  float h32;
+  bool active;
+};
+
+// One unit of the traversal (see tri_step): a Node4, the pre-test of two triangles, or the FP64 test of one.
+__device__ __forceinline__ void any_step(const BvhView &bvh, const Ray &r, const AnyRay &q, Hit &s, AnyTrav &t, WideStack &st) {
+  using u32x4 = unsigned int __attribute__((ext_vector_type(4)));
+  using Bytes = const __attribute__((address_space(1))) unsigned char;
+  using GlobalChunk = const __attribute__((address_space(1))) u32x4;
+  const bool at_leaf = (t.cur & LEAF_BIT) != 0;
+  const bool test = t.cand != 0u;
+  const uint32_t first = t.cur & ~LEAF_BIT;
+  const uint32_t p = first + (uint32_t)__builtin_ctz(t.cand | 0x80000000u);
+  // without pre-test records every triangle of the leaf gets the FP64 test (the fetch then reads triangle `first`)
+  Bytes *base = !at_leaf                            ? (Bytes *)(bvh.nodes4 + t.cur)
+                : test || bvh.tri_filter == nullptr ? (Bytes *)(reinterpret_cast<const TriRec *>(bvh.prims) + p)
+                                                    : (Bytes *)(bvh.tri_filter + first);
+  const bool record = test || (at_leaf && bvh.tri_filter == nullptr);
+  // node lanes read the near row of each axis into chunk a and the far row into chunk 3 + a (see tri_step)
+  const uint32_t sign = at_leaf ? 0u : q.b.sign;
+  const uint32_t n0 = (sign & 1u) * 48u, n1 = ((sign >> 1) & 1u) * 48u, n2 = ((sign >> 2) & 1u) * 48u;
+  u32x4 c0, c1, c2, c3, c4, c5, c6, c7;
+  c0 = *(GlobalChunk *)(base + n0);
+  c1 = *(GlobalChunk *)(base + n1 + 16);
+  c2 = *(GlobalChunk *)(base + n2 + 32);
+  c3 = *(GlobalChunk *)(base + (48u - n0));
+  c4 = *(GlobalChunk *)(base + (64u - n1));
+  if (!record) {  // a triangle record ends with chunk 4
+    c5 = *(GlobalChunk *)(base + (80u - n2));
+    c6 = *(GlobalChunk *)(base + 96);
+    c7 = *(GlobalChunk *)(base + 112);
+  }
+  asm volatile("" : "+v"(c0), "+v"(c1), "+v"(c2), "+v"(c3), "+v"(c4), "+v"(c5), "+v"(c6), "+v"(c7));
+  if (!at_leaf) {
+    float k[4];
+    uint32_t rf[4], cn[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const float a0 = __builtin_fmaf(__uint_as_float(c0[c]), q.b.inv[0], q.b.offn[0]);
+      const float a1 = __builtin_fmaf(__uint_as_float(c1[c]), q.b.inv[1], q.b.offn[1]);
+      const float a2 = __builtin_fmaf(__uint_as_float(c2[c]), q.b.inv[2], q.b.offn[2]);
+      const float f0 = __builtin_fmaf(__uint_as_float(c3[c]), q.b.inv[0], q.b.offf[0]);
+      const float f1 = __builtin_fmaf(__uint_as_float(c4[c]), q.b.inv[1], q.b.offf[1]);
+      const float f2 = __builtin_fmaf(__uint_as_float(c5[c]), q.b.inv[2], q.b.offf[2]);
+      const float A = max_nn(max3_nn(a0, a1, a2), q.b.tmin);
+      const float M = min_nn(min3_nn(f0, f1, f2), t.h32);
+      k[c] = (c7[c] != EMPTY_SLOT && A <= M) ? A : __builtin_inff();
+      rf[c] = c6[c];
+      cn[c] = c7[c];
+    }
+    sort4(k, rf, cn);
+    const float INF = __builtin_inff();
+    const int n = (k[0] < INF ? 1 : 0) + (k[1] < INF ? 1 : 0) + (k[2] < INF ? 1 : 0) + (k[3] < INF ? 1 : 0);
+    if (n) {
+      st.room(n - 1);
+      if (n > 1) st.put(st.sp + n - 2, rf[1], cn[1]);
+      if (n > 2) st.put(st.sp + n - 3, rf[2], cn[2]);
+      if (n > 3) st.put(st.sp, rf[3], cn[3]);
+      st.sp += n - 1;
+      t.cur = rf[0];
+      t.cnt = cn[0];
+      return;
+    }
+  } else if (!test) {
+    bool p0 = true, p1 = true;
+    if (bvh.tri_filter != nullptr) {
+      TriFilt g[2];
+      u32x4 raw[8] = {c0, c1, c2, c3, c4, c5, c6, c7};
+      __builtin_memcpy(g, raw, sizeof g);
+      p0 = tri_filter(g[0], q.D, q.O, q.b.om, q.b.tmin, t.h32);
+      p1 = tri_filter(g[1], q.D, q.O, q.b.om, q.b.tmin, t.h32);
+    }
+    t.cand = (p0 ? 1u : 0u) | (p1 && t.cnt > 1u ? 2u : 0u);
+    if (t.cand) return;
+    if (t.cnt > 2u) {
+      t.cnt -= 2u;
+      t.cur += 2u;
+      return;
+    }
+  } else {
+    TriRec rec;
+    u32x4 raw[5] = {c0, c1, c2, c3, c4};
+    __builtin_memcpy(&rec, raw, sizeof rec);
+    if (isect_tri(rec, r, s, p)) {
+      t.active = false;
+      return;
+    }
+    t.cand &= t.cand - 1u;
+    if (t.cand) return;
+    if (t.cnt > 2u) {
+      t.cnt -= 2u;
+      t.cur += 2u;
+      return;
+    }
+  }
+  if (st.sp > st.bot) {
+    const WideEntry e = st.pop();
+    t.cur = e.ref;
+    t.cnt = e.key;
+    return;
+  }
+  t.active = false;
+}
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BRT_WAVES_PER_EU)))
+k_trace_any(BvhView bvh, RaysView rays, HitsView hits, uint64_t n, uint32_t flags, uint32_t first, double S,
+            unsigned long long *group, uint32_t refill, const uint32_t *order, uint32_t ring, uint32_t chunk,
+            uint32_t fixed) {
+  extern __shared__ unsigned char smem[];
+  __shared__ AnyShare shares[4];
+  constexpr int RW = (int)(sizeof(RaysView) / 8), HW = (int)(sizeof(HitsView) / 8);
+  __shared__ uint64_t views[RW + HW];  // ray and hit columns, read back where they are used (see k_trace_persistent)
+  if (threadIdx.x == 0) {
+    lds_store(views, rays);
+    lds_store(views + RW, hits);
+  }
+  __syncthreads();
+  const uint32_t lane = __lane_id(), wave = threadIdx.x / 64;
+  BRT_LDS volatile AnyShare *sh = (BRT_LDS volatile AnyShare *)&shares[wave];
+  uint64_t spill[WIDE_SPILL];
+  WideStack st;
+  st.ring = (BRT_LDS uint32_t *)smem + (size_t)wave * ring * 128 + lane;
+  st.spill = spill;
+  st.mask = (int)ring - 1;
+  st.reset();
+  Ray r;
+  AnyRay q;
+  Hit s;
+  AnyTrav t;
+  t.active = false;
+  t.cand = 0;
+  bool has_ray = false, shared = false;
+  bool done = false;              // a traced ray, still to be written
+  bool exhausted = false;         // wave-uniform
+  uint32_t pos = 0, pos_end = 0;  // shared rays: this part's positions in the visiting order
+  uint32_t slot = 0, slots = 0;   // the share slot of this lane's ray; slots given out (wave-uniform)
+  uint64_t idx = 0;
+  const auto write_rays = [&]() {  // finished rays are written together (see k_trace_tri)
+    if (done) {
+      done = false;
+      finish_ray<TriRec>(bvh, lds_fresh<HitsView>(views + RW), idx, r, s, flags, first, 1u);
+    }
+  };
+  WavePool pool;
+  if (fixed) pool.take_fixed(((uint64_t)blockIdx.x * (blockDim.x / 64) + wave) * fixed, fixed, n);
+  uint32_t turn = 0;
+  for (;;) {
+    if (!exhausted) {
+      const unsigned long long idle = __ballot(!has_ray);
+      const uint32_t nidle = (uint32_t)__popcll(idle);
+      if (nidle >= refill || nidle == 64u) {
+        write_rays();
+        bool got;
+        uint64_t cand = 0;
+        pool_refill(pool, group + COUNTER_POOL, n, chunk, idle, nidle, lane, got, cand, exhausted);
+        if (got) {
+          idx = order ? (uint64_t)order[cand] : cand;
+          const RaysView V = lds_fresh<RaysView>(views);
+          start_ray<true>(bvh, V, idx, S, r, q.b, s);
+          if (deferred_to_exact(r)) {
+            __atomic_store_n(group + COUNTER_DEFERRED, 1ull, __ATOMIC_RELAXED);
+          } else {
+            has_ray = true;
+            Trav b;
+            trav_begin<true>(bvh, r, q.b, s, b);
+            t = AnyTrav{b.cur, b.cnt, 0u, b.h32, b.active};
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+              q.D[k] = (float)r.d[k];
+              q.O[k] = (float)r.o[k];
+            }
+            st.reset();
+          }
+        }
+      }
+    }
+    const unsigned long long busy = __ballot(has_ray);
+    if (exhausted) {
+      if (!busy) {
+        write_rays();
+        break;
+      }
+      // a part hands on the last eighth of its positions, so it needs eight for the order to stay strict
+      const unsigned long long can = __ballot(has_ray && st.sp > st.bot && (!shared || pos_end - pos >= 8u));
+      const uint32_t nidle = 64u - (uint32_t)__popcll(busy);
+      if (nidle >= SHARE_MIN_IDLE && can && (++turn & 1u) == 0u) {
+        write_rays();  // the helpers' state is overwritten
+        const unsigned long long below = (1ull << lane) - 1ull;
+        const uint32_t ncan = (uint32_t)__popcll(can), k = nidle < ncan ? nidle : ncan;
+        const bool able = ((can >> lane) & 1ull) != 0ull;
+        const uint32_t rank = (uint32_t)__popcll((has_ray ? can : ~busy) & below);
+        const bool donor = able && rank < k, helper = !has_ray && rank < k;
+        const uint32_t pos_end0 = shared ? pos_end : 0xffffffffu;
+        // the r-th helper takes from the r-th donor, whose lane number lane r receives
+        const unsigned long long fresh = __ballot(donor && !shared);
+        uint64_t e = 0;
+        if (donor) {
+          e = st.take_bottom();
+          if (!shared) {
+            shared = true;
+            slot = slots + (uint32_t)__popcll(fresh & below);
+            sh->parts[slot] = 1u;
+            sh->prim[slot] = INVALID_ID;
+            sh->h[slot] = r.tmax;
+            sh->first[slot] = 0xffffffffu;
+            pos = 0u;
+            pos_end = 0xffffffffu;
+          }
+          pos_end -= (pos_end - pos) >> 3;
+        }
+        slots += (uint32_t)__popcll(fresh);
+        wave_fence();
+        if (donor) atomicAdd(&shares[wave].parts[slot], 1u);
+        // (at most 32 donors: lane 63 takes what the others push)
+        const uint32_t by_rank = (uint32_t)__builtin_amdgcn_ds_permute((donor ? (int)rank : 63) << 2, (int)lane);
+        const uint32_t from = lane_get(by_rank, (int)rank);  // with all lanes: a permute reads active lanes only
+        const int src = helper ? (int)from : (int)lane;
+        lane_take(e, src, helper);
+        lane_take(r.o, src, helper);
+        lane_take(r.d, src, helper);
+        lane_take(r.tmin, src, helper);
+        lane_take(r.tmax, src, helper);
+        lane_take(q, src, helper);
+        lane_take(s.h, src, helper);
+        lane_take(t.h32, src, helper);
+        lane_take(idx, src, helper);
+        lane_take(slot, src, helper);
+        {
+          const uint32_t from_end = lane_get(pos_end, src), old_end = lane_get(pos_end0, src);
+          pos = helper ? from_end : pos;
+          pos_end = helper ? old_end : pos_end;
+        }
+        if (helper) {
+          has_ray = true;
+          shared = true;
+          s.leaf_idx = INVALID_ID;
+          t.cur = (uint32_t)e;
+          t.cnt = (uint32_t)(e >> 32);
+          t.cand = 0;
+          t.active = true;
+          st.reset();
+        }
+        wave_fence();
+      }
+    }
+    if (has_ray && t.active) {
+      if (shared && sh->first[slot] < pos) {  // behind a hit
+        t.active = false;
+      } else {
+        any_step(bvh, r, q, s, t, st);
+        if (shared && s.leaf_idx != INVALID_ID) atomicMin(&shares[wave].first[slot], pos);
+      }
+    }
+    bool fin = has_ray && !t.active;
+    if (exhausted) {
+      // the parts of a shared ray are merged one lane at a time; the last one writes the ray
+      unsigned long long m = __ballot(fin && shared);
+      while (m) {
+        const uint32_t l = (uint32_t)__ffsll((long long)m) - 1u;
+        m &= m - 1ull;
+        if (lane == l) {
+          const uint32_t parts = sh->parts[slot] - 1u;
+          sh->parts[slot] = parts;
+          if (s.leaf_idx != INVALID_ID && sh->first[slot] == pos) {
+            sh->h[slot] = s.h;
+            sh->u[slot] = s.u;
+            sh->v[slot] = s.v;
+            sh->prim[slot] = s.leaf_idx;
+          }
+          has_ray = false;
+          shared = false;
+          if (parts == 0u) {
+            s.h = sh->h[slot];
+            s.u = sh->u[slot];
+            s.v = sh->v[slot];
+            s.leaf_idx = sh->prim[slot];
+          } else {
+            fin = false;
+          }
+        }
+        wave_fence();
+      }
+    }
+    done = done || fin;
+    if (fin) has_ray = false;
+  }
+}
+
 // Split-precision pre-test records of the triangles in leaf order (TriFilt), from their FP64 records; the FILTER_PAD
 // records after the last one are zero.
 __global__ void k_tri_filter_records(const TriRec *__restrict__ recs, uint32_t n, TriFilt *out, uint32_t total) {
@@ -2534,6 +2847,24 @@ hipError_t persistent_blocks(K kernel, uint32_t block, size_t lds, uint64_t n, u
   return hipSuccess;
 }
 
+// The FP64 launch over the rays a split-precision launch deferred (default launch shape of the exact path).
+template <class Rec>
+hipError_t launch_deferred(const BvhView &bvh, const RaysViewT<typename Rec::real> &rays,
+                           const HitsViewT<typename Rec::real> &hits, uint64_t n, const TraceLaunch &cfg,
+                           const SplitParams &sp, uint32_t is_tri, hipStream_t stream) {
+  using R = typename Rec::real;
+  const uint32_t ring64 = ring_default<Rec, false>();
+  const size_t lds64 = ring_lds_bytes<false, R>(256, ring64);
+  uint64_t blocks = 0;
+  hipError_t e = persistent_blocks(k_trace_persistent<Rec, false>, 256, lds64, n, blocks);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_trace_persistent<Rec, false>), dim3((uint32_t)blocks), dim3(256), lds64, stream, bvh, rays,
+                     hits, n, cfg.flags | FLAG_DEFERRED_ONLY, cfg.first ? 1u : 0u, is_tri, sp.scene_extent,
+                     cfg.counter + COUNTER_DEFERRED_POOL, refill_default<Rec, false>(), cfg.order, ring64,
+                     cfg.counter + COUNTER_DEFERRED, POOL_CHUNK);
+  return hipGetLastError();
+}
+
 // Enqueues one traversal of a geometry type: the counter group is cleared, then the trace kernel runs. A split-
 // precision launch is followed by the FP64 launch over the rays it deferred (deferred_to_exact), which returns at
 // once when there are none; both run in stream order before the next geometry type, so intersect1's merge order
@@ -2567,23 +2898,13 @@ hipError_t launch_kernel(const BvhView &bvh, const RaysViewT<typename Rec::real>
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !SPLIT) return e;
-  // the FP64 launch over the deferred rays (default launch shape of the exact path)
-  const uint32_t ring64 = ring_default<Rec, false>();
-  const size_t lds64 = ring_lds_bytes<false, R>(256, ring64);
-  uint64_t blocks = 0;
-  e = persistent_blocks(k_trace_persistent<Rec, false>, 256, lds64, n, blocks);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((k_trace_persistent<Rec, false>), dim3((uint32_t)blocks), dim3(256), lds64, stream, bvh, rays,
-                     hits, n, cfg.flags | FLAG_DEFERRED_ONLY, first, is_tri, sp.scene_extent,
-                     grp + COUNTER_DEFERRED_POOL, refill_default<Rec, false>(), cfg.order, ring64,
-                     grp + COUNTER_DEFERRED, POOL_CHUNK);
-  return hipGetLastError();
+  return launch_deferred<Rec>(bvh, rays, hits, n, cfg, sp, is_tri, stream);
 }
 
 // The fast triangle traversal (k_trace_tri) takes closest-hit launches on the persistent schedule, in either precision:
 // 1.31M-triangle mesh, 4,194,304 incoherent rays 3.03 ms, against 5.6-5.8 ms for the exact FP64 kernel and 3.8 ms for
 // nearest-first split precision; a 1920x1080 camera with normals 2.24 against 3.57 ms. Any-hit launches return the first
-// hit of their own visiting order and keep the kernels that define it; the one-ray-per-thread schedule keeps its kernel.
+// hit of their own visiting order; the one-ray-per-thread schedule keeps its kernel.
 bool fast_triangles(const TraceLaunch &cfg) {
   return cfg.schedule == SCHEDULE_PERSISTENT && !(cfg.flags & FLAG_ANY_HIT);
 }
@@ -2595,7 +2916,12 @@ bool fast_triangles(const TraceLaunch &cfg) {
 bool fast_wide(const BvhView &bvh, const TraceLaunch &cfg) {
   return bvh.nodesq && bvh.leaf_boxes && cfg.precision == PREC_FP64 && fast_triangles(cfg);
 }
-constexpr uint32_t TRI_RING = 16, TRI_REFILL = 16;
+// Any hit of triangles in split precision on the persistent schedule takes k_trace_any (figures there). In FP64 the first
+// accepted hit of the reference's order counts, which only boxes tested in FP64 give: the exact kernel.
+bool fast_any(const TraceLaunch &cfg) {
+  return cfg.schedule == SCHEDULE_PERSISTENT && cfg.precision != PREC_FP64 && (cfg.flags & FLAG_ANY_HIT);
+}
+constexpr uint32_t TRI_RING = 16, TRI_REFILL = 16, ANY_REFILL = 32;
 constexpr size_t tri_lds_bytes(uint32_t block, uint32_t ring) { return (size_t)block * ring * sizeof(uint64_t); }
 
 hipError_t launch_tri(const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint64_t n,
@@ -2662,6 +2988,30 @@ hipError_t launch_wide(const BvhView &bvh, const RaysViewT<typename Rec::real> &
                      hits, n, cfg.flags, first, is_tri, sp.scene_extent, grp + COUNTER_DEFERRED_POOL,
                      refill_default<Rec, false>(), cfg.order, ring64, grp + COUNTER_DEFERRED, POOL_CHUNK);
   return hipGetLastError();
+}
+
+// Any hit of triangles in split precision (k_trace_any).
+hipError_t launch_any(const BvhView &bvh, const RaysView &rays, const HitsView &hits, uint64_t n, const TraceLaunch &cfg,
+                      const SplitParams &sp, hipStream_t stream) {
+  const uint32_t block = cfg.block ? cfg.block : 256;
+  const uint32_t ring = cfg.ring ? cfg.ring : TRI_RING;
+  const size_t lds = tri_lds_bytes(block, ring);
+  unsigned long long *grp = cfg.counter;
+  if (!grp) return hipErrorInvalidValue;
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
+  uint64_t blocks = 0;
+  hipError_t e = persistent_blocks(k_trace_any, block, lds, n * 64, blocks);
+  if (e != hipSuccess) return e;
+  const uint32_t wpb = block / 64, fixed = fixed_per_wave(n, blocks * wpb);
+  const uint64_t need = fixed ? (n + fixed * wpb - 1) / (fixed * wpb) : (n + block - 1) / block;
+  if (blocks > need) blocks = need;
+  hipLaunchKernelGGL(k_trace_any, dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits, n, cfg.flags,
+                     cfg.first ? 1u : 0u, sp.scene_extent, grp, cfg.refill ? cfg.refill : ANY_REFILL, cfg.order, ring,
+                     cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return launch_deferred<TriRec>(bvh, rays, hits, n, cfg, sp, 1u, stream);
 }
 
 hipError_t launch_tri_batch(const BatchJob *jobs, uint32_t njobs, uint64_t total, const TraceLaunch &cfg,
@@ -2744,6 +3094,7 @@ hipError_t launch_trace(GeomType type, const BvhView &bvh, const RaysView &rays,
   switch (type) {
   case TRIANGLES:
     if (bvh.nodesq && fast_triangles(cfg)) return launch_tri(bvh, rays, hits, n, cfg, split, stream);
+    if (fast_any(cfg)) return launch_any(bvh, rays, hits, n, cfg, split, stream);
     return launch_typed<TriRec>(bvh, rays, hits, n, cfg, split, 1u, stream);
   case SPHERES: return launch_other<SphRec>(bvh, rays, hits, n, cfg, split, stream);
   case PLANES: return launch_typed<PlaRec>(bvh, rays, hits, n, cfg, split, cfg.overwrite ? 1u : 0u, stream);
