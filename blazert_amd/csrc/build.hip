@@ -349,11 +349,24 @@ __global__ void k_lv_bounds(Level L, const uint32_t *__restrict__ idx, const dou
       mn[k] = dmin(mn[k], __shfl_xor(mn[k], off));
       mx[k] = dmax(mx[k], __shfl_xor(mx[k], off));
     }
+  // one atomic per block and side: they serialise on a large node's six words (16 levels of 1.31M: 558 ->
+  // 255 us)
+  __shared__ double part[BLOCK / 64][6];
   if ((threadIdx.x & 63) == 0)
     for (int k = 0; k < 3; k++) {
-      atomicMin(&nd.klo[k], okey(mn[k]));
-      atomicMax(&nd.khi[k], okey(mx[k]));
+      part[threadIdx.x / 64][k] = mn[k];
+      part[threadIdx.x / 64][3 + k] = mx[k];
     }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    double v = part[0][threadIdx.x];
+    for (int w = 1; w < BLOCK / 64; w++) v = dmin(v, part[w][threadIdx.x]);
+    atomicMin(&nd.klo[threadIdx.x], okey(v));
+  } else if (threadIdx.x < 6) {
+    double v = part[0][threadIdx.x];
+    for (int w = 1; w < BLOCK / 64; w++) v = dmax(v, part[w][threadIdx.x]);
+    atomicMax(&nd.khi[threadIdx.x - 3], okey(v));
+  }
 }
 
 __global__ void k_lv_prep(Level L, uint32_t m, uint32_t min_leaf, uint32_t max_depth) {
@@ -506,20 +519,33 @@ __global__ void k_lv_rank1(Level L, const uint32_t *__restrict__ idx, const doub
   }
 }
 
-// Per node: block offsets of the misplaced counts.
-__global__ void k_lv_rank2(Level L, uint32_t m) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  LNode &nd = L.nodes[i];
+// Per node: block offsets of the misplaced counts, a wave's scan (one thread walking a large node's blocks: 276 us for
+// 16 levels of 1.31M, 75 us this way).
+__global__ void __launch_bounds__(64) k_lv_rank2(Level L) {
+  LNode &nd = L.nodes[blockIdx.x];
   if (nd.leaf || !nd.split) return;
+  const uint32_t lane = threadIdx.x;
   uint32_t sl = 0, sr = 0;
-  for (uint32_t b = nd.blk0; b < nd.blk0 + nd.nblk; b++) {
-    L.off_l[b] = sl;
-    L.off_r[b] = sr;
-    sl += L.blk_l[b];
-    sr += L.blk_r[b];
+  for (uint32_t base = 0; base < nd.nblk; base += 64u) {
+    const uint32_t b = nd.blk0 + base + lane;
+    const bool in = base + lane < nd.nblk;
+    const uint32_t l = in ? L.blk_l[b] : 0u, r = in ? L.blk_r[b] : 0u;
+    uint32_t pl = l, pr = r;  // inclusive sums
+    for (uint32_t off = 1; off < 64u; off <<= 1) {
+      const uint32_t ul = __shfl_up(pl, off), ur = __shfl_up(pr, off);
+      if (lane >= off) {
+        pl += ul;
+        pr += ur;
+      }
+    }
+    if (in) {
+      L.off_l[b] = sl + pl - l;
+      L.off_r[b] = sr + pr - r;
+    }
+    sl += __shfl(pl, 63);
+    sr += __shfl(pr, 63);
   }
-  nd.misplaced = sr;
+  if (lane == 0) nd.misplaced = sr;
 }
 
 // Positions of the right part's passing elements, indexed by their rank from the right end.
@@ -1409,7 +1435,7 @@ hipError_t device_build(const DeviceBuildIn &in, DeviceBuildOut &out, hipStream_
     BRT_LAUNCH(k_lv_count<<<nblocks, BLOCK, 0, st>>>(L, idx, ctr));
     BRT_LAUNCH(k_lv_decide<<<blocks_for(m, 64), 64, 0, st>>>(L, m));
     BRT_LAUNCH(k_lv_rank1<<<nblocks, BLOCK, 0, st>>>(L, idx, ctr));
-    BRT_LAUNCH(k_lv_rank2<<<blocks_for(m, 64), 64, 0, st>>>(L, m));
+    BRT_LAUNCH(k_lv_rank2<<<m, 64, 0, st>>>(L));
     BRT_LAUNCH(k_lv_rank3<<<nblocks, BLOCK, 0, st>>>(L, idx, ctr, pos_r));
     BRT_LAUNCH(k_lv_swap<<<nblocks, BLOCK, 0, st>>>(L, idx, ctr, pos_r));
     BRT_CHECK(hipMemcpyAsync(hn.data(), d_nodes, m * sizeof(LNode), hipMemcpyDeviceToHost, st));
