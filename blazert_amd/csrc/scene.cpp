@@ -1143,7 +1143,7 @@ int device_error(hipError_t e, const char *what) {
 }
 
 // The FP32 pre-test records of a triangle (TriFilt), sphere (SphFilt) or cylinder (CylFilt) geometry, made on the
-// device from its uploaded FP64 records and waited for; none for other types, or when the scene's extent is above
+// device from its uploaded FP64 records; the caller waits for it. None for other types, or when the scene's extent is above
 // FILTER_MAX_EXTENT. BLAZERT_AMD_SPLIT_PRETEST=0 in the environment at upload time leaves them out (every
 // primitive test then runs in FP64; the hits are the same, which the tests check).
 hipError_t make_prim_filter(DeviceScene &d, BvhView &v, uint32_t type, double extent, hipStream_t st,
@@ -1164,7 +1164,6 @@ hipError_t make_prim_filter(DeviceScene &d, BvhView &v, uint32_t type, double ex
   e = type == TRIANGLES ? launch_tri_filter_records(v.prims, v.n_prims, p, st)
       : type == SPHERES  ? launch_sph_filter_records(v.prims, v.n_prims, p, st)
                          : launch_cyl_filter_records(v.prims, v.n_prims, p, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (type == TRIANGLES) v.tri_filter = static_cast<const TriFilt *>(p);
   else if (type == SPHERES) v.sph_filter = static_cast<const SphFilt *>(p);
   else v.cyl_filter = static_cast<const CylFilt *>(p);
@@ -1172,8 +1171,8 @@ hipError_t make_prim_filter(DeviceScene &d, BvhView &v, uint32_t type, double ex
   return e;
 }
 
-// The reference-order FP32 nodes of the fast closest-hit traversals, made on the device from the type's Node4 records and
-// waited for, and the leaves' boxes (not for an FP64 scene's triangles). None (every trace then takes the exact kernels) for
+// The reference-order FP32 nodes of the fast closest-hit traversals, made on the device from the type's Node4 records (the
+// caller waits for it), and the leaves' boxes (not for an FP64 scene's triangles). None (every trace then takes the exact kernels) for
 // planes, for a tree that split precision does not take, one with an inverted or NaN box, or one with a leaf of more than
 // NODEQ_MAX_LEAF primitives.
 hipError_t make_nodesq(DeviceScene &d, BvhView &v, uint32_t type, bool f32, double extent, uint32_t num_n4,
@@ -1195,7 +1194,6 @@ hipError_t make_nodesq(DeviceScene &d, BvhView &v, uint32_t type, bool f32, doub
     v.leaf_boxes = b;
     *device_bytes += box_bytes;
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
   v.nodesq = static_cast<const NodeQ *>(p);
   *device_bytes += bytes;
   return e;
@@ -1224,6 +1222,7 @@ int put_geometry(DeviceScene &d, Geometry &g, uint32_t t) {
       e = make_nodesq(d, v, t, false, g.extent_ok ? g.extent : INFINITY, g.num_n4, ord4,
                       g.stats.max_num_prims_per_leaf, nullptr, &g.stats.device_bytes);
   }
+  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // launches on any stream may read what was made
   if (e != hipSuccess) return device_error(e, "upload failed");
   d.views[t] = v;
   return BRT_OK;
@@ -1249,7 +1248,8 @@ int put_geometry_f32(DeviceScene &d, GeometryF &g, uint32_t t) {
     if (e == hipSuccess)
       e = make_nodesq(d, v, t, true, g.extent, g.num_n4, ord4, g.stats.max_num_prims_per_leaf, nullptr,
                       &g.stats.device_bytes);
-    d.release(v.nodes4);  // only the nodes made from them are used
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // launches on any stream may read what was made
+    d.release(v.nodes4);                                    // only the nodes made from them are used
     d.release(ord4);
     v.nodes4 = nullptr;
   }
@@ -1415,6 +1415,7 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
     if (hipError_t fe = make_nodesq(*d, v, t, false, g.extent_ok ? g.extent : INFINITY, r.num_n4, r.ord4, r.max_prims, st,
                                     &bs.device_bytes))
       return device_error(fe, "fast traversal nodes");
+    if (hipError_t fe = hipStreamSynchronize(st)) return device_error(fe, "fast traversal nodes");
     d->views[t] = v;
     bs.build_time_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   }
