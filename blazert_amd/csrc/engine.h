@@ -77,12 +77,12 @@ constexpr int COUNTER_DEFERRED_POOL = 2;
 constexpr int CLAIM_COUNTERS = 8;
 constexpr int COUNTER_STRIDE = 16;
 constexpr int COUNTER_CLEARED = CLAIM_COUNTERS * COUNTER_STRIDE;  // slots a launch clears (1 KiB)
-// Rays whose fast triangle traversal could not be certified (k_trace_tri) are listed behind the counters, for the
-// exact launch that follows: COUNTER_LISTED counts them, and when there are more than LIST_CAPACITY that launch traces
-// every ray.
+// Rays that a fast traversal leaves to the exact launch behind it are listed behind the counters: COUNTER_LISTED counts
+// them, and when there are more than LIST_CAPACITY that launch traces every ray. A launch with a fixed range of at most 64
+// rays per wave writes one word per wave there instead, a bit for each ray left, and needs no cleared counters.
 constexpr int COUNTER_LISTED = 3;
-constexpr int LIST_CAPACITY = 3968;
-constexpr int COUNTER_GROUP = COUNTER_CLEARED + LIST_CAPACITY;  // slots per group (32 KiB)
+constexpr int LIST_CAPACITY = 8064;
+constexpr int COUNTER_GROUP = COUNTER_CLEARED + LIST_CAPACITY;  // slots per group (64 KiB)
 
 constexpr uint32_t SCHEDULE_PERSISTENT = 0;  // persistent waves with per-lane ray refill (default)
 constexpr uint32_t SCHEDULE_PER_THREAD = 1;  // one ray per thread, grid-stride

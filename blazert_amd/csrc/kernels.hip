@@ -1141,12 +1141,13 @@ __device__ __forceinline__ bool fast_ray(const RaysViewT<typename Rec::real> &V,
   else return wide_ray(r, S);
 }
 
-// One ray per thread (grid-stride).
+// One ray per thread (grid-stride). left: only the rays whose bits a launch of `fixed` rays per wave set there.
 template <class Rec, bool SPLIT>
 __global__ void __launch_bounds__(256) k_trace(BvhView bvh, RaysViewT<typename Rec::real> rays,
                                                HitsViewT<typename Rec::real> hits, uint64_t n, uint32_t flags,
                                                uint32_t first, uint32_t is_tri, double S, const uint32_t *order,
-                                               uint32_t ring, unsigned long long *deferred) {
+                                               uint32_t ring, unsigned long long *deferred,
+                                               const unsigned long long *left = nullptr, uint32_t fixed = 1) {
   using R = typename Rec::real;
   extern __shared__ unsigned char smem[];
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -1157,6 +1158,7 @@ __global__ void __launch_bounds__(256) k_trace(BvhView bvh, RaysViewT<typename R
   RingStack<SPLIT, R> st;
   ring_bind<SPLIT, R>(st, smem, &spill, ring);
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) {
+    if (left && !((left[k / fixed] >> (k % fixed)) & 1ull)) continue;
     const uint64_t i = order ? (uint64_t)order[k] : k;
     RayT<R> r;
     Ray32 q;
@@ -1712,7 +1714,9 @@ __device__ __forceinline__ unsigned long long bound_of(float h32, uint32_t pos) 
 
 // Persistent waves as in k_trace_persistent. BATCH: the rays of many jobs, as in k_trace_batch. LONE: one ray by one wave,
 // without counters; where it would be listed or deferred, `merged` says so (RAY_LEFT) and nothing else is written.
-template <bool BATCH, bool LONE = false>
+// FIXED: the waves of a single-scene launch take `fixed` rays each and mark the rays left in a word of their own (a kernel of
+// its own: in the claiming one that code costs 7%).
+template <bool BATCH, bool LONE = false, bool FIXED = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BRT_WAVES_PER_EU)))
 k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t n,
             uint32_t flags, uint32_t first, double S, unsigned long long *group, uint32_t refill,
@@ -1763,15 +1767,18 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
   uint32_t slot = 0, slots = 0;  // the share slot of this lane's ray; slots given out (wave-uniform)
   uint64_t idx = 0;        // ray index, within its job
   uint32_t j = 0;
+  uint32_t number = 0;  // FIXED: the ray's in the wave's range
+  unsigned long long mask = 0;  // wave-uniform
   // Finished rays are written together, when the wave refills: a ray ends in almost every iteration, and writing it
   // there would run this code for a lane or two each time.
   auto write_rays = [&]() {
+    if constexpr (FIXED) mask_add(mask, done && t.listed, number);
     if (done) {
       done = false;
       if (t.listed) {
         if constexpr (LONE) {
           st_stream(lds_fresh<HitsView>(views + RW).merged, idx, RAY_LEFT);
-        } else {
+        } else if constexpr (!FIXED) {
           const unsigned long long k = atomicAdd(group + COUNTER_LISTED, 1ull);
           if (k < (unsigned long long)LIST_CAPACITY) {
             group[COUNTER_CLEARED + k] = BATCH ? jobs[j].offset + idx : idx;
@@ -1805,8 +1812,9 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
     }
   };
   WavePool pool;
+  const uint64_t global_wave = (uint64_t)blockIdx.x * (blockDim.x / 64) + wave, range = global_wave * fixed;
   if (fixed)  // a small launch: no claims, and the other lanes help from the start
-    pool.take_fixed(((uint64_t)blockIdx.x * (blockDim.x / 64) + wave) * fixed, fixed, n);
+    pool.take_fixed(range, fixed, n);
   uint32_t turn = 0;
   for (;;) {
     if (!exhausted) {
@@ -1817,6 +1825,7 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
         bool got;
         uint64_t cand = 0;
         pool_refill(pool, group + COUNTER_POOL, n, chunk, idle, nidle, lane, got, cand, exhausted);
+        bool defer = false;
         double ext = S;
         TriRoot root{};
         RawRay raw{};
@@ -1851,6 +1860,7 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
             }
           }
         } else if (LONE || got) {
+          if constexpr (FIXED) number = (uint32_t)(cand - range);
           idx = order ? (uint64_t)order[cand] : cand;
           root = tri_root(bvh);
           raw = load_ray(lds_fresh<RaysView>(views), idx);
@@ -1874,16 +1884,20 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
             t.active = t.listed = false;
           } else if constexpr (LONE) {
             st_stream(lds_fresh<HitsView>(views + RW).merged, idx, RAY_LEFT);
+          } else if constexpr (FIXED) {
+            defer = true;
           } else {
             __atomic_store_n(group + COUNTER_DEFERRED, 1ull, __ATOMIC_RELAXED);
           }
         }
+        if constexpr (FIXED) mask_add(mask, defer, number);
       }
     }
     const unsigned long long busy = __ballot(has_ray);
     if (exhausted) {
       if (!busy) {
         write_rays();
+        if (FIXED && lane == 0) group[COUNTER_CLEARED + global_wave] = mask;
         break;
       }
       const unsigned long long can = __ballot(has_ray && st.sp > st.bot);
@@ -1930,6 +1944,7 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
           lane_take(q, src, helper);
           lane_take(idx, src, helper);
           lane_take(slot, src, helper);
+          if constexpr (FIXED) lane_take(number, src, helper);
         }
         lane_take(s.h, src, helper);
         lane_take(t.h32, src, helper);
@@ -2096,13 +2111,27 @@ __device__ __forceinline__ void wide_step(const BvhView &bvh, const RayT<typenam
   };
   u32x4 c0, c1, c2, c3, c4, c5, c6, c7;
   c0 = *(GlobalChunk *)(base + near0);
-  if (!at_leaf || has(1)) c1 = *(GlobalChunk *)(base + near1 + 16);
-  if (!at_leaf || has(2)) c2 = *(GlobalChunk *)(base + near2 + 32);
-  if (!at_leaf || has(3)) c3 = *(GlobalChunk *)(base + 48);
-  if (!at_leaf || has(4)) c4 = *(GlobalChunk *)(base + (64u - near0));
-  if (!at_leaf || has(5)) c5 = *(GlobalChunk *)(base + (64u - near1) + 16);
-  if (!at_leaf || has(6)) c6 = *(GlobalChunk *)(base + (64u - near2) + 32);
-  if (!at_leaf || has(7)) c7 = *(GlobalChunk *)(base + 112);
+  if constexpr (FILTER) {
+    c1 = *(GlobalChunk *)(base + near1 + 16);
+    if (!at_leaf || has(3)) {
+      c2 = *(GlobalChunk *)(base + near2 + 32);
+      c3 = *(GlobalChunk *)(base + 48);
+    }
+    if (!at_leaf || has(7)) {
+      c4 = *(GlobalChunk *)(base + (64u - near0));
+      c5 = *(GlobalChunk *)(base + (64u - near1) + 16);
+      c6 = *(GlobalChunk *)(base + (64u - near2) + 32);
+      c7 = *(GlobalChunk *)(base + 112);
+    }
+  } else {
+    if (!at_leaf || has(1)) c1 = *(GlobalChunk *)(base + near1 + 16);
+    if (!at_leaf || has(2)) c2 = *(GlobalChunk *)(base + near2 + 32);
+    if (!at_leaf || has(3)) c3 = *(GlobalChunk *)(base + 48);
+    if (!at_leaf || has(4)) c4 = *(GlobalChunk *)(base + (64u - near0));
+    if (!at_leaf || has(5)) c5 = *(GlobalChunk *)(base + (64u - near1) + 16);
+    if (!at_leaf || has(6)) c6 = *(GlobalChunk *)(base + (64u - near2) + 32);
+    if (!at_leaf || has(7)) c7 = *(GlobalChunk *)(base + 112);
+  }
   u32x4 more[MORE + 1];
 #pragma unroll
   for (int k = 0; k < MORE; k++)
@@ -2182,7 +2211,7 @@ __device__ __forceinline__ void wide_step(const BvhView &bvh, const RayT<typenam
     for (int k = 0; k < MORE; k++) raw[8 + k] = more[k];
 #pragma unroll
     for (uint32_t g = 0; g < (FILTER ? 1u : FG); g++) {
-      if (g >= t.cnt) break;
+      if (!FILTER && g >= t.cnt) break;
       Rec rec;
       __builtin_memcpy(&rec, raw + g * REC_Q, sizeof rec);
       const HitT<R> old = s;
@@ -2228,7 +2257,7 @@ __device__ __forceinline__ void wide_step(const BvhView &bvh, const RayT<typenam
   t.active = false;
 }
 
-template <class Rec>
+template <class Rec, bool FIXED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BRT_WAVES_PER_EU)))
 k_trace_wide(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<typename Rec::real> hits, uint64_t n,
              uint32_t flags, uint32_t first, uint32_t is_tri, double S, unsigned long long *group, uint32_t refill, const uint32_t *order, uint32_t ring, uint32_t chunk,
@@ -2259,12 +2288,17 @@ k_trace_wide(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<typename
   t.cand = 0;
   bool has_ray = false, done = false, exhausted = false;
   uint64_t idx = 0;
+  uint32_t number = 0;  // see k_trace_tri
+  unsigned long long mask = 0;
   const auto write_rays = [&]() {  // finished rays are written together (see k_trace_tri)
+    if constexpr (FIXED) mask_add(mask, done && t.listed, number);
     if (done) {
       done = false;
       if (t.listed) {
-        const unsigned long long k = atomicAdd(group + COUNTER_LISTED, 1ull);
-        if (k < (unsigned long long)LIST_CAPACITY) group[COUNTER_CLEARED + k] = idx;
+        if constexpr (!FIXED) {
+          const unsigned long long k = atomicAdd(group + COUNTER_LISTED, 1ull);
+          if (k < (unsigned long long)LIST_CAPACITY) group[COUNTER_CLEARED + k] = idx;
+        }
       } else {
         finish_ray<Rec>(bvh, lds_fresh<HitsV>(views + RW), idx, r, s, flags, first, is_tri);
       }
@@ -2277,7 +2311,8 @@ k_trace_wide(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<typename
     x.inv[2] = R(1) / V.dz[idx];
   };
   WavePool pool;
-  if (fixed) pool.take_fixed(((uint64_t)blockIdx.x * (blockDim.x / 64) + wave) * fixed, fixed, n);
+  const uint64_t global_wave = (uint64_t)blockIdx.x * (blockDim.x / 64) + wave, range = global_wave * fixed;
+  if constexpr (FIXED) pool.take_fixed(range, fixed, n);
   for (;;) {
     if (!exhausted) {
       const unsigned long long idle = __ballot(!has_ray);
@@ -2287,7 +2322,9 @@ k_trace_wide(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<typename
         bool got;
         uint64_t cand = 0;
         pool_refill(pool, group + COUNTER_POOL, n, chunk, idle, nidle, lane, got, cand, exhausted);
+        bool defer = false;
         if (got) {
+          if constexpr (FIXED) number = (uint32_t)(cand - range);
           idx = order ? (uint64_t)order[cand] : cand;
           const RawRayT<R> raw = load_ray(lds_fresh<RaysV>(views), idx);
           setup_ray(raw.org, raw.dir, raw.tmin, raw.tmax, r);
@@ -2307,14 +2344,18 @@ k_trace_wide(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<typename
             tri_begin(tri_root(bvh), r, q, s, b);
             t = WideTrav{b.cur, b.cnt, 0u, b.cur & ~LEAF_BIT, b.h32, b.active, false, false};
             st.reset();
+          } else if constexpr (FIXED) {
+            defer = true;
           } else {
             __atomic_store_n(group + COUNTER_DEFERRED, 1ull, __ATOMIC_RELAXED);
           }
         }
+        if constexpr (FIXED) mask_add(mask, defer, number);
       }
     }
     if (exhausted && !__ballot(has_ray)) {
       write_rays();
+      if (FIXED && lane == 0) group[COUNTER_CLEARED + global_wave] = mask;
       break;
     }
     if (has_ray) {
@@ -2456,6 +2497,7 @@ __device__ __forceinline__ void any_step(const BvhView &bvh, const Ray &r, const
   t.active = false;
 }
 
+template <bool FIXED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BRT_WAVES_PER_EU)))
 k_trace_any(BvhView bvh, RaysView rays, HitsView hits, uint64_t n, uint32_t flags, uint32_t first, double S,
             unsigned long long *group, uint32_t refill, const uint32_t *order, uint32_t ring, uint32_t chunk,
@@ -2489,6 +2531,7 @@ k_trace_any(BvhView bvh, RaysView rays, HitsView hits, uint64_t n, uint32_t flag
   uint32_t pos = 0, pos_end = 0;  // shared rays: this part's positions in the visiting order
   uint32_t slot = 0, slots = 0;   // the share slot of this lane's ray; slots given out (wave-uniform)
   uint64_t idx = 0;
+  unsigned long long mask = 0;  // see k_trace_tri
   const auto write_rays = [&]() {  // finished rays are written together (see k_trace_tri)
     if (done) {
       done = false;
@@ -2496,7 +2539,8 @@ k_trace_any(BvhView bvh, RaysView rays, HitsView hits, uint64_t n, uint32_t flag
     }
   };
   WavePool pool;
-  if (fixed) pool.take_fixed(((uint64_t)blockIdx.x * (blockDim.x / 64) + wave) * fixed, fixed, n);
+  const uint64_t global_wave = (uint64_t)blockIdx.x * (blockDim.x / 64) + wave, range = global_wave * fixed;
+  if constexpr (FIXED) pool.take_fixed(range, fixed, n);
   uint32_t turn = 0;
   for (;;) {
     if (!exhausted) {
@@ -2507,12 +2551,14 @@ k_trace_any(BvhView bvh, RaysView rays, HitsView hits, uint64_t n, uint32_t flag
         bool got;
         uint64_t cand = 0;
         pool_refill(pool, group + COUNTER_POOL, n, chunk, idle, nidle, lane, got, cand, exhausted);
+        bool defer = false;
         if (got) {
           idx = order ? (uint64_t)order[cand] : cand;
           const RaysView V = lds_fresh<RaysView>(views);
           start_ray<true>(bvh, V, idx, S, r, q.b, s);
           if (deferred_to_exact(r)) {
-            __atomic_store_n(group + COUNTER_DEFERRED, 1ull, __ATOMIC_RELAXED);
+            defer = true;
+            if constexpr (!FIXED) __atomic_store_n(group + COUNTER_DEFERRED, 1ull, __ATOMIC_RELAXED);
           } else {
             has_ray = true;
             Trav b;
@@ -2526,12 +2572,14 @@ k_trace_any(BvhView bvh, RaysView rays, HitsView hits, uint64_t n, uint32_t flag
             st.reset();
           }
         }
+        if constexpr (FIXED) mask_add(mask, defer, (uint32_t)(cand - range));
       }
     }
     const unsigned long long busy = __ballot(has_ray);
     if (exhausted) {
       if (!busy) {
         write_rays();
+        if (FIXED && lane == 0) group[COUNTER_CLEARED + global_wave] = mask;
         break;
       }
       // a part hands on the last eighth of its positions, so it needs eight for the order to stay strict
@@ -2865,6 +2913,19 @@ hipError_t launch_deferred(const BvhView &bvh, const RaysViewT<typename Rec::rea
   return hipGetLastError();
 }
 
+// The exact launch over the rays that a launch of `fixed` rays per wave left.
+template <class Rec>
+hipError_t launch_left(const BvhView &bvh, const RaysViewT<typename Rec::real> &rays,
+                       const HitsViewT<typename Rec::real> &hits, uint64_t n, const TraceLaunch &cfg, const SplitParams &sp,
+                       uint32_t is_tri, uint32_t fixed, hipStream_t stream) {
+  const uint32_t ring = ring_default<Rec, false>();
+  hipLaunchKernelGGL((k_trace<Rec, false>), dim3((uint32_t)((n + 255) / 256)), dim3(256),
+                     (ring_lds_bytes<false, typename Rec::real>(256, ring)), stream, bvh, rays, hits, n, cfg.flags,
+                     cfg.first ? 1u : 0u, is_tri, sp.scene_extent, cfg.order, ring, cfg.counter + COUNTER_DEFERRED,
+                     cfg.counter + COUNTER_CLEARED, fixed);
+  return hipGetLastError();
+}
+
 // Enqueues one traversal of a geometry type: the counter group is cleared, then the trace kernel runs. A split-
 // precision launch is followed by the FP64 launch over the rays it deferred (deferred_to_exact), which returns at
 // once when there are none; both run in stream order before the next geometry type, so intersect1's merge order
@@ -2894,7 +2955,8 @@ hipError_t launch_kernel(const BvhView &bvh, const RaysViewT<typename Rec::real>
     uint64_t blocks = (n + block - 1) / block;
     if (blocks > (1ull << 30)) blocks = 1ull << 30;
     hipLaunchKernelGGL((k_trace<Rec, SPLIT>), dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits, n,
-                       cfg.flags, first, is_tri, sp.scene_extent, cfg.order, ring, grp + COUNTER_DEFERRED);
+                       cfg.flags, first, is_tri, sp.scene_extent, cfg.order, ring, grp + COUNTER_DEFERRED,
+                       (const unsigned long long *)nullptr, 1u);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !SPLIT) return e;
@@ -2933,18 +2995,21 @@ hipError_t launch_tri(const BvhView &bvh, const RaysView &rays, const HitsView &
   unsigned long long *grp = cfg.counter;
   if (!grp) return hipErrorInvalidValue;
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
   uint64_t blocks = 0;
   hipError_t e = persistent_blocks(k_trace_tri<false>, block, lds, n * 64, blocks);
   if (e != hipSuccess) return e;
-  const uint32_t wpb = block / 64, fixed = fixed_per_wave(n, blocks * wpb);
+  const uint32_t wpb = block / 64;
+  uint32_t fixed = fixed_per_wave(n, blocks * wpb);
+  if (blocks * wpb > (uint64_t)LIST_CAPACITY) fixed = 0;  // (a word per wave)
+  if (!fixed) hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
   const uint64_t need = fixed ? (n + fixed * wpb - 1) / (fixed * wpb) : (n + block - 1) / block;
   if (blocks > need) blocks = need;
-  hipLaunchKernelGGL(k_trace_tri<false>, dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits,
+  hipLaunchKernelGGL((fixed ? k_trace_tri<false, false, true> : k_trace_tri<false>), dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits,
                      (const BatchJob *)nullptr, 0u, n, cfg.flags, first, sp.scene_extent, grp,
                      cfg.refill ? cfg.refill : TRI_REFILL, cfg.order, ring, cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (fixed) return launch_left<TriRec>(bvh, rays, hits, n, cfg, sp, 1u, fixed, stream);
   // the rays it left to the exact kernel (default launch shape of the exact path)
   const uint32_t ring64 = ring_default<TriRec, false>();
   const size_t lds64 = ring_lds_bytes<false, double>(256, ring64);
@@ -2968,18 +3033,21 @@ hipError_t launch_wide(const BvhView &bvh, const RaysViewT<typename Rec::real> &
   unsigned long long *grp = cfg.counter;
   if (!grp) return hipErrorInvalidValue;
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
   uint64_t blocks = 0;
-  hipError_t e = persistent_blocks(k_trace_wide<Rec>, block, lds, n * 64, blocks);
+  hipError_t e = persistent_blocks(k_trace_wide<Rec, false>, block, lds, n * 64, blocks);
   if (e != hipSuccess) return e;
-  const uint32_t wpb = block / 64, fixed = fixed_per_wave(n, blocks * wpb);
+  const uint32_t wpb = block / 64;
+  uint32_t fixed = fixed_per_wave(n, blocks * wpb);
+  if (blocks * wpb > (uint64_t)LIST_CAPACITY) fixed = 0;  // (a word per wave)
+  if (!fixed) hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
   const uint64_t need = fixed ? (n + fixed * wpb - 1) / (fixed * wpb) : (n + block - 1) / block;
   if (blocks > need) blocks = need;
-  hipLaunchKernelGGL(k_trace_wide<Rec>, dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits, n, cfg.flags,
+  hipLaunchKernelGGL((fixed ? k_trace_wide<Rec, true> : k_trace_wide<Rec, false>), dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits, n, cfg.flags,
                      first, is_tri, sp.scene_extent, grp, cfg.refill ? cfg.refill : TRI_REFILL, cfg.order, ring,
                      cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (fixed) return launch_left<Rec>(bvh, rays, hits, n, cfg, sp, is_tri, fixed, stream);
   const uint32_t ring64 = ring_default<Rec, false>();
   const size_t lds64 = ring_lds_bytes<false, R>(256, ring64);
   e = persistent_blocks(k_trace_persistent<Rec, false, true>, 256, lds64, n, blocks);
@@ -2999,18 +3067,21 @@ hipError_t launch_any(const BvhView &bvh, const RaysView &rays, const HitsView &
   unsigned long long *grp = cfg.counter;
   if (!grp) return hipErrorInvalidValue;
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
   uint64_t blocks = 0;
-  hipError_t e = persistent_blocks(k_trace_any, block, lds, n * 64, blocks);
+  hipError_t e = persistent_blocks(k_trace_any<false>, block, lds, n * 64, blocks);
   if (e != hipSuccess) return e;
-  const uint32_t wpb = block / 64, fixed = fixed_per_wave(n, blocks * wpb);
+  const uint32_t wpb = block / 64;
+  uint32_t fixed = fixed_per_wave(n, blocks * wpb);
+  if (blocks * wpb > (uint64_t)LIST_CAPACITY) fixed = 0;  // (a word per wave)
+  if (!fixed) hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
   const uint64_t need = fixed ? (n + fixed * wpb - 1) / (fixed * wpb) : (n + block - 1) / block;
   if (blocks > need) blocks = need;
-  hipLaunchKernelGGL(k_trace_any, dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits, n, cfg.flags,
+  hipLaunchKernelGGL((fixed ? k_trace_any<true> : k_trace_any<false>), dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits, n, cfg.flags,
                      cfg.first ? 1u : 0u, sp.scene_extent, grp, cfg.refill ? cfg.refill : ANY_REFILL, cfg.order, ring,
                      cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (fixed) return launch_left<TriRec>(bvh, rays, hits, n, cfg, sp, 1u, fixed, stream);
   return launch_deferred<TriRec>(bvh, rays, hits, n, cfg, sp, 1u, stream);
 }
 

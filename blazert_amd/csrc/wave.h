@@ -120,6 +120,16 @@ inline uint32_t fixed_per_wave(uint64_t n, uint64_t waves) {
   return per <= 64 ? (uint32_t)per : 0u;
 }
 
+// Adds the numbers of the lanes with `set` to a wave-uniform mask; called by the whole wave.
+__device__ __forceinline__ void mask_add(unsigned long long &mask, bool set, uint32_t number) {
+  unsigned long long m = __ballot(set);
+  while (m) {
+    const int l = __ffsll((long long)m) - 1;
+    mask |= 1ull << (uint32_t)__builtin_amdgcn_readlane((int)number, l);
+    m &= m - 1ull;
+  }
+}
+
 // Called by every lane of a wave with the same pool state when the wave refills. An idle lane handed an index gets
 // it in `idx` and `got`; `exhausted` is set once nothing is left to hand out. `counter` is the first of the
 // launch's CLAIM_COUNTERS counters (COUNTER_STRIDE slots apart).
