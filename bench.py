@@ -458,7 +458,7 @@ def cpu_baseline(osc, org, dirs, ns, threads) -> dict:
 def kernel_sources_hash() -> str:
     import hashlib
     h = hashlib.sha256()
-    for name in ("kernels.hip", "engine.h", "layout.h"):
+    for name in ("kernels.hip", "engine.h", "layout.h", "wave.h"):
         h.update(open(os.path.join(ROOT, "blazert_amd", "csrc", name), "rb").read())
     h.update(open(os.path.join(ROOT, "include", "blazert_amd", "device", "exact.h"), "rb").read())
     return h.hexdigest()[:16]

@@ -2046,8 +2046,8 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
 // What bounds it (8,388,608 incoherent rays): the vector ALU, 74% busy with a quarter of the lanes active, since a wave runs
 // the node, pre-test and FP64 branches in almost every iteration for a few lanes each. Lanes with an FP64 test, or with a
 // pre-test, therefore wait until WIDE_MIN_LANES of the wave have one (or no other lane has anything else to do): 50,000
-// spheres 4.19 -> 3.24 ms (8 lanes: 3.36, 24: 3.62), against 4.44 ms for the exact kernel; 10,000 cylinders 3.65 -> 3.46 ms,
-// against 5.45 ms. (k_trace_tri, bound by the data path of the L1, gains nothing from it.) A wave with no rays left to take
+// spheres 4.19 -> 3.24 ms (8 lanes: 3.36, 24: 3.62), against 4.44 ms for the exact kernel; 10,000 cylinders 4.90 -> 4.59 ms
+// (3.68 with the pre-test against the axis), against 5.45 ms. (k_trace_tri, bound by the data path of the L1, gains nothing from it.) A wave with no rays left to take
 // doesn't wait: there the longest ray counts. In FP32 the primitives are tested without a pre-test.
 constexpr int WIDE_MIN_LANES = 16;
 
@@ -2211,7 +2211,7 @@ __device__ __forceinline__ void wide_step(const BvhView &bvh, const RayT<typenam
     for (int k = 0; k < MORE; k++) raw[8 + k] = more[k];
 #pragma unroll
     for (uint32_t g = 0; g < (FILTER ? 1u : FG); g++) {
-      if (!FILTER && g >= t.cnt) break;
+      if (g >= t.cnt) break;
       Rec rec;
       __builtin_memcpy(&rec, raw + g * REC_Q, sizeof rec);
       const HitT<R> old = s;
@@ -2971,9 +2971,9 @@ bool fast_triangles(const TraceLaunch &cfg) {
   return cfg.schedule == SCHEDULE_PERSISTENT && !(cfg.flags & FLAG_ANY_HIT);
 }
 // Spheres' and cylinders' (k_trace_wide), in FP64 (split precision has a visiting order of its own): 8,388,608 incoherent
-// rays, 50,000 spheres 3.24 against 4.44 ms, 10,000 cylinders 3.48 against 5.45 ms; a 512x512 camera over 1,024 spheres 0.094
+// rays, 50,000 spheres 3.25 against 4.44 ms, 10,000 cylinders 3.68 against 5.45 ms; a 512x512 camera over 1,024 spheres 0.091
 // against 0.137 ms a call. 100 planes 1.75 against 1.61 ms: they keep the exact kernel. In a Scene<float>, incoherent rays:
-// 1,000,003 on 327,680 triangles 0.65 against 0.83 ms, on 50,000 spheres 0.45 against 0.48, 2,000 on 81,920 triangles 0.089
+// 1,000,003 on 327,680 triangles 0.63 against 0.83 ms, on 50,000 spheres 0.45 against 0.48, 2,000 on 81,920 triangles 0.089
 // against 0.192; 1920x1080 camera rays on 1.31M triangles 2.05 against 2.62 ms.
 bool fast_wide(const BvhView &bvh, const TraceLaunch &cfg) {
   return bvh.nodesq && bvh.leaf_boxes && cfg.precision == PREC_FP64 && fast_triangles(cfg);
