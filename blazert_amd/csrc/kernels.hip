@@ -2405,7 +2405,7 @@ __device__ __forceinline__ void any_step(const BvhView &bvh, const Ray &r, const
   const bool at_leaf = (t.cur & LEAF_BIT) != 0;
   const bool test = t.cand != 0u;
   const uint32_t first = t.cur & ~LEAF_BIT;
-  const uint32_t p = first + (uint32_t)__builtin_ctz(t.cand | 0x80000000u);
+  const uint32_t p = leaf_record(first, t.cand);
   // without pre-test records every triangle of the leaf gets the FP64 test (the fetch then reads triangle `first`)
   Bytes *base = !at_leaf                            ? (Bytes *)(bvh.nodes4 + t.cur)
                 : test || bvh.tri_filter == nullptr ? (Bytes *)(reinterpret_cast<const TriRec *>(bvh.prims) + p)

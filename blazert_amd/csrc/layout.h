@@ -89,6 +89,12 @@ static_assert(sizeof(TriFilt) == 64, "TriFilt size");
 constexpr uint32_t FILTER_GROUP = BRT_FILTER_GROUP;  // triangles pre-tested per traversal step
 constexpr uint32_t FILTER_PAD = FILTER_GROUP - 1;
 
+// The primitive whose record a lane at a leaf reads: the lowest candidate of its group, which starts at `first`, or `first`
+// itself while no candidate is known. Never a place behind the leaf, whose records may be the last of their allocation.
+inline __host__ __device__ uint32_t leaf_record(uint32_t first, uint32_t cand) {
+  return cand ? first + (uint32_t)__builtin_ctz(cand) : first;
+}
+
 // Split precision: FP32 pre-test record of a sphere, in leaf order beside the SphRec array: the center rounded to
 // nearest and |r| rounded up. Built on the device from the SphRec array; SPH_FILTER_PAD zero records follow the last one, so a group of
 // SPH_FILTER_GROUP records read from any leaf start stays in bounds.
