@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <functional>
+
 #include "../../include/blazert_amd.h"
 #include "layout.h"
 
@@ -221,10 +223,11 @@ struct ClosestViews {
 // Gathers the triangles' vertices in leaf order (9 doubles per triangle) for the closest-surface query.
 hipError_t launch_leaf_vertices(const uint32_t *order, const uint32_t *faces, const double *vertices, uint32_t n,
                                 double *out, hipStream_t stream);
-// group: the stream's launch counters (used for triangles).
+// claims: called when a search of triangles is too large for one range per wave (fixed_per_wave); gives COUNTER_CLEARED
+// words that no other launch uses before this one has ended, or NULL where there are none to be had.
 hipError_t launch_closest_surface(const ClosestViews &views, const double *px, const double *py, const double *pz,
-                                  uint64_t n, double *dist, uint32_t *prim, uint32_t *geom, unsigned long long *group,
-                                  hipStream_t stream);
+                                  uint64_t n, double *dist, uint32_t *prim, uint32_t *geom,
+                                  const std::function<unsigned long long *()> &claims, hipStream_t stream);
 
 // Device memory of scenes and builds (scene.cpp). hipMalloc and hipFree of a scene's arrays and a build's workspace cost
 // more than building it (1.31M triangles: 50 and 46 calls, 10.5 of 20 ms), so freed blocks are kept for the next one: up

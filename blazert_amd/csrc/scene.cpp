@@ -903,6 +903,8 @@ struct DeviceScene {
   // group first, so they can share it; launches on different streams never share one.
   std::mutex counter_mu;
   std::vector<std::pair<hipStream_t, unsigned long long *>> stream_counters;
+  std::mutex closest_mu;
+  std::vector<std::pair<hipStream_t, unsigned long long *>> closest_claims;  // COUNTER_CLEARED words per stream
   std::mutex inv_mu;
   uint32_t *inv_order[NUM_TYPES]{};  // primitive id -> leaf position, made on the first distance query
   double *leaf_vertices = nullptr;    // triangles' vertices in leaf order, made on the first closest-surface query
@@ -913,6 +915,7 @@ struct DeviceScene {
     for (auto &w : sorts)
       if (w.second->base) (void)hipFree(w.second->base);
     for (auto &c : stream_counters) pool_put(device, c.second, false);
+    for (auto &c : closest_claims) pool_put(device, c.second, false);
     for (void *p : allocs) pool_put(device, p, false);
     pool_release(device);
   }
@@ -928,6 +931,24 @@ struct DeviceScene {
     if (!p || it == allocs.end()) return;
     allocs.erase(it);
     pool_put(device, const_cast<void *>(p), false);
+  }
+  // Counters of the closest-surface searches enqueued on `st`, which run in order; the caller holds closest_mu. NULL (the
+  // search then does without) where that order doesn't hold: under capture, since graphs may be replayed on any stream and
+  // side by side, and for the per-thread default stream, which one handle names for all threads.
+  unsigned long long *closest_counters(hipStream_t st) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (st == hipStreamPerThread || hipStreamIsCapturing(st, &capturing) != hipSuccess ||
+        capturing != hipStreamCaptureStatusNone)
+      return nullptr;
+    for (auto &c : closest_claims)
+      if (c.first == st) return c.second;
+    void *p = nullptr;
+    if (pool_get(device, COUNTER_CLEARED * sizeof(unsigned long long), &p) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    closest_claims.emplace_back(st, static_cast<unsigned long long *>(p));
+    return closest_claims.back().second;
   }
   // The counter group of `st`, allocated on the stream's first launch (NULL if that allocation fails).
   unsigned long long *counter_group(hipStream_t st) {
@@ -1779,10 +1800,14 @@ int brt_closest_surface(const brt_scene *cs, const brt_points *points, uint64_t 
     }
     cv.leaf_vertices = s->dev->leaf_vertices;
   }
-  unsigned long long *group = s->dev->counter_group(static_cast<hipStream_t>(stream));
-  if (!group) return fail(BRT_ERR_OUT_OF_MEMORY, "launch counters");
-  hipError_t e = launch_closest_surface(cv, points->x, points->y, points->z, n, distance, prim_id, geom_id, group,
-                                        static_cast<hipStream_t>(stream));
+  // Held until the search is enqueued, so that a thread's clearing of the counters and its search stay together.
+  std::unique_lock<std::mutex> lk(s->dev->closest_mu, std::defer_lock);
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  const auto claims = [&] {
+    lk.lock();
+    return s->dev->closest_counters(st);
+  };
+  hipError_t e = launch_closest_surface(cv, points->x, points->y, points->z, n, distance, prim_id, geom_id, claims, st);
   if (e != hipSuccess) return device_error(e, "launch failed");
   return BRT_OK;
 }

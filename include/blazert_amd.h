@@ -208,7 +208,11 @@ int brt_distance_to_surface(const brt_scene *scene, uint32_t geom_type, const br
  * and BRT_INVALID_ID when no primitive gives a distance. Extension: the reference has no scene-level distance query
  * (docs/source/roadmap.rst). Asynchronous on `stream`, except that the first call on a scene with triangles
  * allocates (hipMalloc, 72 bytes per triangle) and fills a leaf-order copy of the triangles' vertices, then waits
- * for it; do not graph-capture that first call. */
+ * for it; do not graph-capture that first call. Every other call may be captured, also the first on its stream, and
+ * such graphs may be replayed on any streams, side by side. Outside capture, a search of more points than the GPU
+ * takes in one go (about 262,144) uses 1 KiB of counters per scene and stream, allocated on the stream's first such
+ * search, so a stream's searches should have ended before it is destroyed; where the allocation fails the search does
+ * without them. */
 int brt_closest_surface(const brt_scene *scene, const brt_points *points, uint64_t n, double *distance,
                         uint32_t *prim_id, uint32_t *geom_id, void *stream);
 
