@@ -886,6 +886,15 @@ DevicePool &pool_of(int device) {
   return *p;
 }
 
+// Waits for the device's streams by freeing memory, as freeing the block itself would have. (hipDeviceSynchronize is refused
+// while any thread captures a stream, and ends that capture.) False where that is refused.
+bool wait_for_device() {
+  void *p = nullptr;
+  if (hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 // Frees every kept block; the caller holds the pool's mutex.
 void pool_trim(DevicePool &P) {
   for (auto &b : P.free_blocks) (void)hipFree(b.p);
@@ -995,16 +1004,15 @@ hipError_t pool_get(int device, size_t bytes, void **p) {
   const size_t want = (bytes + step - 1) / step * step;
   DevicePool &P = pool_of(device);
   std::lock_guard<std::mutex> lk(P.mu);
+  // the smallest block that fits, one that is idle before one that may still be in use
   auto best = P.free_blocks.end();
   for (auto it = P.free_blocks.begin(); it != P.free_blocks.end(); ++it)
-    if (it->bytes >= want && it->bytes <= want + want / 4 && (best == P.free_blocks.end() || it->bytes < best->bytes))
+    if (it->bytes >= want && it->bytes <= want + want / 4 &&
+        (best == P.free_blocks.end() || it->idle > best->idle || (it->idle == best->idle && it->bytes < best->bytes)))
       best = it;
-  if (best != P.free_blocks.end()) {
-    if (!best->idle) {
-      const hipError_t e = hipDeviceSynchronize();
-      if (e != hipSuccess) return e;
-      for (auto &b : P.free_blocks) b.idle = true;
-    }
+  if (best != P.free_blocks.end() && !best->idle && wait_for_device())
+    for (auto &b : P.free_blocks) b.idle = true;
+  if (best != P.free_blocks.end() && best->idle) {
     *p = best->p;
     P.held -= best->bytes;
     P.sizes[best->p] = best->bytes;
