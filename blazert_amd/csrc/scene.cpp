@@ -908,10 +908,16 @@ struct DeviceScene {
   int device = -1;
   std::vector<void *> allocs;
   BvhView views[NUM_TYPES]{};
-  // One group of launch counters per stream (COUNTER_GROUP): launches on one stream run in order and each clears its
-  // group first, so they can share it; launches on different streams never share one.
+  // One group of launch counters per stream (COUNTER_GROUP): launches on one stream run in order and each clears or writes
+  // its group first, so they can share it; launches on different streams never share one. A launch is several kernels, which
+  // another thread's must not come between: whoever enqueues them holds `mu`.
+  struct LaunchCounters {
+    hipStream_t stream;
+    unsigned long long *words;
+    std::mutex mu;
+  };
   std::mutex counter_mu;
-  std::vector<std::pair<hipStream_t, unsigned long long *>> stream_counters;
+  std::vector<std::unique_ptr<LaunchCounters>> stream_counters;
   std::mutex closest_mu;
   std::vector<std::pair<hipStream_t, unsigned long long *>> closest_claims;  // COUNTER_CLEARED words per stream
   std::mutex inv_mu;
@@ -923,7 +929,7 @@ struct DeviceScene {
   ~DeviceScene() {
     for (auto &w : sorts)
       if (w.second->base) (void)hipFree(w.second->base);
-    for (auto &c : stream_counters) pool_put(device, c.second, false);
+    for (auto &c : stream_counters) pool_put(device, c->words, false);
     for (auto &c : closest_claims) pool_put(device, c.second, false);
     for (void *p : allocs) pool_put(device, p, false);
     pool_release(device);
@@ -960,17 +966,20 @@ struct DeviceScene {
     return closest_claims.back().second;
   }
   // The counter group of `st`, allocated on the stream's first launch (NULL if that allocation fails).
-  unsigned long long *counter_group(hipStream_t st) {
+  LaunchCounters *counter_group(hipStream_t st) {
     std::lock_guard<std::mutex> lk(counter_mu);
     for (auto &c : stream_counters)
-      if (c.first == st) return c.second;
+      if (c->stream == st) return c.get();
     // a first launch under capture is refused, as the allocation it needs would be; kept memory must not change that
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return nullptr;
+    auto c = std::make_unique<LaunchCounters>();
+    c->stream = st;
     void *p = nullptr;
     if (pool_get(device, COUNTER_GROUP * sizeof(unsigned long long), &p) != hipSuccess) return nullptr;
-    stream_counters.emplace_back(st, static_cast<unsigned long long *>(p));
-    return stream_counters.back().second;
+    c->words = static_cast<unsigned long long *>(p);
+    stream_counters.push_back(std::move(c));
+    return stream_counters.back().get();
   }
   SortWorkspace *sort_workspace(hipStream_t st) {
     std::lock_guard<std::mutex> lk(sort_mu);
@@ -1590,12 +1599,14 @@ int intersect1_t(const brt_scene *s, const R org[3], const R dir[3], R tmin, R t
         q->merged = 0u;
       }
     }
-    TraceLaunch cfg{BRT_PRECISION_FP64, flags | BRT_FLAG_HITS_INOUT, 64, false, SCHEDULE_PER_THREAD, 0,
-                    ms->dev->counter_group(nullptr), nullptr};
-    if (!cfg.counter) {
+    DeviceScene::LaunchCounters *counters = ms->dev->counter_group(nullptr);
+    if (!counters) {
       e = hipErrorOutOfMemory;
       break;
     }
+    std::lock_guard<std::mutex> enqueue(counters->mu);
+    TraceLaunch cfg{BRT_PRECISION_FP64, flags | BRT_FLAG_HITS_INOUT, 64, false, SCHEDULE_PER_THREAD, 0, counters->words,
+                    nullptr};
     if constexpr (std::is_same<R, float>::value)
       e = launch_trace_f32((GeomType)t, ms->dev->views[t], rv, hv, 1, cfg, g.extent, nullptr);
     else
@@ -1951,8 +1962,15 @@ static int intersect_impl(brt_scene *s, const brt_rays *rays, const brt_hits *hi
                     L.refill, nullptr, order};
     cfg.ring = L.stack_ring;
     cfg.pool = L.pool_size;
-    cfg.counter = noalloc ? reinterpret_cast<unsigned long long *>(scratch) : s->dev->counter_group(st);
-    if (!cfg.counter) return fail(BRT_ERR_OUT_OF_MEMORY, "launch counters");
+    std::unique_lock<std::mutex> enqueue;
+    if (noalloc) {
+      cfg.counter = reinterpret_cast<unsigned long long *>(scratch);
+    } else {
+      DeviceScene::LaunchCounters *counters = s->dev->counter_group(st);
+      if (!counters) return fail(BRT_ERR_OUT_OF_MEMORY, "launch counters");
+      enqueue = std::unique_lock<std::mutex>(counters->mu);
+      cfg.counter = counters->words;
+    }
     SplitParams sp{g.extent};
     hipError_t e = launch_trace((GeomType)t, s->dev->views[t], rv, hv, n, cfg, sp, st);
     if (e != hipSuccess) return fail(BRT_ERR_DEVICE, std::string("launch failed: ") + hipGetErrorString(e));
@@ -2007,8 +2025,10 @@ int brt_traverse(const brt_scene *cs, uint32_t geom_type, const brt_rays *rays, 
   cfg.ring = L.stack_ring;
   cfg.pool = L.pool_size;
   cfg.overwrite = true;
-  cfg.counter = s->dev->counter_group(static_cast<hipStream_t>(stream));
-  if (!cfg.counter) return fail(BRT_ERR_OUT_OF_MEMORY, "launch counters");
+  DeviceScene::LaunchCounters *counters = s->dev->counter_group(static_cast<hipStream_t>(stream));
+  if (!counters) return fail(BRT_ERR_OUT_OF_MEMORY, "launch counters");
+  std::lock_guard<std::mutex> enqueue(counters->mu);
+  cfg.counter = counters->words;
   SplitParams sp{g.extent};
   hipError_t e = launch_trace((GeomType)geom_type, s->dev->views[geom_type], rv, hv, n, cfg, sp,
                               static_cast<hipStream_t>(stream));
@@ -2059,8 +2079,10 @@ int brt_intersect_f32(const brt_scene *cs, const brt_rays_f32 *rays, const brt_h
     TraceLaunch cfg{L.precision, L.flags, L.block_size, first, L.schedule, L.refill, nullptr, nullptr};
     cfg.ring = L.stack_ring;
     cfg.pool = L.pool_size;
-    cfg.counter = s->dev->counter_group(st);
-    if (!cfg.counter) return fail(BRT_ERR_OUT_OF_MEMORY, "launch counters");
+    DeviceScene::LaunchCounters *counters = s->dev->counter_group(st);
+    if (!counters) return fail(BRT_ERR_OUT_OF_MEMORY, "launch counters");
+    std::lock_guard<std::mutex> enqueue(counters->mu);
+    cfg.counter = counters->words;
     hipError_t e = launch_trace_f32((GeomType)t, s->dev->views[t], rv, hv, n, cfg, s->geoF[t].extent, st);
     if (e != hipSuccess) return fail(BRT_ERR_DEVICE, std::string("launch failed: ") + hipGetErrorString(e));
     first = false;
@@ -2418,8 +2440,10 @@ int brt_mirror_trace(const brt_scene *cs, const brt_rays *rays, uint64_t n, uint
                     nullptr};
     cfg.ring = L.stack_ring;
     cfg.pool = L.pool_size;
-    cfg.counter = s->dev->counter_group(st);
-    if (!cfg.counter) return fail(BRT_ERR_OUT_OF_MEMORY, "launch counters");
+    DeviceScene::LaunchCounters *counters = s->dev->counter_group(st);
+    if (!counters) return fail(BRT_ERR_OUT_OF_MEMORY, "launch counters");
+    std::lock_guard<std::mutex> enqueue(counters->mu);
+    cfg.counter = counters->words;
     SplitParams sp{s->geo[TRIANGLES].extent};
     hipError_t e = launch_trace(TRIANGLES, bvh, rv, hv, n, cfg, sp, st);
     double *pos[3] = {out->px + off, out->py + off, out->pz + off};
