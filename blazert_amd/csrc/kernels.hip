@@ -1500,7 +1500,8 @@ __device__ __forceinline__ void make_rayq(const Ray &r, double len2, double S, R
 // the hit distance before it, `slack` what the ray's direction falls short of unit length. The FP64 test's errors are
 // those of tri_filter's table with u = 2^-53; 32 u covers them and the rounding of the record's edges and of the
 // normalised direction. The distance h = t / |det| is then known to err / |det|, err = 4 (Et + Ed h), twice over; `rel` is
-// that relative to h.
+// that relative to h. The boxes' exits are distances along the direction as given, up to 1 + 2^-21 long where tmin is not 0
+// (fast_ray), so the hit has to lie behind tmin by more than that.
 struct Certificate {
   bool sure;
   float rel;
@@ -1516,7 +1517,7 @@ __device__ __forceinline__ Certificate certified(const TriRec &T, const double o
   const double err = 4.0 * (Et + Ed * (t * (1.0 / ad)));
   Certificate c;
   c.sure = u > Eu && v > Ev && w > Eu + Ev + Ed && ad >= 0x1p12 * Ed && t >= 0x1p12 * Et &&
-           t - err >= ad * tmin * (1.0 + 0x1p-46) && t + err < thr * (1.0 - (0x1p-46 + slack));
+           t - err >= ad * tmin * (1.0 + 0x1p-20) && t + err < thr * (1.0 - (0x1p-46 + slack));
   c.rel = (float)(err * (1.0 / t)) * (1.0f + 0x1p-20f);
   return c;
 }
