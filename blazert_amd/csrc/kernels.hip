@@ -250,7 +250,8 @@ __device__ __forceinline__ bool sph_filter(const SphFilt &S, const float D[3], c
 // T^2 <= a^2 k^2 + b^2 j^2 for T = j y0 - k x0, a cap's point is on or in the ellipse and so is an origin inside, up to
 // roundings of 2e-15 (P^2 + max(a,b)^2) in T^2. T = (o - c) . (d x axis) for the record's axis, and the right side is at most
 // max(a,b)^2 (|d x axis|^2 + 1e-5) for a rotation within 1e-6 of orthonormal (others have infinite radii and pass). In FP32 T
-// is within 27 u P, u = 2^-24; the test rejects when it is outside by 32 u P, whose square covers the FP64 roundings too.
+// is within 27 u P, u = 2^-24; the test rejects when it is outside by 32 u P, whose square covers the FP64 roundings too. A
+// semi-axis below 1e-15, with which the right side could fall in the FP32 denormal range, is recorded as infinite.
 __device__ __forceinline__ bool cyl_filter(const CylFilt &C, const float D[3], const float O[3], float om) {
   const float u = 5.9604644775390625e-08f;
   const SphFilt sphere{{C.c[0], C.c[1], C.c[2]}, C.r};
@@ -2742,7 +2743,7 @@ __global__ void k_sph_filter_records(const SphRec *__restrict__ recs, uint32_t n
 // the test, on or inside the elliptic shell of semi-axes a, b; for an orthonormal R that point lies within
 // sqrt(max(a,b)^2 + (h/2)^2) of c. Both radii are enlarged by 2^-10 of themselves, the sphere's also by 2^-20 of the
 // coordinate magnitude, far above any rounding of the FP64 test, and are infinite (never reject) when R R^T differs from
-// the identity by more than 1e-6 or an input is not finite.
+// the identity by more than 1e-6 or an input is not finite; so is a semi-axis whose square leaves the FP32 range.
 __global__ void k_cyl_filter_records(const CylRec *__restrict__ recs, uint32_t n, CylFilt *out, uint32_t total) {
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
@@ -2761,6 +2762,7 @@ __global__ void k_cyl_filter_records(const CylRec *__restrict__ recs, uint32_t n
       double rad = rb * (1.0 + 0x1p-10) + 0x1p-20 * (cm + rb);
       double shell = ab * (1.0 + 0x1p-10);
       if (!(dev <= 1e-6) || !(rad < 1e300)) rad = shell = __builtin_inf();
+      if (shell < 1e-15) shell = __builtin_inf();
       for (int k = 0; k < 3; k++) {  // first column of R x second
         const int x = (k + 1) % 3, y = (k + 2) % 3;
         f.axis[k] = (float)(C.R[3 * x] * C.R[3 * y + 1] - C.R[3 * y] * C.R[3 * x + 1]);
