@@ -408,7 +408,9 @@ __device__ void closest_scan(const BvhView &bvh, const double *p, Best &best) {
 // triangle and any vector w, |p - q| >= min_i (p - v_i).w / |w| over its vertices; w is taken from the centroid to p, which is
 // nearly exact for a triangle that is small against its distance, and as the plane's normal. Those dot products are within
 // 26 u Sm |w| of exact (each p - v_i within 4 u Sm per component, each dot within 3 u of its factors' norms).
-// slack = 32 u Sm covers both, and the FP64 distance's own 1e-10 Sm.
+// slack = 32 u Sm covers both, and the FP64 distance's own 1e-10 Sm. The gaps are compared as squares: from
+// WIDE_MIN_EXTENT on, slack alone keeps the squared limit above 3e-36, where the FP32 range still has all digits.
+constexpr double WIDE_MIN_EXTENT = 1e-12;
 constexpr uint32_t WIDE_RING = 16;
 constexpr uint32_t WIDE_BLOCK = 256;
 
@@ -789,7 +791,7 @@ hipError_t launch_closest_surface(const ClosestViews &views, const double *px, c
   if (n == 0) return hipSuccess;
   int from = 0;
   const BvhView &tri = views.view[TRIANGLES];
-  if (views.present[TRIANGLES] && tri.nodesq && tri.tri_filter) {
+  if (views.present[TRIANGLES] && tri.nodesq && tri.tri_filter && views.extent[TRIANGLES] >= WIDE_MIN_EXTENT) {
     int dev = 0, cus = 0, per_cu = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
