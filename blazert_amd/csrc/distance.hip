@@ -408,6 +408,8 @@ __device__ void closest_scan(const BvhView &bvh, const double *p, Best &best) {
 // triangle and any vector w, |p - q| >= min_i (p - v_i).w / |w| over its vertices; w is taken from the centroid to p, which is
 // nearly exact for a triangle that is small against its distance, and as the plane's normal. Those dot products are within
 // 26 u Sm |w| of exact (each p - v_i within 4 u Sm per component, each dot within 3 u of its factors' norms).
+// The normal serves for one vertex only where its own FP64 rounding, 2^-50 of the edges' product sa sb, turns it by less than
+// u from the edges: for |n| > ed = 10 u sa sb, which leaves out triangles that are lines but for a rounding.
 // slack = 32 u Sm covers both, and the FP64 distance's own 1e-10 Sm. The gaps are compared as squares: from
 // WIDE_MIN_EXTENT on, slack alone keeps the squared limit above 3e-36, where the FP32 range still has all digits.
 constexpr double WIDE_MIN_EXTENT = 1e-12;
@@ -454,7 +456,8 @@ __device__ __forceinline__ bool tri_in_reach(const TriFilt &T, const float P[3],
   const float nn = dot(T.n[0], T.n[1], T.n[2], T.n[0], T.n[1], T.n[2]);
   const float l2 = (lim * lim) * (1.0f + 16.0f * u);
   // products below 1e-30 may have lost digits to the denormal range: no rejection (nor on infinities and NaN)
-  return !((m > 0.0f) & (m * m > l2 * ww) & (l2 * ww > 1e-30f)) & !((cn * cn > l2 * nn) & (l2 * nn > 1e-30f));
+  return !((m > 0.0f) & (m * m > l2 * ww) & (l2 * ww > 1e-30f)) &
+         !((cn * cn > l2 * nn) & (l2 * nn > 1e-30f) & (nn > T.ed * T.ed));
 }
 
 __device__ __forceinline__ void order_pair(uint32_t &ka, uint32_t &ra, uint32_t &kb, uint32_t &rb) {
