@@ -79,11 +79,14 @@ constexpr int COUNTER_DEFERRED_POOL = 2;
 constexpr int CLAIM_COUNTERS = 8;
 constexpr int COUNTER_STRIDE = 16;
 constexpr int COUNTER_CLEARED = CLAIM_COUNTERS * COUNTER_STRIDE;  // slots a launch clears (1 KiB)
-// Rays that a fast traversal leaves to the exact launch behind it are listed behind the counters: COUNTER_LISTED counts
-// them, and when there are more than LIST_CAPACITY that launch traces every ray. A launch with a fixed range of at most 64
-// rays per wave writes one word per wave there instead, a bit for each ray left, and needs no cleared counters.
+// What a fast traversal leaves to the exact launch behind it: COUNTER_DEFERRED says that rays were passed over, and others are
+// listed behind the counters, COUNTER_LISTED counting them. Both have a slot on each of the CLAIM_COUNTERS lines, and each line
+// its own part of the list, for the blocks that start claiming there: one line for all of them is busy for longer than such
+// rays take. When a part overflows, the launch behind traces every ray. A launch with a fixed range of at most 64 rays per wave
+// writes one word per wave there instead, a bit for each ray left, and needs no cleared counters.
 constexpr int COUNTER_LISTED = 3;
 constexpr int LIST_CAPACITY = 8064;
+constexpr int LIST_PART = LIST_CAPACITY / CLAIM_COUNTERS;
 constexpr int COUNTER_GROUP = COUNTER_CLEARED + LIST_CAPACITY;  // slots per group (64 KiB)
 
 constexpr uint32_t SCHEDULE_PERSISTENT = 0;  // persistent waves with per-lane ray refill (default)
