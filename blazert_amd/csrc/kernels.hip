@@ -35,6 +35,7 @@ constexpr uint32_t FLAG_ANY_HIT = 2u;
 // Internal: an FP64 launch that traces only the rays a split-precision launch of the same geometry type deferred
 // (see deferred_to_exact), and none at all when that launch deferred nothing.
 constexpr uint32_t FLAG_DEFERRED_ONLY = 1u << 31;
+constexpr uint32_t FLAG_SPLIT = 1u << 30;  // k_trace_tri and the launch behind it: split precision
 // Exact paths: primitives of a leaf tested per traversal step, per primitive type (triangles, spheres, planes,
 // cylinders). They are tested in leaf order, each against the hit distance the previous one left, so the count
 // changes speed only.
@@ -1089,11 +1090,12 @@ __device__ __forceinline__ void start_ray(const BvhView &bvh, const RaysViewT<R>
 }
 
 // Rays whose reference traversal the FP32 bounds enclose: no slab term can be NaN or leave the FP32 range, tmin >= 0
-// and a direction of unit length (its slab distances are then the hit distances; a longer one only makes the reference
-// skip less, except through tmin).
-__device__ __forceinline__ bool fast_ray(const Ray &r, double len2, double S) {
-  bool ok = (r.sign & RAY_NAN_FREE) && r.tmin >= 0.0 && len2 >= 1.0 - 0x1p-20 && len2 <= 1e20 &&
-            (len2 <= 1.0 + 0x1p-20 || r.tmin == 0.0);
+// and a direction of at least unit length (its slab distances are then the hit distances, or shorter: the reference skips no
+// more by them, except through tmin, see certified).
+// Split precision takes shorter ones too: it need not tell the boxes that the reference reaches from those a rounding away.
+constexpr double SHORT_LEN2 = 1.0 - 0x1p-20;
+__device__ __forceinline__ bool fast_ray(const Ray &r, double len2, double S, bool split) {
+  bool ok = (r.sign & RAY_NAN_FREE) && r.tmin >= 0.0 && (split || len2 >= SHORT_LEN2) && len2 <= 1e20;
 #pragma unroll
   for (int k = 0; k < 3; k++) ok = ok && fabs(r.inv[k]) * (S + fabs(r.o[k])) <= 1e36 && fabs(r.inv[k]) <= 1e30;
   return ok && fabs(r.o[0]) <= FILTER_MAX_EXTENT && fabs(r.o[1]) <= FILTER_MAX_EXTENT &&
@@ -1133,12 +1135,12 @@ __device__ __forceinline__ double squared_length(const RawRay &w) {
 
 // The type's predicate from the ray's columns.
 template <class Rec>
-__device__ __forceinline__ bool fast_ray(const RaysViewT<typename Rec::real> &V, uint64_t i, double S) {
+__device__ __forceinline__ bool fast_ray(const RaysViewT<typename Rec::real> &V, uint64_t i, double S, bool split) {
   using R = typename Rec::real;
   const RawRayT<R> w = load_ray(V, i);
   RayT<R> r;
   setup_ray(w.org, w.dir, w.tmin, w.tmax, r);
-  if constexpr (Rec::kind == TRIANGLES && sizeof(R) == 8) return fast_ray(r, squared_length(w), S);
+  if constexpr (Rec::kind == TRIANGLES && sizeof(R) == 8) return fast_ray(r, squared_length(w), S, split);
   else return wide_ray(r, S);
 }
 
@@ -1220,15 +1222,12 @@ __device__ __forceinline__ T lds_fresh(const uint64_t *src) {
   return out;
 }
 
-// Sets the launch's flag of rays passed over, once per wave and on the block's own line: stores to one line are served one after
-// the other. 2,073,600 rays of an axis-parallel camera, all passed over, take this kernel 0.14 ms (0.27 with one line, 1.5 with
-// a store per ray). Called by the whole wave; `noted` is wave-uniform.
-__device__ __forceinline__ void note_passed(bool passed, bool &noted, unsigned long long *group, uint32_t lane) {
-  if (!noted && __ballot(passed)) {
-    noted = true;
-    if (lane == 0) {
-      __atomic_store_n(group + (blockIdx.x % CLAIM_COUNTERS) * COUNTER_STRIDE + COUNTER_DEFERRED, 1ull, __ATOMIC_RELAXED);
-    }
+// Sets the launch's flag of rays passed over, when a wave that has passed some ends, and on the block's own line: stores to one
+// line are served one after the other. 2,073,600 rays of an axis-parallel camera, all passed over, take k_trace_tri 0.14 ms
+// (0.27 with one line, 1.5 with a store per ray).
+__device__ __forceinline__ void note_passed(bool noted, unsigned long long *group, uint32_t lane) {
+  if (noted && lane == 0) {
+    __atomic_store_n(group + (blockIdx.x % CLAIM_COUNTERS) * COUNTER_STRIDE + COUNTER_DEFERRED, 1ull, __ATOMIC_RELAXED);
   }
 }
 
@@ -1335,7 +1334,7 @@ k_trace_persistent(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<ty
           } else {
             idx = order ? (uint64_t)order[cand] : cand;
             start_ray<SPLIT>(bvh, rays_view(), idx, S, r, q, s);
-            if constexpr (AFTER_FAST) trace = left.all || !fast_ray<Rec>(rays_view(), idx, S);
+            if constexpr (AFTER_FAST) trace = left.all || !fast_ray<Rec>(rays_view(), idx, S, (flags & FLAG_SPLIT) != 0u);
           }
           if (SPLIT && deferred_to_exact(r)) {
             __atomic_store_n(deferred, 1ull, __ATOMIC_RELAXED);
@@ -1453,7 +1452,7 @@ k_trace_batch(const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t total,
             bv = J.bvh;
             start_ray<SPLIT>(bv, J.rays, idx, J.extent, r, q, s);
             bool trace = true;
-            if constexpr (AFTER_FAST) trace = from_list || left.all || !fast_ray<Rec>(J.rays, idx, J.extent);
+            if constexpr (AFTER_FAST) trace = from_list || left.all || !fast_ray<Rec>(J.rays, idx, J.extent, (flags & FLAG_SPLIT) != 0u);
             if (SPLIT && deferred_to_exact(r)) {
               __atomic_store_n(deferred, 1ull, __ATOMIC_RELAXED);
             } else if (trace && (!deferred_only || deferred_to_exact(r))) {
@@ -1522,8 +1521,9 @@ struct RayQ {
   float offn[3], offf[3];  // entry / exit plane offsets, rounded apart (make_ray32)
   float D[3], O[3];        // unit direction and origin, for the pre-test
   float om, tmin;
-  float slack;             // >= 1 - |raw direction|
-  // bits 0-4: shift of the octant's order mask, bit 5: its word, bits 6-8: direction signs, bit 9: mask complemented
+  float slack;             // >= 1 - |raw direction| where that is positive, else <= it
+  // bits 0-4: shift of the octant's order mask, bit 5: its word, bits 6-8: direction signs, bit 9: mask complemented, bit 10:
+  // a direction too short for its hits' distances to be merged (split precision)
   uint32_t code;
 };
 
@@ -1541,17 +1541,18 @@ __device__ __forceinline__ void make_rayq(const Ray &r, double len2, double S, R
   }
   q.om = a.om;
   q.tmin = fmaxf(a.tmin, 0.0f);
-  q.slack = len2 < 1.0 ? f32_up(1.0 - len2) : 0.0f;
+  const bool brief = len2 < SHORT_LEN2;
+  q.slack = brief ? 0.0f : len2 < 1.0 ? f32_up(1.0 - len2) : f32_down(1.0 - __builtin_sqrt(len2));
   const uint32_t s = r.sign & 7u, c = (s & 4u) ? (~s & 3u) : s;
-  q.code = ((c & 1u) << 4) | ((c >> 1) << 5) | (s << 6) | ((s >> 2) << 9);
+  q.code = ((c & 1u) << 4) | ((c >> 1) << 5) | (s << 6) | ((s >> 2) << 9) | (brief ? 1024u : 0u);
 }
 
 // Whether an accepted hit is one that the reference's traversal must reach as well (see above). `thr` is |det| times
 // the hit distance before it, `slack` what the ray's direction falls short of unit length. The FP64 test's errors are
 // those of tri_filter's table with u = 2^-53; 32 u covers them and the rounding of the record's edges and of the
 // normalised direction. The distance h = t / |det| is then known to err / |det|, err = 4 (Et + Ed h), twice over; `rel` is
-// that relative to h. The boxes' exits are distances along the direction as given, up to 1 + 2^-21 long where tmin is not 0
-// (fast_ray), so the hit has to lie behind tmin by more than that.
+// that relative to h. The boxes' exits are distances along the direction as given, so a hit has to lie behind tmin by that
+// direction's length where it is longer than one.
 struct Certificate {
   bool sure;
   float rel;
@@ -1567,7 +1568,8 @@ __device__ __forceinline__ Certificate certified(const TriRec &T, const double o
   const double err = 4.0 * (Et + Ed * (t * (1.0 / ad)));
   Certificate c;
   c.sure = u > Eu && v > Ev && w > Eu + Ev + Ed && ad >= 0x1p12 * Ed && t >= 0x1p12 * Et &&
-           t - err >= ad * tmin * (1.0 + 0x1p-20) && t + err < thr * (1.0 - (0x1p-46 + slack));
+           t - err >= ad * tmin * (1.0 + 0x1p-46) * (1.0 - fmin(slack, 0.0)) &&
+           t + err < thr * (1.0 - (0x1p-46 + fmax(slack, 0.0)));
   c.rel = (float)(err * (1.0 / t)) * (1.0f + 0x1p-20f);
   return c;
 }
@@ -1914,7 +1916,7 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
         if (LONE || got) {
           setup_ray(raw.org, raw.dir, raw.tmin, raw.tmax, r);
           const double len2 = squared_length(raw);
-          if (fast_ray(r, len2, ext)) {
+          if (fast_ray(r, len2, ext, (flags & FLAG_SPLIT) != 0u)) {
             has_ray = got;
             make_rayq(r, len2, ext, q);
             s.h = r.tmax;
@@ -1935,7 +1937,12 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
           }
         }
         if constexpr (FIXED) mask_add(mask, defer, number);
-        else if constexpr (!LONE) note_passed(defer, noted, group, lane);
+        else if constexpr (!LONE) {
+          if (!noted && __ballot(defer)) {
+            noted = true;
+            note_passed(true, group, lane);
+          }
+        }
       }
     }
     const unsigned long long busy = __ballot(has_ray);
@@ -1945,7 +1952,7 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
         if (FIXED && lane == 0) group[COUNTER_CLEARED + global_wave] = mask;
         break;
       }
-      const unsigned long long can = __ballot(has_ray && st.sp > st.bot);
+      const unsigned long long can = __ballot(has_ray && st.sp > st.bot && !(q.code & 1024u));
       const uint32_t nidle = 64u - (uint32_t)__popcll(busy);
       // in every other iteration: sharing costs about as many instructions as a traversal step (every one: 3-5% slower);
       // a lone ray has the instruction slots to itself and shares in every one (41.4 -> 38.4 us a call; not at all: 46.0 us)
@@ -2046,7 +2053,7 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
             const float rel = fmaxf(t.rel, sh->rel[slot]);
             sh->rel[slot] = rel;
             // (the nearer one may lie in a box whose entry, along a direction shorter than one, is behind the other)
-            const double close = 2.0 * ((double)rel + (double)q.slack) + 0x1p-46;
+            const double close = 2.0 * ((double)rel + (double)fmaxf(q.slack, 0.0f)) + 0x1p-46;
             if (fabs(s.h - h) <= close * s.h) parts |= 0x80000000u;
             if (s.h < h) {
               sh->h[slot] = s.h;
@@ -2394,12 +2401,13 @@ k_trace_wide(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<typename
           }
         }
         if constexpr (FIXED) mask_add(mask, defer, number);
-        else note_passed(defer, noted, group, lane);
+        else noted = noted || __ballot(defer) != 0ull;
       }
     }
     if (exhausted && !__ballot(has_ray)) {
       write_rays();
       if (FIXED && lane == 0) group[COUNTER_CLEARED + global_wave] = mask;
+      if constexpr (!FIXED) note_passed(noted, group, lane);
       break;
     }
     if (has_ray) {
@@ -2617,7 +2625,7 @@ k_trace_any(BvhView bvh, RaysView rays, HitsView hits, uint64_t n, uint32_t flag
           }
         }
         if constexpr (FIXED) mask_add(mask, defer, (uint32_t)(cand - range));
-        else note_passed(defer, noted, group, lane);
+        else noted = noted || __ballot(defer) != 0ull;
       }
     }
     const unsigned long long busy = __ballot(has_ray);
@@ -2625,6 +2633,7 @@ k_trace_any(BvhView bvh, RaysView rays, HitsView hits, uint64_t n, uint32_t flag
       if (!busy) {
         write_rays();
         if (FIXED && lane == 0) group[COUNTER_CLEARED + global_wave] = mask;
+        if constexpr (!FIXED) note_passed(noted, group, lane);
         break;
       }
       // a part hands on the last eighth of its positions, so it needs eight for the order to stay strict
@@ -3037,6 +3046,7 @@ hipError_t launch_tri(const BvhView &bvh, const RaysView &rays, const HitsView &
   const uint32_t block = cfg.block ? cfg.block : 256;
   const uint32_t ring = cfg.ring ? cfg.ring : TRI_RING;
   const uint32_t first = cfg.first ? 1u : 0u;
+  const uint32_t flags = cfg.flags | (cfg.precision != PREC_FP64 ? FLAG_SPLIT : 0u);
   const size_t lds = tri_lds_bytes(block, ring);
   unsigned long long *grp = cfg.counter;
   if (!grp) return hipErrorInvalidValue;
@@ -3051,7 +3061,7 @@ hipError_t launch_tri(const BvhView &bvh, const RaysView &rays, const HitsView &
   const uint64_t need = fixed ? (n + fixed * wpb - 1) / (fixed * wpb) : (n + block - 1) / block;
   if (blocks > need) blocks = need;
   hipLaunchKernelGGL((fixed ? k_trace_tri<false, false, true> : k_trace_tri<false>), dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits,
-                     (const BatchJob *)nullptr, 0u, n, cfg.flags, first, sp.scene_extent, grp,
+                     (const BatchJob *)nullptr, 0u, n, flags, first, sp.scene_extent, grp,
                      cfg.refill ? cfg.refill : TRI_REFILL, cfg.order, ring, cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -3062,7 +3072,7 @@ hipError_t launch_tri(const BvhView &bvh, const RaysView &rays, const HitsView &
   e = persistent_blocks(k_trace_persistent<TriRec, false, true>, 256, lds64, n, blocks);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((k_trace_persistent<TriRec, false, true>), dim3((uint32_t)blocks), dim3(256), lds64, stream, bvh,
-                     rays, hits, n, cfg.flags, first, 1u, sp.scene_extent, grp + COUNTER_DEFERRED_POOL,
+                     rays, hits, n, flags, first, 1u, sp.scene_extent, grp + COUNTER_DEFERRED_POOL,
                      refill_default<TriRec, false>(), cfg.order, ring64, grp + COUNTER_DEFERRED, POOL_CHUNK);
   return hipGetLastError();
 }
@@ -3136,6 +3146,7 @@ hipError_t launch_tri_batch(const BatchJob *jobs, uint32_t njobs, uint64_t total
   const uint32_t block = cfg.block ? cfg.block : 256;
   const uint32_t ring = cfg.ring ? cfg.ring : TRI_RING;
   const size_t lds = tri_lds_bytes(block, ring);
+  const uint32_t flags = cfg.flags | (cfg.precision != PREC_FP64 ? FLAG_SPLIT : 0u);
   unsigned long long *grp = cfg.counter;
   if (!grp || njobs == 0) return hipErrorInvalidValue;
   if (total == 0) return hipSuccess;
@@ -3147,7 +3158,7 @@ hipError_t launch_tri_batch(const BatchJob *jobs, uint32_t njobs, uint64_t total
   if (blocks > need) blocks = need;
   hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
   hipLaunchKernelGGL(k_trace_tri<true>, dim3((uint32_t)blocks), dim3(block), lds, stream, BvhView{}, RaysView{},
-                     HitsView{}, jobs, njobs, total, cfg.flags, 0u, 0.0, grp, cfg.refill ? cfg.refill : TRI_REFILL,
+                     HitsView{}, jobs, njobs, total, flags, 0u, 0.0, grp, cfg.refill ? cfg.refill : TRI_REFILL,
                      (const uint32_t *)nullptr, ring, cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -3156,7 +3167,7 @@ hipError_t launch_tri_batch(const BatchJob *jobs, uint32_t njobs, uint64_t total
   e = persistent_blocks(k_trace_batch<TriRec, false, true>, 256, lds64, total, blocks);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((k_trace_batch<TriRec, false, true>), dim3((uint32_t)blocks), dim3(256), lds64, stream, jobs,
-                     njobs, total, cfg.flags, grp + COUNTER_DEFERRED_POOL, refill_default<TriRec, false>(), ring64,
+                     njobs, total, flags, grp + COUNTER_DEFERRED_POOL, refill_default<TriRec, false>(), ring64,
                      grp + COUNTER_DEFERRED, POOL_CHUNK);
   return hipGetLastError();
 }
