@@ -85,9 +85,9 @@ constexpr int COUNTER_CLEARED = CLAIM_COUNTERS * COUNTER_STRIDE;  // slots a lau
 // rays take. When a part overflows, the launch behind traces every ray. A launch with a fixed range of at most 64 rays per wave
 // writes one word per wave there instead, a bit for each ray left, and needs no cleared counters.
 constexpr int COUNTER_LISTED = 3;
-constexpr int LIST_CAPACITY = 8064;
+constexpr int LIST_CAPACITY = 32640;
 constexpr int LIST_PART = LIST_CAPACITY / CLAIM_COUNTERS;
-constexpr int COUNTER_GROUP = COUNTER_CLEARED + LIST_CAPACITY;  // slots per group (64 KiB)
+constexpr int COUNTER_GROUP = COUNTER_CLEARED + LIST_CAPACITY;  // slots per group (256 KiB)
 
 constexpr uint32_t SCHEDULE_PERSISTENT = 0;  // persistent waves with per-lane ray refill (default)
 constexpr uint32_t SCHEDULE_PER_THREAD = 1;  // one ray per thread, grid-stride

@@ -1699,8 +1699,12 @@ __device__ __forceinline__ void tri_step(const TriTrees &T, const Ray &r, const 
           c = certified(rec, r.o, r.tmin, (double)q.slack, u, v, w, tt, ad, thr);
         })) {
       t.h32 = f32_up(s.h);
-      t.listed = t.listed || !c.sure;
       t.rel = fmaxf(t.rel, c.rel);
+      if (!c.sure) {  // the exact kernel's
+        t.listed = true;
+        t.active = false;
+        return;
+      }
     }
     t.cand &= t.cand - 1u;
     if (t.cand) return;
