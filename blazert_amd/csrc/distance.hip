@@ -477,9 +477,11 @@ struct ClosestShare {
   uint32_t parts[SHARE_SLOTS];  // parts still running
 };
 
-// What bounds it: 1,048,576 points in [-2,2]^3 around 1.31M triangles take 3.65 ms (6.5 with binary FP64 nodes and FP64
+// What bounds it: 1,048,576 points in [-2,2]^3 around 1.31M triangles take 3.41 ms (6.5 with binary FP64 nodes and FP64
 // distances only, one point per thread), about 90 steps a point with a far from even spread; lines beyond L2 at 3.7 TB/s.
-// 1,000 points on 82k triangles 351 -> 130 us, 50,000 on 328k 735 -> 463 us.
+// 1,000 points on 82k triangles 351 -> 130 us, 50,000 on 328k 735 -> 463 us. Searches of a few steps each gain least, since a
+// wave's lanes are then seldom at one kind of step: 1,000,000 points within 0.001 of 82k triangles 1.68 ms (1.60 one per
+// thread), of a flat grid of 524,288 triangles 0.59 (0.31). Waiting lanes take these from 1.75 and 0.62, and the first from 3.70.
 //
 // Persistent waves as in the ray traversal (or `fixed` points per wave): lanes whose point is done start the wave's next
 // ones, and once there are none, idle lanes take over stack entries of the busy ones, whose best distances they share.
@@ -595,7 +597,15 @@ k_closest_triangles(ClosestViews V, const double *__restrict__ px, const double 
       }
     }
     bool fin = false;
-    if (busy) {
+    bool go = busy;
+    if (!exhausted) {  // lanes with a pre-test or an FP64 distance wait until WIDE_MIN_LANES have one, or nothing else is left
+      const bool leaf = busy && (cur & LEAF_BIT) != 0, test = leaf && cand != 0u, group = leaf && cand == 0u;
+      const int tests = __popcll(__ballot(test)), groups = __popcll(__ballot(group));
+      const int nodes = __popcll(__ballot(busy)) - tests - groups;
+      if (test && tests < WIDE_MIN_LANES && nodes + groups != 0) go = false;
+      if (group && groups < WIDE_MIN_LANES && nodes != 0) go = false;
+    }
+    if (go) {
       if (shared) {
         const double d = __longlong_as_double((long long)sh->bound[slot]);
         lim = fminf(lim, f32_up((double)f32_up(d) + (double)slack));

@@ -2107,8 +2107,6 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
 // spheres 4.19 -> 3.24 ms (8 lanes: 3.36, 24: 3.62), against 4.44 ms for the exact kernel; 10,000 cylinders 4.90 -> 4.59 ms
 // (3.68 with the pre-test against the axis), against 5.45 ms. (k_trace_tri, bound by the data path of the L1, gains nothing from it.) A wave with no rays left to take
 // doesn't wait: there the longest ray counts. In FP32 the primitives are tested without a pre-test.
-constexpr int WIDE_MIN_LANES = 16;
-
 // Primitives without a pre-test tested per step. Triangles in FP32, 1,000,003 incoherent rays on 327,680: 1 per step 0.88,
 // 2: 0.71, 3: 0.68, 4: 0.65 ms.
 template <class Rec>

@@ -173,6 +173,9 @@ __device__ __forceinline__ void pool_refill(WavePool &P, unsigned long long *cou
   P.next += take;
   if (P.last && P.next == P.end) exhausted = true;
 }
+// Lanes of k_trace_wide and k_closest_triangles with an FP64 test, or with a pre-test, wait for as many of the wave (see there).
+constexpr int WIDE_MIN_LANES = 16;
+
 // Work sharing in a wave with nothing left to start: from SHARE_MIN_IDLE idle lanes on, these take over stack entries of
 // the busy ones. At most SHARE_SLOTS queries of a wave are then ever shared.
 constexpr uint32_t SHARE_MIN_IDLE = 32;
