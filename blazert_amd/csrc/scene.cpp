@@ -1255,12 +1255,13 @@ int put_geometry(DeviceScene &d, Geometry &g, uint32_t t) {
   if (e == hipSuccess) e = make_prim_filter(d, v, t, g.extent, nullptr, &g.stats.device_bytes);
   if (e == hipSuccess) {
     const uint32_t *ord4 = nullptr;
-    e = d.put(g.ord4, &ord4);
+    if (t != PLANES) e = d.put(g.ord4, &ord4);
     if (e == hipSuccess)
       e = make_nodesq(d, v, t, false, g.extent_ok ? g.extent : INFINITY, g.num_n4, ord4,
                       g.stats.max_num_prims_per_leaf, nullptr, &g.stats.device_bytes);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // launches on any stream may read what was made
+    d.release(ord4);                                         // only the nodes made from it are used
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // launches on any stream may read what was made
   if (e != hipSuccess) return device_error(e, "upload failed");
   d.views[t] = v;
   return BRT_OK;
@@ -1454,6 +1455,7 @@ int commit_on_device(brt_scene *s, hipStream_t st) {
                                     &bs.device_bytes))
       return device_error(fe, "fast traversal nodes");
     if (hipError_t fe = hipStreamSynchronize(st)) return device_error(fe, "fast traversal nodes");
+    d->release(r.ord4);
     d->views[t] = v;
     bs.build_time_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   }
