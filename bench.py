@@ -579,15 +579,17 @@ def user_geometry_leg(args, dev) -> dict:
     tr = osph.intersect_batch(org[:nsmp], dirs[:nsmp], normals=False, trace=True,
                               nthreads=len(os.sched_getaffinity(0)))["trace"]
     bpr = S_RAY_HIT + float(tr["node_visits"].mean()) * S_NODE64 + float(tr["prim_tests"].mean()) * 36
-    roof = {k: {"bound": "hbm", "achieved": round(bpr * n / (t * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS,
-                "unit": "GB/s", "frac": round(bpr * n / (t * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}
-            for k, t in (("user", ms_user), ("builtin", ms_builtin))}
+    user_gbs = bpr * n / (ms_user * 1e-3) / 1e9
+    roof = {"bound": "hbm", "achieved": round(user_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": round(user_gbs / HBM_PEAK_GBS, 4)}
     log(f"user collection {n / ms_user / 1e3:.1f} Mrays/s ({ms_user:.3f} ms) vs built-in spheres "
         f"{n / ms_builtin / 1e3:.1f} Mrays/s, identical: {exact}")
     return {"value": round(n / ms_user / 1e3, 3), "unit": "Mrays/s", "ms_per_step": round(ms_user, 4),
             "builtin_spheres_mrays_s": round(n / ms_builtin / 1e3, 3), "builtin_ms": round(ms_builtin, 4),
             "identical_to_builtin_all_rays": exact, "hits": hits, "tree_build_s": round(build_s, 3),
-            "bytes_per_ray": round(bpr, 1), "roofline_user": roof["user"], "roofline_builtin": roof["builtin"],
+            "bytes_per_ray": round(bpr, 1), "roofline_user": roof,
+            # (the built-in kernel reads FP32 boxes and records instead of these bytes: no roofline)
+            "builtin_algorithmic_gbs": round(bpr * n / (ms_builtin * 1e-3) / 1e9, 1),
             "workload": "1,048,576 spheres (r in [0.1, 0.5]) in [-40, 40]^3, 4,194,304 incoherent rays from inside, "
                         "example sphere intersector through include/blazert_amd/user_geometry.h"}
 
@@ -761,25 +763,28 @@ def main():
                  and np.array_equal(g_sub_p[ok], ref["prim_id"][ok]))
     achieved = bpr64 * n / (ms64 * 1e-3) / 1e9
     traffic, traffic32, traffic_note = measured_traffic()
-    out["roofline"] = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                       "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": traffic_note,
-                       "bytes_per_ray": round(bpr64, 1), "node_visits_per_ray": round(visits, 2),
-                       "tri_tests_per_ray": round(ptests, 2)}
+    # achieved: the measured traffic where it is known. The reference traversal's bytes (FP64 boxes, every triangle's record)
+    # stand beside it: the kernels read FP32 boxes and pre-test records instead, so that rate can pass the peak.
+    def hbm(traffic, ms):
+        gbs = round(traffic / (ms * 1e-3) / 1e9, 1) if traffic else None
+        return {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "frac": round(gbs / HBM_PEAK_GBS, 4) if traffic else None, "traffic": traffic,
+                "traffic_source": traffic_note}
+
+    out["roofline"] = {**hbm(traffic, ms64), "algorithmic_gbs": round(achieved, 1), "bytes_per_ray": round(bpr64, 1),
+                       "node_visits_per_ray": round(visits, 2), "tri_tests_per_ray": round(ptests, 2)}
     # split precision: the same work numerator (the reference traversal's node visits and triangle tests) with the
     # split path's node record size, 32 B of FP32 box + topology per node
     bpr32 = S_RAY_HIT + visits * S_NODE32 + ptests * S_TRI
     ach32 = bpr32 * n / (ms32 * 1e-3) / 1e9
-    out["split_precision"]["roofline"] = {"bound": "hbm", "achieved": round(ach32, 1), "peak": HBM_PEAK_GBS,
-                                          "unit": "GB/s", "frac": round(ach32 / HBM_PEAK_GBS, 4),
-                                          "bytes_per_ray": round(bpr32, 1), "traffic": traffic32,
-                                          "traffic_source": traffic_note}
+    out["split_precision"]["roofline"] = {**hbm(traffic32, ms32), "algorithmic_gbs": round(ach32, 1),
+                                          "bytes_per_ray": round(bpr32, 1)}
     ceil = ceilings(**CEIL)
     out["ceilings"] = ceil
     chase = ceil["dependent_line_chains_gbs"]
     for rf, tb, ms in ((out["roofline"], traffic, ms64), (out["split_precision"]["roofline"], traffic32, ms32)):
         rf["dependent_line_ceiling_gbs"] = chase
         if tb:
-            rf["traffic_gbs"] = round(tb / (ms * 1e-3) / 1e9, 1)
             rf["traffic_frac_of_dependent_line_ceiling"] = round(tb / (ms * 1e-3) / 1e9 / chase, 4)
     out["parity"] = {"sample_rays": ns, "fp64_bit_exact_vs_oracle": exact,
                      "reference_stack_overflow_rays": int((~ok).sum())}
