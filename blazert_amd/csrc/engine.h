@@ -156,16 +156,17 @@ struct SplitParams {
   double scene_extent;
 };
 
-// Split precision: writes the FP32 pre-test records (TriFilt, n + FILTER_PAD of them) of n leaf-order TriRecs.
+// Writes the FP32 pre-test records (TriFilt, n + FILTER_PAD of them) of n leaf-order TriRecs.
 hipError_t launch_tri_filter_records(const void *recs, uint32_t n, void *out, hipStream_t stream);
-// Split precision: writes the FP32 pre-test records (SphFilt, n + SPH_FILTER_PAD of them) of n leaf-order SphRecs.
+// Writes the FP32 pre-test records (SphFilt, n + SPH_FILTER_PAD of them) of n leaf-order SphRecs.
 hipError_t launch_sph_filter_records(const void *recs, uint32_t n, void *out, hipStream_t stream);
-// Split precision: writes the bounding-sphere pre-test records (SphFilt, n + SPH_FILTER_PAD) of n leaf-order CylRecs.
+// Writes the FP32 pre-test records (CylFilt, n + SPH_FILTER_PAD of them) of n leaf-order CylRecs.
 hipError_t launch_cyl_filter_records(const void *recs, uint32_t n, void *out, hipStream_t stream);
 
-// Triangles: assembles the reference-order nodes (NodeQ) from n Node4 records and their visiting orders (two words per
-// record, visit_order4).
+// Writes the leaves' boxes, each at its first primitive's place in leaf order (six numbers of the scene's type).
 hipError_t launch_leaf_boxes(const BvhView &bvh, bool f32, void *out, hipStream_t stream);
+// Assembles the reference-order nodes (NodeQ) from n Node4 records and their visiting orders (two words per record,
+// visit_order4).
 hipError_t launch_nodeq_records(const Node4 *nodes4, const uint32_t *ord, uint32_t n, NodeQ *out, hipStream_t stream);
 
 // Clears the counters of a group on the stream.

@@ -172,7 +172,8 @@ __device__ __forceinline__ bool slab32(const float *b, const Ray32 &q, float &ke
 //   w = |det| - u - v: the sum of those plus 2 u (|det| + |u| + |v|) <= 0.2 Ed + 0.18 (Eu + Ev)
 // The bounds used (Ed = ed, Et = 1.2 ed Pm, and for u, v and w alike E = kw Pm + cw, with kw = 1.2 * 16 u (sa + sb) and
 // cw = 1.3 ed + tol) keep a margin for the rounding of the bounds themselves; ed and Et hold an absolute 1e-29, E the
-// reference's tolerance, for results in the FP32 denormal range. The reference accepts u, v, w >= -4 DBL_EPSILON (tol), t >= |det| tmin and |det| h > t with the signs
+// reference's tolerance, for results in the FP32 denormal range. The reference accepts u, v, w >= -4 DBL_EPSILON (tol),
+// t >= |det| tmin and |det| h > t with the signs
 // taken from det; where the sign of det is not certain (|det| <= Ed) the triangle passes. Scenes and ray origins
 // above FILTER_MAX_EXTENT are not pre-tested, so no value here overflows; every rejection is a comparison that is
 // false for NaN operands.
@@ -1500,8 +1501,10 @@ k_trace_batch(const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t total,
 // checked (certified): one that lies inside its triangle by more than the rounding of the test, and clear of the earlier
 // hit distance and of tmin by more than the error of its own distance, lies inside every box above it by more than the
 // rounding of the slab test (whose far planes are widened by 4 eps), so the reference tests it too, with the same hit
-// distance, and accepts it. A ray with a hit that fails the check writes nothing and is listed for the exact kernel that
-// follows on the stream. Rays outside the assumptions of the argument (fast_ray) go there as well.
+// distance, and accepts it. A ray with a hit that fails the check ends there (what it would find next is of no use), writes
+// nothing and is listed for the exact kernel that follows on the stream: 1,048,576 rays aimed at vertices and edges are traced
+// at 0.6 of the exact kernel's own speed. Testing the accepted hit's leaf box in FP64 instead spills registers in this loop and
+// costs 8-12% on rays that need no check. Rays outside the assumptions of the argument (fast_ray) go there as well.
 //
 // What bounds it (4,194,304 incoherent rays, 1.31M triangles): the data path of the vector L1 (87% busy: every step reads a
 // 128-byte record per lane in eight loads) and the vector ALU (73%, a quarter of the lanes active), with 5.7 TB/s of
@@ -1514,8 +1517,9 @@ k_trace_batch(const BatchJob *__restrict__ jobs, uint32_t njobs, uint64_t total,
 // accepted hit is certified as before, and one nearer than the hit of the parts before it would have been accepted in
 // the reference's order too. A part also skips what lies behind a hit of a part before it (never of one after it). The
 // parts' hits are merged by distance when the last of them ends, and a ray whose parts have two hits within their error
-// bounds of each other, and what its direction falls short of unit length, is listed. Sharing takes the incoherent set from 3.57 to 3.16 ms and 50,000 rays on 328k triangles
-// from 450 to 268 us; the camera set, whose rays mostly end at their first hit, loses 4%.
+// bounds of each other, and what its direction falls short of unit length, is listed. Sharing takes the incoherent set from
+// 3.57 to 3.16 ms and 50,000 rays on 328k triangles from 450 to 268 us; the camera set, whose rays mostly end at their first
+// hit, loses 4%.
 struct RayQ {
   float inv[3];
   float offn[3], offf[3];  // entry / exit plane offsets, rounded apart (make_ray32)
@@ -2090,7 +2094,8 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
 
 // ------------------------------------------------------------------------------------------------ leaf checks, fast
 // Closest hits of spheres and cylinders, and of a Scene<float>'s triangles, bit-identical to the exact kernel
-// (k_trace_persistent<Rec, false>), with the FP32 boxes and the visiting order of k_trace_tri. No certificate is needed: when a primitive reports a hit and its leaf has
+// (k_trace_persistent<Rec, false>), with the FP32 boxes and the visiting order of k_trace_tri. No certificate is needed: when
+// a primitive reports a hit and its leaf has
 // not been checked yet, the reference's own slab and pop tests of the leaf's box, in the scene type and at the hit distance as
 // it stands, decide whether the reference tests the leaf at all. That leaf's test decides for the boxes above it too. They hold its box
 // and every operation of the slab test is monotone, so they pass the slab test with it, with an entry distance no larger. As
@@ -2105,7 +2110,8 @@ k_trace_tri(BvhView bvh, RaysView rays, HitsView hits, const BatchJob *__restric
 // the node, pre-test and FP64 branches in almost every iteration for a few lanes each. Lanes with an FP64 test, or with a
 // pre-test, therefore wait until WIDE_MIN_LANES of the wave have one (or no other lane has anything else to do): 50,000
 // spheres 4.19 -> 3.24 ms (8 lanes: 3.36, 24: 3.62), against 4.44 ms for the exact kernel; 10,000 cylinders 4.90 -> 4.59 ms
-// (3.68 with the pre-test against the axis), against 5.45 ms. (k_trace_tri, bound by the data path of the L1, gains nothing from it.) A wave with no rays left to take
+// (3.30 with the pre-test against the axis), against 5.45 ms. (k_trace_tri, bound by the data path of the L1, gains nothing
+// from it.) A wave with no rays left to take
 // doesn't wait: there the longest ray counts. In FP32 the primitives are tested without a pre-test.
 // Primitives without a pre-test tested per step. Triangles in FP32, 1,000,003 incoherent rays on 327,680: 1 per step 0.88,
 // 2: 0.71, 3: 0.68, 4: 0.65 ms.
@@ -2316,7 +2322,8 @@ __device__ __forceinline__ void wide_step(const BvhView &bvh, const RayT<typenam
 template <class Rec, bool FIXED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BRT_WAVES_PER_EU)))
 k_trace_wide(BvhView bvh, RaysViewT<typename Rec::real> rays, HitsViewT<typename Rec::real> hits, uint64_t n,
-             uint32_t flags, uint32_t first, uint32_t is_tri, double S, unsigned long long *group, uint32_t refill, const uint32_t *order, uint32_t ring, uint32_t chunk,
+             uint32_t flags, uint32_t first, uint32_t is_tri, double S, unsigned long long *group, uint32_t refill,
+             const uint32_t *order, uint32_t ring, uint32_t chunk,
              uint32_t fixed) {
   using R = typename Rec::real;
   using RaysV = RaysViewT<R>;
@@ -2913,7 +2920,6 @@ __global__ void k_init_hits(HitsViewT<R> hits, uint64_t n) {
   }
 }
 
-// Blocks of a persistent launch: as many as fit on the device at once, but no more than the rays need.
 // (n, 3) rows to three columns of n. Memory bound: the rows are read once (the second and third loads of a wave hit the
 // lines of the first) and each column written in whole lines.
 constexpr uint32_t ROWS_PER_THREAD = 4;
@@ -2939,6 +2945,7 @@ __global__ void __launch_bounds__(256) k_rows_to_columns(const T *__restrict__ r
   }
 }
 
+// Blocks of a persistent launch: as many as fit on the device at once, but no more than the rays need.
 template <class K>
 hipError_t persistent_blocks(K kernel, uint32_t block, size_t lds, uint64_t n, uint64_t &blocks) {
   int dev = 0, cus = 0, per_cu = 0;
@@ -3028,15 +3035,16 @@ bool fast_triangles(const TraceLaunch &cfg) {
   return cfg.schedule == SCHEDULE_PERSISTENT && !(cfg.flags & FLAG_ANY_HIT);
 }
 // Spheres' and cylinders' (k_trace_wide), in FP64 (split precision has a visiting order of its own): 8,388,608 incoherent
-// rays, 50,000 spheres 3.25 against 4.44 ms, 10,000 cylinders 3.68 against 5.45 ms; a 512x512 camera over 1,024 spheres 0.091
+// rays, 50,000 spheres 3.3 against 4.44 ms, 10,000 cylinders 3.30 against 5.45 ms; a 512x512 camera over 1,024 spheres 0.091
 // against 0.137 ms a call. 100 planes 1.75 against 1.61 ms: they keep the exact kernel. In a Scene<float>, incoherent rays:
 // 1,000,003 on 327,680 triangles 0.63 against 0.83 ms, on 50,000 spheres 0.45 against 0.48, 2,000 on 81,920 triangles 0.089
 // against 0.192; 1920x1080 camera rays on 1.31M triangles 2.05 against 2.62 ms.
 bool fast_wide(const BvhView &bvh, const TraceLaunch &cfg) {
   return bvh.nodesq && bvh.leaf_boxes && cfg.precision == PREC_FP64 && fast_triangles(cfg);
 }
-// Any hit of triangles in split precision on the persistent schedule takes k_trace_any (figures there). In FP64 the first
-// accepted hit of the reference's order counts, which only boxes tested in FP64 give: the exact kernel.
+// Any hit of triangles in split precision on the persistent schedule takes k_trace_any (figures there). In FP64 the hit that
+// counts is the first one accepted in the reference's order, and k_trace_any takes parts of a ray in any order: the exact
+// kernel. (The first certified hit of k_trace_tri would be that hit too; no such launch has been built.)
 bool fast_any(const TraceLaunch &cfg) {
   return cfg.schedule == SCHEDULE_PERSISTENT && cfg.precision != PREC_FP64 && (cfg.flags & FLAG_ANY_HIT);
 }
@@ -3062,7 +3070,8 @@ hipError_t launch_tri(const BvhView &bvh, const RaysView &rays, const HitsView &
   if (!fixed) hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
   const uint64_t need = fixed ? (n + fixed * wpb - 1) / (fixed * wpb) : (n + block - 1) / block;
   if (blocks > need) blocks = need;
-  hipLaunchKernelGGL((fixed ? k_trace_tri<false, false, true> : k_trace_tri<false>), dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits,
+  hipLaunchKernelGGL((fixed ? k_trace_tri<false, false, true> : k_trace_tri<false>), dim3((uint32_t)blocks), dim3(block),
+                     lds, stream, bvh, rays, hits,
                      (const BatchJob *)nullptr, 0u, n, flags, first, sp.scene_extent, grp,
                      cfg.refill ? cfg.refill : TRI_REFILL, cfg.order, ring, cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
   e = hipGetLastError();
@@ -3100,7 +3109,8 @@ hipError_t launch_wide(const BvhView &bvh, const RaysViewT<typename Rec::real> &
   if (!fixed) hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
   const uint64_t need = fixed ? (n + fixed * wpb - 1) / (fixed * wpb) : (n + block - 1) / block;
   if (blocks > need) blocks = need;
-  hipLaunchKernelGGL((fixed ? k_trace_wide<Rec, true> : k_trace_wide<Rec, false>), dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits, n, cfg.flags,
+  hipLaunchKernelGGL((fixed ? k_trace_wide<Rec, true> : k_trace_wide<Rec, false>), dim3((uint32_t)blocks), dim3(block),
+                     lds, stream, bvh, rays, hits, n, cfg.flags,
                      first, is_tri, sp.scene_extent, grp, cfg.refill ? cfg.refill : TRI_REFILL, cfg.order, ring,
                      cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
   e = hipGetLastError();
@@ -3134,7 +3144,8 @@ hipError_t launch_any(const BvhView &bvh, const RaysView &rays, const HitsView &
   if (!fixed) hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, stream, grp);
   const uint64_t need = fixed ? (n + fixed * wpb - 1) / (fixed * wpb) : (n + block - 1) / block;
   if (blocks > need) blocks = need;
-  hipLaunchKernelGGL((fixed ? k_trace_any<true> : k_trace_any<false>), dim3((uint32_t)blocks), dim3(block), lds, stream, bvh, rays, hits, n, cfg.flags,
+  hipLaunchKernelGGL((fixed ? k_trace_any<true> : k_trace_any<false>), dim3((uint32_t)blocks), dim3(block), lds, stream, bvh,
+                     rays, hits, n, cfg.flags,
                      cfg.first ? 1u : 0u, sp.scene_extent, grp, cfg.refill ? cfg.refill : ANY_REFILL, cfg.order, ring,
                      cfg.pool ? cfg.pool : POOL_CHUNK, fixed);
   e = hipGetLastError();

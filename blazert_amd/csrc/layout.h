@@ -27,7 +27,8 @@ enum GeomType : uint32_t { TRIANGLES = 0, SPHERES = 1, PLANES = 2, CYLINDERS = 3
 
 // FP32 4-wide node for split-precision traversal, 128 B: the binary tree collapsed greedily (starting from a node's
 // two children, the internal slot of largest surface area is replaced by its own two children until four slots are
-// filled or all are leaves), so one record holds up to four child boxes, rounded outward (min down, max up). Planes are child-minor: lo[axis][child]. A child reference is a
+// filled or all are leaves), so one record holds up to four child boxes, rounded outward (min down, max up). Planes are child-minor:
+// lo[axis][child]. A child reference is a
 // Node4 index or LEAF_BIT | first primitive with the leaf count beside it; unused slots have cnt = EMPTY_SLOT.
 constexpr uint32_t EMPTY_SLOT = 0xFFFFFFFFu;
 struct alignas(128) Node4 {

@@ -67,7 +67,7 @@ typedef struct brt_build_stats {
   double build_time_s;
   uint32_t num_primitives;
   uint32_t geom_id;
-  uint64_t device_bytes; /* nodes (FP64 + FP32) + primitive records + ids + post-processing data */
+  uint64_t device_bytes; /* nodes (FP64 + FP32), primitive and pre-test records, ids and post-processing data */
   uint32_t built_on_device; /* 1: built by brt_scene_commit_device's GPU builder, 0: by the host builder */
   uint32_t reserved;
 } brt_build_stats;
@@ -108,16 +108,22 @@ typedef struct brt_hits {
 #define BRT_SORT_OCTANT_MORTON 1u
 #define BRT_SORT_MORTON 2u
 
+/* The defaults depend on the kernel a launch takes. Closest hits of triangles, of FP64 spheres and cylinders and of every
+ * Scene<float> type but planes, and any hit of split-precision triangles, take kernels over 4-wide FP32 boxes on
+ * BRT_SCHEDULE_PERSISTENT; everything else takes the general kernels, as do trees with a leaf of more than 255
+ * primitives, boxes that are NaN or inverted, or coordinates of 1e30 and more. */
 typedef struct brt_launch {
   uint32_t precision;  /* BRT_PRECISION_* */
   uint32_t flags;      /* BRT_FLAG_* */
-  uint32_t block_size; /* threads per block: 64, 128, 192 or 256; 0 = library default (256; 128 for FP64 spheres) */
+  uint32_t block_size; /* threads per block: 64, 128, 192 or 256; 0 = library default (256; 128 for FP64
+                          spheres on the general kernels) */
   uint32_t schedule;   /* BRT_SCHEDULE_* */
   uint32_t refill;     /* persistent: refill a wave once this many of its 64 lanes are idle; 0 = default (32 for
-                          any-hit FP64 triangles and FP32 triangles, 16 otherwise) */
+                          any hit of triangles and for FP64 and FP32 triangles on the general kernels, 16
+                          otherwise) */
   uint32_t sort;       /* BRT_SORT_*: trace rays in a sorted order (results are written in input order) */
-  uint32_t stack_ring; /* traversal-stack entries per lane kept in LDS: 4, 8 or 16; 0 = 16 for FP64 and
-                          split-precision triangles (8 for any-hit FP64), 8 otherwise.
+  uint32_t stack_ring; /* traversal-stack entries per lane kept in LDS: 4, 8 or 16; 0 = 16 on the kernels
+                          over 4-wide boxes and for split-precision triangles, 8 otherwise.
                           Deeper entries spill to private memory; a deeper ring spills less but takes more LDS */
   uint32_t pool_size;  /* persistent: ray indices a wave claims at once: 32, 64 or 128; 0 = 64. Smaller claims
                           balance image-order (coherent) rays better, larger ones cost fewer atomics on the launch's
@@ -140,7 +146,9 @@ int brt_device_count(void);
 
 /* BlazertScene<T>() with build_options (blazert/scene.h:42,73); opts may be NULL for the defaults. */
 int brt_scene_create(const brt_build_options *opts, brt_scene **out);
-/* Releases host and device memory of the scene. */
+/* Releases host and device memory of the scene. Device memory of scenes and device builds comes from a pool per GPU: up to
+ * 2 GiB of what they give back (a device commit's workspace included) stays allocated for the next scene or build, out of
+ * reach of other allocators in the process, until the last scene on that GPU is destroyed. */
 int brt_scene_destroy(brt_scene *scene);
 
 /* add_mesh (blazert/scene.h:227-240): vertices xyz (3*nv doubles), faces (3*nf uint32).
@@ -222,8 +230,9 @@ int brt_rows_to_columns(const void *rows, uint32_t elem_bytes, uint64_t n, void 
 
 /* Batched intersect1 (blazert/scene.h:161-211) for n rays resident on the device, enqueued on `stream`
  * (a hipStream_t, NULL = default stream). launch may be NULL (FP64, no flags, persistent). Asynchronous.
- * The launches keep a few device counters per scene and stream, allocated on the first launch on that stream
- * (do not graph-capture that first launch); launches on one stream run in order, so any number may be in flight.
+ * The launches keep 256 KiB of device counters per scene and stream, allocated on the first launch on that stream
+ * (do not graph-capture that first launch); launches on one stream run in order, so any number may be in flight, from
+ * any threads.
  * With BRT_PRECISION_FP32_TRAV_FP64_HIT, rays whose reference slab test can produce NaN terms (a zero, non-finite
  * or reciprocal-overflowing direction component, a non-finite origin, a NaN tmin) are traced by the FP64 path. */
 int brt_intersect(const brt_scene *scene, const brt_rays *rays, const brt_hits *hits, uint64_t n,
@@ -232,7 +241,7 @@ int brt_intersect(const brt_scene *scene, const brt_rays *rays, const brt_hits *
 /* brt_intersect that allocates nothing. No counterpart in the reference: it is for callers that cannot allocate
  * device memory (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc). Same arguments and
  * hits as brt_intersect, bit for bit. Its launch counters and its ray-sort workspace live in one static device
- * array of the library (24 MiB per GPU that loads the library, held until the process ends) instead of per-stream
+ * array of the library (24.25 MiB per GPU that loads the library, held until the process ends) instead of per-stream
  * and per-scene allocations. Limits, each refused with an error before any device work: the scene must already be
  * on the current device (BRT_ERR_STATE; brt_scene_upload, brt_scene_commit_device or a brt_intersect put it
  * there), and a sorted launch takes at most 2^20 rays (BRT_ERR_UNSUPPORTED); unsorted launches take any n. All
